@@ -24,24 +24,24 @@ struct Vol {          // spatial shape (per batch item)
 // out_f32: y is FP32 (no bias, no ReLU: used for the input gradient).
 hipError_t conv3d_fwd(const Act &x, const uint16_t *W, const float *bias, Act y, Vol v,
                       bool relu, bool out_f32, hipStream_t st);
-// dW[tap][co][ci] += sum_p dy[p][co] x[p + tap][ci] (FP32 accumulator, padded
-// cin like the weights); db[co] += sum_p dy[p][co].
+// dW[tap][co][ci] = sum_p dy[p][co] x[p + tap][ci] (FP32, [27][cout][cin]);
+// db[co] = sum_p dy[p][co].  scratch holds kGradScratch floats.
+constexpr long kGradScratch = 8L << 20;
 hipError_t conv3d_wgrad(const Act &x, const Act &dy, float *dW, float *db, Vol v,
-                        hipStream_t st);
+                        float *scratch, hipStream_t st);
 // Weights of the transposed convolution: Wt[tap][ci][co] = W[26-tap][co][ci]
 // (cin/cout swapped, pads to 32 on the new input channels).
 hipError_t conv3d_flip_weights(const uint16_t *W, uint16_t *Wt, int cin, int cout,
                                hipStream_t st);
 // FP32 master weights [27][cout][cin] -> BF16 padded [27][cout][cin_pad].
 hipError_t pack_weights(const float *Wf, uint16_t *W, int cin, int cout, hipStream_t st);
-// Padded FP32 gradient [27][cout][cin_pad] -> [27][cout][cin].
-hipError_t unpack_grad(const float *gp, float *g, int cin, int cout, hipStream_t st);
 
 // First layer: 1 FP32 input channel -> cout BF16 channels, ReLU.
 hipError_t conv3d_first_fwd(const float *x, const float *W, const float *b, Act y, Vol v,
                             hipStream_t st);
+// Its weight and bias gradient (16 channels; overwrites dW [27][16] and db).
 hipError_t conv3d_first_wgrad(const float *x, const Act &dy, float *dW, float *db, Vol v,
-                              hipStream_t st);
+                              float *scratch, hipStream_t st);
 // Head: 1x1x1 conv cin -> 1 FP32 plus the residual input: out = x0 + W.y + b.
 hipError_t head_fwd(const Act &y, const float *W, const float *b, const float *x0, float *out,
                     Vol v, hipStream_t st);

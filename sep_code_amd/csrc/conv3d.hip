@@ -8,9 +8,11 @@
 // B[8(l/16)+i][l%16] (i < 8; K = 16: 4(l/16)+i, i < 4), and receives
 // D[4(l/16)+j][l%16] (j < 4) (checked on the device against a host product).  In channels-last layout
 // the 8 K values of a lane are 8 consecutive channels of one position: one
-// 16-byte load.  The weight gradient is a GEMM over positions (K) staged
-// through LDS transposed so both operands are again 16-byte lane loads.
+// 16-byte load.  The weight gradient is a GEMM over positions (K) whose
+// operands are read from LDS with the transposing read (k_wgrad).
 #include "conv3d.h"
+
+#include <algorithm>
 
 namespace brtm {
 namespace {
@@ -188,89 +190,178 @@ k_conv_fwd(const uint16_t *__restrict__ x, int xcs, const uint16_t *__restrict__
 }
 
 // ------------------------------------------------------------- weight GEMM
-template <int CIN_P, int COUT>
-__global__ void __launch_bounds__(256)
-k_conv_wgrad(const uint16_t *__restrict__ x, int xcs, int cin, const uint16_t *__restrict__ dy,
-             int dycs, float *dW, int N, int D, int H, int Wd, long chunk) {
-  constexpr int MT = COUT / 16, NTC = CIN_P / 16, T = MT * NTC, TPW = (T + 3) / 4;
-  constexpr int LP = 40;  // 32 positions + pad, rows stay 16-byte aligned
-  __shared__ __attribute__((aligned(16))) uint16_t As[COUT][LP];
-  __shared__ __attribute__((aligned(16))) uint16_t Bs[CIN_P][LP];
-  const int tap = blockIdx.y;
-  const int dz = tap / 9 - 1, dyy = (tap / 3) % 3 - 1, dx = tap % 3 - 1;
-  const long npos = (long)N * D * H * Wd;
-  const long p0 = (long)blockIdx.x * chunk;
-  const long p1 = p0 + chunk < npos ? p0 + chunk : npos;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int col = lane & 15, kq = lane >> 4;
-  f32x4 acc[TPW];
-#pragma unroll
-  for (int i = 0; i < TPW; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (long p = p0; p < p1; p += 32) {
-    for (int i = tid; i < 32 * COUT; i += 256) {
-      const int pp = i / COUT, co = i % COUT;
-      const long q = p + pp;
-      As[co][pp] = q < p1 ? dy[q * dycs + co] : (uint16_t)0;
-    }
-    for (int i = tid; i < 32 * CIN_P; i += 256) {
-      const int pp = i / CIN_P, ci = i % CIN_P;
-      const long q = p + pp;
-      uint16_t v = 0;
-      if (q < p1 && ci < cin) {
-        const int xx = (int)(q % Wd);
-        long r = q / Wd;
-        const int yv = (int)(r % H);
-        r /= H;
-        const int zv = (int)(r % D);
-        const int z2 = zv + dz, y2 = yv + dyy, x2 = xx + dx;
-        if (z2 >= 0 && z2 < D && y2 >= 0 && y2 < H && x2 >= 0 && x2 < Wd)
-          v = x[(q + ((long)dz * H + dyy) * Wd + dx) * xcs + ci];
-      }
-      Bs[ci][pp] = v;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < TPW; ++k) {
-      const int t = wave + 4 * k;
-      if (t < T) {
-        const int mt = t / NTC, nt = t % NTC;
-        const bf16x8 a = ld8(&As[mt * 16 + col][8 * kq]);
-        const bf16x8 b = ld8(&Bs[nt * 16 + col][8 * kq]);
-        acc[k] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc[k], 0, 0, 0);
-      }
-    }
-    __syncthreads();
+// dW[tap][co][ci] = sum_p dy[p][co] x[p + tap][ci]: for each tap a GEMM whose
+// K runs over positions, so both operands are channels-last tiles read with
+// K along the slow index.  ds_read_b64_tr_b16 reads them transposed: a
+// 16-lane group takes a 4-position x 16-channel block and lane j gets channel
+// j's four positions, at any position offset, so a tap's x shift costs
+// nothing.
+//
+// A workgroup stages R rows of dy (SEG positions) and the R + 2 input rows
+// around them of plane z + dz - 1 (SEG + 2 positions) once and uses them for
+// nine taps: wave dx (three waves) owns the taps (dz, *, dx), a fragment of
+// an input row serves the three dy taps, whose dy rows wait in registers.
+// The workgroup strides over the units of the volume with its sums in
+// registers and writes one partial sum per element; k_grad_sum adds the
+// partials in order (no atomics: the gradient is the same in every run).  The
+// bias gradient is one more product, dy by ones, on the wave of the centre
+// tap.  Before this a workgroup per tap re-read both tensors 27 times and
+// transposed them with 2-byte LDS stores: 2.00 ms for 16->16 and 3.79 ms for
+// 48->16 at 4 x 64^3, now 0.055 and 0.22 ms (two workgroups of 80 KB of LDS
+// per CU, the stage and the products in turn).
+//
+// SEG positions per K run: 64 on the full-resolution level, 32 and 16 on the
+// coarser ones (their row lengths are multiples of these for every patch).
+// LDS rows are an odd multiple of 32 bytes, which spreads the eight rows two
+// lane groups read together over all banks.
+__host__ __device__ constexpr int lds_row(int c) { return (c / 16) % 2 ? c : c + 16; }
+
+typedef __attribute__((address_space(3))) i16x4 lds_i16x4;
+__device__ __forceinline__ i16x4 ld_tr(const uint16_t *p) {
+  return __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4 *)p);
+}
+
+template <int K32>  // 1: 32 positions per product, 0: 16
+struct GradFrag {
+  i16x4 v[K32 + 1];
+  // positions 4g .. 4g+3 (and 16 + 4g ..) of the row at p, this lane's channel
+  __device__ __forceinline__ void load(const uint16_t *p, int stride) {
+    v[0] = ld_tr(p);
+    if constexpr (K32) v[1] = ld_tr(p + 16 * stride);
   }
+  __device__ __forceinline__ void ones() {
+    for (int h = 0; h < K32 + 1; ++h) v[h] = i16x4{0x3f80, 0x3f80, 0x3f80, 0x3f80};
+  }
+  __device__ __forceinline__ static f32x4 mul(const GradFrag &a, const GradFrag &b, f32x4 c) {
+    if constexpr (K32)
+      return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a.v),
+                                                     __builtin_bit_cast(bf16x8, b.v), c, 0, 0, 0);
+    else
+      return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a.v[0], b.v[0], c, 0, 0, 0);
+  }
+};
+
+template <int CIN, int COUT, int SEG, int R>
+__global__ void __launch_bounds__(192)
+k_wgrad(const uint16_t *__restrict__ x, int xcs, const uint16_t *__restrict__ dy, int dycs,
+        float *__restrict__ part, int D, int H, int Wd, long units) {
+  constexpr int MT = COUT / 16, NT = CIN / 16, KS = SEG >= 32 ? SEG / 32 : 1;
+  constexpr int XS = lds_row(CIN), DS = lds_row(COUT), XP = SEG + 2;
+  typedef GradFrag<(SEG >= 32)> Frag;
+  __shared__ __attribute__((aligned(16))) uint16_t Xs[R + 2][XP][XS];
+  __shared__ __attribute__((aligned(16))) uint16_t Ds[R][SEG][DS];
+  const int tid = threadIdx.x, lane = tid & 63, dx = tid >> 6, dz = blockIdx.y;
+  const int g = lane >> 4, j = lane & 15;
+  const int xo = (4 * g + (j >> 2) + dx) * XS + 4 * (j & 3);
+  const int ao = (4 * g + (j >> 2)) * DS + 4 * (j & 3);
+  const bool bias = dz == 1 && dx == 1;
+  f32x4 acc[3][MT][NT], accb[MT];
 #pragma unroll
-  for (int k = 0; k < TPW; ++k) {
-    const int t = wave + 4 * k;
-    if (t < T) {
-      const int mt = t / NTC, nt = t % NTC;
+  for (int m = 0; m < MT; ++m) {
+    accb[m] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int co = mt * 16 + 4 * kq + j, ci = nt * 16 + col;
-        if (ci < cin) atomicAdd(dW + ((long)tap * COUT + co) * CIN_P + ci, acc[k][j]);
-      }
+    for (int t = 0; t < 3; ++t)
+#pragma unroll
+      for (int n = 0; n < NT; ++n) acc[t][m][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  Frag one;
+  one.ones();
+  const int nseg = Wd / SEG, nyc = H / R;
+  for (long u = blockIdx.x; u < units; u += gridDim.x) {
+    const int xs = (int)(u % nseg) * SEG;
+    long r = u / nseg;
+    const int y0 = (int)(r % nyc) * R;
+    r /= nyc;
+    const int z = (int)(r % D), z2 = z + dz - 1;
+    const long nn = r / D;
+    if (z2 < 0 || z2 >= D) continue;  // the whole workgroup: a zero plane
+    __syncthreads();                  // the previous unit has been read
+    const uint16_t *xp = x + (nn * D + z2) * H * Wd * xcs;
+    constexpr int XC = CIN / 8, NX = (R + 2) * XP * XC;
+#pragma unroll 4
+    for (int i = tid; i < NX; i += 192) {
+      const int c = i % XC, p = (i / XC) % XP, rr = i / (XC * XP);
+      const int yy = y0 + rr - 1, xx = xs + p - 1;
+      uint4 v = make_uint4(0, 0, 0, 0);
+      if (yy >= 0 && yy < H && xx >= 0 && xx < Wd)
+        v = *reinterpret_cast<const uint4 *>(xp + ((long)yy * Wd + xx) * xcs + 8 * c);
+      *reinterpret_cast<uint4 *>(&Xs[rr][p][8 * c]) = v;
     }
+    const uint16_t *dp = dy + (((nn * D + z) * H + y0) * Wd + xs) * dycs;
+    constexpr int DC = COUT / 8, ND = R * SEG * DC;
+#pragma unroll 4
+    for (int i = tid; i < ND; i += 192) {
+      const int c = i % DC, p = (i / DC) % SEG, rr = i / (DC * SEG);
+      *reinterpret_cast<uint4 *>(&Ds[rr][p][8 * c]) =
+          *reinterpret_cast<const uint4 *>(dp + ((long)rr * Wd + p) * dycs + 8 * c);
+    }
+    __syncthreads();
+    Frag a[3][KS][MT];
+#pragma unroll
+    for (int xr = 0; xr < R + 2; ++xr) {
+      if (xr < R) {
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+          for (int m = 0; m < MT; ++m) {
+            a[xr % 3][ks][m].load(&Ds[xr][ks * 32][16 * m] + ao, DS);
+            if (bias) accb[m] = Frag::mul(a[xr % 3][ks][m], one, accb[m]);
+          }
+      }
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+        for (int n = 0; n < NT; ++n) {
+          Frag b;
+          b.load(&Xs[xr][ks * 32][16 * n] + xo, XS);
+#pragma unroll
+          for (int t = 0; t < 3; ++t) {
+            if (xr - t < 0 || xr - t >= R) continue;
+#pragma unroll
+            for (int m = 0; m < MT; ++m)
+              acc[t][m][n] = Frag::mul(a[(xr - t + 3) % 3][ks][m], b, acc[t][m][n]);
+          }
+        }
+    }
+  }
+  constexpr int NW = 27 * CIN * COUT;
+  float *o = part + (long)blockIdx.x * (NW + COUT);
+#pragma unroll
+  for (int t = 0; t < 3; ++t)
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+      for (int n = 0; n < NT; ++n)
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+          o[((dz * 9 + t * 3 + dx) * COUT + 16 * m + 4 * g + k) * CIN + 16 * n + j] =
+              acc[t][m][n][k];
+  if (bias && j == 0) {
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+      for (int k = 0; k < 4; ++k) o[NW + 16 * m + 4 * g + k] = accb[m][k];
   }
 }
 
-__global__ void k_bias_grad(const uint16_t *__restrict__ dy, int dycs, int c, long npos,
-                            float *db) {
-  // thread t accumulates channel t % c over positions t / c, stride blockDim/c
-  __shared__ float red[256];
-  const int per = 256 / c;  // positions per block pass (c divides 256)
-  const int ch = threadIdx.x % c, sub = threadIdx.x / c;
+// out[e] = sum of the S partials part[s][e] (e < nw into dW, the rest into
+// db): 64 elements by 4 runs of s per workgroup.
+__global__ void __launch_bounds__(256)
+k_grad_sum(const float *__restrict__ part, int S, int nw, int nb, float *dW, float *db) {
+  __shared__ float red[4][64];
+  const int q = threadIdx.x >> 6, l = threadIdx.x & 63;
+  const int e = blockIdx.x * 64 + l, n = nw + nb;
   float s = 0.f;
-  if (sub < per)
-    for (long p = (long)blockIdx.x * per + sub; p < npos; p += (long)gridDim.x * per)
-      s += bf2f(dy[p * dycs + ch]);
-  red[threadIdx.x] = s;
+  if (e < n) {
+#pragma unroll 8
+    for (int k = q; k < S; k += 4) s += part[(long)k * n + e];
+  }
+  red[q][l] = s;
   __syncthreads();
-  if (threadIdx.x < c) {
-    float t = 0.f;
-    for (int k = 0; k < per; ++k) t += red[k * c + threadIdx.x];
-    atomicAdd(db + threadIdx.x, t);
+  if (q == 0 && e < n) {
+    s = (red[0][l] + red[1][l]) + (red[2][l] + red[3][l]);
+    if (e < nw) dW[e] = s;
+    else db[e - nw] = s;
   }
 }
 
@@ -295,17 +386,6 @@ __global__ void k_pack(const float *Wf, uint16_t *W, int cin, int cout) {
     const int ci = (int)(i % cin_p);
     const long r = i / cin_p;  // tap*cout + co
     W[i] = ci < cin ? f2bf(Wf[r * cin + ci]) : (uint16_t)0;
-  }
-}
-
-__global__ void k_unpack(const float *gp, float *g, int cin, int cout) {
-  const int cin_p = cpad(cin);
-  const long n = 27L * cout * cin;
-  for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (long)gridDim.x * blockDim.x) {
-    const int ci = (int)(i % cin);
-    const long r = i / cin;
-    g[i] = gp[r * cin_p + ci];
   }
 }
 
@@ -415,40 +495,75 @@ __global__ void k_first_fwd4(const float *__restrict__ x, const float *__restric
   }
 }
 
-__global__ void k_first_wgrad(const float *__restrict__ x, const uint16_t *__restrict__ dy,
-                              int dycs, int cout, float *dW, float *db, int N, int D, int H,
-                              int Wd) {
-  // blockIdx.y = tap (27) or 27 for the bias; thread accumulates all channels
-  const int tap = blockIdx.y;
-  const long npos = (long)N * D * H * Wd;
-  float acc[64];
-  for (int c = 0; c < cout; ++c) acc[c] = 0.f;
-  for (long p = (long)blockIdx.x * blockDim.x + threadIdx.x; p < npos;
-       p += (long)gridDim.x * blockDim.x) {
-    float xv = 1.f;
-    if (tap < 27) {
-      const int xx = (int)(p % Wd);
-      long r = p / Wd;
-      const int yv = (int)(r % H);
-      r /= H;
-      const int zv = (int)(r % D);
-      const int z2 = zv + tap / 9 - 1, y2 = yv + (tap / 3) % 3 - 1, x2 = xx + tap % 3 - 1;
-      const bool ok = z2 >= 0 && z2 < D && y2 >= 0 && y2 < H && x2 >= 0 && x2 < Wd;
-      xv = ok ? x[p + ((long)(tap / 9 - 1) * H + (tap / 3) % 3 - 1) * Wd + tap % 3 - 1] : 0.f;
-    }
-    for (int c = 0; c < cout; ++c) acc[c] = fmaf(bf2f(dy[p * dycs + c]), xv, acc[c]);
-  }
-  __shared__ float red[256];
-  for (int c = 0; c < cout; ++c) {
-    red[threadIdx.x] = acc[c];
+// First layer's weight and bias gradient: dW[tap][co] = sum_p x[p + tap]
+// dy[p][co] on the FP32 matrix unit (v_mfma_f32_16x16x4_f32, K = 4 positions:
+// the input stays FP32): 16 channels by 27 taps, the 28th column is ones and
+// gives the bias.  Lane l holds A[l%16][l/16] and B[l/16][l%16].  A workgroup
+// stages 8 rows of 64 positions and the input around them, keeps its sums in
+// registers over its units and writes one partial (k_grad_sum adds them).
+// One tap per workgroup and 64 accumulators per thread took 1.06 ms at 4 x
+// 64^3, this 0.036 ms.
+__global__ void __launch_bounds__(256)
+k_first_wgrad(const float *__restrict__ x, const uint16_t *__restrict__ dy, int dycs,
+              float *__restrict__ part, int D, int H, int Wd, long units) {
+  constexpr int R = 8, SEG = 64, XP = 68;
+  __shared__ float Xs[3][R + 2][XP];
+  __shared__ __attribute__((aligned(16))) uint16_t Ds[R][SEG][16];
+  __shared__ float red[4][28 * 16];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int g = lane >> 4, j = lane & 15;
+  const int t1 = 16 + j;
+  // offsets of taps j and 16 + j from the position's cell in Xs
+  auto off = [](int t) { return ((t / 9) * (R + 2) + (t / 3) % 3) * XP + t % 3; };
+  const int o0 = off(j), o1 = t1 < 27 ? off(t1) : 0;
+  f32x4 acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = {0.f, 0.f, 0.f, 0.f};
+  const int nseg = Wd / SEG, nyc = H / R;
+  for (long u = blockIdx.x; u < units; u += gridDim.x) {
+    const int xs = (int)(u % nseg) * SEG;
+    long r = u / nseg;
+    const int y0 = (int)(r % nyc) * R;
+    r /= nyc;
+    const int z = (int)(r % D);
+    const long nn = r / D;
     __syncthreads();
-    for (int o = blockDim.x / 2; o > 0; o >>= 1) {
-      if ((int)threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
-      __syncthreads();
+#pragma unroll 4
+    for (int i = tid; i < 3 * (R + 2) * (SEG + 2); i += 256) {
+      const int p = i % (SEG + 2), rr = (i / (SEG + 2)) % (R + 2), pz = i / ((SEG + 2) * (R + 2));
+      const int zz = z + pz - 1, yy = y0 + rr - 1, xx = xs + p - 1;
+      const bool ok = zz >= 0 && zz < D && yy >= 0 && yy < H && xx >= 0 && xx < Wd;
+      Xs[pz][rr][p] = ok ? x[((nn * D + zz) * H + yy) * Wd + xx] : 0.f;
     }
-    if (threadIdx.x == 0) atomicAdd(tap < 27 ? dW + tap * cout + c : db + c, red[0]);
+    const uint16_t *dp = dy + (((nn * D + z) * H + y0) * Wd + xs) * dycs;
+#pragma unroll
+    for (int i = tid; i < R * SEG * 2; i += 256) {
+      const int c = i & 1, p = (i >> 1) % SEG, rr = i / (2 * SEG);
+      *reinterpret_cast<uint4 *>(&Ds[rr][p][8 * c]) =
+          *reinterpret_cast<const uint4 *>(dp + ((long)rr * Wd + p) * dycs + 8 * c);
+    }
     __syncthreads();
+#pragma unroll
+    for (int h = 0; h < R / 4; ++h) {
+      const int row = wave * (R / 4) + h;
+      const float *xr = &Xs[0][row][0] + g;
+#pragma unroll 4
+      for (int p = 0; p < SEG; p += 4) {
+        const float a = bf2f(Ds[row][p + g][j]);
+        const float b0 = xr[p + o0];
+        float b1 = xr[p + o1];
+        b1 = t1 < 27 ? b1 : (t1 == 27 ? 1.f : 0.f);
+        acc0 = __builtin_amdgcn_mfma_f32_16x16x4f32(a, b0, acc0, 0, 0, 0);
+        acc1 = __builtin_amdgcn_mfma_f32_16x16x4f32(a, b1, acc1, 0, 0, 0);
+      }
+    }
   }
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    red[wave][j * 16 + 4 * g + k] = acc0[k];
+    if (t1 < 28) red[wave][t1 * 16 + 4 * g + k] = acc1[k];
+  }
+  __syncthreads();
+  for (int e = tid; e < 28 * 16; e += 256)
+    part[(long)blockIdx.x * (28 * 16) + e] = (red[0][e] + red[1][e]) + (red[2][e] + red[3][e]);
 }
 
 // -------------------------------------------------------------------- head
@@ -677,23 +792,29 @@ hipError_t fwd_t(const Act &x, const uint16_t *W, const float *b, Act y, Vol v, 
   return fwd_y<CIN, COUT, 1>(x, W, b, y, v, relu, f32, st);
 }
 
-template <int CIN_P, int COUT>
-hipError_t wgrad_t(const Act &x, const Act &dy, float *dW, Vol v, hipStream_t st) {
-  const long npos = (long)v.n * v.spatial();
-  const long chunk = 2048;
-  const dim3 grid((unsigned)((npos + chunk - 1) / chunk), 27);
-  k_conv_wgrad<CIN_P, COUT><<<grid, 256, 0, st>>>((const uint16_t *)x.p, x.cs, x.c,
-                                                  (const uint16_t *)dy.p, dy.cs, dW, v.n, v.d,
-                                                  v.h, v.w, chunk);
+// Workgroups of a weight gradient: up to 256 (times the three dz), fewer
+// where the volume has fewer units or the partials would pass kGradScratch.
+template <int CIN, int COUT, int SEG, int R>
+hipError_t wgrad_t(const Act &x, const Act &dy, float *dW, float *db, Vol v, float *scratch,
+                   hipStream_t st) {
+  constexpr int NW = 27 * CIN * COUT;
+  if (v.w % SEG || v.h % R) return hipErrorInvalidValue;
+  const long units = (long)v.n * v.d * (v.h / R) * (v.w / SEG);
+  const int S = (int)std::min({units, 256L, kGradScratch / (NW + COUT)});
+  k_wgrad<CIN, COUT, SEG, R><<<dim3(S, 3), 192, 0, st>>>(
+      (const uint16_t *)x.p, x.cs, (const uint16_t *)dy.p, dy.cs, scratch, v.d, v.h, v.w, units);
+  k_grad_sum<<<(NW + COUT + 63) / 64, 256, 0, st>>>(scratch, S, NW, COUT, dW, db);
   return hipGetLastError();
 }
 
 }  // namespace
 
-// The (cin_pad, cout) pairs of the network's weight gradients (for the
-// forward convolutions and their transposes).
-#define BRTM_CONV_PAIRS(X) \
-  X(32, 16) X(32, 32) X(32, 64) X(64, 64) X(96, 32) X(64, 16) X(64, 32) X(32, 96) X(32, 48)
+// The weight gradients of the network: (cin, cout, positions per K run, rows
+// per unit).  The level fixes the run; 96 input channels take four rows so
+// that two workgroups fit a CU's LDS.
+#define BRTM_WGRAD_SHAPES(X)                                                     \
+  X(16, 16, 64, 8) X(48, 16, 64, 8) X(16, 32, 32, 8) X(32, 32, 32, 8) X(96, 32, 32, 4) \
+  X(32, 64, 16, 8) X(64, 64, 16, 8)
 
 // The (cin, cout) pairs of the forward convolutions (16->16, 16->32, 32->32,
 // 32->64, 64->64, 96->32, 48->16) and of the transposed ones (input
@@ -713,18 +834,13 @@ hipError_t conv3d_fwd(const Act &x, const uint16_t *W, const float *bias, Act y,
 }
 
 hipError_t conv3d_wgrad(const Act &x, const Act &dy, float *dW, float *db, Vol v,
-                        hipStream_t st) {
-  if (x.c % 8 || x.cs % 8 || dy.c % 16 || 256 % dy.c) return hipErrorInvalidValue;
-  const int cp = cpad(x.c);
-  hipError_t e = hipErrorInvalidValue;
-#define X(CP, CO) \
-  if (cp == CP && dy.c == CO) e = wgrad_t<CP, CO>(x, dy, dW, v, st);
-  BRTM_CONV_PAIRS(X)
+                        float *scratch, hipStream_t st) {
+  if (x.cs % 8 || dy.cs % 8) return hipErrorInvalidValue;
+#define X(CI, CO, SEG, R) \
+  if (x.c == CI && dy.c == CO) return wgrad_t<CI, CO, SEG, R>(x, dy, dW, db, v, scratch, st);
+  BRTM_WGRAD_SHAPES(X)
 #undef X
-  if (e != hipSuccess) return e;
-  const long npos = (long)v.n * v.spatial();
-  k_bias_grad<<<512, 256, 0, st>>>((const uint16_t *)dy.p, dy.cs, dy.c, npos, db);
-  return hipGetLastError();
+  return hipErrorInvalidValue;
 }
 
 hipError_t conv3d_flip_weights(const uint16_t *W, uint16_t *Wt, int cin, int cout,
@@ -735,11 +851,6 @@ hipError_t conv3d_flip_weights(const uint16_t *W, uint16_t *Wt, int cin, int cou
 
 hipError_t pack_weights(const float *Wf, uint16_t *W, int cin, int cout, hipStream_t st) {
   k_pack<<<grid1(27L * cout * cpad(cin)), 256, 0, st>>>(Wf, W, cin, cout);
-  return hipGetLastError();
-}
-
-hipError_t unpack_grad(const float *gp, float *g, int cin, int cout, hipStream_t st) {
-  k_unpack<<<grid1(27L * cout * cin), 256, 0, st>>>(gp, g, cin, cout);
   return hipGetLastError();
 }
 
@@ -758,10 +869,13 @@ hipError_t conv3d_first_fwd(const float *x, const float *W, const float *b, Act 
 }
 
 hipError_t conv3d_first_wgrad(const float *x, const Act &dy, float *dW, float *db, Vol v,
-                              hipStream_t st) {
-  if (dy.c > 64) return hipErrorInvalidValue;
-  k_first_wgrad<<<dim3(256, 28), 256, 0, st>>>(x, (const uint16_t *)dy.p, dy.cs, dy.c, dW, db,
-                                               v.n, v.d, v.h, v.w);
+                              float *scratch, hipStream_t st) {
+  if (dy.c != 16 || dy.cs % 8 || v.w % 64 || v.h % 8) return hipErrorInvalidValue;
+  const long units = (long)v.n * v.d * (v.h / 8) * (v.w / 64);
+  const int S = (int)std::min(units, 512L);
+  k_first_wgrad<<<S, 256, 0, st>>>(x, (const uint16_t *)dy.p, dy.cs, scratch, v.d, v.h, v.w,
+                                   units);
+  k_grad_sum<<<7, 256, 0, st>>>(scratch, S, 27 * 16, 16, dW, db);
   return hipGetLastError();
 }
 

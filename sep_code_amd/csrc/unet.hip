@@ -128,7 +128,8 @@ struct brtm_unet {
   long nparams = 0;
   long w0 = 0, b0 = 0, wl[9] = {}, bl[9] = {}, wh = 0, bh = 0;
   DevBuf params, grads, am, av;
-  DevBuf wbf[9], wtf[9], gpad[9];
+  DevBuf wbf[9], wtf[9];
+  DevBuf gscratch;  // partial weight gradients
   DevBuf e1a, cat1, p1, e2a, cat2, p2, b1, b2, d2a, d2b, d1a, d1b, out;
   DevBuf g_out, dy_d1b, dy_d1a, dy_cat1, dy_d2b, dy_d2a, dy_cat2, dy_b2, dy_b1, dy_p2, dy_e2a,
       dy_p1, dy_e1a, dpre;
@@ -198,7 +199,7 @@ int forward(brtm_unet *u, const float *x, int nb) {
 }
 
 // Backward of one MFMA layer l: given the FP32 gradient of its (ReLU) output
-// gy (stride gcs) and its output activation y, accumulate its parameter
+// gy (stride gcs) and its output activation y, write its parameter
 // gradients from input x and (if gx) write the input gradient gx (FP32,
 // all cin channels, stride cin).
 int layer_bwd(brtm_unet *u, int l, const float *gy, int gcs, const Act &y, const Act &x, float *gx,
@@ -207,7 +208,8 @@ int layer_bwd(brtm_unet *u, int l, const float *gy, int gcs, const Act &y, const
   const int cin = kConv[l].cin, cout = kConv[l].cout;
   Act dp = act(u->dpre, cout, cout);
   BRTM_HIP(relu_bwd(gy, gcs, y, dp, v, st));
-  BRTM_HIP(conv3d_wgrad(x, dp, u->gpad[l].as<float>(), u->grads.as<float>() + u->bl[l], v, st));
+  float *G = u->grads.as<float>();
+  BRTM_HIP(conv3d_wgrad(x, dp, G + u->wl[l], G + u->bl[l], v, u->gscratch.as<float>(), st));
   if (gx) {
     Act out{gx, cin, cin};
     BRTM_HIP(conv3d_fwd(dp, u->wtf[l].as<uint16_t>(), nullptr, out, v, false, true, st));
@@ -223,9 +225,8 @@ int backward(brtm_unet *u, const float *x, int nb) {
              n3 = (long)nb * v3.spatial();
   float *G = u->grads.as<float>();
   const float *pr = u->prm();
-  BRTM_HIP(hipMemsetAsync(G, 0, sizeof(float) * u->nparams, st));
-  for (int l = 0; l < 9; ++l)
-    BRTM_HIP(hipMemsetAsync(u->gpad[l].ptr, 0, u->gpad[l].bytes, st));
+  // the head's gradient accumulates; every other one is written whole
+  BRTM_HIP(hipMemsetAsync(G + u->wh, 0, sizeof(float) * (C1 + 1), st));
   BRTM_HIP(hipMemsetAsync(u->dy_d2b.ptr, 0, sizeof(float) * n2 * C2, st));
   BRTM_HIP(hipMemsetAsync(u->dy_b2.ptr, 0, sizeof(float) * n3 * C3, st));
   // head
@@ -260,9 +261,7 @@ int backward(brtm_unet *u, const float *x, int nb) {
   // first layer: ReLU backward then weight gradient (no input gradient)
   Act dp = act(u->dpre, C1, C1);
   BRTM_HIP(relu_bwd(u->dy_e1a.as<float>(), C1, act(u->e1a, C1, C1), dp, v1, st));
-  BRTM_HIP(conv3d_first_wgrad(x, dp, G + u->w0, G + u->b0, v1, st));
-  for (int l = 0; l < 9; ++l)
-    BRTM_HIP(unpack_grad(u->gpad[l].as<float>(), G + u->wl[l], kConv[l].cin, kConv[l].cout, st));
+  BRTM_HIP(conv3d_first_wgrad(x, dp, G + u->w0, G + u->b0, v1, u->gscratch.as<float>(), st));
   (void)n1;
   return BRTM_OK;
 }
@@ -333,8 +332,8 @@ int brtm_unet_create(brtm_ctx *ctx, int batch, int patch, unsigned long long see
   for (int l = 0; l < 9; ++l) {
     A(u->wbf[l], bf * 27 * kConv[l].cout * pad32(kConv[l].cin));
     A(u->wtf[l], bf * 27 * kConv[l].cin * pad32(kConv[l].cout));
-    A(u->gpad[l], f4 * 27 * kConv[l].cout * pad32(kConv[l].cin));
   }
+  A(u->gscratch, f4 * kGradScratch);
   A(u->e1a, bf * B * P3 * C1);
   A(u->cat1, bf * B * P3 * 48);
   A(u->p1, bf * B * P3b * C1);
