@@ -98,6 +98,18 @@ constexpr int kAutoPrefetch = 1;
 // launches, which the hint would forfeit: 11 % slower at 256^3.
 constexpr double kStreamMinStepBytes = 512.0 * 1024 * 1024;
 
+// Largest grids of the VL step without LDS.  Its taps go through L1 and L2,
+// which pays while the fields stay in the Infinity Cache.  Plain / FP32
+// imaging / FP16 imaging / FP16 Born steps in us, before and with it: 48^3 8.8
+// / 9.6 / 11.6 / 11.5 and 3.2 / 3.6 / 3.6 / 3.5; 128^3 10.6 / 11.9 / 16.3 / 15.8
+// and 8.4 / 11.1 / 10.6 / 9.8; 208^3 (9.0 M cells) 31 / 63 / 47 / 45 and 26 / 40
+// / 37 / 33.  At 288 x 240 x 208 (14.4 M) it takes 41 / 77 / 61 / 57, the ring's
+// 64 x 16 tiles 36 / 62 / 63 / 55.  Where n1 is no multiple of 4 the
+// alternative is the one- or two-cell kernel: 257 x 201 x 233 (12 M) 41 / 66 /
+// 60 / 52 against 36 / 54 / 51 / 44, 301^3 (27 M) 100 / 173 / 172 / 150 against
+// 113 / 178 / 174 / 149.
+constexpr long kDirectMaxCells = 10L << 20, kDirectMaxCellsOdd = 16L << 20;
+
 #define BRTM_TRY(x)              \
   do {                           \
     int rc_ = (x);               \
@@ -148,6 +160,13 @@ int step(brtm_ctx *c, int form, int act, int fmt, const float *p, const float *p
   P.pf = c->prefetch == 0 ? kAutoPrefetch : c->prefetch;
   P.stream = c->stream_loads < 0 ? (16.0 * (double)c->ncell > kStreamMinStepBytes)
                                  : c->stream_loads != 0;
+  // The automatic choice: the kernel without LDS while the fields stay in the
+  // caches, the four-cell ring where n1 allows it, else as below.
+  const bool autosel =
+      form == FORM_VL && c->ty_tile == 0 && c->x_per_lane == 0 && c->halo_ring < 0;
+  const bool direct =
+      autosel && c->ncell <= (c->n1 % 4 == 0 ? kDirectMaxCells : kDirectMaxCellsOdd);
+  const bool auto4 = autosel && !direct && c->n1 % 4 == 0;
   // Tile rows / workgroup target per variant (measured on MI355X at 512^3):
   // plain steps prefer tall tiles, 16-bit snapshot variants short ones.
   int ty = c->ty_tile, tb = c->target_blocks;
@@ -167,7 +186,7 @@ int step(brtm_ctx *c, int form, int act, int fmt, const float *p, const float *p
     else if (want >= 2 && c->n1 % 2 == 0) xl = 2;
   }
   // halo ring: automatic (-1) means on for the 4-cell kernel
-  bool ring = c->halo_ring < 0 ? xl == 4 : c->halo_ring != 0;
+  const bool ring = c->halo_ring < 0 ? xl == 4 : c->halo_ring != 0;
   if (ty == 0) {
     if (xl == 4) { ty = (ring && act == ACT_IMG && fmt == FMT_F32) ? 8 : 16; tb = 256; }
     else if (xl == 2) { ty = 16; tb = 2048; }
@@ -177,24 +196,14 @@ int step(brtm_ctx *c, int form, int act, int fmt, const float *p, const float *p
   }
   if (xl == 4 && ty == 32) ty = 16;  // the 4-cell kernel's tiles are 8 or 16 rows
   plan_step(P, ty, tb, 64 * xl);
-  // Small grids: when the automatic shape leaves compute units without a
-  // workgroup, 64-wide 8-row tiles give several times as many (128^3: 480
-  // workgroups instead of 120, the plain step 10.7 us instead of 12.8).
-  if (c->ty_tile == 0 && c->x_per_lane == 0 && c->halo_ring < 0 &&
-      (long)P.ntx * P.nty * P.ntz < c->ncu) {
-    xl = 1;
-    ring = false;
-    ty = 8;
-    tb = 2048;
-    plan_step(P, ty, tb, 64);
-  }
   const bool timed =
       c->ktime_on && form == c->ktime_form && act == c->ktime_act && fmt == c->ktime_fmt;
   BRTM_TRY(ktime_begin(c, timed));
-  // receivers inside the step: the four-cell ring kernel, or the one-cell
-  // kernel's 8-row small-grid shape; one receiver plane
+  // receivers inside the step: the four-cell ring kernel, the kernel without
+  // LDS, or the one-cell kernel's 8-row shape; one receiver plane
   const bool src = rec == REC_SOURCE;
-  const bool rec_kernel = (xl == 4 && ring) || (xl == 1 && !ring && ty == 8);
+  const bool rec_kernel =
+      direct || auto4 || (xl == 4 && ring) || (xl == 1 && !ring && ty == 8);
   const bool in_step = rec != REC_NONE && fused && c->rec_fusion && rec_kernel &&
                        form == FORM_VL &&
                        (src ? c->src_plane && c->nsrc > 0 : c->rec_plane && c->nrec > 0);
@@ -210,7 +219,13 @@ int step(brtm_ctx *c, int form, int act, int fmt, const float *p, const float *p
     std::memcpy(P.rsinc, &c->sinc[src ? 0 : 1][8 * (it % jt)], sizeof(P.rsinc));
   }
   const int kmode = !in_step ? REC_NONE : (src ? REC_INJECT : rec);
-  if (xl == 1 && form == FORM_VL && ring)
+  if (direct) {
+    // two slices per thread once that still leaves 12 waves per compute unit
+    const long waves2 = ((c->n1 - 5L) / 4) * (c->n2 - 8) * ((c->n3 - 7) / 2) / 64;
+    BRTM_HIP(launch_step_direct(act, fmt, P, waves2 >= 12L * c->ncu ? 2 : 1, c->stream, kmode));
+  } else if (auto4)
+    BRTM_HIP(launch_step_auto4(act, fmt, P, c->ncu, c->stream, kmode));
+  else if (xl == 1 && form == FORM_VL && ring)
     BRTM_HIP(launch_step_ring(act, fmt, P, ty, c->stream));
   else if (xl == 4)
     BRTM_HIP(launch_step_x4(act, fmt, P, ty, ring, c->stream, kmode));

@@ -14,8 +14,8 @@ enum StepForm { FORM_VL = 0, FORM_LV = 1 };
 //   ACT_IMG  img += cimg . s . p_new        (zero-lag imaging, VL only)
 //   ACT_BORN p_new += cimg . s . m          (Born secondary source)
 enum StepAct { ACT_NONE = 0, ACT_IMG = 1, ACT_BORN = 2 };
-// Receivers handled inside the step (the four-cell ring kernel, and the
-// one-cell kernel's 8-row small-grid shape):
+// Receivers handled inside the step (the four-cell ring kernel, the kernel
+// without LDS, and the one-cell kernel's 8-row shape):
 //   REC_INJECT   pn += sum_k rsinc[k] rtr(r, rid+k) before imaging and the store
 //   REC_EXTRACT  rtr(r, rid+k) += rsinc[k] . pn . (rscale[r] or 1)
 // for the cells of plane rz whose rmap entry is a receiver index r >= 0.
@@ -77,6 +77,14 @@ hipError_t launch_step_x2(int act, int fmt, StepParams P, int ty_tile, hipStream
 // ring only) handles the receivers inside the step.
 hipError_t launch_step_x4(int act, int fmt, StepParams P, int ty_tile, bool ring,
                           hipStream_t st, int rec = REC_NONE);
+// The four-cell ring step in the tile shape and z chunks that fill ncu
+// compute units best (plans P itself).
+hipError_t launch_step_auto4(int act, int fmt, const StepParams &P, int ncu, hipStream_t st,
+                             int rec = REC_NONE);
+// The VL step without LDS for grids that stay in the caches (any n1): zc
+// (1 or 2) slices per thread; rec as above.
+hipError_t launch_step_direct(int act, int fmt, const StepParams &P, int zc, hipStream_t st,
+                              int rec = REC_NONE);
 // Two consecutive plain VL steps in one pass: p^{n+1} = step(p = p^n,
 // po = p^{n-1}) into pn and p^{n+2} = step(p^{n+1}, p^n) into pn2, with the
 // sponge, and (rec = REC_INJECT) the source points of plane rz injected after

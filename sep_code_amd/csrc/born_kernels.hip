@@ -22,6 +22,7 @@
 
 #include <hip/hip_fp16.h>
 
+#include <algorithm>
 #include <type_traits>
 
 namespace brtm {
@@ -706,37 +707,34 @@ __device__ __forceinline__ f32x4 ld4_stream(const float *a, int i) {
   return __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(a + i));
 }
 
-// Four consecutive snapshot values decoded to FP32; STREAM selects the
-// streaming (nontemporal) load.
-template <int FMT, bool STREAM = false>
-__device__ __forceinline__ f32x4 snap4_at(const void *s, const float *sscale, int i, int z) {
-  f32x4 r = {0.f, 0.f, 0.f, 0.f};
-  if constexpr (FMT == FMT_F32) {
-    const f32x4 *a = reinterpret_cast<const f32x4 *>(static_cast<const float *>(s) + i);
-    if constexpr (STREAM) r = __builtin_nontemporal_load(a);
-    else r = *a;
+// Four 16-bit snapshot codes as FP32.
+template <int FMT>
+__device__ __forceinline__ f32x4 decode4(const u32x2 &u, float sc) {
+  f32x4 r;
+  if constexpr (FMT == FMT_BF16) {
+    r.x = __uint_as_float(u.x << 16) * sc;
+    r.y = __uint_as_float(u.x & 0xffff0000u) * sc;
+    r.z = __uint_as_float(u.y << 16) * sc;
+    r.w = __uint_as_float(u.y & 0xffff0000u) * sc;
   } else {
-    // 16-bit codes: four of them in 8 bytes
-    const u32x2 *a = reinterpret_cast<const u32x2 *>(static_cast<const uint16_t *>(s) + i);
-    u32x2 u;
-    if constexpr (STREAM) u = __builtin_nontemporal_load(a);
-    else u = *a;
-    const float sc = sscale[z];
-    if constexpr (FMT == FMT_BF16) {
-      r.x = __uint_as_float(u.x << 16) * sc;
-      r.y = __uint_as_float(u.x & 0xffff0000u) * sc;
-      r.z = __uint_as_float(u.y << 16) * sc;
-      r.w = __uint_as_float(u.y & 0xffff0000u) * sc;
-    } else if constexpr (FMT == FMT_F16) {
-      const float2 lo = __half22float2(__builtin_bit_cast(__half2, (unsigned int)u.x));
-      const float2 hi = __half22float2(__builtin_bit_cast(__half2, (unsigned int)u.y));
-      r.x = lo.x * sc;
-      r.y = lo.y * sc;
-      r.z = hi.x * sc;
-      r.w = hi.y * sc;
-    }
+    const float2 lo = __half22float2(__builtin_bit_cast(__half2, (unsigned int)u.x));
+    const float2 hi = __half22float2(__builtin_bit_cast(__half2, (unsigned int)u.y));
+    r.x = lo.x * sc;
+    r.y = lo.y * sc;
+    r.z = hi.x * sc;
+    r.w = hi.y * sc;
   }
   return r;
+}
+
+// Four consecutive snapshot values decoded to FP32 (i a multiple of 4).
+template <int FMT>
+__device__ __forceinline__ f32x4 snap4_at(const void *s, const float *sscale, int i, int z) {
+  if constexpr (FMT == FMT_F32)
+    return *reinterpret_cast<const f32x4 *>(static_cast<const float *>(s) + i);
+  else
+    return decode4<FMT>(
+        *reinterpret_cast<const u32x2 *>(static_cast<const uint16_t *>(s) + i), sscale[z]);
 }
 
 template <int TY, int RPT, int FMT, int ACT>
@@ -932,31 +930,77 @@ k_step_x4(const StepParams P) {
 // ---------------------------------------------------------------------------
 // Four cells per lane on the six-plane LDS ring (the two ideas above
 // together): 16-byte accesses, and each halo loaded in the same iteration as
-// the neighbouring tiles' z-queue loads of that slice.  16-row tiles take
-// 149 KB of LDS, which the one workgroup per CU that the registers allow
-// can have.
+// the neighbouring tiles' z-queue loads of that slice.  A wave covers LX lanes
+// by 64 / LX rows, so a tile is 4 LX cells by NWV (64 / LX) RPT rows:
+//   LX 64, 8 waves: 256 x 8 (100 KB of LDS; RPT 2: 256 x 16, 149 KB), one
+//     workgroup per CU;
+//   LX 32, 12 waves: 128 x 24 (102 KB), one workgroup per CU, and LX 16, 4
+//     waves: 64 x 16 (41 KB), three per CU: for rows that 256-wide tiles fit
+//     badly (launch_step_auto4 chooses).
 // ---------------------------------------------------------------------------
-template <int TY, int RPT, int FMT, int ACT, int REC = REC_NONE, int PF = 1, bool STREAM = false>
-__global__ void __launch_bounds__(64 * (TY / RPT))
+// A lane's accesses to one x-y plane: its byte offset inside the plane is
+// fixed for the whole z sweep, and kOff marks a lane that has none (the load
+// gives zero, the store does nothing).
+constexpr unsigned int kOff = 0x80000000u;  // beyond any plane (n1 n2 < 2^28)
+
+template <bool NT>
+__device__ __forceinline__ f32x4 plane_ld4(const float *base, unsigned int off, bool on) {
+  f32x4 v = {0.f, 0.f, 0.f, 0.f};
+  if (on && off != kOff) {
+    const f32x4 *a = reinterpret_cast<const f32x4 *>(reinterpret_cast<const char *>(base) + off);
+    if constexpr (NT) v = __builtin_nontemporal_load(a);
+    else v = *a;
+  }
+  return v;
+}
+__device__ __forceinline__ void plane_st4(float *base, unsigned int off, const f32x4 &v) {
+  if (off != kOff)
+    __builtin_nontemporal_store(
+        v, reinterpret_cast<f32x4 *>(reinterpret_cast<char *>(base) + off));
+}
+
+// The snapshot and the image or model come through buffer loads, whose range
+// check gives the zeros without a branch: their four loads then issue in one
+// run with the others.  FP16 imaging / FP16 Born at 512^3: 600 / 491 us against
+// 710 / 553 us with masked loads like the ones above; the masked form is the
+// better one for p, p_old, V and the stores (plain step 358 against 370 us).
+typedef __amdgpu_buffer_rsrc_t plane_rsrc;
+constexpr int kNt = 2;  // the nontemporal bit of a buffer access
+__device__ __forceinline__ plane_rsrc plane_of(const void *base, int bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, bytes, 0x00020000);
+}
+template <bool NT>
+__device__ __forceinline__ f32x4 buffer_ld4(plane_rsrc r, unsigned int off) {
+  return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, NT ? kNt : 0));
+}
+
+template <int LX, int NWV, int RPT, int FMT, int ACT, int REC = REC_NONE, int PF = 1,
+          bool STREAM = false>
+__global__ void __launch_bounds__(64 * NWV)
 k_step_x4r(const StepParams P) {
   static_assert((ACT == ACT_NONE) == (FMT == FMT_NONE), "an action needs a snapshot format");
   static_assert(PF == 1 || (PF == 2 && ACT == ACT_NONE),
                 "two slices of prefetch only for the plain step (registers)");
   static_assert(!(REC == REC_INJECT && ACT == ACT_BORN) && !(REC == REC_EXTRACT && ACT == ACT_IMG),
                 "injection goes with the adjoint, extraction with Born modelling");
-  constexpr int NWV = TY / RPT;
-  constexpr int HY = 8 / NWV;
-  static_assert(8 % NWV == 0, "waves must divide the 8 halo rows");
-  constexpr int LW = 264;
+  constexpr int WR = 64 / LX;          // rows per wave
+  constexpr int TY = NWV * WR * RPT;   // rows per tile
+  constexpr int TW = 4 * LX;           // cells per tile row
+  constexpr int NT = 64 * NWV;
+  // y halo: 8 rows of LX groups, HY per thread; x halo: two groups per row,
+  // loaded by the first lanes of the row's wave, one load per row of a thread
+  constexpr int HY = (8 * LX + NT - 1) / NT, NH = HY + RPT;
+  constexpr int LW = TW + 8;
   constexpr int NR = 6;
   __shared__ __attribute__((aligned(16))) float ring[NR][TY + 8][LW];
   __shared__ float wsh[kWMax];
 
-  const int lane = threadIdx.x;
-  const int wy = threadIdx.y;
+  const int tid = threadIdx.y * 64 + threadIdx.x;
+  const int lx = threadIdx.x % LX;
+  const int ry = threadIdx.y * WR * RPT + threadIdx.x / LX;  // the thread's first row
   const int n1 = P.n1, n2 = P.n2, n3 = P.n3, nw = P.nw;
   const int s3 = n1 * n2;
-  for (int e = wy * 64 + lane; e < nw; e += 64 * NWV) wsh[e] = P.wtab[e];
+  for (int e = tid; e < nw; e += NT) wsh[e] = P.wtab[e];
 
   const int nb = P.ntx * P.nty * P.ntz;
   const int bid = blockIdx.x;
@@ -966,155 +1010,166 @@ k_step_x4r(const StepParams P) {
   const int ty = (t / P.ntx) % P.nty;
   const int tz = t / (P.ntx * P.nty);
 
-  const int x = tx * 256 + 4 * lane;
+  const int x = tx * TW + 4 * lx;
   const int y0 = ty * TY;
-  const int yb = y0 + wy * RPT;
+  const int yb = y0 + ry;
   const int z0 = 4 + tz * P.zc;
   const int z1 = min(z0 + P.zc, n3 - 4);
-  const bool xmem = x < n1;
-  const bool xin = (x >= 4) && (x < n1 - 4);
   int ex[4];
 #pragma unroll
   for (int j = 0; j < 4; ++j) ex[j] = edist(x + j, n1);
 
-  auto ld4 = [&](const float *a, int i, bool ok) -> f32x4 {
-    f32x4 v = {0.f, 0.f, 0.f, 0.f};
-    if (ok) v = *reinterpret_cast<const f32x4 *>(a + i);
-    return v;
+  // byte offsets in a plane: the thread's groups (loads; stores only inside
+  // the update set) and its halo groups with their place in LDS
+  const bool xmem = x < n1, xin = x >= 4 && x < n1 - 4;
+  unsigned int lo[RPT], so[RPT], ho[NH];
+#pragma unroll
+  for (int r = 0; r < RPT; ++r) {
+    const int y = yb + r * WR;
+    lo[r] = xmem && y < n2 ? 4u * (y * n1 + x) : kOff;
+    so[r] = xin && y >= 4 && y < n2 - 4 ? 4u * (y * n1 + x) : kOff;
+  }
+  int hrow[NH], hcol[NH];
+  bool hput[NH];
+#pragma unroll
+  for (int j = 0; j < HY; ++j) {
+    const int h = tid + j * NT, row = h / LX, gx = tx * TW + 4 * (h % LX);
+    const int gy = row < 4 ? y0 - 4 + row : y0 + TY + (row - 4);
+    hput[j] = (j + 1) * NT <= 8 * LX || h < 8 * LX;
+    hrow[j] = row < 4 ? row : TY + row;
+    hcol[j] = 4 + 4 * (h % LX);
+    ho[j] = hput[j] && gx < n1 && gy >= 0 && gy < n2 ? 4u * (gy * n1 + gx) : kOff;
+  }
+#pragma unroll
+  for (int r = 0; r < RPT; ++r) {
+    const int h = threadIdx.x, row = threadIdx.y * WR * RPT + r * WR + (h >> 1);
+    const int gx = (h & 1) ? tx * TW + TW : tx * TW - 4, gy = y0 + row;
+    hput[HY + r] = h < 2 * WR;
+    hrow[HY + r] = 4 + row;
+    hcol[HY + r] = (h & 1) ? TW + 4 : 0;
+    ho[HY + r] = hput[HY + r] && gx >= 0 && gx < n1 && gy < n2 ? 4u * (gy * n1 + gx) : kOff;
+  }
+
+  // (readfirstlane keeps the plane's base in scalar registers: a 32-bit lane
+  // offset is then all the address a lane needs)
+  auto plane = [&](auto *a, int z) { return a + (long)s3 * __builtin_amdgcn_readfirstlane(z); };
+  auto load_halo = [&](int z, bool on, f32x4 *oh) {
+#pragma unroll
+    for (int j = 0; j < NH; ++j) oh[j] = plane_ld4<false>(plane(P.p, z), ho[j], on);
+  };
+  auto put_plane = [&](int z, const f32x4 *c, const f32x4 *hh) {
+    float(*pl)[LW] = ring[z % NR];
+#pragma unroll
+    for (int r = 0; r < RPT; ++r)
+      *reinterpret_cast<f32x4 *>(&pl[4 + ry + r * WR][4 + 4 * lx]) = c[r];
+#pragma unroll
+    for (int j = 0; j < NH; ++j)
+      if (hput[j]) *reinterpret_cast<f32x4 *>(&pl[hrow[j]][hcol[j]]) = hh[j];
   };
   // the lane's own streams (read once, by this tile only)
-  auto ldc = [&](const float *a, int i, bool ok) -> f32x4 {
-    f32x4 v = {0.f, 0.f, 0.f, 0.f};
-    if (ok) {
-      if constexpr (STREAM) v = ld4_stream(a, i);
-      else v = *reinterpret_cast<const f32x4 *>(a + i);
+  auto load_center = [&](int z, bool on, f32x4 *opo, f32x4 *oV, f32x4 *oS, f32x4 *oX) {
+#pragma unroll
+    for (int r = 0; r < RPT; ++r) {
+      opo[r] = plane_ld4<STREAM>(plane(P.po, z), lo[r], on);
+      oV[r] = plane_ld4<STREAM>(plane(P.V, z), lo[r], on);
     }
-    return v;
+    if constexpr (ACT != ACT_NONE) {
+      const int pb = on ? 4 * s3 : 0;  // bytes of a plane
+      // an FP32 snapshot streams at every size (64.6 against 70.4 us for
+      // FP32 imaging at 256^3); 16-bit ones only with STREAM (BF16 imaging
+      // at 256^3: 77.4 against 74.6 us)
+      if constexpr (FMT == FMT_F32) {
+        const plane_rsrc rs = plane_of(plane(static_cast<const float *>(P.snap), z), pb);
+#pragma unroll
+        for (int r = 0; r < RPT; ++r) oS[r] = buffer_ld4<true>(rs, lo[r]);
+      } else {
+        const plane_rsrc rs = plane_of(plane(static_cast<const uint16_t *>(P.snap), z), pb / 2);
+        const float sc = P.sscale[z];
+#pragma unroll
+        for (int r = 0; r < RPT; ++r)
+          oS[r] = decode4<FMT>(
+              __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(
+                                            rs, lo[r] >> 1, 0, STREAM ? kNt : 0)),
+              sc);
+      }
+      // the image streams at every size (FP32 / BF16 imaging at 256^3:
+      // 62.3 / 71.6 against 65.2 / 74.6 us); the model only with STREAM
+      // (the Born step at 256^3: 66.0 against 64.5 us)
+      const plane_rsrc rx = plane_of(plane(ACT == ACT_IMG ? P.img : P.m, z), pb);
+#pragma unroll
+      for (int r = 0; r < RPT; ++r) oX[r] = buffer_ld4 < STREAM || ACT == ACT_IMG > (rx, lo[r]);
+    }
   };
 
   f32x4 q[RPT][9];
 #pragma unroll
-  for (int r = 0; r < RPT; ++r) {
-    const int y = yb + r;
-    const bool ok = xmem && y < n2;
+  for (int k = 0; k < 9; ++k) {
 #pragma unroll
-    for (int k = 0; k < 9; ++k) q[r][k] = ld4(P.p, (z0 - 4 + k) * s3 + y * n1 + x, ok);
+    for (int r = 0; r < RPT; ++r) q[r][k] = plane_ld4<false>(plane(P.p, z0 - 4 + k), lo[r], true);
   }
 
-  int hyy[HY], hyrow[HY];
-#pragma unroll
-  for (int j = 0; j < HY; ++j) {
-    const int h = wy * HY + j;
-    hyy[j] = h < 4 ? y0 - 4 + h : y0 + TY + (h - 4);
-    hyrow[j] = h < 4 ? h : TY + h;
-  }
-  const bool hxl = lane < 2;
-  const int hxx = lane == 0 ? tx * 256 - 4 : tx * 256 + 256;
-  const int hxcol = lane == 0 ? 0 : 260;
-  const bool hxok = hxl && hxx >= 0 && hxx < n1;
-
-  auto load_halo = [&](int z, f32x4 *ohy, f32x4 *ohx) {
-#pragma unroll
-    for (int j = 0; j < HY; ++j)
-      ohy[j] = ld4(P.p, z * s3 + hyy[j] * n1 + x, xmem && hyy[j] >= 0 && hyy[j] < n2);
-#pragma unroll
-    for (int r = 0; r < RPT; ++r)
-      ohx[r] = ld4(P.p, z * s3 + (yb + r) * n1 + hxx, hxok && (yb + r) < n2);
-  };
-  auto put_plane = [&](int z, const f32x4 *c, const f32x4 *hy, const f32x4 *hx) {
-    float(*pl)[LW] = ring[z % NR];
-#pragma unroll
-    for (int r = 0; r < RPT; ++r)
-      *reinterpret_cast<f32x4 *>(&pl[4 + wy * RPT + r][4 + 4 * lane]) = c[r];
-#pragma unroll
-    for (int j = 0; j < HY; ++j) *reinterpret_cast<f32x4 *>(&pl[hyrow[j]][4 + 4 * lane]) = hy[j];
-    if (hxl) {
-#pragma unroll
-      for (int r = 0; r < RPT; ++r) *reinterpret_cast<f32x4 *>(&pl[4 + wy * RPT + r][hxcol]) = hx[r];
-    }
-  };
-  auto load_center = [&](int z, f32x4 *opo, f32x4 *oV, f32x4 *oS, f32x4 *oX) {
-#pragma unroll
-    for (int r = 0; r < RPT; ++r) {
-      const int y = yb + r;
-      const bool ok = xmem && y < n2;
-      const int i = z * s3 + y * n1 + x;
-      opo[r] = ldc(P.po, i, ok);
-      oV[r] = ldc(P.V, i, ok);
-      if constexpr (ACT != ACT_NONE) {
-        const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-        // an FP32 snapshot streams at every size (64.6 against 70.4 us for
-        // FP32 imaging at 256^3); 16-bit ones only with STREAM (BF16 imaging
-        // at 256^3: 77.4 against 74.6 us)
-        oS[r] = ok ? snap4_at<FMT, STREAM || FMT == FMT_F32>(P.snap, P.sscale, i, z) : zero;
-        // the image streams at every size (FP32 / BF16 imaging at 256^3:
-        // 62.3 / 71.6 against 65.2 / 74.6 us); the model only with STREAM
-        // (the Born step at 256^3: 66.0 against 64.5 us)
-        const float *xs = ACT == ACT_IMG ? P.img : P.m;
-        if constexpr (STREAM || ACT == ACT_IMG) oX[r] = ok ? ld4_stream(xs, i) : zero;
-        else oX[r] = ld4(xs, i, ok);
-      }
-    }
-  };
-
-  // prologue: planes z0 .. z0+3 into the ring; the halo of z0+4 waits in hy/hx
-  f32x4 hy[HY], hx[RPT];
+  // prologue: planes z0 .. z0+3 into the ring; the halo of z0+4 waits in hh
+  f32x4 hh[NH];
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
-    f32x4 th[HY], tx_[RPT], c[RPT];
-    load_halo(z0 + k, th, tx_);
+    f32x4 th[NH], c[RPT];
+    load_halo(z0 + k, true, th);
 #pragma unroll
     for (int r = 0; r < RPT; ++r) c[r] = q[r][4 + k];
-    put_plane(z0 + k, c, th, tx_);
+    put_plane(z0 + k, c, th);
   }
-  load_halo(z0 + 4, hy, hx);
+  load_halo(z0 + 4, true, hh);
   f32x4 cpo[RPT], cV[RPT], cS[RPT], cX[RPT];
-  load_center(z0, cpo, cV, cS, cX);
+  load_center(z0, true, cpo, cV, cS, cX);
   // PF = 2: the inputs of slice z+1 were loaded one iteration earlier and
   // wait in the p* registers while the loads of slice z+2 are in flight
-  f32x4 pq[RPT], phy[HY], phx[RPT], ppo[RPT], pV[RPT], pS[RPT], pX[RPT];
+  f32x4 pq[RPT], ph[NH], ppo[RPT], pV[RPT], pS[RPT], pX[RPT];
   if constexpr (PF == 2) {
-    if (z0 + 1 < z1) {
+    const bool on = z0 + 1 < z1;
+    const int zf = on ? z0 + 1 : z0;
 #pragma unroll
-      for (int r = 0; r < RPT; ++r) {
-        const int y = yb + r;
-        pq[r] = ld4(P.p, (z0 + 5) * s3 + y * n1 + x, xmem && y < n2);
-      }
-      load_halo(z0 + 5, phy, phx);
-      load_center(z0 + 1, ppo, pV, pS, pX);
-    }
+    for (int r = 0; r < RPT; ++r) pq[r] = plane_ld4<false>(plane(P.p, zf + 4), lo[r], on);
+    load_halo(zf + 4, on, ph);
+    load_center(zf, on, ppo, pV, pS, pX);
   }
 
   const float c0 = P.c[0];
   for (int z = z0; z < z1; ++z) {
+    // Everything of the previous iteration has arrived (vmcnt(0)), its stores
+    // too, before this one's loads are issued.  Where the accesses are in
+    // branches the compiler cannot count them and would otherwise wait for
+    // this slice's own loads in the middle of its arithmetic; waiting here
+    // costs less in the plain step (320^3: 102 against 109 us) and in
+    // 256-wide tiles, and more in the narrow tiles' imaging and Born steps
+    // (384^3, FP32 imaging: 282 against 270 us), which leave it out.
+    if constexpr (LX == 64 || ACT == ACT_NONE) __builtin_amdgcn_s_waitcnt(0x0f70);
     {
       f32x4 c[RPT];
 #pragma unroll
       for (int r = 0; r < RPT; ++r) c[r] = q[r][8];
-      put_plane(z + 4, c, hy, hx);
+      put_plane(z + 4, c, hh);
     }
-    const int zn = z + 1;
-    const int zf = z + PF;  // the slice whose inputs are loaded now
-    f32x4 nq[RPT], nhy[HY], nhx[RPT];
+    // the slice whose inputs are loaded now (nothing past the chunk's last)
+    const bool on = z + PF < z1;
+    const int zf = on ? z + PF : z;
+    f32x4 nq[RPT], nh[NH];
     f32x4 npo[RPT], nV[RPT], nS[RPT], nX[RPT];
-    if (zf < z1) {
 #pragma unroll
-      for (int r = 0; r < RPT; ++r) {
-        const int y = yb + r;
-        nq[r] = ld4(P.p, (zf + 4) * s3 + y * n1 + x, xmem && y < n2);
-      }
-      load_halo(zf + 4, nhy, nhx);
-      load_center(zf, npo, nV, nS, nX);
-    }
+    for (int r = 0; r < RPT; ++r) nq[r] = plane_ld4<false>(plane(P.p, zf + 4), lo[r], on);
+    load_halo(zf + 4, on, nh);
+    load_center(zf, on, npo, nV, nS, nX);
     __syncthreads();
 
     float(*pl)[LW] = ring[z % NR];
     const int ez = edist(z, n3);
 #pragma unroll
     for (int r = 0; r < RPT; ++r) {
-      const int y = yb + r;
-      const int row = 4 + wy * RPT + r;
-      const int col = 4 + 4 * lane;
+      const int y = yb + r * WR;
+      const int row = 4 + ry + r * WR;
+      const int col = 4 + 4 * lx;
+      // skipping a row as a whole keeps its LDS reads and stores together: 365
+      // us against 371 us for the plain 512^3 step with its source inside
+      if (so[r] == kOff) continue;
       const f32x4 C = q[r][4];
       const f32x4 L = *reinterpret_cast<const f32x4 *>(&pl[row][col - 4]);
       const f32x4 R = *reinterpret_cast<const f32x4 *>(&pl[row][col + 4]);
@@ -1136,84 +1191,224 @@ k_step_x4r(const StepParams P) {
           acc[j] = fmaf(c3, zz[j], acc[j]);
         }
       }
-      if (xin && y >= 4 && y < n2 - 4) {
-        const int eyz = min(edist(y, n2), ez);
-        const int i = z * s3 + y * n1 + x;
-        f32x4 pn;
+      const int eyz = min(edist(y, n2), ez);
+      f32x4 pn;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int e = min(ex[j], eyz);
-          const float w = e < nw ? wsh[e] : 1.f;
-          float v = w * fmaf(cV[r][j], acc[j], 2.f * C[j]) - (w * w) * cpo[r][j];
-          if constexpr (ACT == ACT_BORN) v = fmaf(P.cimg * cS[r][j], cX[r][j], v);
-          pn[j] = v;
-        }
-        if constexpr (REC != REC_NONE) {
-          // the receiver plane: the same arithmetic as k_inject / k_extract
-          // for the (at most one) receiver of each cell
-          if (z == P.rz) {
-            const int4 rr = *reinterpret_cast<const int4 *>(P.rmap + y * n1 + x);
-            const int ri[4] = {rr.x, rr.y, rr.z, rr.w};
+      for (int j = 0; j < 4; ++j) {
+        const int e = min(ex[j], eyz);
+        const float w = e < nw ? wsh[e] : 1.f;
+        pn[j] = w * fmaf(cV[r][j], acc[j], 2.f * C[j]) - (w * w) * cpo[r][j];
+      }
+      if constexpr (ACT == ACT_BORN) {
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-              if (ri[j] < 0) continue;
-              if constexpr (REC == REC_INJECT) {
-                float acc = 0.f;
+        for (int j = 0; j < 4; ++j) pn[j] = fmaf(P.cimg * cS[r][j], cX[r][j], pn[j]);
+      }
+      if constexpr (REC != REC_NONE) {
+        // the receiver plane: the same arithmetic as k_inject / k_extract
+        // for the (at most one) receiver of each cell
+        if (z == P.rz) {
+          const int4 rr = *reinterpret_cast<const int4 *>(P.rmap + y * n1 + x);
+          const int ri[4] = {rr.x, rr.y, rr.z, rr.w};
 #pragma unroll
-                for (int k = 0; k < 8; ++k)
-                  if (P.rsinc[k] != 0.f)
-                    acc = fmaf(P.rsinc[k], P.rtr[ri[j] * P.rsp + (P.rid + k) * P.rst], acc);
-                pn[j] += acc;
-              } else {
-                const float v = P.rscale ? pn[j] * P.rscale[ri[j]] : pn[j];
+          for (int j = 0; j < 4; ++j) {
+            if (ri[j] < 0) continue;
+            if constexpr (REC == REC_INJECT) {
+              float acc = 0.f;
 #pragma unroll
-                for (int k = 0; k < 8; ++k)
-                  if (P.rsinc[k] != 0.f) P.rtr[ri[j] * P.rsp + (P.rid + k) * P.rst] += v * P.rsinc[k];
-              }
+              for (int k = 0; k < 8; ++k)
+                if (P.rsinc[k] != 0.f)
+                  acc = fmaf(P.rsinc[k], P.rtr[ri[j] * P.rsp + (P.rid + k) * P.rst], acc);
+              pn[j] += acc;
+            } else {
+              const float v = P.rscale ? pn[j] * P.rscale[ri[j]] : pn[j];
+#pragma unroll
+              for (int k = 0; k < 8; ++k)
+                if (P.rsinc[k] != 0.f) P.rtr[ri[j] * P.rsp + (P.rid + k) * P.rst] += v * P.rsinc[k];
             }
           }
         }
-        __builtin_nontemporal_store(pn, reinterpret_cast<f32x4 *>(P.pn + i));
-        if constexpr (ACT == ACT_IMG) {
-          f32x4 im;
+      }
+      plane_st4(plane(P.pn, z), so[r], pn);
+      if constexpr (ACT == ACT_IMG) {
+        f32x4 im;
 #pragma unroll
-          for (int j = 0; j < 4; ++j) im[j] = fmaf(P.cimg * cS[r][j], pn[j], cX[r][j]);
-          __builtin_nontemporal_store(im, reinterpret_cast<f32x4 *>(P.img + i));
-        }
+        for (int j = 0; j < 4; ++j) im[j] = fmaf(P.cimg * cS[r][j], pn[j], cX[r][j]);
+        plane_st4(plane(P.img, z), so[r], im);
       }
     }
 
-    if (zn < z1) {
 #pragma unroll
-      for (int r = 0; r < RPT; ++r) {
+    for (int r = 0; r < RPT; ++r) {
 #pragma unroll
-        for (int k = 0; k < 8; ++k) q[r][k] = q[r][k + 1];
-        if constexpr (PF == 2) {
-          q[r][8] = pq[r];
-          cpo[r] = ppo[r];
-          cV[r] = pV[r];
-          hx[r] = phx[r];
-          pq[r] = nq[r];
-          ppo[r] = npo[r];
-          pV[r] = nV[r];
-          phx[r] = nhx[r];
-        } else {
-          q[r][8] = nq[r];
-          cpo[r] = npo[r];
-          cV[r] = nV[r];
-          cS[r] = nS[r];
-          cX[r] = nX[r];
-          hx[r] = nhx[r];
+      for (int k = 0; k < 8; ++k) q[r][k] = q[r][k + 1];
+      if constexpr (PF == 2) {
+        q[r][8] = pq[r];
+        cpo[r] = ppo[r];
+        cV[r] = pV[r];
+        pq[r] = nq[r];
+        ppo[r] = npo[r];
+        pV[r] = nV[r];
+      } else {
+        q[r][8] = nq[r];
+        cpo[r] = npo[r];
+        cV[r] = nV[r];
+        cS[r] = nS[r];
+        cX[r] = nX[r];
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < NH; ++j) {
+      if constexpr (PF == 2) {
+        hh[j] = ph[j];
+        ph[j] = nh[j];
+      } else {
+        hh[j] = nh[j];
+      }
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// The VL step without LDS, for grids whose fields stay in the caches.
+//
+// A thread owns four consecutive x (from x = 4) of ZC consecutive z and loads
+// every tap itself: all loads are independent, so a wave waits for about one
+// trip to memory instead of one per slice of a z sweep, and there is no
+// barrier.  Lanes run over the update set's (x group, y) pairs in order, so
+// no lane idles at the tile edges of small or odd grids; neighbouring rows
+// of a workgroup share their y taps in L1.  Rows are read 16 bytes at a time
+// at any dword alignment (n1 need not be a multiple of 4; ALIGNED only
+// widens the 16-bit snapshot, map and store accesses).
+// ---------------------------------------------------------------------------
+typedef f32x4 f32x4u __attribute__((aligned(4)));
+
+template <int ZC, int FMT, int ACT, int REC, bool ALIGNED>
+__global__ void __launch_bounds__(256)
+k_step_direct(const StepParams P) {
+  static_assert((ACT == ACT_NONE) == (FMT == FMT_NONE), "an action needs a snapshot format");
+  static_assert(!(REC == REC_INJECT && ACT == ACT_BORN) && !(REC == REC_EXTRACT && ACT == ACT_IMG),
+                "injection goes with the adjoint, extraction with Born modelling");
+  const int n1 = P.n1, n2 = P.n2, n3 = P.n3, nw = P.nw;
+  const int s3 = n1 * n2;
+  // XCD k takes a contiguous run of (plane block, z chunk) tiles, the z
+  // chunks of a plane block first: they share its z taps
+  const int nb = P.ntx * P.ntz;
+  const int bid = blockIdx.x;
+  const int q8 = nb >> 3, r8 = nb & 7, xcd = bid & 7, jj = bid >> 3;
+  const int t = (xcd < r8) ? xcd * (q8 + 1) + jj : r8 * (q8 + 1) + (xcd - r8) * q8 + jj;
+  const int gx = (n1 - 5) >> 2;  // x groups: ceil((n1 - 8) / 4)
+  const int e = (t / P.ntz) * 256 + threadIdx.x;
+  const int z0 = 4 + (t % P.ntz) * ZC;
+  const int y = 4 + e / gx, x = 4 + (e % gx) * 4;
+  if (y >= n2 - 4) return;
+  const int i0 = z0 * s3 + y * n1 + x;
+  auto ld = [](const float *a) -> f32x4 { return *reinterpret_cast<const f32x4u *>(a); };
+
+  // z taps of the ZC slices, then each slice's own streams.  The chunk's
+  // slices beyond the update set are clamped to its last one (loaded, not
+  // stored).
+  const int zl = min(ZC, n3 - 4 - z0);
+  f32x4 q[ZC + 8], po[ZC], V[ZC], S[ZC], X[ZC];
+#pragma unroll
+  for (int k = 0; k < ZC + 8; ++k) q[k] = ld(P.p + (i0 + (min(k, zl + 7) - 4) * s3));
+#pragma unroll
+  for (int k = 0; k < ZC; ++k) {
+    const int zk = min(k, zl - 1), i = i0 + zk * s3;
+    po[k] = ld(P.po + i);
+    V[k] = ld(P.V + i);
+    if constexpr (ACT != ACT_NONE) {
+      X[k] = ld((ACT == ACT_IMG ? P.img : P.m) + i);
+      if constexpr (FMT == FMT_F32) {
+        S[k] = ld(static_cast<const float *>(P.snap) + i);
+      } else if constexpr (ALIGNED) {
+        S[k] = snap4_at<FMT>(P.snap, P.sscale, i, z0 + zk);
+      } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) S[k][j] = snap_at<FMT>(P.snap, P.sscale, i + j, z0 + zk);
+      }
+    }
+  }
+  int exy[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) exy[j] = min(edist(x + j, n1), edist(y, n2));
+  const int nv = min(4, n1 - 4 - x);  // cells of the group in the update set
+  const float c0 = P.c[0];
+  f32x4 pn[ZC];
+#pragma unroll
+  for (int k = 0; k < ZC; ++k) {
+    const int zk = min(k, zl - 1), z = z0 + zk;
+    const float *pc = P.p + (i0 + zk * s3);
+    const f32x4 L = ld(pc - 4), R = ld(pc + 4), C = q[k + 4];
+    f32x4 up[4], dn[4];
+#pragma unroll
+    for (int m = 1; m <= 4; ++m) {
+      up[m - 1] = ld(pc - m * n1);
+      dn[m - 1] = ld(pc + m * n1);
+    }
+    const float a[12] = {L.x, L.y, L.z, L.w, C.x, C.y, C.z, C.w, R.x, R.y, R.z, R.w};
+    float acc[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[j] = c0 * a[4 + j];
+#pragma unroll
+    for (int m = 1; m <= 4; ++m) {
+      const float c1 = P.c[1 + 3 * (m - 1)], c2 = P.c[2 + 3 * (m - 1)], c3 = P.c[3 + 3 * (m - 1)];
+      const f32x4 ud = up[m - 1] + dn[m - 1];
+      const f32x4 zz = q[k + 4 - m] + q[k + 4 + m];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        acc[j] = fmaf(c1, a[4 + j - m] + a[4 + j + m], acc[j]);
+        acc[j] = fmaf(c2, ud[j], acc[j]);
+        acc[j] = fmaf(c3, zz[j], acc[j]);
+      }
+    }
+    const int ez = edist(z, n3);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int ee = max(min(exy[j], ez), 0);
+      const float w = ee < nw ? P.wtab[ee] : 1.f;
+      float v = w * fmaf(V[k][j], acc[j], 2.f * C[j]) - (w * w) * po[k][j];
+      if constexpr (ACT == ACT_BORN) v = fmaf(P.cimg * S[k][j], X[k][j], v);
+      pn[k][j] = v;
+    }
+    if constexpr (REC != REC_NONE) {
+      if (z == P.rz && k < zl) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int ri = j < nv ? P.rmap[y * n1 + x + j] : -1;
+          if (ri < 0) continue;
+          if constexpr (REC == REC_INJECT) {
+            float add = 0.f;
+#pragma unroll
+            for (int h = 0; h < 8; ++h)
+              if (P.rsinc[h] != 0.f)
+                add = fmaf(P.rsinc[h], P.rtr[ri * P.rsp + (P.rid + h) * P.rst], add);
+            pn[k][j] += add;
+          } else {
+            const float v = P.rscale ? pn[k][j] * P.rscale[ri] : pn[k][j];
+#pragma unroll
+            for (int h = 0; h < 8; ++h)
+              if (P.rsinc[h] != 0.f) P.rtr[ri * P.rsp + (P.rid + h) * P.rst] += v * P.rsinc[h];
+          }
         }
       }
+    }
+  }
 #pragma unroll
-      for (int j = 0; j < HY; ++j) {
-        if constexpr (PF == 2) {
-          hy[j] = phy[j];
-          phy[j] = nhy[j];
-        } else {
-          hy[j] = nhy[j];
-        }
+  for (int k = 0; k < ZC; ++k) {
+    if (k >= zl) break;
+    const int i = i0 + k * s3;
+    f32x4 im;
+    if constexpr (ACT == ACT_IMG) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) im[j] = fmaf(P.cimg * S[k][j], pn[k][j], X[k][j]);
+    }
+    if (nv == 4) {
+      *reinterpret_cast<f32x4u *>(P.pn + i) = pn[k];
+      if constexpr (ACT == ACT_IMG) *reinterpret_cast<f32x4u *>(P.img + i) = im;
+    } else {
+      for (int j = 0; j < nv; ++j) {
+        P.pn[i + j] = pn[k][j];
+        if constexpr (ACT == ACT_IMG) P.img[i + j] = im[j];
       }
     }
   }
@@ -1925,29 +2120,31 @@ hipError_t launch_ring_t(int act, int fmt, const StepParams &P, hipStream_t st) 
   return hipErrorInvalidValue;
 }
 
-// The ring step with its receiver mode, lookahead and load policy.
-template <int TY, int RPT, int FMT, int ACT, bool STREAM>
-hipError_t launch_x4r(const StepParams &P, hipStream_t st, int rec, dim3 grid, dim3 block) {
-  if constexpr (ACT == ACT_NONE) {
+// The ring step with its receiver mode, lookahead (256-wide tiles only) and
+// load policy.
+template <int LX, int NWV, int RPT, int FMT, int ACT, bool STREAM>
+hipError_t launch_x4r(const StepParams &P, hipStream_t st, int rec) {
+  const dim3 block(64, NWV), grid(P.ntx * P.nty * P.ntz);
+  if constexpr (ACT == ACT_NONE && LX == 64) {
     if (P.pf == 2 && rec == REC_NONE) {
-      k_step_x4r<TY, RPT, FMT, ACT, REC_NONE, 2, STREAM><<<grid, block, 0, st>>>(P);
+      k_step_x4r<LX, NWV, RPT, FMT, ACT, REC_NONE, 2, STREAM><<<grid, block, 0, st>>>(P);
       return hipGetLastError();
     }
     if (P.pf == 2 && rec == REC_INJECT) {
-      k_step_x4r<TY, RPT, FMT, ACT, REC_INJECT, 2, STREAM><<<grid, block, 0, st>>>(P);
+      k_step_x4r<LX, NWV, RPT, FMT, ACT, REC_INJECT, 2, STREAM><<<grid, block, 0, st>>>(P);
       return hipGetLastError();
     }
   }
   if (rec == REC_NONE) {
-    k_step_x4r<TY, RPT, FMT, ACT, REC_NONE, 1, STREAM><<<grid, block, 0, st>>>(P);
+    k_step_x4r<LX, NWV, RPT, FMT, ACT, REC_NONE, 1, STREAM><<<grid, block, 0, st>>>(P);
   } else if (rec == REC_INJECT) {
     if constexpr (ACT != ACT_BORN)
-      k_step_x4r<TY, RPT, FMT, ACT, REC_INJECT, 1, STREAM><<<grid, block, 0, st>>>(P);
+      k_step_x4r<LX, NWV, RPT, FMT, ACT, REC_INJECT, 1, STREAM><<<grid, block, 0, st>>>(P);
     else
       return hipErrorInvalidValue;
   } else if (rec == REC_EXTRACT) {
     if constexpr (ACT != ACT_IMG)
-      k_step_x4r<TY, RPT, FMT, ACT, REC_EXTRACT, 1, STREAM><<<grid, block, 0, st>>>(P);
+      k_step_x4r<LX, NWV, RPT, FMT, ACT, REC_EXTRACT, 1, STREAM><<<grid, block, 0, st>>>(P);
     else
       return hipErrorInvalidValue;
   } else {
@@ -1956,40 +2153,42 @@ hipError_t launch_x4r(const StepParams &P, hipStream_t st, int rec, dim3 grid, d
   return hipGetLastError();
 }
 
-template <bool RING, int TY, int RPT, int FMT, int ACT>
-hipError_t launch_x4_kernel(const StepParams &P, hipStream_t st, int rec) {
-  const dim3 block(64, TY / RPT);
-  const dim3 grid(P.ntx * P.nty * P.ntz);
-  if constexpr (RING) {
-    return P.stream ? launch_x4r<TY, RPT, FMT, ACT, true>(P, st, rec, grid, block)
-                    : launch_x4r<TY, RPT, FMT, ACT, false>(P, st, rec, grid, block);
-  } else {
-    if (rec != REC_NONE) return hipErrorInvalidValue;
-    k_step_x4<TY, RPT, FMT, ACT><<<grid, block, 0, st>>>(P);
-  }
-  return hipGetLastError();
-}
-
-template <bool RING, int TY, int RPT, int ACT>
-hipError_t launch_x4_a(int fmt, const StepParams &P, hipStream_t st, int rec) {
-  switch (fmt) {
-    case FMT_F32: return launch_x4_kernel<RING, TY, RPT, FMT_F32, ACT>(P, st, rec);
-    case FMT_BF16: return launch_x4_kernel<RING, TY, RPT, FMT_BF16, ACT>(P, st, rec);
-    case FMT_F16: return launch_x4_kernel<RING, TY, RPT, FMT_F16, ACT>(P, st, rec);
+// act and fmt as one of the step's seven (action, format) pairs.
+template <template <int, int> class L, class... A>
+hipError_t by_action(int act, int fmt, A &&...a) {
+  switch (act * 4 + fmt) {
+    case ACT_NONE * 4 + FMT_NONE: return L<FMT_NONE, ACT_NONE>::run(a...);
+    case ACT_IMG * 4 + FMT_F32: return L<FMT_F32, ACT_IMG>::run(a...);
+    case ACT_IMG * 4 + FMT_BF16: return L<FMT_BF16, ACT_IMG>::run(a...);
+    case ACT_IMG * 4 + FMT_F16: return L<FMT_F16, ACT_IMG>::run(a...);
+    case ACT_BORN * 4 + FMT_F32: return L<FMT_F32, ACT_BORN>::run(a...);
+    case ACT_BORN * 4 + FMT_BF16: return L<FMT_BF16, ACT_BORN>::run(a...);
+    case ACT_BORN * 4 + FMT_F16: return L<FMT_F16, ACT_BORN>::run(a...);
     default: return hipErrorInvalidValue;
   }
 }
 
-template <bool RING, int TY, int RPT>
-hipError_t launch_x4_t(int act, int fmt, const StepParams &P, hipStream_t st, int rec) {
-  if (act == ACT_NONE) {
-    if (fmt != FMT_NONE) return hipErrorInvalidValue;
-    return launch_x4_kernel<RING, TY, RPT, FMT_NONE, ACT_NONE>(P, st, rec);
-  }
-  if (act == ACT_BORN) return launch_x4_a<RING, TY, RPT, ACT_BORN>(fmt, P, st, rec);
-  if (act == ACT_IMG) return launch_x4_a<RING, TY, RPT, ACT_IMG>(fmt, P, st, rec);
-  return hipErrorInvalidValue;
-}
+template <int LX, int NWV, int RPT>
+struct RingShapeOf {
+  template <int FMT, int ACT>
+  struct L {
+    static hipError_t run(const StepParams &P, hipStream_t st, int rec) {
+      return P.stream ? launch_x4r<LX, NWV, RPT, FMT, ACT, true>(P, st, rec)
+                      : launch_x4r<LX, NWV, RPT, FMT, ACT, false>(P, st, rec);
+    }
+  };
+};
+
+template <int TY, int RPT>
+struct FlatShapeOf {
+  template <int FMT, int ACT>
+  struct L {
+    static hipError_t run(const StepParams &P, hipStream_t st) {
+      k_step_x4<TY, RPT, FMT, ACT><<<dim3(P.ntx * P.nty * P.ntz), dim3(64, TY / RPT), 0, st>>>(P);
+      return hipGetLastError();
+    }
+  };
+};
 
 template <int FORM, int TY, int RPT, int ACT, int REC = REC_NONE>
 hipError_t launch_step_a(int fmt, const StepParams &P, hipStream_t st) {
@@ -2061,11 +2260,117 @@ hipError_t launch_step_x4(int act, int fmt, StepParams P, int ty_tile, bool ring
   // 8-row tiles with one row per thread, or 16-row tiles with two (ty_tile
   // 16 or 32); four cells per lane leave no registers for taller tiles.
   if (ring) {
-    if (ty_tile == 8) return launch_x4_t<true, 8, 1>(act, fmt, P, st, rec);
-    return launch_x4_t<true, 16, 2>(act, fmt, P, st, rec);
+    if (ty_tile == 8) return by_action<RingShapeOf<64, 8, 1>::L>(act, fmt, P, st, rec);
+    return by_action<RingShapeOf<64, 8, 2>::L>(act, fmt, P, st, rec);
   }
-  if (ty_tile == 8) return launch_x4_t<false, 8, 1>(act, fmt, P, st, rec);
-  return launch_x4_t<false, 16, 2>(act, fmt, P, st, rec);
+  if (rec != REC_NONE) return hipErrorInvalidValue;
+  if (ty_tile == 8) return by_action<FlatShapeOf<8, 1>::L>(act, fmt, P, st);
+  return by_action<FlatShapeOf<16, 2>::L>(act, fmt, P, st);
+}
+
+// z chunks of a ring step whose workgroups run `capacity` at a time: a round
+// of workgroups takes a chunk's slices plus about nine for its prologue, so
+// the chunk count that fills one to four rounds with the fewest slices wins.
+// Returns the slices all rounds take together.
+static long plan_rounds(StepParams &P, int ty, int xw, int capacity) {
+  P.ntx = (P.n1 + xw - 1) / xw;
+  P.nty = (P.n2 + ty - 1) / ty;
+  const int nz = P.n3 - 8;
+  const long tiles = (long)P.ntx * P.nty;
+  long best = -1;
+  for (int r = 1; r <= 4; ++r) {
+    const long want = std::max(1L, std::min((long)nz, capacity * (long)r / tiles));
+    const int zc = (int)((nz + want - 1) / want), ntz = (nz + zc - 1) / zc;
+    const long rounds = (tiles * ntz + capacity - 1) / capacity;
+    const long cost = rounds * (zc + 9);
+    if (best < 0 || cost < best) {
+      best = cost;
+      P.zc = zc;
+      P.ntz = ntz;
+    }
+  }
+  return best;
+}
+
+hipError_t launch_step_auto4(int act, int fmt, const StepParams &P, int ncu, hipStream_t st,
+                             int rec) {
+  if (P.nw > kWMax || P.n3 < 9 || P.n2 < 9 || P.n1 < 12 || (P.n1 & 3)) return hipErrorInvalidValue;
+  if (rec != REC_NONE && (!P.rmap || !P.rtr || P.nrec <= 0 || P.rz < 4 || P.rz >= P.n3 - 4))
+    return hipErrorInvalidValue;
+  // Tile shapes, and what a slice of one round of workgroups costs next to a
+  // slice of 256 x 8 tiles (plain steps at 256^3 to 512^3):
+  //   256 x 8   1.00  one 8-wave workgroup per CU
+  //   256 x 16  1.66  the same with two rows per thread, plain steps only (in
+  //                   the others its second row costs twice: FP16 imaging at
+  //                   512^3 630 us against 590 us in 256 x 8)
+  //   128 x 24  1.33  one 12-wave workgroup per CU
+  //   64 x 16   1.38  three 4-wave workgroups per CU
+  // The shape whose rounds cost least is taken: where 256-wide tiles fit the
+  // rows they win (256^3: plain 38.6 us against 39.9 us in 128 x 24 and 42.0
+  // us in the 256 x 16 tiles used there before; 512^3 256 x 16), elsewhere the
+  // narrow ones: 384^3 149 us in 128 x 24 (287-323 us in 256 x 16 with a
+  // second round of 32 workgroups before), 320^3 101 us and 288 x 240 x 208 36
+  // us in 64 x 16 (120 and 46 us in the two-cell kernel before).
+  // (imaging and Born steps move more per slice, which the narrow shapes' finer
+  // halos cost more: FP32 imaging at 512^3 640 us in 256 x 8, 750 us in 64 x 16)
+  const bool plain = act == ACT_NONE;
+  StepParams Q[4] = {P, P, P, P};
+  const double cost[4] = {1.00 * plan_rounds(Q[0], 8, 256, ncu),
+                          plain ? 1.66 * plan_rounds(Q[1], 16, 256, ncu) : 1e30,
+                          (plain ? 1.33 : 1.45) * plan_rounds(Q[2], 24, 128, ncu),
+                          (plain ? 1.38 : 1.60) * plan_rounds(Q[3], 16, 64, 3 * ncu)};
+  switch (std::min_element(cost, cost + 4) - cost) {
+    case 0: return by_action<RingShapeOf<64, 8, 1>::L>(act, fmt, Q[0], st, rec);
+    case 1: return by_action<RingShapeOf<64, 8, 2>::L>(act, fmt, Q[1], st, rec);
+    case 2: return by_action<RingShapeOf<32, 12, 1>::L>(act, fmt, Q[2], st, rec);
+    default: return by_action<RingShapeOf<16, 4, 1>::L>(act, fmt, Q[3], st, rec);
+  }
+}
+
+template <int ZC, int FMT, int ACT, int REC>
+hipError_t launch_direct_k(const StepParams &P, hipStream_t st) {
+  const dim3 grid(P.ntx * P.ntz);
+  if (P.n1 % 4 == 0) k_step_direct<ZC, FMT, ACT, REC, true><<<grid, 256, 0, st>>>(P);
+  else k_step_direct<ZC, FMT, ACT, REC, false><<<grid, 256, 0, st>>>(P);
+  return hipGetLastError();
+}
+
+template <int ZC, int FMT, int ACT>
+hipError_t launch_direct_r(const StepParams &P, hipStream_t st, int rec) {
+  if (rec == REC_NONE) return launch_direct_k<ZC, FMT, ACT, REC_NONE>(P, st);
+  if constexpr (ACT != ACT_BORN)
+    if (rec == REC_INJECT) return launch_direct_k<ZC, FMT, ACT, REC_INJECT>(P, st);
+  if constexpr (ACT != ACT_IMG)
+    if (rec == REC_EXTRACT) return launch_direct_k<ZC, FMT, ACT, REC_EXTRACT>(P, st);
+  return hipErrorInvalidValue;
+}
+
+template <int ZC>
+struct DirectOf {
+  template <int FMT, int ACT>
+  struct L {
+    static hipError_t run(const StepParams &P, hipStream_t st, int rec) {
+      return launch_direct_r<ZC, FMT, ACT>(P, st, rec);
+    }
+  };
+};
+
+template <int ZC>
+hipError_t launch_direct_t(int act, int fmt, StepParams P, hipStream_t st, int rec) {
+  const long groups = (long)((P.n1 - 5) / 4) * (P.n2 - 8);
+  P.ntx = (int)((groups + 255) / 256);
+  P.ntz = (P.n3 - 8 + ZC - 1) / ZC;
+  if ((long)P.ntx * P.ntz > 0x7fffffffL) return hipErrorInvalidValue;
+  return by_action<DirectOf<ZC>::template L>(act, fmt, P, st, rec);
+}
+
+hipError_t launch_step_direct(int act, int fmt, const StepParams &P, int zc, hipStream_t st,
+                              int rec) {
+  if (P.nw > kWMax || P.n3 < 9 || P.n2 < 9 || P.n1 < 9) return hipErrorInvalidValue;
+  if (rec != REC_NONE && (!P.rmap || !P.rtr || P.nrec <= 0 || P.rz < 4 || P.rz >= P.n3 - 4))
+    return hipErrorInvalidValue;
+  if (zc == 1) return launch_direct_t<1>(act, fmt, P, st, rec);
+  return launch_direct_t<2>(act, fmt, P, st, rec);
 }
 
 template <int REC>
