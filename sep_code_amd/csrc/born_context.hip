@@ -29,11 +29,71 @@ namespace brtm {
 static thread_local std::string g_err;
 void set_error(const std::string &msg) { g_err = msg; }
 
+std::shared_mutex g_capturing;
+
+namespace {
+std::mutex g_live_mu;
+std::vector<brtm_ctx *> g_live;  // contexts whose pools may hold memory
+
+void flush_pools() {
+  std::lock_guard<std::mutex> lock(g_live_mu);
+  for (brtm_ctx *c : g_live) c->pool.flush();
+}
+}  // namespace
+
+bool VecPool::take(size_t n, DevBuf *out) {
+  std::lock_guard<std::mutex> lock(mu_);
+  size_t best = free_.size();
+  for (size_t i = 0; i < free_.size(); ++i)
+    if (free_[i].bytes >= n && free_[i].bytes - n <= n / 8 &&
+        (best == free_.size() || free_[i].bytes < free_[best].bytes))
+      best = i;
+  if (best == free_.size()) return false;
+  bytes_ -= free_[best].bytes;
+  *out = std::move(free_[best]);
+  free_.erase(free_.begin() + best);
+  return true;
+}
+
+void VecPool::put(DevBuf &&b) {
+  if (!b.ptr) return;
+  DevBuf gone;  // freed outside the lock
+  std::unique_lock<std::shared_mutex> quiet(g_capturing, std::try_to_lock);
+  if (!quiet || hipDeviceSynchronize() != hipSuccess) {
+    gone = std::move(b);
+    return;
+  }
+  std::lock_guard<std::mutex> lock(mu_);
+  if (bytes_ + b.bytes > cap) {
+    gone = std::move(b);
+    return;
+  }
+  bytes_ += b.bytes;
+  free_.push_back(std::move(b));
+}
+
+void VecPool::flush() {
+  std::vector<DevBuf> gone;
+  std::lock_guard<std::mutex> lock(mu_);
+  gone.swap(free_);
+  bytes_ = 0;
+}
+
+size_t VecPool::held() {
+  std::lock_guard<std::mutex> lock(mu_);
+  return bytes_;
+}
+
 int DevBuf::alloc(size_t n) {
   if (ptr && bytes >= n) return BRTM_OK;
   release();
   if (n == 0) return BRTM_OK;
   hipError_t e = hipMalloc(&ptr, n);
+  if (e == hipErrorOutOfMemory) {  // what the pools keep is given back first
+    (void)hipGetLastError();
+    flush_pools();
+    e = hipMalloc(&ptr, n);
+  }
   if (e != hipSuccess) {
     ptr = nullptr;
     (void)hipGetLastError();
@@ -383,10 +443,12 @@ static int run_loop(brtm_ctx *c, F &&body) {
     BRTM_HIP(hipStreamSynchronize(c->stream));
     free_graphs(c);
   }
+  std::shared_lock<std::shared_mutex> capturing(g_capturing);
   BRTM_HIP(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
   const int rc = body();
   hipGraph_t g = nullptr;
   const hipError_t e = hipStreamEndCapture(c->stream, &g);
+  capturing.unlock();
   if (rc != BRTM_OK || e != hipSuccess) {
     if (g) (void)hipGraphDestroy(g);
     if (rc != BRTM_OK) return rc;
@@ -820,6 +882,12 @@ int brtm_create(int device, brtm_ctx **out) {
     ctx_release(c);
     return rc;
   }
+  size_t mfree = 0, mtotal = 0;
+  if (hipMemGetInfo(&mfree, &mtotal) == hipSuccess) c->pool.cap = mtotal / 16;
+  {
+    std::lock_guard<std::mutex> lock(g_live_mu);
+    g_live.push_back(c);
+  }
   *out = c;
   return BRTM_OK;
 }
@@ -829,11 +897,17 @@ int brtm_destroy(brtm_ctx *c) {
   BRTM_REQUIRE(!c->destroyed, BRTM_ESTATE, "brtm_destroy called twice on one context");
   (void)hipSetDevice(c->device);
   if (c->stream) (void)hipStreamSynchronize(c->stream);
+  {
+    std::lock_guard<std::mutex> lock(g_live_mu);
+    g_live.erase(std::remove(g_live.begin(), g_live.end(), c), g_live.end());
+  }
   // The device memory goes now; objects still alive on the context keep
   // only its host record (stream, events) until they are destroyed.
+  c->pool.cap = 0;
+  c->pool.flush();
   c->stores.clear();
   for (DevBuf *b : {&c->d_wtab, &c->V, &c->fa, &c->fb, &c->fc, &c->fd, &c->img, &c->mdl,
-                    &c->seg, &c->mvw, &c->rscale, &c->partials, &c->dotv, &c->slocs, &c->strc,
+                    &c->seg, &c->mvw, &c->rscale, &c->partials, &c->dotv, &c->gram, &c->slocs, &c->strc,
                     &c->rlocs, &c->rmap, &c->smap, &c->traces})
     b->release();
   c->have_space = c->have_vel = false;
@@ -853,6 +927,7 @@ int brtm_create_space(brtm_ctx *c, float d1, float d2, float d3, float bc_a, flo
                "sponge parameters out of range (0 <= bc_a <= 256, bc_b >= 0)");
   BRTM_HIP(hipSetDevice(c->device));
   BRTM_HIP(hipStreamSynchronize(c->stream));  // buffers below are reallocated
+  c->pool.flush();                            // a new grid has other vectors
   c->n1 = n1;
   c->n2 = n2;
   c->n3 = n3;
@@ -1366,10 +1441,11 @@ int brtm_device_bytes(brtm_ctx *c, double *bytes) {
   BRTM_REQUIRE(c && bytes, BRTM_EINVAL, "NULL argument");
   double b = 0;
   for (DevBuf *x : {&c->d_wtab, &c->V, &c->fa, &c->fb, &c->fc, &c->fd, &c->img, &c->mdl,
-                    &c->seg, &c->partials, &c->dotv, &c->slocs, &c->strc, &c->rlocs, &c->rmap, &c->smap,
+                    &c->seg, &c->partials, &c->dotv, &c->gram, &c->slocs, &c->strc, &c->rlocs, &c->rmap, &c->smap,
                     &c->traces, &c->mvw, &c->rscale})
     b += (double)x->bytes;
   for (auto &s : c->stores) b += (double)s.data.bytes + (double)s.scale.bytes;
+  b += (double)c->pool.held();
   *bytes = b;
   return BRTM_OK;
 }

@@ -3,6 +3,8 @@
 #include <hip/hip_runtime.h>
 
 #include <atomic>
+#include <mutex>
+#include <shared_mutex>
 #include <string>
 #include <vector>
 
@@ -48,6 +50,32 @@ struct DevBuf {
   void release();
   template <class T> T *as() const { return static_cast<T *>(ptr); }
 };
+
+// Buffers of destroyed vectors, kept for the next ones of about their size:
+// allocating and freeing the vectors of a solver (22 of them, 2.3 GB, at 16 M
+// samples and history 8) took 9 to 47 ms per solve, several times the
+// solve's kernels.  Holds at most a sixteenth of the device's memory; given
+// back when the context is destroyed, gets a new grid, or any allocation of
+// the library finds no memory.  A context's vectors are used on its stream,
+// so a buffer taken again is ordered after its last use there, and put()
+// waits for the device first, as freeing it would have.
+class VecPool {
+ public:
+  bool take(size_t n, DevBuf *out);
+  void put(DevBuf &&b);  // frees b when it does not fit
+  void flush();
+  size_t held();
+  size_t cap = 0;
+
+ private:
+  std::mutex mu_;
+  std::vector<DevBuf> free_;
+  size_t bytes_ = 0;
+};
+
+// Held shared while a propagation loop is being captured: a device-wide wait
+// is not allowed then.
+extern std::shared_mutex g_capturing;
 
 // One shot's source wavefield.
 struct Store {
@@ -111,6 +139,8 @@ struct brtm_ctx {
   bool born_direct_lv = false;
   int seg_slots = 0;
   brtm::DevBuf partials, dotv;
+  brtm::DevBuf gram;  // scratch of the solvers' one-pass products
+  brtm::VecPool pool;
   // this device's copy of the allocation-free entry point's scratch array
   // (its device address, from hipGetSymbolAddress at brtm_create)
   double *noalloc_scratch = nullptr;
@@ -216,4 +246,7 @@ namespace brtm {
 int check_vec(const brtm_vec *v, long n, const char *what);
 // The context a Born operator propagates on.
 brtm_ctx *op_context(const brtm_op *op);
+// brtm_vec_create; zero = false leaves the contents undefined (for vectors
+// that are written whole before they are read).
+int vec_create(brtm_ctx *ctx, long n, bool zero, brtm_vec **out);
 }  // namespace brtm

@@ -145,6 +145,18 @@ hipError_t launch_square_accumulate(int fmt, const void *src, const float *sscal
 constexpr int kDotBlocks = 1024;
 hipError_t launch_dot(const float *a, const float *b, long n, double *partials,
                       double *out, hipStream_t st);
+// The products a CG step needs, in one pass: the pairs v[a] . v[b] (b <= a,
+// row by row), then v[a] . r, K <= kGramMax vectors of n floats.  The results
+// are the doubles at scratch + kGramProducts * kGramBlocks.
+constexpr int kGramMax = 9, kGramProducts = kGramMax * (kGramMax + 1) / 2 + kGramMax;
+constexpr int kGramBlocks = 768;
+constexpr size_t kGramScratch = (size_t)kGramProducts * (kGramBlocks + 1);  // doubles
+hipError_t launch_gram(int K, const float *const *v, const float *r, long n, double *scratch,
+                       hipStream_t st);
+// s = sum_k c[k] x[k], acc += s (s may be one of the x); norm: acc . acc and
+// acc . e (0 without e) of the new acc, at the same place as above.
+hipError_t launch_combine(int nb, const float *const *x, const double *c, float *s, float *acc,
+                          const float *e, long n, bool norm, double *scratch, hipStream_t st);
 hipError_t launch_axpby(float *y, const float *x, double a, double b, long n,
                         hipStream_t st);  // y = a*y + b*x
 hipError_t launch_mul(float *y, const float *x, long n, hipStream_t st);  // y *= x

@@ -1856,45 +1856,204 @@ __global__ void k_square_acc(int fmt, const void *src, const float *sscale, floa
 // FP64 dot product: fixed grid, per-block partials, single-block finish, so
 // the result is deterministic run to run.
 // ---------------------------------------------------------------------------
-__global__ void k_dot_partial(const float *__restrict__ a, const float *__restrict__ b, long n,
-                              double *partials) {
-  double acc = 0.0;
-  for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (long)gridDim.x * blockDim.x)
-    acc += (double)a[i] * (double)b[i];
-  __shared__ double red[256];
-  red[threadIdx.x] = acc;
-  __syncthreads();
-  for (int o = blockDim.x / 2; o > 0; o >>= 1) {
-    if ((int)threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) partials[blockIdx.x] = red[0];
+__device__ __forceinline__ double wave_sum(double v) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+  return v;
 }
 
-__global__ void k_dot_final(const double *partials, int np, double *out) {
-  __shared__ double red[256];
-  double acc = 0.0;
-  for (int i = threadIdx.x; i < np; i += blockDim.x) acc += partials[i];
-  red[threadIdx.x] = acc;
-  __syncthreads();
-  for (int o = blockDim.x / 2; o > 0; o >>= 1) {
-    if ((int)threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
-    __syncthreads();
+// Products of up to kGramMax + 1 vectors in one pass over them: all pairs of
+// v[0..K) and their products with v[K], in FP64.  A flexible-CG step with
+// eight stored steps needs 54 products of ten vectors; one by one that read
+// every vector eleven times with a host wait each (3.3 ms of dots an iteration
+// at 33 M elements), here each is read once: 16 bytes per lane and vector in
+// flight, 54 FP64 sums per lane.  Bound by HBM.
+struct GramParams {
+  const float *v[kGramMax + 1];
+  long n;
+  double *part;  // [K (K + 1) / 2 + K][gridDim.x]
+};
+
+template <int K, bool VEC>
+__global__ void __launch_bounds__(256) k_gram(const GramParams P) {
+  constexpr int NP = K * (K + 1) / 2 + K;
+  double acc[NP];
+#pragma unroll
+  for (int p = 0; p < NP; ++p) acc[p] = 0.0;
+  auto add = [&](const float *x) {
+    int p = 0;
+    double d[K + 1];
+#pragma unroll
+    for (int k = 0; k <= K; ++k) d[k] = (double)x[k];
+#pragma unroll
+    for (int a = 0; a < K; ++a)
+#pragma unroll
+      for (int b = 0; b <= a; ++b) acc[p] = fma(d[a], d[b], acc[p]), ++p;
+#pragma unroll
+    for (int a = 0; a < K; ++a) acc[p] = fma(d[a], d[K], acc[p]), ++p;
+  };
+  const long i0 = (long)blockIdx.x * 256 + threadIdx.x, step = (long)gridDim.x * 256;
+  if constexpr (VEC) {
+    for (long i = i0; i < (P.n >> 2); i += step) {
+      f32x4 x[K + 1];
+#pragma unroll
+      for (int k = 0; k <= K; ++k) x[k] = reinterpret_cast<const f32x4 *>(P.v[k])[i];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        float y[K + 1];
+#pragma unroll
+        for (int k = 0; k <= K; ++k) y[k] = x[k][j];
+        add(y);
+      }
+    }
   }
-  if (threadIdx.x == 0) *out = red[0];
+  for (long i = (VEC ? P.n & ~3L : 0L) + i0; i < P.n; i += step) {
+    float y[K + 1];
+#pragma unroll
+    for (int k = 0; k <= K; ++k) y[k] = P.v[k][i];
+    add(y);
+  }
+  __shared__ double red[4][NP];
+#pragma unroll
+  for (int p = 0; p < NP; ++p) {
+    const double v = wave_sum(acc[p]);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6][p] = v;
+  }
+  __syncthreads();
+  for (int p = threadIdx.x; p < NP; p += 256)
+    P.part[(long)p * gridDim.x + blockIdx.x] = (red[0][p] + red[1][p]) + (red[2][p] + red[3][p]);
 }
 
-__global__ void k_axpby(float *y, const float *__restrict__ x, double a, double b, long n) {
-  for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (long)gridDim.x * blockDim.x)
+// out[p] = sum of the np partials of row p (one workgroup per row).
+__global__ void __launch_bounds__(256) k_rows_final(const double *part, int np, double *out) {
+  double acc = 0.0;
+  for (int i = threadIdx.x; i < np; i += 256) acc += part[(long)blockIdx.x * np + i];
+  __shared__ double red[4];
+  acc = wave_sum(acc);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
+  __syncthreads();
+  if (threadIdx.x == 0) out[blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
+}
+
+// A CG step: s = sum_k c[k] x[k] (in FP64, rounded once), then acc += s; with
+// NORM the products acc . acc and (e not null) acc . e of the new acc as well.
+// One pass instead of a copy, a scaling, an axpy per stored step, an add and
+// two dots.
+struct CombineParams {
+  const float *x[kGramMax];
+  double c[kGramMax];
+  float *s, *acc;
+  const float *e;
+  long n;
+  double *part;  // [2][gridDim.x]
+};
+
+template <int NB, bool VEC, bool NORM>
+__global__ void __launch_bounds__(256) k_combine(const CombineParams P) {
+  double rr = 0.0, re = 0.0;
+  const long i0 = (long)blockIdx.x * 256 + threadIdx.x, step = (long)gridDim.x * 256;
+  if constexpr (VEC) {
+    for (long i = i0; i < (P.n >> 2); i += step) {
+      f32x4 x[NB], a = {0.f, 0.f, 0.f, 0.f}, e = a, s;
+#pragma unroll
+      for (int k = 0; k < NB; ++k) x[k] = reinterpret_cast<const f32x4 *>(P.x[k])[i];
+      if (P.acc) a = reinterpret_cast<const f32x4 *>(P.acc)[i];
+      if (NORM && P.e) e = reinterpret_cast<const f32x4 *>(P.e)[i];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        double v = 0.0;
+#pragma unroll
+        for (int k = 0; k < NB; ++k) v = fma(P.c[k], (double)x[k][j], v);
+        s[j] = (float)v;
+        a[j] += s[j];
+        if constexpr (NORM) {
+          rr = fma((double)a[j], (double)a[j], rr);
+          re = fma((double)a[j], (double)e[j], re);
+        }
+      }
+      reinterpret_cast<f32x4 *>(P.s)[i] = s;
+      if (P.acc) reinterpret_cast<f32x4 *>(P.acc)[i] = a;
+    }
+  }
+  for (long i = (VEC ? P.n & ~3L : 0L) + i0; i < P.n; i += step) {
+    double v = 0.0;
+#pragma unroll
+    for (int k = 0; k < NB; ++k) v = fma(P.c[k], (double)P.x[k][i], v);
+    const float s = (float)v;
+    const float a = (P.acc ? P.acc[i] : 0.f) + s;
+    if constexpr (NORM) {
+      rr = fma((double)a, (double)a, rr);
+      if (P.e) re = fma((double)a, (double)P.e[i], re);
+    }
+    P.s[i] = s;
+    if (P.acc) P.acc[i] = a;
+  }
+  if constexpr (NORM) {
+    __shared__ double red[2][4];
+    rr = wave_sum(rr);
+    re = wave_sum(re);
+    if ((threadIdx.x & 63) == 0) {
+      red[0][threadIdx.x >> 6] = rr;
+      red[1][threadIdx.x >> 6] = re;
+    }
+    __syncthreads();
+    if (threadIdx.x < 2)
+      P.part[(long)threadIdx.x * gridDim.x + blockIdx.x] =
+          (red[threadIdx.x][0] + red[threadIdx.x][1]) + (red[threadIdx.x][2] + red[threadIdx.x][3]);
+  }
+}
+
+// One product (brtm_vec_dot): 16-byte loads where both vectors are aligned.
+template <bool VEC>
+__global__ void __launch_bounds__(256)
+k_dot_partial(const float *__restrict__ a, const float *__restrict__ b, long n, double *partials) {
+  double acc = 0.0;
+  const long i0 = (long)blockIdx.x * 256 + threadIdx.x, step = (long)gridDim.x * 256;
+  if constexpr (VEC) {
+#pragma unroll 2
+    for (long i = i0; i < (n >> 2); i += step) {
+      const f32x4 x = reinterpret_cast<const f32x4 *>(a)[i], y = reinterpret_cast<const f32x4 *>(b)[i];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc = fma((double)x[j], (double)y[j], acc);
+    }
+  }
+  for (long i = (VEC ? n & ~3L : 0L) + i0; i < n; i += step)
+    acc = fma((double)a[i], (double)b[i], acc);
+  __shared__ double red[4];
+  acc = wave_sum(acc);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
+  __syncthreads();
+  if (threadIdx.x == 0) partials[blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
+}
+
+// y = a y + b x, y *= x: 16 bytes per lane where both are aligned.
+template <bool VEC>
+__global__ void k_axpby(float *y, const float *x, double a, double b, long n) {
+  const long i0 = (long)blockIdx.x * blockDim.x + threadIdx.x, step = (long)gridDim.x * blockDim.x;
+  if constexpr (VEC) {
+    for (long i = i0; i < (n >> 2); i += step) {
+      f32x4 u = reinterpret_cast<f32x4 *>(y)[i];
+      const f32x4 v = reinterpret_cast<const f32x4 *>(x)[i];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) u[j] = (float)(a * (double)u[j] + b * (double)v[j]);
+      reinterpret_cast<f32x4 *>(y)[i] = u;
+    }
+  }
+  for (long i = (VEC ? n & ~3L : 0L) + i0; i < n; i += step)
     y[i] = (float)(a * (double)y[i] + b * (double)x[i]);
 }
 
-__global__ void k_mul(float *y, const float *__restrict__ x, long n) {
-  for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (long)gridDim.x * blockDim.x)
-    y[i] *= x[i];
+template <bool VEC>
+__global__ void k_mul(float *y, const float *x, long n) {
+  const long i0 = (long)blockIdx.x * blockDim.x + threadIdx.x, step = (long)gridDim.x * blockDim.x;
+  if constexpr (VEC) {
+    for (long i = i0; i < (n >> 2); i += step) {
+      f32x4 u = reinterpret_cast<f32x4 *>(y)[i];
+      u *= reinterpret_cast<const f32x4 *>(x)[i];
+      reinterpret_cast<f32x4 *>(y)[i] = u;
+    }
+  }
+  for (long i = (VEC ? n & ~3L : 0L) + i0; i < n; i += step) y[i] *= x[i];
 }
 
 // Zero the cells outside the update set (the 4-cell halo every step leaves
@@ -2492,20 +2651,135 @@ hipError_t launch_square_accumulate(int fmt, const void *src, const float *sscal
   return hipGetLastError();
 }
 
+static bool aligned16(const void *p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
+
 hipError_t launch_dot(const float *a, const float *b, long n, double *partials, double *out,
                       hipStream_t st) {
-  k_dot_partial<<<kDotBlocks, 256, 0, st>>>(a, b, n, partials);
-  k_dot_final<<<1, 256, 0, st>>>(partials, kDotBlocks, out);
+  if (aligned16(a) && aligned16(b))
+    k_dot_partial<true><<<kDotBlocks, 256, 0, st>>>(a, b, n, partials);
+  else
+    k_dot_partial<false><<<kDotBlocks, 256, 0, st>>>(a, b, n, partials);
+  k_rows_final<<<1, 256, 0, st>>>(partials, kDotBlocks, out);
+  return hipGetLastError();
+}
+
+template <int K>
+static void launch_gram_k(const GramParams &P, bool vec, hipStream_t st) {
+  if (vec) k_gram<K, true><<<kGramBlocks, 256, 0, st>>>(P);
+  else k_gram<K, false><<<kGramBlocks, 256, 0, st>>>(P);
+  k_rows_final<<<K * (K + 1) / 2 + K, 256, 0, st>>>(P.part, kGramBlocks,
+                                                    P.part + (long)kGramProducts * kGramBlocks);
+}
+
+hipError_t launch_gram(int K, const float *const *v, const float *r, long n, double *scratch,
+                       hipStream_t st) {
+  if (K < 1 || K > kGramMax) return hipErrorInvalidValue;
+  GramParams P{};
+  bool vec = aligned16(r);
+  for (int k = 0; k < K; ++k) {
+    P.v[k] = v[k];
+    vec = vec && aligned16(v[k]);
+  }
+  P.v[K] = r;
+  P.n = n;
+  P.part = scratch;
+  switch (K) {
+    case 1: launch_gram_k<1>(P, vec, st); break;
+    case 2: launch_gram_k<2>(P, vec, st); break;
+    case 3: launch_gram_k<3>(P, vec, st); break;
+    case 4: launch_gram_k<4>(P, vec, st); break;
+    case 5: launch_gram_k<5>(P, vec, st); break;
+    case 6: launch_gram_k<6>(P, vec, st); break;
+    case 7: launch_gram_k<7>(P, vec, st); break;
+    case 8: launch_gram_k<8>(P, vec, st); break;
+    default: launch_gram_k<9>(P, vec, st); break;
+  }
+  return hipGetLastError();
+}
+
+template <int NB>
+static void launch_combine_k(const CombineParams &P, bool vec, bool norm, hipStream_t st) {
+  if (norm) {
+    if (vec) k_combine<NB, true, true><<<kGramBlocks, 256, 0, st>>>(P);
+    else k_combine<NB, false, true><<<kGramBlocks, 256, 0, st>>>(P);
+    k_rows_final<<<2, 256, 0, st>>>(P.part, kGramBlocks,
+                                    P.part + (long)kGramProducts * kGramBlocks);
+  } else {
+    const int g = grid_for((P.n + 3) / 4, 256);
+    if (vec) k_combine<NB, true, false><<<g, 256, 0, st>>>(P);
+    else k_combine<NB, false, false><<<g, 256, 0, st>>>(P);
+  }
+}
+
+hipError_t launch_combine(int nb, const float *const *x, const double *c, float *s, float *acc,
+                          const float *e, long n, bool norm, double *scratch, hipStream_t st) {
+  if (nb < 1) return hipErrorInvalidValue;
+  // more vectors than one launch takes: the sum so far is one of the next
+  // launch's inputs
+  int k0 = 0;
+  bool first = true;
+  while (nb - k0 > (first ? kGramMax : kGramMax - 1)) {
+    const int m = first ? kGramMax : kGramMax - 1;
+    const float *xs[kGramMax];
+    double cs[kGramMax];
+    int t = 0;
+    if (!first) {
+      xs[t] = s;
+      cs[t++] = 1.0;
+    }
+    for (int k = 0; k < m; ++k) {
+      xs[t] = x[k0 + k];
+      cs[t++] = c[k0 + k];
+    }
+    const hipError_t er = launch_combine(t, xs, cs, s, nullptr, nullptr, n, false, scratch, st);
+    if (er != hipSuccess) return er;
+    k0 += m;
+    first = false;
+  }
+  CombineParams P{};
+  int t = 0;
+  if (!first) {
+    P.x[t] = s;
+    P.c[t++] = 1.0;
+  }
+  for (int k = k0; k < nb; ++k) {
+    P.x[t] = x[k];
+    P.c[t++] = c[k];
+  }
+  P.s = s;
+  P.acc = acc;
+  P.e = e;
+  P.n = n;
+  P.part = scratch;
+  bool vec = aligned16(s) && aligned16(acc) && aligned16(e);
+  for (int k = 0; k < t; ++k) vec = vec && aligned16(P.x[k]);
+  switch (t) {
+    case 1: launch_combine_k<1>(P, vec, norm, st); break;
+    case 2: launch_combine_k<2>(P, vec, norm, st); break;
+    case 3: launch_combine_k<3>(P, vec, norm, st); break;
+    case 4: launch_combine_k<4>(P, vec, norm, st); break;
+    case 5: launch_combine_k<5>(P, vec, norm, st); break;
+    case 6: launch_combine_k<6>(P, vec, norm, st); break;
+    case 7: launch_combine_k<7>(P, vec, norm, st); break;
+    case 8: launch_combine_k<8>(P, vec, norm, st); break;
+    default: launch_combine_k<9>(P, vec, norm, st); break;
+  }
   return hipGetLastError();
 }
 
 hipError_t launch_axpby(float *y, const float *x, double a, double b, long n, hipStream_t st) {
-  k_axpby<<<grid_for(n, 256), 256, 0, st>>>(y, x, a, b, n);
+  if (aligned16(y) && aligned16(x))
+    k_axpby<true><<<grid_for((n + 3) / 4, 256), 256, 0, st>>>(y, x, a, b, n);
+  else
+    k_axpby<false><<<grid_for(n, 256), 256, 0, st>>>(y, x, a, b, n);
   return hipGetLastError();
 }
 
 hipError_t launch_mul(float *y, const float *x, long n, hipStream_t st) {
-  k_mul<<<grid_for(n, 256), 256, 0, st>>>(y, x, n);
+  if (aligned16(y) && aligned16(x))
+    k_mul<true><<<grid_for((n + 3) / 4, 256), 256, 0, st>>>(y, x, n);
+  else
+    k_mul<false><<<grid_for(n, 256), 256, 0, st>>>(y, x, n);
   return hipGetLastError();
 }
 

@@ -42,6 +42,31 @@ int check_vec(const brtm_vec *v, long n, const char *what) {
 
 brtm_ctx *op_context(const brtm_op *op) { return op ? op->ctx : nullptr; }
 
+int vec_create(brtm_ctx *ctx, long n, bool zero, brtm_vec **out) {
+  BRTM_REQUIRE(ctx && out && n > 0, BRTM_EINVAL, "bad vector arguments");
+  BRTM_LIVE(ctx);
+  BRTM_HIP(hipSetDevice(ctx->device));
+  brtm_vec *v = new brtm_vec();
+  v->hold.reset(ctx);
+  v->ctx = ctx;
+  v->n = n;
+  const size_t bytes = sizeof(float) * (size_t)n;
+  int rc = ctx->pool.take(bytes, &v->buf) ? BRTM_OK : v->buf.alloc(bytes);
+  if (rc != BRTM_OK) {
+    delete v;
+    return rc;
+  }
+  v->ptr = v->buf.as<float>();
+  hipError_t e = zero ? hipMemsetAsync(v->p(), 0, bytes, ctx->stream) : hipSuccess;
+  if (e != hipSuccess) {
+    delete v;
+    set_error(hipGetErrorString(e));
+    return BRTM_EHIP;
+  }
+  *out = v;
+  return BRTM_OK;
+}
+
 namespace {
 
 __global__ void k_random(float *v, long n, unsigned long long seed) {
@@ -140,27 +165,7 @@ extern "C" {
 
 // ---------------------------------------------------------------- vectors
 int brtm_vec_create(brtm_ctx *ctx, long n, brtm_vec **out) {
-  BRTM_REQUIRE(ctx && out && n > 0, BRTM_EINVAL, "bad vector arguments");
-  BRTM_LIVE(ctx);
-  BRTM_HIP(hipSetDevice(ctx->device));
-  brtm_vec *v = new brtm_vec();
-  v->hold.reset(ctx);
-  v->ctx = ctx;
-  v->n = n;
-  int rc = v->buf.alloc(sizeof(float) * (size_t)n);
-  if (rc != BRTM_OK) {
-    delete v;
-    return rc;
-  }
-  v->ptr = v->buf.as<float>();
-  hipError_t e = hipMemsetAsync(v->p(), 0, sizeof(float) * (size_t)n, ctx->stream);
-  if (e != hipSuccess) {
-    delete v;
-    set_error(hipGetErrorString(e));
-    return BRTM_EHIP;
-  }
-  *out = v;
-  return BRTM_OK;
+  return vec_create(ctx, n, true, out);
 }
 
 int brtm_vec_destroy(brtm_vec *v) {
@@ -168,6 +173,7 @@ int brtm_vec_destroy(brtm_vec *v) {
   // the context's host record outlives brtm_destroy while v holds it
   (void)hipSetDevice(v->ctx->device);
   (void)hipStreamSynchronize(v->ctx->stream);
+  v->ctx->pool.put(std::move(v->buf));
   delete v;
   return BRTM_OK;
 }

@@ -55,6 +55,7 @@ struct brtm_solver {
            *ss = nullptr, *z = nullptr;
   std::vector<brtm_vec *> hs, hS;      // flexible-CG history, newest first
   int H = 0, nh = 0;
+  bool scratch_unset = false;          // (s, ss) is a history slot nothing was written to
   bool first = true;                   // cgstep::forget (Born/cgstep.cpp:16-26)
   double rr0_rr0 = 0;                  // |rr0|^2
   const brtm_vec *offset = nullptr;    // offset of the first judged solve
@@ -83,13 +84,40 @@ int grid_n(long n) {
 }
 
 // out = (add ? out : 0) + s * (w ? w . in : in); out is not read when add = 0.
-__global__ void k_scaled(float *out, const float *__restrict__ in, const float *__restrict__ w,
-                         float s, int add, long n) {
-  for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (long)gridDim.x * blockDim.x) {
+// VEC: 16 bytes per lane (all of out, in and w aligned).
+template <bool VEC>
+__global__ void k_scaled(float *out, const float *in, const float *__restrict__ w, float s, int add,
+                         long n) {
+  const long i0 = (long)blockIdx.x * blockDim.x + threadIdx.x, step = (long)gridDim.x * blockDim.x;
+  if constexpr (VEC) {
+    typedef float f32x4 __attribute__((ext_vector_type(4)));
+    for (long i = i0; i < (n >> 2); i += step) {
+      f32x4 v = reinterpret_cast<const f32x4 *>(in)[i], o = {0.f, 0.f, 0.f, 0.f};
+      if (w) v = reinterpret_cast<const f32x4 *>(w)[i] * v;
+      if (add) o = reinterpret_cast<f32x4 *>(out)[i];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float t = s * v[j];
+        o[j] = add ? o[j] + t : t;
+      }
+      reinterpret_cast<f32x4 *>(out)[i] = o;
+    }
+  }
+  for (long i = (VEC ? n & ~3L : 0L) + i0; i < n; i += step) {
     float v = s * (w ? w[i] * in[i] : in[i]);
     out[i] = add ? out[i] + v : v;
   }
+}
+
+int scaled(float *out, const float *in, const float *w, float s, int add, long n,
+           hipStream_t st) {
+  auto aligned = [](const void *p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
+  if (aligned(out) && aligned(in) && aligned(w))
+    k_scaled<true><<<grid_n((n + 3) / 4), 256, 0, st>>>(out, in, w, s, add, n);
+  else
+    k_scaled<false><<<grid_n(n), 256, 0, st>>>(out, in, w, s, add, n);
+  BRTM_HIP(hipGetLastError());
+  return BRTM_OK;
 }
 
 // tmute on [trace][nt]: one block row per trace (strided over gridDim.y),
@@ -126,11 +154,8 @@ int apply_raw(brtm_linop *A, bool adjoint, int add, const brtm_vec *in, brtm_vec
       return adjoint ? brtm_op_adjoint(A->op, add, out, in) : brtm_op_forward(A->op, add, in, out);
     case brtm_linop::IDENTITY:
     case brtm_linop::DIAG:
-      k_scaled<<<grid_n(out->n), 256, 0, st>>>(out->p(), in->p(),
-                                               A->kind == brtm_linop::DIAG ? A->w->p() : nullptr,
-                                               s, add, out->n);
-      BRTM_HIP(hipGetLastError());
-      return BRTM_OK;
+      return scaled(out->p(), in->p(), A->kind == brtm_linop::DIAG ? A->w->p() : nullptr, s, add,
+                    out->n, st);
     case brtm_linop::TMUTE: {
       dim3 grid((unsigned)((A->nt + 255) / 256), (unsigned)std::min<long>(A->ntrace, 65535));
       k_tmute<<<grid, 256, 0, st>>>(out->p(), in->p(), A->tstart.as<int>(), A->nt, A->nrx,
@@ -240,17 +265,71 @@ int check_parts(int n, brtm_linop *const *ops) {
   return BRTM_OK;
 }
 
+// n doubles from the device, waiting for the stream.
+int fetch(brtm_ctx *c, const double *src, int n, double *out) {
+  BRTM_HIP(hipMemcpyAsync(out, src, sizeof(double) * n, hipMemcpyDeviceToHost, c->stream));
+  BRTM_HIP(hipStreamSynchronize(c->stream));
+  return BRTM_OK;
+}
+
+// M = the K x K products of the range vectors B, bv their products with rr:
+// one pass over the vectors and one wait (up to kGramMax of them; beyond, a
+// dot each and still one wait).
+int gram(brtm_solver *S, int K, const brtm_vec *const *B, double *M, double *bv) {
+  brtm_ctx *c = S->ctx;
+  constexpr int kMost = BRTM_CG_MAX_HISTORY + 1;
+  double h[kMost * (kMost + 1) / 2 + kMost];
+  const int np = K * (K + 1) / 2 + K;
+  if (K <= kGramMax) {
+    const float *v[kGramMax];
+    for (int a = 0; a < K; ++a) v[a] = B[a]->p();
+    LS_TRY(c->gram.alloc(sizeof(double) * kGramScratch));
+    double *scratch = c->gram.as<double>();
+    BRTM_HIP(launch_gram(K, v, S->rr->p(), S->rr->n, scratch, c->stream));
+    LS_TRY(fetch(c, scratch + (long)kGramProducts * kGramBlocks, np, h));
+  } else {
+    LS_TRY(c->gram.alloc(sizeof(double) * std::max<size_t>(kGramScratch, kDotBlocks + np)));
+    double *part = c->gram.as<double>(), *out = part + kDotBlocks;
+    int p = 0;
+    for (int a = 0; a < K; ++a)
+      for (int b = 0; b <= a; ++b)
+        BRTM_HIP(launch_dot(B[a]->p(), B[b]->p(), S->rr->n, part, out + p++, c->stream));
+    for (int a = 0; a < K; ++a)
+      BRTM_HIP(launch_dot(B[a]->p(), S->rr->p(), S->rr->n, part, out + p++, c->stream));
+    LS_TRY(fetch(c, out, np, h));
+  }
+  int p = 0;
+  for (int a = 0; a < K; ++a)
+    for (int b = 0; b <= a; ++b) M[a * K + b] = M[b * K + a] = h[p++];
+  for (int a = 0; a < K; ++a) bv[a] = h[p++];
+  return BRTM_OK;
+}
+
+// s = sum c xd, m += s; ss = sum c xr, rr += ss; norms = rr . rr, rr . e.
+int take_step(brtm_solver *S, int nb, const float *const *xd, const float *const *xr,
+              const double *c, const brtm_vec *e, double norms[2]) {
+  brtm_ctx *ctx = S->ctx;
+  LS_TRY(ctx->gram.alloc(sizeof(double) * kGramScratch));
+  double *scratch = ctx->gram.as<double>();
+  BRTM_HIP(launch_combine(nb, xd, c, S->s->p(), S->m->p(), nullptr, S->m->n, false, scratch,
+                          ctx->stream));
+  BRTM_HIP(launch_combine(nb, xr, c, S->ss->p(), S->rr->p(), e ? e->p() : nullptr, S->rr->n, true,
+                          scratch, ctx->stream));
+  return fetch(ctx, scratch + (long)kGramProducts * kGramBlocks, 2, norms);
+}
+
 // One iteration of lin_solver::solve (Born/lin_solver.cpp:123-141):
 // g = A' rr, direction = P(g) (or g), gg = A direction, then the step.
-// Returns BRTM_OK with *stop set on a breakdown.
-int iterate(brtm_solver *S, const brtm_cg_params *prm, brtm_cg_stats *st, double *alfa_out,
-            double *beta_out, bool *stop) {
+// Returns BRTM_OK with *stop set on a breakdown; norms receives rr . rr and
+// (e given) rr . e after the step.
+int iterate(brtm_solver *S, const brtm_cg_params *prm, brtm_cg_stats *st, const brtm_vec *e,
+            double norms[2], double *alfa_out, double *beta_out, bool *stop) {
   const double small = 1e-20;
   brtm_linop *A = S->oper;
   LS_TRY(apply(A, true, 0, S->rr, S->g));
   brtm_vec *dir = S->g;
   if (prm->precond) {
-    if (!S->z) LS_TRY(brtm_vec_create(S->ctx, A->nd, &S->z));
+    if (!S->z) LS_TRY(vec_create(S->ctx, A->nd, true, &S->z));
     if (prm->precond(prm->precond_user, S->g, S->z) != 0) {
       set_error("preconditioner failed");
       return BRTM_ESTATE;
@@ -270,33 +349,28 @@ int iterate(brtm_solver *S, const brtm_cg_params *prm, brtm_cg_stats *st, double
     for (int i = 0; i < S->nh; ++i) B[i + 1] = S->hS[i];
     double M[(BRTM_CG_MAX_HISTORY + 1) * (BRTM_CG_MAX_HISTORY + 1)], bv[BRTM_CG_MAX_HISTORY + 1],
         x[BRTM_CG_MAX_HISTORY + 1];
-    for (int a = 0; a < K; ++a) {
-      for (int b = 0; b <= a; ++b) {
-        LS_TRY(brtm_vec_dot(B[a], B[b], &M[a * K + b]));
-        M[b * K + a] = M[a * K + b];
-      }
-      LS_TRY(brtm_vec_dot(B[a], S->rr, &bv[a]));
-      bv[a] = -bv[a];
-    }
+    LS_TRY(gram(S, K, B, M, bv));
+    for (int a = 0; a < K; ++a) bv[a] = -bv[a];
     if (std::fabs(M[0]) < small || gram_solve(K, M, bv, x) == 0) {
       *stop = true;
       return BRTM_OK;
     }
-    // new step into the scratch pair (s, ss)
-    LS_TRY(brtm_vec_copy(S->s, dir));
-    LS_TRY(brtm_vec_scale(S->s, x[0]));
-    LS_TRY(brtm_vec_copy(S->ss, S->gg));
-    LS_TRY(brtm_vec_scale(S->ss, x[0]));
+    // new step into the scratch pair (s, ss); a dropped vector is not read
+    const float *xd[BRTM_CG_MAX_HISTORY + 1] = {dir->p()}, *xr[BRTM_CG_MAX_HISTORY + 1] = {
+        S->gg->p()};
+    double c[BRTM_CG_MAX_HISTORY + 1] = {x[0]};
+    int nb = 1;
     for (int i = 0; i < S->nh; ++i) {
       if (x[i + 1] == 0) continue;
-      LS_TRY(brtm_vec_scale_add(S->s, 1.0, S->hs[i], x[i + 1]));
-      LS_TRY(brtm_vec_scale_add(S->ss, 1.0, S->hS[i], x[i + 1]));
+      xd[nb] = S->hs[i]->p();
+      xr[nb] = S->hS[i]->p();
+      c[nb++] = x[i + 1];
     }
-    LS_TRY(brtm_vec_add(S->m, S->s));
-    LS_TRY(brtm_vec_add(S->rr, S->ss));
+    LS_TRY(take_step(S, nb, xd, xr, c, e, norms));
     // push: the new step becomes hs[0]; the dropped (or unused) slot
     // becomes the next scratch pair
     const int slot = S->nh < S->H ? S->nh : S->H - 1;
+    S->scratch_unset = S->nh < S->H;
     std::swap(S->s, S->hs[slot]);
     std::swap(S->ss, S->hS[slot]);
     std::rotate(S->hs.begin(), S->hs.begin() + slot, S->hs.begin() + slot + 1);
@@ -306,37 +380,31 @@ int iterate(brtm_solver *S, const brtm_cg_params *prm, brtm_cg_stats *st, double
     beta = S->nh > 1 ? x[1] : 0.0;
   } else {
     // cgstep::step_it (Born/cgstep.cpp:14-58)
-    double gg_gg = 0;
-    LS_TRY(brtm_vec_dot(S->gg, S->gg, &gg_gg));
+    const brtm_vec *B[2] = {S->gg, S->ss};
+    double M[4], bv[2];
+    LS_TRY(gram(S, S->first ? 1 : 2, B, M, bv));
+    const double gg_gg = M[0];
     if (S->first) {
       if (std::fabs(gg_gg) < small) {
         *stop = true;
         return BRTM_OK;
       }
-      double gg_rr = 0;
-      LS_TRY(brtm_vec_dot(S->gg, S->rr, &gg_rr));
       beta = 0;
-      alfa = -gg_rr / gg_gg;
+      alfa = -bv[0] / gg_gg;
     } else {
-      double ss_ss = 0, gg_ss = 0, gg_rr = 0, ss_rr = 0;
-      LS_TRY(brtm_vec_dot(S->ss, S->ss, &ss_ss));
-      LS_TRY(brtm_vec_dot(S->gg, S->ss, &gg_ss));
-      LS_TRY(brtm_vec_dot(S->gg, S->rr, &gg_rr));
-      LS_TRY(brtm_vec_dot(S->ss, S->rr, &ss_rr));
+      const double ss_ss = M[3], gg_ss = M[1], gg_rr = -bv[0], ss_rr = -bv[1];
       if (std::fabs(gg_gg) < small || std::fabs(ss_ss) < small) {
         *stop = true;
         return BRTM_OK;
       }
       const double determ = gg_gg * ss_ss * (1.0 - gg_ss / gg_gg * gg_ss / ss_ss);
-      gg_rr = -gg_rr;
-      ss_rr = -ss_rr;
       alfa = (ss_ss * gg_rr - gg_ss * ss_rr) / determ;
       beta = (-gg_ss * gg_rr + gg_gg * ss_rr) / determ;
     }
-    LS_TRY(brtm_vec_scale_add(S->s, beta, dir, alfa));      // s  = beta s  + alfa g
-    LS_TRY(brtm_vec_scale_add(S->ss, beta, S->gg, alfa));   // ss = beta ss + alfa gg
-    LS_TRY(brtm_vec_add(S->m, S->s));                       // m += s
-    LS_TRY(brtm_vec_add(S->rr, S->ss));                     // rr += ss
+    // s = beta s + alfa g, ss = beta ss + alfa gg; m += s, rr += ss
+    const float *xd[2] = {dir->p(), S->s->p()}, *xr[2] = {S->gg->p(), S->ss->p()};
+    const double c[2] = {alfa, beta};
+    LS_TRY(take_step(S, S->first ? 1 : 2, xd, xr, c, e, norms));
   }
   S->first = false;
   *alfa_out = alfa;
@@ -348,6 +416,11 @@ int iterate(brtm_solver *S, const brtm_cg_params *prm, brtm_cg_stats *st, double
 int set_history(brtm_solver *S, int history) {
   const int H = history >= 2 ? history : 0;
   if (H == S->H) return BRTM_OK;
+  if (S->scratch_unset) {  // cgstep reads (s, ss): no previous step
+    LS_TRY(brtm_vec_zero(S->s));
+    LS_TRY(brtm_vec_zero(S->ss));
+    S->scratch_unset = false;
+  }
   for (brtm_vec *v : S->hs) brtm_vec_destroy(v);
   for (brtm_vec *v : S->hS) brtm_vec_destroy(v);
   S->hs.assign(H, nullptr);
@@ -355,8 +428,8 @@ int set_history(brtm_solver *S, int history) {
   S->H = H;
   S->nh = 0;
   for (int i = 0; i < H; ++i) {
-    LS_TRY(brtm_vec_create(S->ctx, S->oper->nd, &S->hs[i]));
-    LS_TRY(brtm_vec_create(S->ctx, S->oper->nr, &S->hS[i]));
+    LS_TRY(vec_create(S->ctx, S->oper->nd, false, &S->hs[i]));
+    LS_TRY(vec_create(S->ctx, S->oper->nr, false, &S->hS[i]));
   }
   return BRTM_OK;
 }
@@ -685,21 +758,16 @@ int brtm_solver_solve(brtm_solver *S, const brtm_cg_params *prm, double *resid_h
     LS_TRY(brtm_vec_dot(e, e, &ee));
   }
   const double dnorm = std::sqrt(S->rr0_rr0);
-  auto judged = [&](double rr_rr, double *out) -> int {
-    if (!e) {
-      *out = dnorm > 0 ? std::sqrt(rr_rr) / dnorm : 0.0;
-      return BRTM_OK;
-    }
-    double re = 0;
-    const int r2 = brtm_vec_dot(S->rr, e, &re);
-    *out = S->jnorm > 0 ? std::sqrt(std::max(rr_rr + 2 * re + ee, 0.0)) / S->jnorm : 0.0;
-    return r2;
+  auto judged = [&](double rr_rr, double re) {
+    if (!e) return dnorm > 0 ? std::sqrt(rr_rr) / dnorm : 0.0;
+    return S->jnorm > 0 ? std::sqrt(std::max(rr_rr + 2 * re + ee, 0.0)) / S->jnorm : 0.0;
   };
   // |rr| / |d|: the residual of the data as given (noisy when e is set)
   auto data_rel = [&](double rr_rr) { return dnorm > 0 ? std::sqrt(rr_rr) / dnorm : 0.0; };
-  double rr_rr = 0;
+  double rr_rr = 0, rr_e = 0;
   LS_TRY(brtm_vec_dot(S->rr, S->rr, &rr_rr));
-  LS_TRY(judged(rr_rr, &st.rel_resid));
+  if (e) LS_TRY(brtm_vec_dot(S->rr, e, &rr_e));
+  st.rel_resid = judged(rr_rr, rr_e);
   st.data_rel_resid = data_rel(rr_rr);
   if (resid_hist) resid_hist[0] = st.rel_resid;
   if (prm->data_resid_hist) prm->data_resid_hist[0] = st.data_rel_resid;
@@ -710,18 +778,17 @@ int brtm_solver_solve(brtm_solver *S, const brtm_cg_params *prm, double *resid_h
       st.breakdown = 1;
       break;
     }
-    double alfa = 0, beta = 0;
+    double alfa = 0, beta = 0, norms[2] = {0, 0};
     bool stop = false;
-    rc = iterate(S, prm, &st, &alfa, &beta, &stop);
+    rc = iterate(S, prm, &st, e, norms, &alfa, &beta, &stop);
     if (rc != BRTM_OK) break;
     if (stop) {
       st.breakdown = 1;
       break;
     }
     st.iterations = iter + 1;
-    rc = brtm_vec_dot(S->rr, S->rr, &rr_rr);
-    if (rc == BRTM_OK) rc = judged(rr_rr, &st.rel_resid);
-    if (rc != BRTM_OK) break;
+    rr_rr = norms[0];
+    st.rel_resid = judged(rr_rr, norms[1]);
     st.data_rel_resid = data_rel(rr_rr);
     if (resid_hist) resid_hist[iter + 1] = st.rel_resid;
     if (prm->data_resid_hist) prm->data_resid_hist[iter + 1] = st.data_rel_resid;
