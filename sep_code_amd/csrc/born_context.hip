@@ -131,11 +131,8 @@ int illumination(brtm_ctx *c, float *acc) {
   const int sfmt = fmt_of_store(S.kind);
   BRTM_REQUIRE(sfmt != FMT_NONE && S.count > 0, BRTM_ESTATE,
                "illumination needs a snapshot store (f32, bf16 or f16) for the shot");
-  for (int k = 0; k < S.count; ++k) {
-    const void *snap = S.data.as<char>() + fmt_bytes(sfmt) * (size_t)c->ncell * k;
-    const float *ss = sfmt == FMT_F32 ? nullptr : S.scale.as<float>() + (size_t)c->n3 * k;
-    BRTM_HIP(launch_square_accumulate(sfmt, snap, ss, acc, c->n1 * c->n2, c->n3, c->stream));
-  }
+  BRTM_HIP(launch_square_accumulate(sfmt, S.data.ptr, S.scale.as<float>(), S.count, acc,
+                                    c->n1 * c->n2, c->n3, c->stream));
   return BRTM_OK;
 }
 
@@ -488,8 +485,15 @@ int source_prop(brtm_ctx *c, int jt, int nt, int jimg, int kind, int ckpt, float
   const bool direct = ck_direct || fmt == FMT_F32;
   const size_t need = ck_direct ? 2 * fbytes * (size_t)ck_count
                                 : fbytes * (size_t)((nt - 1) / jimg + 1);
+  // 16-bit snapshots are encoded whole: their buffers are kept when the new
+  // ones fill them to within an eighth (allocating a 256^3 shot's 1 GB anew
+  // took 20 ms with other contexts alive)
+  const size_t need16 = fmt_bytes(FMT_F16) * (size_t)c->ncell * (size_t)((nt - 1) / jimg + 1);
+  const bool keep16 = (fmt == FMT_BF16 || fmt == FMT_F16) &&
+                      (S.kind == BRTM_STORE_BF16 || S.kind == BRTM_STORE_F16) &&
+                      S.data.bytes >= need16 && S.data.bytes - need16 <= need16 / 8;
   const bool keep = direct && S.kind == kind && S.halo_zero && S.data.bytes >= need;
-  if (!keep) S.release();
+  if (!keep && !keep16) S.release();
   S.kind = kind;
   S.nt = nt;
   S.jt = jt;
@@ -499,7 +503,10 @@ int source_prop(brtm_ctx *c, int jt, int nt, int jimg, int kind, int ckpt, float
   if (fmt != FMT_NONE) {
     S.count = (nt - 1) / jimg + 1;
     BRTM_TRY(S.data.alloc(fmt_bytes(fmt) * (size_t)c->ncell * S.count));
-    if (fmt != FMT_F32) BRTM_TRY(S.scale.alloc(sizeof(float) * (size_t)c->n3 * S.count));
+    if (fmt != FMT_F32) {
+      BRTM_TRY(S.scale.alloc(sizeof(float) * (size_t)c->n3 * S.count));
+      BRTM_TRY(c->encmax.alloc(encode_scratch(c->n3)));
+    }
     // FP32 snapshots are written by the steps themselves and read back as
     // the next step's input, so their halos must be zero (once per buffer)
     if (fmt == FMT_F32 && !keep) {
@@ -570,7 +577,8 @@ int source_prop(brtm_ctx *c, int jt, int nt, int jimg, int kind, int ckpt, float
     if (fmt != FMT_NONE && fmt != FMT_F32 && it % jimg == 0) {
       const int k = it / jimg;
       BRTM_HIP(launch_encode(fmt, out, S.data.as<char>() + 2 * (size_t)c->ncell * k,
-                             S.scale.as<float>() + (size_t)c->n3 * k, n12, c->n3, c->stream));
+                             S.scale.as<float>() + (size_t)c->n3 * k, c->encmax.as<float>(), n12,
+                             c->n3, c->stream));
     }
     return BRTM_OK;
   };
@@ -907,7 +915,7 @@ int brtm_destroy(brtm_ctx *c) {
   c->pool.flush();
   c->stores.clear();
   for (DevBuf *b : {&c->d_wtab, &c->V, &c->fa, &c->fb, &c->fc, &c->fd, &c->img, &c->mdl,
-                    &c->seg, &c->mvw, &c->rscale, &c->partials, &c->dotv, &c->gram, &c->slocs, &c->strc,
+                    &c->seg, &c->mvw, &c->rscale, &c->partials, &c->dotv, &c->gram, &c->encmax, &c->slocs, &c->strc,
                     &c->rlocs, &c->rmap, &c->smap, &c->traces})
     b->release();
   c->have_space = c->have_vel = false;
@@ -1441,7 +1449,7 @@ int brtm_device_bytes(brtm_ctx *c, double *bytes) {
   BRTM_REQUIRE(c && bytes, BRTM_EINVAL, "NULL argument");
   double b = 0;
   for (DevBuf *x : {&c->d_wtab, &c->V, &c->fa, &c->fb, &c->fc, &c->fd, &c->img, &c->mdl,
-                    &c->seg, &c->partials, &c->dotv, &c->gram, &c->slocs, &c->strc, &c->rlocs, &c->rmap, &c->smap,
+                    &c->seg, &c->partials, &c->dotv, &c->gram, &c->encmax, &c->slocs, &c->strc, &c->rlocs, &c->rmap, &c->smap,
                     &c->traces, &c->mvw, &c->rscale})
     b += (double)x->bytes;
   for (auto &s : c->stores) b += (double)s.data.bytes + (double)s.scale.bytes;

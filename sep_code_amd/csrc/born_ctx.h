@@ -140,6 +140,7 @@ struct brtm_ctx {
   int seg_slots = 0;
   brtm::DevBuf partials, dotv;
   brtm::DevBuf gram;  // scratch of the solvers' one-pass products
+  brtm::DevBuf encmax;  // partial slice maxima of the snapshot encoder
   brtm::VecPool pool;
   // this device's copy of the allocation-free entry point's scratch array
   // (its device address, from hipGetSymbolAddress at brtm_create)

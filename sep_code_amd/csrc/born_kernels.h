@@ -131,15 +131,17 @@ hipError_t launch_receiver_scale(const float *V, const float *wtab, int nw, cons
                                  int npts, float *rs, int n1, int n2, int n3, hipStream_t st);
 
 // Snapshot encoding: per-slice max |s| then quantise to fmt.
-hipError_t launch_encode(int fmt, const float *s, void *dst, float *sscale, int n12, int n3,
-                         hipStream_t st);
+// part: encode_scratch(n3) bytes.
+hipError_t launch_encode(int fmt, const float *s, void *dst, float *sscale, float *part, int n12,
+                         int n3, hipStream_t st);
+size_t encode_scratch(int n3);
 // Decode one snapshot to FP32 (tests, diagnostics).
 hipError_t launch_decode(int fmt, const void *src, const float *sscale, float *dst, int n12,
                          int n3, hipStream_t st);
 
-// acc += s^2 over one snapshot (illumination).
-hipError_t launch_square_accumulate(int fmt, const void *src, const float *sscale, float *acc,
-                                   int n12, int n3, hipStream_t st);
+// acc += sum of s^2 over `count` consecutive snapshots (illumination).
+hipError_t launch_square_accumulate(int fmt, const void *src, const float *sscale, int count,
+                                    float *acc, int n12, int n3, hipStream_t st);
 
 // FP64 reductions / vector kernels.
 constexpr int kDotBlocks = 1024;
