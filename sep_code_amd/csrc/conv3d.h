@@ -20,10 +20,10 @@ struct Vol {          // spatial shape (per batch item)
   long spatial() const { return (long)d * h * w; }
 };
 
-// y = act(conv3x3x3(x, W) + b), zero padding 1.  relu: ReLU on the output;
-// out_f32: y is FP32 (no bias, no ReLU: used for the input gradient).
+// y = ReLU(conv3x3x3(x, W) + b), zero padding 1; out_f32: y is FP32 (no bias,
+// no ReLU: the input gradient).
 hipError_t conv3d_fwd(const Act &x, const uint16_t *W, const float *bias, Act y, Vol v,
-                      bool relu, bool out_f32, hipStream_t st);
+                      bool out_f32, hipStream_t st);
 // dW[tap][co][ci] = sum_p dy[p][co] x[p + tap][ci] (FP32, [27][cout][cin]);
 // db[co] = sum_p dy[p][co].  scratch holds kGradScratch floats.
 constexpr long kGradScratch = 8L << 20;

@@ -1,7 +1,7 @@
 // 3-D convolutions of the learned preconditioner on gfx950 MFMA.
 //
-// Forward (and input-gradient) convolutions are implicit GEMMs: M = output
-// channels, N = 16 consecutive x positions (of YT rows) per wave, K = the 27
+// Forward (and input-gradient) convolutions are implicit GEMMs (k_conv): M =
+// output channels, N = 16 consecutive x positions per row, K = the 27
 // taps x input channels, one v_mfma_f32_16x16x32_bf16 per (16-channel output
 // tile, row, tap, 32-channel chunk) and one v_mfma_f32_16x16x16_bf16 per
 // 16-channel remainder.  Operand lanes: lane l holds A[l%16][8(l/16)+i] and
@@ -48,145 +48,202 @@ int grid1(long n, int bs = 256) {
 }
 
 // ------------------------------------------------------------- forward GEMM
-// A wave computes 16 x positions of YT consecutive rows at one z, all output
-// channels.  K runs tap by tap: for each (dz, dx) and 32-channel chunk the
-// wave loads the YT + 2 input rows y0-1 .. y0+YT once (a lane's 8 K values
-// are 8 consecutive channels of one position: one 16-byte load) and the
-// three dy taps use them, so an input row is loaded once for three MFMAs of
-// each row tile.  The weight operand of a tap is loaded once for the YT row
-// tiles.  A 16-channel remainder (CIN = 16, 48) runs on the K = 16 MFMA
-// (v_mfma_f32_16x16x16_bf16: 4 K values per lane, one 8-byte load) instead
-// of being padded to 32.
-template <int CIN, int COUT, int YT, bool RELU, bool OUTF32>
-__global__ void __launch_bounds__(256)
-k_conv_fwd(const uint16_t *__restrict__ x, int xcs, const uint16_t *__restrict__ W,
-           const float *__restrict__ bias, void *y, int ycs, int N, int D, int H, int Wd) {
-  static_assert(CIN % 16 == 0 && COUT % 16 == 0, "channel counts");
+// Elements between two positions (or two weight rows) in LDS: lanes 0..15 of
+// a 16-byte read are that far apart, and strides of an odd number of 16-byte
+// units or of at most 64 bytes spread them over all banks.
+__host__ __device__ constexpr int pos_stride(int c) { return c > 48 ? c + 8 : c; }
+
+// v, in a form that the compiler cannot move out of a loop.
+__device__ __forceinline__ int opaque(int v) {
+  asm volatile("" : "+v"(v));
+  return v;
+}
+
+// What happens to a finished output tile.
+enum { OUT_ACT = 0, OUT_GRAD = 1 };  // bias + ReLU to BF16; FP32 as it is
+
+// A workgroup sweeps z over zl output planes of a tile of 16 WX positions by
+// YT WY rows.  Each input plane of the tile (with its halo, zeros outside the
+// volume) is staged in LDS once and serves all 27 taps of the three output
+// planes around it, whose sums wait in registers; the next plane is loaded
+// into registers meanwhile.  A wave computes 16 positions of YT rows and MTW
+// 16-channel output tiles: for a (dx, 32-channel chunk) the YT + 2 row
+// fragments are read once for the nine (dz, dy) taps, and a weight fragment
+// once for the YT rows.  Weights wait in LDS (WL) where they fit beside the
+// plane, else they come through the vector cache.  A 16-channel remainder
+// (CIN = 16, 48) runs on the K = 16 MFMA.  Every output's sum runs over
+// (dz, dx, chunk, dy) in this order, whatever the tile.
+//
+// What bounds it: the matrix unit (46 us for 48->16 at 8 x 64^3, the K = 16
+// products at half rate) and the LDS reads that feed it.  A wave that loaded
+// its rows from the vector cache for each dz, dx and chunk moved three times
+// the fragments through a 64-byte-per-clock cache: at 8 x 64^3 48->16 took 219
+// us, now 129; 16->16 93, now 57; 96->32 (32^3) 108, now 76; 32->32 41, now
+// 23; 64->64 (16^3) 62, now 23; 32->64 21, now 18.
+template <int CIN, int COUT, int MTW, int YT, int WX, int WY, bool WL, int OUT>
+__global__ void __launch_bounds__(64 * WX * WY * (COUT / 16 / MTW), 2)
+k_conv(const uint16_t *__restrict__ x, int xcs, const uint16_t *__restrict__ W,
+       const float *__restrict__ bias, void *y, int ycs, int zl, int D, int H, int Wd) {
   constexpr int CIN_P = (CIN + 31) / 32 * 32;
-  constexpr int MT = COUT / 16;
+  constexpr int NT = 64 * WX * WY * (COUT / 16 / MTW);
   constexpr int NC = CIN / 32;          // 32-channel chunks
   constexpr bool R16 = CIN % 32 == 16;  // and a 16-channel remainder
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int wt = Wd >> 4, hg = H / YT;
-  // XCD-aware order: workgroup b runs on XCD b % 8, so XCD k takes a
-  // contiguous run of tiles (x fastest, then rows, then z).  Neighbouring
-  // rows and planes, whose inputs the 27 taps share, then meet in that XCD's
-  // L2 instead of being fetched again by another XCD.
-  const int nb = gridDim.x, q8 = nb >> 3, r8 = nb & 7;
-  const int bid = blockIdx.x, xcd = bid & 7, jj = bid >> 3;
-  const int blk = (xcd < r8) ? xcd * (q8 + 1) + jj : r8 * (q8 + 1) + (xcd - r8) * q8 + jj;
-  const long tile = (long)blk * 4 + wave;
-  if (tile >= (long)N * D * hg * wt) return;  // whole wave; no barriers below
-  const int xt = (int)(tile % wt);
-  long r = tile / wt;
-  const int y0 = (int)(r % hg) * YT;
-  r /= hg;
-  const int zz = (int)(r % D);
-  const int nn = (int)(r / D);
-  const int x0 = xt * 16;
+  constexpr int R = YT * WY, X = 16 * WX, PS = pos_stride(CIN), RS = (X + 2) * PS;
+  constexpr int WS = WL ? PS : CIN_P;
+  __shared__ __attribute__((aligned(16))) uint16_t Xs[(R + 2) * RS];
+  __shared__ __attribute__((aligned(16))) uint16_t Ws[WL ? 27 * COUT * PS : 8];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int col = lane & 15, kq = lane >> 4;
-  f32x4 acc[MT][YT];
+  const int wx = wave % WX, wy = (wave / WX) % WY, wm = wave / (WX * WY);
+  // XCD-aware order: workgroup b runs on XCD b % 8, so XCD k takes a
+  // contiguous run of tiles and neighbouring tiles' halos meet in its L2.
+  const int nb = gridDim.x, q8 = nb >> 3, r8 = nb & 7;
+  const int xcd = blockIdx.x & 7, jj = blockIdx.x >> 3;
+  int r = (xcd < r8) ? xcd * (q8 + 1) + jj : r8 * (q8 + 1) + (xcd - r8) * q8 + jj;
+  const int x0 = r % (Wd / X) * X;
+  r /= Wd / X;
+  const int y0 = r % (H / R) * R;
+  r /= H / R;
+  const int z0 = r % (D / zl) * zl;
+  const long n0 = (long)(r / (D / zl)) * D;  // plane 0 of this batch item
+
+  constexpr int XC = CIN / 8, NX = (R + 2) * (X + 2) * XC, PT = (NX + NT - 1) / NT;
+  uint4 pre[PT];  // this thread's 16-byte chunks of a plane
+  const long plane = (long)H * Wd * xcs;
+  const uint32_t bytes = ((uint32_t)(H * Wd - 1) * xcs + CIN) * 2;
+  auto fetch = [&](int z) {
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint16_t *>(x + (n0 + z) * plane), 0, bytes, 0x00020000);
+    // the chunks' places are recomputed for each plane: kept over the plane
+    // loop they took registers that the sums need
+    const int t_ = opaque(tid);
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt)
+    for (int i = 0; i < PT; ++i) {
+      const int e = t_ + i * NT;
+      const int c = e % XC, p = (e / XC) % (X + 2), rr = e / (XC * (X + 2));
+      const int yy = y0 + rr - 1, xx = x0 + p - 1;
+      const bool ok = e < NX && yy >= 0 && yy < H && xx >= 0 && xx < Wd;
+      const uint32_t off = ok ? (uint32_t)(yy * Wd + xx) * xcs * 2 + 16 * c : 0x80000000u;
+      pre[i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rs, off, 0, 0));
+    }
+  };
+
+  const int zf = z0 > 0 ? z0 - 1 : 0, ze = z0 + zl < D ? z0 + zl : D - 1;
+  fetch(zf);
+  if constexpr (WL) {
+    for (int i = tid; i < 27 * COUT * XC; i += NT)
+      *reinterpret_cast<uint4 *>(&Ws[i / XC * PS + i % XC * 8]) =
+          *reinterpret_cast<const uint4 *>(W + (long)(i / XC) * CIN_P + i % XC * 8);
+  }
+  const uint16_t *wb = (WL ? Ws : W) + (wm * MTW * 16 + col) * WS;
+  const uint16_t *xb = Xs + (wy * YT) * RS + (wx * 16 + col) * PS;
+
+  f32x4 acc[3][MTW][YT];  // outputs zp + 1, zp, zp - 1 of input plane zp
 #pragma unroll
-    for (int t = 0; t < YT; ++t) acc[mt][t] = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int dz = 0; dz < 3; ++dz) {
-    const int z2 = zz + dz - 1;
-    if (z2 < 0 || z2 >= D) continue;  // the same for the whole wave
-    const long zb = ((long)nn * D + z2) * H;
+  for (int d = 0; d < 3; ++d)
+#pragma unroll
+    for (int m = 0; m < MTW; ++m)
+#pragma unroll
+      for (int t = 0; t < YT; ++t) acc[d][m][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  auto store = [&](int z) {
+    // a lane's four channels 4kq .. 4kq+3 of an output tile are adjacent: one
+    // 8-byte (BF16) or 16-byte (FP32) store
+#pragma unroll
+    for (int t = 0; t < YT; ++t) {
+      const long o = (((n0 + z) * H + y0 + wy * YT + t) * Wd + x0 + wx * 16 + col) * ycs;
+#pragma unroll
+      for (int m = 0; m < MTW; ++m) {
+        const int c0 = (wm * MTW + m) * 16 + 4 * kq;
+        const f32x4 v = acc[2][m][t];
+        if constexpr (OUT == OUT_GRAD) {
+          *reinterpret_cast<f32x4 *>(static_cast<float *>(y) + o + c0) = v;
+        } else {
+          const float4 b = *reinterpret_cast<const float4 *>(bias + c0);
+          const float v0 = fmaxf(v[0] + b.x, 0.f), v1 = fmaxf(v[1] + b.y, 0.f);
+          const float v2 = fmaxf(v[2] + b.z, 0.f), v3 = fmaxf(v[3] + b.w, 0.f);
+          *reinterpret_cast<uint2 *>(static_cast<uint16_t *>(y) + o + c0) =
+              make_uint2((uint32_t)f2bf(v0) | ((uint32_t)f2bf(v1) << 16),
+                         (uint32_t)f2bf(v2) | ((uint32_t)f2bf(v3) << 16));
+        }
+      }
+    }
+  };
+
+  // products of the staged plane; on[d]: output zp + 1 - d is this sweep's
+  auto products = [&](bool on0, bool on1, bool on2) {
+    const uint16_t *wq = wb + opaque(0);  // no weights kept over the plane loop
 #pragma unroll
     for (int dx = 0; dx < 3; ++dx) {
-      const int x2 = x0 + col + dx - 1;
-      const bool okx = x2 >= 0 && x2 < Wd;
 #pragma unroll
       for (int cg = 0; cg < NC; ++cg) {
         const int c = cg * 32 + 8 * kq;
         bf16x8 bv[YT + 2];
 #pragma unroll
-        for (int rr = 0; rr < YT + 2; ++rr) {
-          const int y2 = y0 + rr - 1;
-          bv[rr] = okx && y2 >= 0 && y2 < H ? ld8(x + ((zb + y2) * Wd + x2) * xcs + c) : zero8();
+        for (int i = 0; i < YT + 2; ++i) bv[i] = ld8(xb + i * RS + dx * PS + c);
+#pragma unroll
+        for (int dz = 0; dz < 3; ++dz) {
+          if (!(dz == 0 ? on0 : dz == 1 ? on1 : on2)) continue;
+#pragma unroll
+          for (int dy = 0; dy < 3; ++dy)
+#pragma unroll
+            for (int m = 0; m < MTW; ++m) {
+              const bf16x8 a = ld8(wq + ((dz * 9 + dy * 3 + dx) * COUT + m * 16) * WS + c);
+#pragma unroll
+              for (int t = 0; t < YT; ++t)
+                acc[dz][m][t] =
+                    __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bv[t + dy], acc[dz][m][t], 0, 0, 0);
+            }
         }
-#pragma unroll
-        for (int dy = 0; dy < 3; ++dy) {
-          const int tap = dz * 9 + dy * 3 + dx;
-          bf16x8 a[MT];
-#pragma unroll
-          for (int mt = 0; mt < MT; ++mt)
-            a[mt] = ld8(W + ((long)tap * COUT + mt * 16 + col) * CIN_P + c);
-#pragma unroll
-          for (int t = 0; t < YT; ++t)
-#pragma unroll
-            for (int mt = 0; mt < MT; ++mt)
-              acc[mt][t] =
-                  __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[mt], bv[t + dy], acc[mt][t], 0, 0, 0);
-        }
+        __builtin_amdgcn_sched_barrier(0);
       }
       if constexpr (R16) {
         const int c = NC * 32 + 4 * kq;
         i16x4 bv[YT + 2];
 #pragma unroll
-        for (int rr = 0; rr < YT + 2; ++rr) {
-          const int y2 = y0 + rr - 1;
-          bv[rr] = okx && y2 >= 0 && y2 < H ? ld4h(x + ((zb + y2) * Wd + x2) * xcs + c) : zero4h();
+        for (int i = 0; i < YT + 2; ++i) bv[i] = ld4h(xb + i * RS + dx * PS + c);
+#pragma unroll
+        for (int dz = 0; dz < 3; ++dz) {
+          if (!(dz == 0 ? on0 : dz == 1 ? on1 : on2)) continue;
+#pragma unroll
+          for (int dy = 0; dy < 3; ++dy)
+#pragma unroll
+            for (int m = 0; m < MTW; ++m) {
+              const i16x4 a = ld4h(wq + ((dz * 9 + dy * 3 + dx) * COUT + m * 16) * WS + c);
+#pragma unroll
+              for (int t = 0; t < YT; ++t)
+                acc[dz][m][t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, bv[t + dy],
+                                                                          acc[dz][m][t], 0, 0, 0);
+            }
         }
-#pragma unroll
-        for (int dy = 0; dy < 3; ++dy) {
-          const int tap = dz * 9 + dy * 3 + dx;
-          i16x4 a[MT];
-#pragma unroll
-          for (int mt = 0; mt < MT; ++mt)
-            a[mt] = ld4h(W + ((long)tap * COUT + mt * 16 + col) * CIN_P + c);
-#pragma unroll
-          for (int t = 0; t < YT; ++t)
-#pragma unroll
-            for (int mt = 0; mt < MT; ++mt)
-              acc[mt][t] =
-                  __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[mt], bv[t + dy], acc[mt][t], 0, 0, 0);
-        }
+        __builtin_amdgcn_sched_barrier(0);
       }
     }
-  }
-  // a lane's four channels 4kq .. 4kq+3 of a 16-channel tile are adjacent:
-  // one 8-byte (BF16) or 16-byte (FP32) store when the channel stride
-  // keeps them aligned
-  const bool vec = (ycs & 3) == 0;
+  };
+
+  for (int zp = zf; zp <= ze; ++zp) {
+    __syncthreads();  // the previous plane has been read
+    const int t_ = opaque(tid);
 #pragma unroll
-  for (int t = 0; t < YT; ++t) {
-    const long opos = (((long)nn * D + zz) * H + y0 + t) * Wd + x0 + col;
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-      const int c0 = mt * 16 + 4 * kq;
-      float v[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        v[j] = acc[mt][t][j];
-        if constexpr (!OUTF32) {
-          v[j] += bias[c0 + j];
-          if (RELU) v[j] = fmaxf(v[j], 0.f);
-        }
-      }
-      if constexpr (OUTF32) {
-        float *o = static_cast<float *>(y) + opos * ycs + c0;
-        if (vec) {
-          *reinterpret_cast<float4 *>(o) = make_float4(v[0], v[1], v[2], v[3]);
-        } else {
-#pragma unroll
-          for (int j = 0; j < 4; ++j) o[j] = v[j];
-        }
-      } else {
-        uint16_t *o = static_cast<uint16_t *>(y) + opos * ycs + c0;
-        if (vec) {
-          *reinterpret_cast<uint2 *>(o) =
-              make_uint2((uint32_t)f2bf(v[0]) | ((uint32_t)f2bf(v[1]) << 16),
-                         (uint32_t)f2bf(v[2]) | ((uint32_t)f2bf(v[3]) << 16));
-        } else {
-#pragma unroll
-          for (int j = 0; j < 4; ++j) o[j] = f2bf(v[j]);
-        }
-      }
+    for (int i = 0; i < PT; ++i) {
+      const int e = t_ + i * NT;
+      if (e < NX) *reinterpret_cast<uint4 *>(&Xs[e / XC * PS + e % XC * 8]) = pre[i];
     }
+    __syncthreads();
+    if (zp < ze) fetch(zp + 1);
+    const bool on0 = zp + 1 < z0 + zl, on1 = zp >= z0 && zp < z0 + zl, on2 = zp > z0;
+    products(on0, on1, on2);
+    if (on2) store(zp - 1);
+#pragma unroll
+    for (int m = 0; m < MTW; ++m)
+#pragma unroll
+      for (int t = 0; t < YT; ++t) {
+        acc[2][m][t] = acc[1][m][t];
+        acc[1][m][t] = acc[0][m][t];
+        acc[0][m][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+      }
   }
+  if (z0 + zl == D) store(D - 1);  // no plane follows
 }
 
 // ------------------------------------------------------------- weight GEMM
@@ -761,35 +818,23 @@ __global__ void k_adam(float *p, const float *__restrict__ g, float *m, float *v
   }
 }
 
-template <int CIN, int COUT, int YT>
-hipError_t fwd_y(const Act &x, const uint16_t *W, const float *b, Act y, Vol v, bool relu,
-                 bool f32, hipStream_t st) {
-  const long tiles = (long)v.n * v.d * (v.h / YT) * (v.w / 16);
-  const int grid = (int)((tiles + 3) / 4);
+// Output planes per sweep: as many as leave two workgroups for a compute unit.
+template <int CIN, int COUT, int MTW, int YT, int WX, int WY, bool WL>
+hipError_t conv_t(const Act &x, const uint16_t *W, const float *b, Act y, Vol v, bool f32,
+                  hipStream_t st) {
+  if (v.w % (16 * WX) || v.h % (YT * WY)) return hipErrorInvalidValue;
+  constexpr int NT = 64 * WX * WY * (COUT / 16 / MTW);
+  const long tiles = (long)v.n * (v.h / (YT * WY)) * (v.w / (16 * WX));
+  int zl = 16;
+  while (zl > 1 && (v.d % zl || tiles * (v.d / zl) < (NT > 256 ? 256 : 512))) zl /= 2;
+  const int grid = (int)(tiles * (v.d / zl));
   if (f32)
-    k_conv_fwd<CIN, COUT, YT, false, true><<<grid, 256, 0, st>>>(
-        (const uint16_t *)x.p, x.cs, W, b, y.p, y.cs, v.n, v.d, v.h, v.w);
-  else if (relu)
-    k_conv_fwd<CIN, COUT, YT, true, false><<<grid, 256, 0, st>>>(
-        (const uint16_t *)x.p, x.cs, W, b, y.p, y.cs, v.n, v.d, v.h, v.w);
+    k_conv<CIN, COUT, MTW, YT, WX, WY, WL, OUT_GRAD><<<grid, NT, 0, st>>>(
+        (const uint16_t *)x.p, x.cs, W, b, y.p, y.cs, zl, v.d, v.h, v.w);
   else
-    k_conv_fwd<CIN, COUT, YT, false, false><<<grid, 256, 0, st>>>(
-        (const uint16_t *)x.p, x.cs, W, b, y.p, y.cs, v.n, v.d, v.h, v.w);
+    k_conv<CIN, COUT, MTW, YT, WX, WY, WL, OUT_ACT><<<grid, NT, 0, st>>>(
+        (const uint16_t *)x.p, x.cs, W, b, y.p, y.cs, zl, v.d, v.h, v.w);
   return hipGetLastError();
-}
-
-// Four rows per wave where that still gives 1024 workgroups, else one; eight
-// for the 16-output-channel layers (one output tile: the rows are the
-// wave's only independent MFMA chains).
-template <int CIN, int COUT>
-hipError_t fwd_t(const Act &x, const uint16_t *W, const float *b, Act y, Vol v, bool relu,
-                 bool f32, hipStream_t st) {
-  const long blocks4 = (long)v.n * v.d * (v.h / 4) * (v.w / 16) / 4;
-  if constexpr (COUT == 16) {
-    if (v.h % 8 == 0 && blocks4 >= 2048) return fwd_y<CIN, COUT, 8>(x, W, b, y, v, relu, f32, st);
-  }
-  if (v.h % 4 == 0 && blocks4 >= 1024) return fwd_y<CIN, COUT, 4>(x, W, b, y, v, relu, f32, st);
-  return fwd_y<CIN, COUT, 1>(x, W, b, y, v, relu, f32, st);
 }
 
 // Workgroups of a weight gradient: up to 256 (times the three dz), fewer
@@ -816,19 +861,21 @@ hipError_t wgrad_t(const Act &x, const Act &dy, float *dW, float *db, Vol v, flo
   X(16, 16, 64, 8) X(48, 16, 64, 8) X(16, 32, 32, 8) X(32, 32, 32, 8) X(96, 32, 32, 4) \
   X(32, 64, 16, 8) X(64, 64, 16, 8)
 
-// The (cin, cout) pairs of the forward convolutions (16->16, 16->32, 32->32,
-// 32->64, 64->64, 96->32, 48->16) and of the transposed ones (input
-// gradients: 32->16, 64->32, 32->96, 16->48).
-#define BRTM_CONV_FWD_PAIRS(X)                                                          \
-  X(16, 16) X(16, 32) X(32, 32) X(32, 64) X(64, 64) X(96, 32) X(48, 16) X(32, 16) X(64, 32) \
-  X(32, 96) X(16, 48)
+// The forward convolutions and the transposed ones (input gradients): (cin,
+// cout, output tiles and rows per wave, waves in x and y, weights in LDS).
+#define BRTM_CONV_SHAPES(X)                                                          \
+  X(16, 16, 1, 8, 4, 2, true) X(48, 16, 1, 8, 4, 2, true) X(16, 48, 3, 4, 4, 2, true) \
+  X(16, 32, 2, 4, 2, 2, true) X(32, 32, 2, 4, 2, 4, true) X(32, 16, 1, 4, 2, 4, true) \
+  X(96, 32, 2, 4, 2, 2, false) X(32, 96, 3, 4, 2, 2, false)                          \
+  X(32, 64, 2, 4, 1, 2, false) X(64, 64, 2, 4, 1, 2, false) X(64, 32, 1, 4, 1, 2, false)
 
 hipError_t conv3d_fwd(const Act &x, const uint16_t *W, const float *bias, Act y, Vol v,
-                      bool relu, bool out_f32, hipStream_t st) {
-  if (v.w % 16 || x.c % 16 || x.cs % 8 || y.c % 16) return hipErrorInvalidValue;
-#define X(CI, CO) \
-  if (x.c == CI && y.c == CO) return fwd_t<CI, CO>(x, W, bias, y, v, relu, out_f32, st);
-  BRTM_CONV_FWD_PAIRS(X)
+                      bool out_f32, hipStream_t st) {
+  if (x.cs % 8 || y.cs % 4) return hipErrorInvalidValue;
+#define X(CI, CO, MTW, YT, WX, WY, WL) \
+  if (x.c == CI && y.c == CO)          \
+    return conv_t<CI, CO, MTW, YT, WX, WY, WL>(x, W, bias, y, v, out_f32, st);
+  BRTM_CONV_SHAPES(X)
 #undef X
   return hipErrorInvalidValue;
 }

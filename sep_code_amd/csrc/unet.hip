@@ -179,21 +179,19 @@ int forward(brtm_unet *u, const float *x, int nb) {
   auto W = [&](int l) { return u->wbf[l].as<uint16_t>(); };
   auto Bv = [&](int l) { return pr + u->bl[l]; };
   BRTM_HIP(conv3d_first_fwd(x, pr + u->w0, pr + u->b0, act(u->e1a, C1, C1), v1, st));
-  BRTM_HIP(conv3d_fwd(act(u->e1a, C1, C1), W(0), Bv(0), act(u->cat1, C1, 48, 32), v1, true,
-                      false, st));
+  BRTM_HIP(conv3d_fwd(act(u->e1a, C1, C1), W(0), Bv(0), act(u->cat1, C1, 48, 32), v1, false, st));
   BRTM_HIP(avgpool_fwd(act(u->cat1, C1, 48, 32), act(u->p1, C1, C1), v1, st));
-  BRTM_HIP(conv3d_fwd(act(u->p1, C1, C1), W(1), Bv(1), act(u->e2a, C2, C2), v2, true, false, st));
-  BRTM_HIP(conv3d_fwd(act(u->e2a, C2, C2), W(2), Bv(2), act(u->cat2, C2, 96, 64), v2, true, false,
-                      st));
+  BRTM_HIP(conv3d_fwd(act(u->p1, C1, C1), W(1), Bv(1), act(u->e2a, C2, C2), v2, false, st));
+  BRTM_HIP(conv3d_fwd(act(u->e2a, C2, C2), W(2), Bv(2), act(u->cat2, C2, 96, 64), v2, false, st));
   BRTM_HIP(avgpool_fwd(act(u->cat2, C2, 96, 64), act(u->p2, C2, C2), v2, st));
-  BRTM_HIP(conv3d_fwd(act(u->p2, C2, C2), W(3), Bv(3), act(u->b1, C3, C3), v3, true, false, st));
-  BRTM_HIP(conv3d_fwd(act(u->b1, C3, C3), W(4), Bv(4), act(u->b2, C3, C3), v3, true, false, st));
+  BRTM_HIP(conv3d_fwd(act(u->p2, C2, C2), W(3), Bv(3), act(u->b1, C3, C3), v3, false, st));
+  BRTM_HIP(conv3d_fwd(act(u->b1, C3, C3), W(4), Bv(4), act(u->b2, C3, C3), v3, false, st));
   BRTM_HIP(upsample_fwd(act(u->b2, C3, C3), act(u->cat2, C3, 96, 0), v3, st));
-  BRTM_HIP(conv3d_fwd(act(u->cat2, 96, 96), W(5), Bv(5), act(u->d2a, C2, C2), v2, true, false, st));
-  BRTM_HIP(conv3d_fwd(act(u->d2a, C2, C2), W(6), Bv(6), act(u->d2b, C2, C2), v2, true, false, st));
+  BRTM_HIP(conv3d_fwd(act(u->cat2, 96, 96), W(5), Bv(5), act(u->d2a, C2, C2), v2, false, st));
+  BRTM_HIP(conv3d_fwd(act(u->d2a, C2, C2), W(6), Bv(6), act(u->d2b, C2, C2), v2, false, st));
   BRTM_HIP(upsample_fwd(act(u->d2b, C2, C2), act(u->cat1, C2, 48, 0), v2, st));
-  BRTM_HIP(conv3d_fwd(act(u->cat1, 48, 48), W(7), Bv(7), act(u->d1a, C1, C1), v1, true, false, st));
-  BRTM_HIP(conv3d_fwd(act(u->d1a, C1, C1), W(8), Bv(8), act(u->d1b, C1, C1), v1, true, false, st));
+  BRTM_HIP(conv3d_fwd(act(u->cat1, 48, 48), W(7), Bv(7), act(u->d1a, C1, C1), v1, false, st));
+  BRTM_HIP(conv3d_fwd(act(u->d1a, C1, C1), W(8), Bv(8), act(u->d1b, C1, C1), v1, false, st));
   BRTM_HIP(head_fwd(act(u->d1b, C1, C1), pr + u->wh, pr + u->bh, x, u->out.as<float>(), v1, st));
   return BRTM_OK;
 }
@@ -212,7 +210,7 @@ int layer_bwd(brtm_unet *u, int l, const float *gy, int gcs, const Act &y, const
   BRTM_HIP(conv3d_wgrad(x, dp, G + u->wl[l], G + u->bl[l], v, u->gscratch.as<float>(), st));
   if (gx) {
     Act out{gx, cin, cin};
-    BRTM_HIP(conv3d_fwd(dp, u->wtf[l].as<uint16_t>(), nullptr, out, v, false, true, st));
+    BRTM_HIP(conv3d_fwd(dp, u->wtf[l].as<uint16_t>(), nullptr, out, v, true, st));
   }
   return BRTM_OK;
 }
