@@ -1,7 +1,7 @@
 // 3-D convolution kernels of the learned image-domain preconditioner
 // (gfx950).  Activations are channels-last [n][z][y][x][c] BF16 with an
 // explicit channel stride (so a layer can read or write a channel slice of a
-// concatenation buffer); weights are [27 taps][cout][cin_pad] BF16 with
+// buffer); weights are [27 taps][cout][cin_pad] BF16 with
 // cin_pad = cin rounded up to 32; accumulation is FP32 on MFMA.
 #pragma once
 #include <hip/hip_runtime.h>
@@ -22,12 +22,14 @@ struct Vol {          // spatial shape (per batch item)
 
 // y = ReLU(conv3x3x3(x, W) + b), zero padding 1; out_f32: y is FP32 (no bias,
 // no ReLU: the input gradient).
-hipError_t conv3d_fwd(const Act &x, const uint16_t *W, const float *bias, Act y, Vol v,
-                      bool out_f32, hipStream_t st);
+// up: the first input channels when they come from a volume of half the size
+// through nearest-neighbour upsampling (channels contiguous), or no channels.
+hipError_t conv3d_fwd(const Act &x, const Act &up, const uint16_t *W, const float *bias, Act y,
+                      Vol v, bool out_f32, hipStream_t st);
 // dW[tap][co][ci] = sum_p dy[p][co] x[p + tap][ci] (FP32, [27][cout][cin]);
 // db[co] = sum_p dy[p][co].  scratch holds kGradScratch floats.
 constexpr long kGradScratch = 8L << 20;
-hipError_t conv3d_wgrad(const Act &x, const Act &dy, float *dW, float *db, Vol v,
+hipError_t conv3d_wgrad(const Act &x, const Act &up, const Act &dy, float *dW, float *db, Vol v,
                         float *scratch, hipStream_t st);
 // Weights of the transposed convolution: Wt[tap][ci][co] = W[26-tap][co][ci]
 // (cin/cout swapped, pads to 32 on the new input channels).
@@ -56,8 +58,7 @@ hipError_t relu_bwd(const float *dy, int dy_cs, const Act &y, Act dpre, Vol v,
 hipError_t avgpool_fwd(const Act &x, Act y, Vol v, hipStream_t st);
 hipError_t avgpool_bwd(const float *dy, int dy_cs, float *dx, int dx_cs, int c, Vol v,
                        hipStream_t st);
-// Nearest x2 upsampling (v is the input shape) and its adjoint (accumulates).
-hipError_t upsample_fwd(const Act &x, Act y, Vol v, hipStream_t st);
+// Adjoint of nearest x2 upsampling (v is the coarse shape; accumulates).
 hipError_t upsample_bwd(const float *dy, int dy_cs, float *dx, int dx_cs, int c, Vol v,
                         hipStream_t st);
 // dst (FP32, stride dcs) += src (FP32, stride scs) over c channels.

@@ -74,16 +74,20 @@ enum { OUT_ACT = 0, OUT_GRAD = 1 };  // bias + ReLU to BF16; FP32 as it is
 // (CIN = 16, 48) runs on the K = 16 MFMA.  Every output's sum runs over
 // (dz, dx, chunk, dy) in this order, whatever the tile.
 //
+// The first CU input channels are a tensor of half the resolution, read
+// through the nearest-neighbour upsampling as it is staged (the concatenated
+// tensor is never stored: 28 us a layer for writing it, and its reads).
+//
 // What bounds it: the matrix unit (46 us for 48->16 at 8 x 64^3, the K = 16
 // products at half rate) and the LDS reads that feed it.  A wave that loaded
 // its rows from the vector cache for each dz, dx and chunk moved three times
 // the fragments through a 64-byte-per-clock cache: at 8 x 64^3 48->16 took 219
-// us, now 129; 16->16 93, now 57; 96->32 (32^3) 108, now 76; 32->32 41, now
+// us, now 117; 16->16 93, now 50; 96->32 (32^3) 108, now 73; 32->32 41, now
 // 23; 64->64 (16^3) 62, now 23; 32->64 21, now 18.
-template <int CIN, int COUT, int MTW, int YT, int WX, int WY, bool WL, int OUT>
+template <int CIN, int CU, int COUT, int MTW, int YT, int WX, int WY, bool WL, int OUT>
 __global__ void __launch_bounds__(64 * WX * WY * (COUT / 16 / MTW), 2)
-k_conv(const uint16_t *__restrict__ x, int xcs, const uint16_t *__restrict__ W,
-       const float *__restrict__ bias, void *y, int ycs, int zl, int D, int H, int Wd) {
+k_conv(const uint16_t *__restrict__ x, int xcs, const uint16_t *__restrict__ up,
+       const uint16_t *__restrict__ W, const float *__restrict__ bias, void *y, int ycs, int zl, int D, int H, int Wd) {
   constexpr int CIN_P = (CIN + 31) / 32 * 32;
   constexpr int NT = 64 * WX * WY * (COUT / 16 / MTW);
   constexpr int NC = CIN / 32;          // 32-channel chunks
@@ -107,16 +111,33 @@ k_conv(const uint16_t *__restrict__ x, int xcs, const uint16_t *__restrict__ W,
   const int z0 = r % (D / zl) * zl;
   const long n0 = (long)(r / (D / zl)) * D;  // plane 0 of this batch item
 
-  constexpr int XC = CIN / 8, NX = (R + 2) * (X + 2) * XC, PT = (NX + NT - 1) / NT;
-  uint4 pre[PT];  // this thread's 16-byte chunks of a plane
-  const long plane = (long)H * Wd * xcs;
-  const uint32_t bytes = ((uint32_t)(H * Wd - 1) * xcs + CIN) * 2;
+  // 16-byte chunks of a plane: the upsampled channels first, then the others
+  constexpr int UC = CU / 8, XC = CIN / 8 - UC, NP = (R + 2) * (X + 2);
+  constexpr int NU = NP * UC, NX = NP * XC, PU = (NU + NT - 1) / NT, PT = (NX + NT - 1) / NT;
+  uint4 preu[PU + 1], pre[PT];
+  const long plane = (long)H * Wd * xcs, uplane = (long)(H / 2) * (Wd / 2) * CU;
+  const uint32_t bytes = ((uint32_t)(H * Wd - 1) * xcs + 8 * XC) * 2;
   auto fetch = [&](int z) {
     const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<uint16_t *>(x + (n0 + z) * plane), 0, bytes, 0x00020000);
     // the chunks' places are recomputed for each plane: kept over the plane
     // loop they took registers that the sums need
     const int t_ = opaque(tid);
+    if constexpr (CU > 0) {
+      const __amdgpu_buffer_rsrc_t ru = __builtin_amdgcn_make_buffer_rsrc(
+          const_cast<uint16_t *>(up + ((n0 + z) >> 1) * uplane), 0, (uint32_t)uplane * 2,
+          0x00020000);
+#pragma unroll
+      for (int i = 0; i < PU; ++i) {
+        const int e = t_ + i * NT;
+        const int c = e % UC, p = (e / UC) % (X + 2), rr = e / (UC * (X + 2));
+        const int yy = y0 + rr - 1, xx = x0 + p - 1;
+        const bool ok = e < NU && yy >= 0 && yy < H && xx >= 0 && xx < Wd;
+        const uint32_t off =
+            ok ? (uint32_t)((yy >> 1) * (Wd >> 1) + (xx >> 1)) * CU * 2 + 16 * c : 0x80000000u;
+        preu[i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(ru, off, 0, 0));
+      }
+    }
 #pragma unroll
     for (int i = 0; i < PT; ++i) {
       const int e = t_ + i * NT;
@@ -131,9 +152,10 @@ k_conv(const uint16_t *__restrict__ x, int xcs, const uint16_t *__restrict__ W,
   const int zf = z0 > 0 ? z0 - 1 : 0, ze = z0 + zl < D ? z0 + zl : D - 1;
   fetch(zf);
   if constexpr (WL) {
-    for (int i = tid; i < 27 * COUT * XC; i += NT)
-      *reinterpret_cast<uint4 *>(&Ws[i / XC * PS + i % XC * 8]) =
-          *reinterpret_cast<const uint4 *>(W + (long)(i / XC) * CIN_P + i % XC * 8);
+    constexpr int WC = CIN / 8;
+    for (int i = tid; i < 27 * COUT * WC; i += NT)
+      *reinterpret_cast<uint4 *>(&Ws[i / WC * PS + i % WC * 8]) =
+          *reinterpret_cast<const uint4 *>(W + (long)(i / WC) * CIN_P + i % WC * 8);
   }
   const uint16_t *wb = (WL ? Ws : W) + (wm * MTW * 16 + col) * WS;
   const uint16_t *xb = Xs + (wy * YT) * RS + (wx * 16 + col) * PS;
@@ -224,10 +246,17 @@ k_conv(const uint16_t *__restrict__ x, int xcs, const uint16_t *__restrict__ W,
   for (int zp = zf; zp <= ze; ++zp) {
     __syncthreads();  // the previous plane has been read
     const int t_ = opaque(tid);
+    if constexpr (CU > 0) {
+#pragma unroll
+      for (int i = 0; i < PU; ++i) {
+        const int e = t_ + i * NT;
+        if (e < NU) *reinterpret_cast<uint4 *>(&Xs[e / UC * PS + e % UC * 8]) = preu[i];
+      }
+    }
 #pragma unroll
     for (int i = 0; i < PT; ++i) {
       const int e = t_ + i * NT;
-      if (e < NX) *reinterpret_cast<uint4 *>(&Xs[e / XC * PS + e % XC * 8]) = pre[i];
+      if (e < NX) *reinterpret_cast<uint4 *>(&Xs[e / XC * PS + e % XC * 8 + CU]) = pre[i];
     }
     __syncthreads();
     if (zp < ze) fetch(zp + 1);
@@ -298,9 +327,10 @@ struct GradFrag {
   }
 };
 
-template <int CIN, int COUT, int SEG, int R>
+template <int CIN, int CU, int COUT, int SEG, int R>
 __global__ void __launch_bounds__(192)
-k_wgrad(const uint16_t *__restrict__ x, int xcs, const uint16_t *__restrict__ dy, int dycs,
+k_wgrad(const uint16_t *__restrict__ x, int xcs, const uint16_t *__restrict__ up,
+        const uint16_t *__restrict__ dy, int dycs,
         float *__restrict__ part, int D, int H, int Wd, long units) {
   constexpr int MT = COUT / 16, NT = CIN / 16, KS = SEG >= 32 ? SEG / 32 : 1;
   constexpr int XS = lds_row(CIN), DS = lds_row(COUT), XP = SEG + 2;
@@ -334,14 +364,19 @@ k_wgrad(const uint16_t *__restrict__ x, int xcs, const uint16_t *__restrict__ dy
     if (z2 < 0 || z2 >= D) continue;  // the whole workgroup: a zero plane
     __syncthreads();                  // the previous unit has been read
     const uint16_t *xp = x + (nn * D + z2) * H * Wd * xcs;
+    const uint16_t *upl = up + ((nn * D + z2) >> 1) * (H / 2) * (Wd / 2) * CU;
     constexpr int XC = CIN / 8, NX = (R + 2) * XP * XC;
 #pragma unroll 4
     for (int i = tid; i < NX; i += 192) {
       const int c = i % XC, p = (i / XC) % XP, rr = i / (XC * XP);
       const int yy = y0 + rr - 1, xx = xs + p - 1;
       uint4 v = make_uint4(0, 0, 0, 0);
-      if (yy >= 0 && yy < H && xx >= 0 && xx < Wd)
-        v = *reinterpret_cast<const uint4 *>(xp + ((long)yy * Wd + xx) * xcs + 8 * c);
+      if (yy >= 0 && yy < H && xx >= 0 && xx < Wd) {
+        const uint16_t *s = xp + ((long)yy * Wd + xx) * xcs + 8 * c - CU;
+        if (CU > 0 && c < CU / 8)  // the upsampled channels (k_conv)
+          s = upl + ((long)(yy >> 1) * (Wd >> 1) + (xx >> 1)) * CU + 8 * c;
+        v = *reinterpret_cast<const uint4 *>(s);
+      }
       *reinterpret_cast<uint4 *>(&Xs[rr][p][8 * c]) = v;
     }
     const uint16_t *dp = dy + (((nn * D + z) * H + y0) * Wd + xs) * dycs;
@@ -494,60 +529,67 @@ __global__ void k_first_fwd(const float *__restrict__ x, const float *__restrict
 
 // Four consecutive x positions per thread (Wd % 4 == 0, 16-byte aligned x and
 // y, cout % 8 == 0): each of the nine (z, y) rows of the 3x3x3 neighbourhood
-// is one 16-byte load plus its two end cells, a quarter of the loads of one
-// position per thread.  The taps and their order are k_first_fwd's: the same
-// arithmetic for every output.
-__global__ void k_first_fwd4(const float *__restrict__ x, const float *__restrict__ W,
-                             const float *__restrict__ b, uint16_t *y, int ycs, int cout, int N,
-                             int D, int H, int Wd) {
+// is one 16-byte load plus its two end cells, and a weight, which all lanes
+// share, is loaded once for the four positions (once for each of them, with
+// the loads in the way of the products, took 85.6 us at 8 x 64^3 x 16, now
+// 38.2; the products alone are 23 us of the vector unit).  The taps and their
+// order are k_first_fwd's: the same arithmetic for every output.
+__global__ void __launch_bounds__(256)
+k_first_fwd4(const float *__restrict__ x, const float *__restrict__ W,
+             const float *__restrict__ b, uint16_t *__restrict__ y, int ycs, int cout, int D,
+             int H, int Wd, long nq) {
   const int wq = Wd >> 2;
-  const long nq = (long)N * D * H * wq;
-  for (long q = (long)blockIdx.x * blockDim.x + threadIdx.x; q < nq;
-       q += (long)gridDim.x * blockDim.x) {
-    const int x0 = (int)(q % wq) * 4;
-    long r = q / wq;
-    const int yv = (int)(r % H);
-    r /= H;
-    const int zv = (int)(r % D);
-    const long nn = r / D;
-    // nb[dz * 3 + dy][k]: the input at (zv + dz - 1, yv + dy - 1, x0 + k - 1)
-    float nb[9][6];
+  const long q = (long)blockIdx.x * 256 + threadIdx.x;
+  if (q >= nq) return;
+  const int x0 = (int)(q % wq) * 4;
+  long r = q / wq;
+  const int yv = (int)(r % H);
+  r /= H;
+  const int zv = (int)(r % D);
+  const long nn = r / D;
+  // nb[dz * 3 + dy][k]: the input at (zv + dz - 1, yv + dy - 1, x0 + k - 1)
+  float nb[9][6];
 #pragma unroll
-    for (int t = 0; t < 9; ++t) {
-      const int z2 = zv + t / 3 - 1, y2 = yv + t % 3 - 1;
-      float4 c = make_float4(0.f, 0.f, 0.f, 0.f);
-      float lo = 0.f, hi = 0.f;
-      if (z2 >= 0 && z2 < D && y2 >= 0 && y2 < H) {
-        const float *row = x + ((nn * D + z2) * H + y2) * Wd;
-        c = *reinterpret_cast<const float4 *>(row + x0);
-        if (x0 > 0) lo = row[x0 - 1];
-        if (x0 + 4 < Wd) hi = row[x0 + 4];
-      }
-      nb[t][0] = lo;
-      nb[t][1] = c.x;
-      nb[t][2] = c.y;
-      nb[t][3] = c.z;
-      nb[t][4] = c.w;
-      nb[t][5] = hi;
+  for (int t = 0; t < 9; ++t) {
+    const int z2 = zv + t / 3 - 1, y2 = yv + t % 3 - 1;
+    float4 c = make_float4(0.f, 0.f, 0.f, 0.f);
+    float lo = 0.f, hi = 0.f;
+    if (z2 >= 0 && z2 < D && y2 >= 0 && y2 < H) {
+      const float *row = x + ((nn * D + z2) * H + y2) * Wd;
+      c = *reinterpret_cast<const float4 *>(row + x0);
+      if (x0 > 0) lo = row[x0 - 1];
+      if (x0 + 4 < Wd) hi = row[x0 + 4];
     }
-    const long p0 = 4 * q;  // the position of x0
+    nb[t][0] = lo;
+    nb[t][1] = c.x;
+    nb[t][2] = c.y;
+    nb[t][3] = c.z;
+    nb[t][4] = c.w;
+    nb[t][5] = hi;
+  }
+  uint16_t *o = y + 4 * q * ycs;
+  for (int c0 = 0; c0 < cout; c0 += 8) {
+    float s[4][8];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int h = 0; h < 8; ++h) s[j][h] = b[c0 + h];
+#pragma unroll
+    for (int tap = 0; tap < 27; ++tap)
+#pragma unroll
+      for (int h = 0; h < 8; ++h) {
+        const float w = W[tap * cout + c0 + h];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) s[j][h] = fmaf(w, nb[tap / 3][j + tap % 3], s[j][h]);
+      }
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      for (int c0 = 0; c0 < cout; c0 += 8) {
-        uint32_t w[4];
+      uint32_t w[4];
 #pragma unroll
-        for (int h = 0; h < 4; ++h) {
-          float s0 = b[c0 + 2 * h], s1 = b[c0 + 2 * h + 1];
-#pragma unroll
-          for (int tap = 0; tap < 27; ++tap) {
-            const float v = nb[tap / 3][j + tap % 3];
-            s0 = fmaf(W[tap * cout + c0 + 2 * h], v, s0);
-            s1 = fmaf(W[tap * cout + c0 + 2 * h + 1], v, s1);
-          }
-          w[h] = (uint32_t)f2bf(fmaxf(s0, 0.f)) | ((uint32_t)f2bf(fmaxf(s1, 0.f)) << 16);
-        }
-        *reinterpret_cast<uint4 *>(y + (p0 + j) * ycs + c0) = make_uint4(w[0], w[1], w[2], w[3]);
-      }
+      for (int h = 0; h < 4; ++h)
+        w[h] = (uint32_t)f2bf(fmaxf(s[j][2 * h], 0.f)) |
+               ((uint32_t)f2bf(fmaxf(s[j][2 * h + 1], 0.f)) << 16);
+      *reinterpret_cast<uint4 *>(o + j * ycs + c0) = make_uint4(w[0], w[1], w[2], w[3]);
     }
   }
 }
@@ -689,28 +731,40 @@ __global__ void k_relu_bwd(const float *__restrict__ dy, int dycs,
   }
 }
 
-__global__ void k_pool_fwd(const uint16_t *__restrict__ x, int xcs, uint16_t *y, int ycs, int c,
-                           int N, int D, int H, int Wd) {
-  const int d2 = D / 2, h2 = H / 2, w2 = Wd / 2;
-  const long n = (long)N * d2 * h2 * w2 * c;
-  for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (long)gridDim.x * blockDim.x) {
-    const int k = (int)(i % c);
-    long r = i / c;
-    const int xx = (int)(r % w2);
-    r /= w2;
-    const int yv = (int)(r % h2);
-    r /= h2;
-    const int zv = (int)(r % d2);
-    const int nn = (int)(r / d2);
-    float s = 0.f;
-    for (int o = 0; o < 8; ++o) {
-      const long q = (((long)nn * D + 2 * zv + (o >> 2)) * H + 2 * yv + ((o >> 1) & 1)) * Wd +
-                     2 * xx + (o & 1);
-      s += bf2f(x[q * xcs + k]);
-    }
-    y[(i / c) * ycs + k] = f2bf(0.125f * s);
+// 2x2x2 average of 8 channels of one coarse position per thread, 16 bytes a
+// load (memory bound: 28.7 us with one channel per thread at 8 x 64^3 x 16,
+// now 9.4).
+__global__ void __launch_bounds__(256)
+k_pool_fwd(const uint16_t *__restrict__ x, int xcs, uint16_t *__restrict__ y, int ycs, int c8,
+           long n, int H, int Wd) {
+  const long i = (long)blockIdx.x * 256 + threadIdx.x;
+  if (i >= n) return;
+  const int h2 = H / 2, w2 = Wd / 2;
+  const int k = (int)(i % c8) * 8;
+  const long p = i / c8;
+  const int xx = (int)(p % w2);
+  long r = p / w2;
+  const int yv = (int)(r % h2);
+  r /= h2;  // coarse plane of the batch: 2 r, 2 r + 1 are its fine planes
+  uint4 v[8];
+#pragma unroll
+  for (int o = 0; o < 8; ++o) {
+    const long q = ((2 * r + (o >> 2)) * H + 2 * yv + ((o >> 1) & 1)) * Wd + 2 * xx + (o & 1);
+    v[o] = *reinterpret_cast<const uint4 *>(x + q * xcs + k);
   }
+  uint32_t w[4];
+#pragma unroll
+  for (int h = 0; h < 4; ++h) {
+    float lo = 0.f, hi = 0.f;
+#pragma unroll
+    for (int o = 0; o < 8; ++o) {
+      const uint32_t u = h == 0 ? v[o].x : h == 1 ? v[o].y : h == 2 ? v[o].z : v[o].w;
+      lo += __uint_as_float(u << 16);
+      hi += __uint_as_float(u & 0xffff0000u);
+    }
+    w[h] = (uint32_t)f2bf(0.125f * lo) | ((uint32_t)f2bf(0.125f * hi) << 16);
+  }
+  *reinterpret_cast<uint4 *>(y + p * ycs + k) = make_uint4(w[0], w[1], w[2], w[3]);
 }
 
 __global__ void k_pool_bwd(const float *__restrict__ dy, int dycs, float *dx, int dxcs, int c,
@@ -728,46 +782,6 @@ __global__ void k_pool_bwd(const float *__restrict__ dy, int dycs, float *dx, in
     const int nn = (int)(t / D);
     const long q = (((long)nn * (D / 2) + zv / 2) * (H / 2) + yv / 2) * (Wd / 2) + xx / 2;
     dx[r * dxcs + k] += 0.125f * dy[q * dycs + k];
-  }
-}
-
-__global__ void k_up_fwd(const uint16_t *__restrict__ x, int xcs, uint16_t *y, int ycs, int c,
-                         int N, int D, int H, int Wd) {
-  // v = coarse shape; fine = 2x
-  const long n = (long)N * 8 * D * H * Wd * c;
-  for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (long)gridDim.x * blockDim.x) {
-    const int k = (int)(i % c);
-    long r = i / c;
-    const int xx = (int)(r % (2 * Wd));
-    long t = r / (2 * Wd);
-    const int yv = (int)(t % (2 * H));
-    t /= 2 * H;
-    const int zv = (int)(t % (2 * D));
-    const int nn = (int)(t / (2 * D));
-    const long q = (((long)nn * D + zv / 2) * H + yv / 2) * Wd + xx / 2;
-    y[r * ycs + k] = x[q * xcs + k];
-  }
-}
-
-// The same with 16-byte moves of 8 channels (c, both strides and both
-// slice offsets multiples of 8 channels).
-__global__ void k_up_fwd8(const uint16_t *__restrict__ x, int xcs, uint16_t *y, int ycs, int c8,
-                          int N, int D, int H, int Wd) {
-  const long n = (long)N * 8 * D * H * Wd * c8;
-  for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (long)gridDim.x * blockDim.x) {
-    const int k = (int)(i % c8) * 8;
-    long r = i / c8;
-    const int xx = (int)(r % (2 * Wd));
-    long t = r / (2 * Wd);
-    const int yv = (int)(t % (2 * H));
-    t /= 2 * H;
-    const int zv = (int)(t % (2 * D));
-    const int nn = (int)(t / (2 * D));
-    const long q = (((long)nn * D + zv / 2) * H + yv / 2) * Wd + xx / 2;
-    *reinterpret_cast<uint4 *>(y + r * ycs + k) =
-        *reinterpret_cast<const uint4 *>(x + q * xcs + k);
   }
 }
 
@@ -819,8 +833,8 @@ __global__ void k_adam(float *p, const float *__restrict__ g, float *m, float *v
 }
 
 // Output planes per sweep: as many as leave two workgroups for a compute unit.
-template <int CIN, int COUT, int MTW, int YT, int WX, int WY, bool WL>
-hipError_t conv_t(const Act &x, const uint16_t *W, const float *b, Act y, Vol v, bool f32,
+template <int CIN, int CU, int COUT, int MTW, int YT, int WX, int WY, bool WL>
+hipError_t conv_t(const Act &x, const uint16_t *up, const uint16_t *W, const float *b, Act y, Vol v, bool f32,
                   hipStream_t st) {
   if (v.w % (16 * WX) || v.h % (YT * WY)) return hipErrorInvalidValue;
   constexpr int NT = 64 * WX * WY * (COUT / 16 / MTW);
@@ -829,62 +843,70 @@ hipError_t conv_t(const Act &x, const uint16_t *W, const float *b, Act y, Vol v,
   while (zl > 1 && (v.d % zl || tiles * (v.d / zl) < (NT > 256 ? 256 : 512))) zl /= 2;
   const int grid = (int)(tiles * (v.d / zl));
   if (f32)
-    k_conv<CIN, COUT, MTW, YT, WX, WY, WL, OUT_GRAD><<<grid, NT, 0, st>>>(
-        (const uint16_t *)x.p, x.cs, W, b, y.p, y.cs, zl, v.d, v.h, v.w);
+    k_conv<CIN, CU, COUT, MTW, YT, WX, WY, WL, OUT_GRAD><<<grid, NT, 0, st>>>(
+        (const uint16_t *)x.p, x.cs, up, W, b, y.p, y.cs, zl, v.d, v.h, v.w);
   else
-    k_conv<CIN, COUT, MTW, YT, WX, WY, WL, OUT_ACT><<<grid, NT, 0, st>>>(
-        (const uint16_t *)x.p, x.cs, W, b, y.p, y.cs, zl, v.d, v.h, v.w);
+    k_conv<CIN, CU, COUT, MTW, YT, WX, WY, WL, OUT_ACT><<<grid, NT, 0, st>>>(
+        (const uint16_t *)x.p, x.cs, up, W, b, y.p, y.cs, zl, v.d, v.h, v.w);
   return hipGetLastError();
 }
 
 // Workgroups of a weight gradient: up to 256 (times the three dz), fewer
 // where the volume has fewer units or the partials would pass kGradScratch.
-template <int CIN, int COUT, int SEG, int R>
-hipError_t wgrad_t(const Act &x, const Act &dy, float *dW, float *db, Vol v, float *scratch,
+template <int CIN, int CU, int COUT, int SEG, int R>
+hipError_t wgrad_t(const Act &x, const uint16_t *up, const Act &dy, float *dW, float *db, Vol v, float *scratch,
                    hipStream_t st) {
   constexpr int NW = 27 * CIN * COUT;
   if (v.w % SEG || v.h % R) return hipErrorInvalidValue;
   const long units = (long)v.n * v.d * (v.h / R) * (v.w / SEG);
   const int S = (int)std::min({units, 256L, kGradScratch / (NW + COUT)});
-  k_wgrad<CIN, COUT, SEG, R><<<dim3(S, 3), 192, 0, st>>>(
-      (const uint16_t *)x.p, x.cs, (const uint16_t *)dy.p, dy.cs, scratch, v.d, v.h, v.w, units);
+  k_wgrad<CIN, CU, COUT, SEG, R><<<dim3(S, 3), 192, 0, st>>>(
+      (const uint16_t *)x.p, x.cs, up, (const uint16_t *)dy.p, dy.cs, scratch, v.d, v.h, v.w, units);
   k_grad_sum<<<(NW + COUT + 63) / 64, 256, 0, st>>>(scratch, S, NW, COUT, dW, db);
   return hipGetLastError();
 }
 
 }  // namespace
 
-// The weight gradients of the network: (cin, cout, positions per K run, rows
-// per unit).  The level fixes the run; 96 input channels take four rows so
-// that two workgroups fit a CU's LDS.
-#define BRTM_WGRAD_SHAPES(X)                                                     \
-  X(16, 16, 64, 8) X(48, 16, 64, 8) X(16, 32, 32, 8) X(32, 32, 32, 8) X(96, 32, 32, 4) \
-  X(32, 64, 16, 8) X(64, 64, 16, 8)
+// The weight gradients of the network: (cin, of these upsampled, cout,
+// positions per K run, rows per unit).  The level fixes the run; 96 input
+// channels take four rows so that two workgroups fit a CU's LDS.
+#define BRTM_WGRAD_SHAPES(X)                                                    \
+  X(16, 0, 16, 64, 8) X(48, 32, 16, 64, 8) X(16, 0, 32, 32, 8) X(32, 0, 32, 32, 8) \
+  X(96, 64, 32, 32, 4) X(32, 0, 64, 16, 8) X(64, 0, 64, 16, 8)
 
 // The forward convolutions and the transposed ones (input gradients): (cin,
-// cout, output tiles and rows per wave, waves in x and y, weights in LDS).
-#define BRTM_CONV_SHAPES(X)                                                          \
-  X(16, 16, 1, 8, 4, 2, true) X(48, 16, 1, 8, 4, 2, true) X(16, 48, 3, 4, 4, 2, true) \
-  X(16, 32, 2, 4, 2, 2, true) X(32, 32, 2, 4, 2, 4, true) X(32, 16, 1, 4, 2, 4, true) \
-  X(96, 32, 2, 4, 2, 2, false) X(32, 96, 3, 4, 2, 2, false)                          \
-  X(32, 64, 2, 4, 1, 2, false) X(64, 64, 2, 4, 1, 2, false) X(64, 32, 1, 4, 1, 2, false)
+// of these upsampled, cout, output tiles and rows per wave, waves in x and y,
+// weights in LDS).
+#define BRTM_CONV_SHAPES(X)                                                                \
+  X(16, 0, 16, 1, 8, 4, 2, true) X(48, 32, 16, 1, 8, 4, 2, true) X(16, 0, 48, 3, 4, 4, 2, true) \
+  X(16, 0, 32, 2, 4, 2, 2, true) X(32, 0, 32, 2, 4, 2, 4, true) X(32, 0, 16, 1, 4, 2, 4, true) \
+  X(96, 64, 32, 2, 4, 2, 2, false) X(32, 0, 96, 3, 4, 2, 2, false)                          \
+  X(32, 0, 64, 2, 4, 1, 2, false) X(64, 0, 64, 2, 4, 1, 2, false) X(64, 0, 32, 1, 4, 1, 2, false)
 
-hipError_t conv3d_fwd(const Act &x, const uint16_t *W, const float *bias, Act y, Vol v,
-                      bool out_f32, hipStream_t st) {
+// Whether (x, up) are CI input channels of which the first CU are upsampled.
+static bool is_input(const Act &x, const Act &up, int ci, int cu) {
+  return up.c == cu && x.c == ci - cu && (cu == 0 || up.cs == cu);
+}
+
+hipError_t conv3d_fwd(const Act &x, const Act &up, const uint16_t *W, const float *bias, Act y,
+                      Vol v, bool out_f32, hipStream_t st) {
   if (x.cs % 8 || y.cs % 4) return hipErrorInvalidValue;
-#define X(CI, CO, MTW, YT, WX, WY, WL) \
-  if (x.c == CI && y.c == CO)          \
-    return conv_t<CI, CO, MTW, YT, WX, WY, WL>(x, W, bias, y, v, out_f32, st);
+#define X(CI, CU, CO, MTW, YT, WX, WY, WL)                                                \
+  if (is_input(x, up, CI, CU) && y.c == CO)                                               \
+    return conv_t<CI, CU, CO, MTW, YT, WX, WY, WL>(x, (const uint16_t *)up.p, W, bias, y, v, \
+                                                   out_f32, st);
   BRTM_CONV_SHAPES(X)
 #undef X
   return hipErrorInvalidValue;
 }
 
-hipError_t conv3d_wgrad(const Act &x, const Act &dy, float *dW, float *db, Vol v,
+hipError_t conv3d_wgrad(const Act &x, const Act &up, const Act &dy, float *dW, float *db, Vol v,
                         float *scratch, hipStream_t st) {
   if (x.cs % 8 || dy.cs % 8) return hipErrorInvalidValue;
-#define X(CI, CO, SEG, R) \
-  if (x.c == CI && dy.c == CO) return wgrad_t<CI, CO, SEG, R>(x, dy, dW, db, v, scratch, st);
+#define X(CI, CU, CO, SEG, R)                                                                \
+  if (is_input(x, up, CI, CU) && dy.c == CO)                                                 \
+    return wgrad_t<CI, CU, CO, SEG, R>(x, (const uint16_t *)up.p, dy, dW, db, v, scratch, st);
   BRTM_WGRAD_SHAPES(X)
 #undef X
   return hipErrorInvalidValue;
@@ -906,9 +928,10 @@ hipError_t conv3d_first_fwd(const float *x, const float *W, const float *b, Act 
   const bool quad = v.w % 4 == 0 && y.c % 8 == 0 && y.cs % 8 == 0 &&
                     reinterpret_cast<uintptr_t>(x) % 16 == 0 &&
                     reinterpret_cast<uintptr_t>(y.p) % 16 == 0;
+  const long nq = (long)v.n * v.spatial() / 4;
   if (quad)
-    k_first_fwd4<<<grid1((long)v.n * v.spatial() / 4), 256, 0, st>>>(
-        x, W, b, (uint16_t *)y.p, y.cs, y.c, v.n, v.d, v.h, v.w);
+    k_first_fwd4<<<(int)((nq + 255) / 256), 256, 0, st>>>(x, W, b, (uint16_t *)y.p, y.cs, y.c,
+                                                          v.d, v.h, v.w, nq);
   else
     k_first_fwd<<<grid1((long)v.n * v.spatial()), 256, 0, st>>>(x, W, b, (uint16_t *)y.p, y.cs,
                                                                  y.c, v.n, v.d, v.h, v.w);
@@ -950,9 +973,11 @@ hipError_t relu_bwd(const float *dy, int dy_cs, const Act &y, Act dpre, Vol v, h
 }
 
 hipError_t avgpool_fwd(const Act &x, Act y, Vol v, hipStream_t st) {
-  const long n = (long)v.n * (v.d / 2) * (v.h / 2) * (v.w / 2) * x.c;
-  k_pool_fwd<<<grid1(n), 256, 0, st>>>((const uint16_t *)x.p, x.cs, (uint16_t *)y.p, y.cs, x.c,
-                                       v.n, v.d, v.h, v.w);
+  if (x.c % 8 || x.cs % 8 || y.cs % 8 || v.d % 2 || v.h % 2 || v.w % 2)
+    return hipErrorInvalidValue;
+  const long n = (long)v.n * (v.d / 2) * (v.h / 2) * (v.w / 2) * (x.c / 8);
+  k_pool_fwd<<<(int)((n + 255) / 256), 256, 0, st>>>((const uint16_t *)x.p, x.cs,
+                                                     (uint16_t *)y.p, y.cs, x.c / 8, n, v.h, v.w);
   return hipGetLastError();
 }
 
@@ -960,20 +985,6 @@ hipError_t avgpool_bwd(const float *dy, int dy_cs, float *dx, int dx_cs, int c, 
                        hipStream_t st) {
   k_pool_bwd<<<grid1((long)v.n * v.spatial() * c), 256, 0, st>>>(dy, dy_cs, dx, dx_cs, c, v.n,
                                                                    v.d, v.h, v.w);
-  return hipGetLastError();
-}
-
-hipError_t upsample_fwd(const Act &x, Act y, Vol v, hipStream_t st) {
-  const bool vec = x.c % 8 == 0 && x.cs % 8 == 0 && y.cs % 8 == 0 &&
-                   reinterpret_cast<uintptr_t>(x.p) % 16 == 0 &&
-                   reinterpret_cast<uintptr_t>(y.p) % 16 == 0;
-  if (vec) {
-    k_up_fwd8<<<grid1((long)v.n * 8 * v.spatial() * (x.c / 8)), 256, 0, st>>>(
-        (const uint16_t *)x.p, x.cs, (uint16_t *)y.p, y.cs, x.c / 8, v.n, v.d, v.h, v.w);
-    return hipGetLastError();
-  }
-  k_up_fwd<<<grid1((long)v.n * 8 * v.spatial() * x.c), 256, 0, st>>>(
-      (const uint16_t *)x.p, x.cs, (uint16_t *)y.p, y.cs, x.c, v.n, v.d, v.h, v.w);
   return hipGetLastError();
 }
 

@@ -74,35 +74,59 @@ __global__ void k_extract(const float *__restrict__ vol, int m1, int m2, int m3,
   }
 }
 
-// Central (P - 2 ov)^3 of a patch into the volume, scaled.
-__global__ void k_insert(const float *__restrict__ src, int P, int ov, float *vol, int m1, int m2,
-                         int m3, int o1, int o2, int o3, float scale) {
-  const int S = P - 2 * ov;
-  const long n = (long)S * S * S;
-  for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (long)gridDim.x * blockDim.x) {
-    const int a = (int)(i % S) + ov, b = (int)((i / S) % S) + ov, c = (int)(i / ((long)S * S)) + ov;
-    const int x = o1 + a, y = o2 + b, z = o3 + c;
-    if (x >= 0 && x < m1 && y >= 0 && y < m2 && z >= 0 && z < m3)
-      vol[((long)z * m2 + y) * m1 + x] = scale * src[((long)c * P + b) * P + a];
+// Patches of a volume cut in blocks of S = P - 2 ov cells, k1 x k2 x ... of
+// them: patch p starts ov cells before block p.
+struct Blocks {
+  int m1, m2, m3, P, ov, k1, k2;
+  __device__ __forceinline__ void origin(int p, int &o1, int &o2, int &o3) const {
+    const int S = P - 2 * ov;
+    o1 = p % k1 * S - ov;
+    o2 = p / k1 % k2 * S - ov;
+    o3 = p / (k1 * k2) * S - ov;
   }
+};
+
+// Patches p0 .. p0 + gridDim.y - 1, scaled, zeros outside the volume; odd:
+// their negatives behind them (one launch for a batch: one of 4.6 us for each
+// patch and sign before).
+__global__ void __launch_bounds__(256)
+k_extract_all(const float *__restrict__ vol, Blocks g, int p0, float scale, bool odd, float *dst) {
+  int o1, o2, o3;
+  g.origin(p0 + blockIdx.y, o1, o2, o3);
+  const int P = g.P;
+  const long i = ((long)blockIdx.x * 256 + threadIdx.x) * 4, n = (long)P * P * P;
+  if (i >= n) return;
+  const int a = (int)(i % P), b = (int)((i / P) % P), c = (int)(i / ((long)P * P));
+  const int x = o1 + a, y = o2 + b, z = o3 + c;
+  const bool row = y >= 0 && y < g.m2 && z >= 0 && z < g.m3;
+  const float *v = vol + ((long)z * g.m2 + y) * g.m1 + x;
+  float f[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k)
+    f[k] = scale * (row && x + k >= 0 && x + k < g.m1 ? v[k] : 0.f);
+  float *d = dst + blockIdx.y * n + i;
+  *reinterpret_cast<float4 *>(d) = make_float4(f[0], f[1], f[2], f[3]);
+  if (odd)
+    *reinterpret_cast<float4 *>(d + gridDim.y * n) = make_float4(-f[0], -f[1], -f[2], -f[3]);
 }
 
-// As k_insert, of the odd part (net(x) - net(-x)) / 2 of two outputs.
-__global__ void k_insert_odd(const float *__restrict__ sp, const float *__restrict__ sm, int P,
-                             int ov, float *vol, int m1, int m2, int m3, int o1, int o2, int o3,
-                             float scale) {
-  const int S = P - 2 * ov;
-  const long n = (long)S * S * S;
-  for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (long)gridDim.x * blockDim.x) {
-    const int a = (int)(i % S) + ov, b = (int)((i / S) % S) + ov, c = (int)(i / ((long)S * S)) + ov;
-    const int x = o1 + a, y = o2 + b, z = o3 + c;
-    if (x >= 0 && x < m1 && y >= 0 && y < m2 && z >= 0 && z < m3) {
-      const long j = ((long)c * P + b) * P + a;
-      vol[((long)z * m2 + y) * m1 + x] = 0.5f * scale * (sp[j] - sm[j]);
-    }
-  }
+// Central (P - 2 ov)^3 of each patch's output into the volume, scaled; odd:
+// of the odd part (net(x) - net(-x)) / 2 of two outputs.
+__global__ void __launch_bounds__(256)
+k_insert_all(const float *__restrict__ src, Blocks g, int p0, float scale, bool odd, float *vol) {
+  int o1, o2, o3;
+  g.origin(p0 + blockIdx.y, o1, o2, o3);
+  const int P = g.P, S = P - 2 * g.ov;
+  const long n = (long)P * P * P;
+  const long i = (long)blockIdx.x * 256 + threadIdx.x;
+  if (i >= (long)S * S * S) return;
+  const int a = (int)(i % S) + g.ov, b = (int)((i / S) % S) + g.ov,
+            c = (int)(i / ((long)S * S)) + g.ov;
+  const int x = o1 + a, y = o2 + b, z = o3 + c;
+  if (x >= g.m1 || y >= g.m2 || z >= g.m3) return;  // never negative: block p's cells
+  const float *s = src + blockIdx.y * n + ((long)c * P + b) * P + a;
+  vol[((long)z * g.m2 + y) * g.m1 + x] =
+      odd ? 0.5f * scale * (s[0] - s[gridDim.y * n]) : scale * s[0];
 }
 
 struct Rng {
@@ -130,7 +154,7 @@ struct brtm_unet {
   DevBuf params, grads, am, av;
   DevBuf wbf[9], wtf[9];
   DevBuf gscratch;  // partial weight gradients
-  DevBuf e1a, cat1, p1, e2a, cat2, p2, b1, b2, d2a, d2b, d1a, d1b, out;
+  DevBuf e1a, skip1, p1, e2a, skip2, p2, b1, b2, d2a, d2b, d1a, d1b, out;
   DevBuf g_out, dy_d1b, dy_d1a, dy_cat1, dy_d2b, dy_d2a, dy_cat2, dy_b2, dy_b1, dy_p2, dy_e2a,
       dy_p1, dy_e1a, dpre;
   DevBuf partials, lossv, xpatch, ypatch;
@@ -179,38 +203,43 @@ int forward(brtm_unet *u, const float *x, int nb) {
   auto W = [&](int l) { return u->wbf[l].as<uint16_t>(); };
   auto Bv = [&](int l) { return pr + u->bl[l]; };
   BRTM_HIP(conv3d_first_fwd(x, pr + u->w0, pr + u->b0, act(u->e1a, C1, C1), v1, st));
-  BRTM_HIP(conv3d_fwd(act(u->e1a, C1, C1), W(0), Bv(0), act(u->cat1, C1, 48, 32), v1, false, st));
-  BRTM_HIP(avgpool_fwd(act(u->cat1, C1, 48, 32), act(u->p1, C1, C1), v1, st));
-  BRTM_HIP(conv3d_fwd(act(u->p1, C1, C1), W(1), Bv(1), act(u->e2a, C2, C2), v2, false, st));
-  BRTM_HIP(conv3d_fwd(act(u->e2a, C2, C2), W(2), Bv(2), act(u->cat2, C2, 96, 64), v2, false, st));
-  BRTM_HIP(avgpool_fwd(act(u->cat2, C2, 96, 64), act(u->p2, C2, C2), v2, st));
-  BRTM_HIP(conv3d_fwd(act(u->p2, C2, C2), W(3), Bv(3), act(u->b1, C3, C3), v3, false, st));
-  BRTM_HIP(conv3d_fwd(act(u->b1, C3, C3), W(4), Bv(4), act(u->b2, C3, C3), v3, false, st));
-  BRTM_HIP(upsample_fwd(act(u->b2, C3, C3), act(u->cat2, C3, 96, 0), v3, st));
-  BRTM_HIP(conv3d_fwd(act(u->cat2, 96, 96), W(5), Bv(5), act(u->d2a, C2, C2), v2, false, st));
-  BRTM_HIP(conv3d_fwd(act(u->d2a, C2, C2), W(6), Bv(6), act(u->d2b, C2, C2), v2, false, st));
-  BRTM_HIP(upsample_fwd(act(u->d2b, C2, C2), act(u->cat1, C2, 48, 0), v2, st));
-  BRTM_HIP(conv3d_fwd(act(u->cat1, 48, 48), W(7), Bv(7), act(u->d1a, C1, C1), v1, false, st));
-  BRTM_HIP(conv3d_fwd(act(u->d1a, C1, C1), W(8), Bv(8), act(u->d1b, C1, C1), v1, false, st));
+  // layer l, from x (and up, of half the size) to y
+  auto conv = [&](int l, const Act &x, const Act &up, const Act &y, const Vol &v) {
+    return conv3d_fwd(x, up, W(l), Bv(l), y, v, false, st);
+  };
+  const Act none{nullptr, 0, 0};
+  const Act s1 = act(u->skip1, C1, C1), s2 = act(u->skip2, C2, C2), b2 = act(u->b2, C3, C3),
+            d2b = act(u->d2b, C2, C2);
+  BRTM_HIP(conv(0, act(u->e1a, C1, C1), none, s1, v1));
+  BRTM_HIP(avgpool_fwd(s1, act(u->p1, C1, C1), v1, st));
+  BRTM_HIP(conv(1, act(u->p1, C1, C1), none, act(u->e2a, C2, C2), v2));
+  BRTM_HIP(conv(2, act(u->e2a, C2, C2), none, s2, v2));
+  BRTM_HIP(avgpool_fwd(s2, act(u->p2, C2, C2), v2, st));
+  BRTM_HIP(conv(3, act(u->p2, C2, C2), none, act(u->b1, C3, C3), v3));
+  BRTM_HIP(conv(4, act(u->b1, C3, C3), none, b2, v3));
+  BRTM_HIP(conv(5, s2, b2, act(u->d2a, C2, C2), v2));
+  BRTM_HIP(conv(6, act(u->d2a, C2, C2), none, d2b, v2));
+  BRTM_HIP(conv(7, s1, d2b, act(u->d1a, C1, C1), v1));
+  BRTM_HIP(conv(8, act(u->d1a, C1, C1), none, act(u->d1b, C1, C1), v1));
   BRTM_HIP(head_fwd(act(u->d1b, C1, C1), pr + u->wh, pr + u->bh, x, u->out.as<float>(), v1, st));
   return BRTM_OK;
 }
 
 // Backward of one MFMA layer l: given the FP32 gradient of its (ReLU) output
 // gy (stride gcs) and its output activation y, write its parameter
-// gradients from input x and (if gx) write the input gradient gx (FP32,
-// all cin channels, stride cin).
-int layer_bwd(brtm_unet *u, int l, const float *gy, int gcs, const Act &y, const Act &x, float *gx,
-              const Vol &v) {
+// gradients from its input (x and, of half the size, up) and (if gx) write
+// the input gradient gx (FP32, all cin channels, stride cin).
+int layer_bwd(brtm_unet *u, int l, const float *gy, int gcs, const Act &y, const Act &x,
+              const Act &up, float *gx, const Vol &v) {
   hipStream_t st = u->ctx->stream;
   const int cin = kConv[l].cin, cout = kConv[l].cout;
   Act dp = act(u->dpre, cout, cout);
   BRTM_HIP(relu_bwd(gy, gcs, y, dp, v, st));
   float *G = u->grads.as<float>();
-  BRTM_HIP(conv3d_wgrad(x, dp, G + u->wl[l], G + u->bl[l], v, u->gscratch.as<float>(), st));
+  BRTM_HIP(conv3d_wgrad(x, up, dp, G + u->wl[l], G + u->bl[l], v, u->gscratch.as<float>(), st));
   if (gx) {
     Act out{gx, cin, cin};
-    BRTM_HIP(conv3d_fwd(dp, u->wtf[l].as<uint16_t>(), nullptr, out, v, true, st));
+    BRTM_HIP(conv3d_fwd(dp, Act{nullptr, 0, 0}, u->wtf[l].as<uint16_t>(), nullptr, out, v, true, st));
   }
   return BRTM_OK;
 }
@@ -227,35 +256,36 @@ int backward(brtm_unet *u, const float *x, int nb) {
   BRTM_HIP(hipMemsetAsync(G + u->wh, 0, sizeof(float) * (C1 + 1), st));
   BRTM_HIP(hipMemsetAsync(u->dy_d2b.ptr, 0, sizeof(float) * n2 * C2, st));
   BRTM_HIP(hipMemsetAsync(u->dy_b2.ptr, 0, sizeof(float) * n3 * C3, st));
+  const Act none{nullptr, 0, 0}, s1 = act(u->skip1, C1, C1), s2 = act(u->skip2, C2, C2);
   // head
   BRTM_HIP(head_bwd(act(u->d1b, C1, C1), pr + u->wh, u->g_out.as<float>(),
                     u->dy_d1b.as<float>(), C1, G + u->wh, G + u->bh, v1, st));
   // d1b, d1a
-  U_TRY(layer_bwd(u, 8, u->dy_d1b.as<float>(), C1, act(u->d1b, C1, C1), act(u->d1a, C1, C1),
+  U_TRY(layer_bwd(u, 8, u->dy_d1b.as<float>(), C1, act(u->d1b, C1, C1), act(u->d1a, C1, C1), none,
                   u->dy_d1a.as<float>(), v1));
-  U_TRY(layer_bwd(u, 7, u->dy_d1a.as<float>(), C1, act(u->d1a, C1, C1), act(u->cat1, 48, 48),
+  U_TRY(layer_bwd(u, 7, u->dy_d1a.as<float>(), C1, act(u->d1a, C1, C1), s1, act(u->d2b, C2, C2),
                   u->dy_cat1.as<float>(), v1));
-  // up1: cat1[0:32] came from d2b
+  // up1: its first 32 inputs came from d2b
   BRTM_HIP(upsample_bwd(u->dy_cat1.as<float>(), 48, u->dy_d2b.as<float>(), C2, C2, v2, st));
-  U_TRY(layer_bwd(u, 6, u->dy_d2b.as<float>(), C2, act(u->d2b, C2, C2), act(u->d2a, C2, C2),
+  U_TRY(layer_bwd(u, 6, u->dy_d2b.as<float>(), C2, act(u->d2b, C2, C2), act(u->d2a, C2, C2), none,
                   u->dy_d2a.as<float>(), v2));
-  U_TRY(layer_bwd(u, 5, u->dy_d2a.as<float>(), C2, act(u->d2a, C2, C2), act(u->cat2, 96, 96),
+  U_TRY(layer_bwd(u, 5, u->dy_d2a.as<float>(), C2, act(u->d2a, C2, C2), s2, act(u->b2, C3, C3),
                   u->dy_cat2.as<float>(), v2));
-  // up2: cat2[0:64] came from b2
+  // up2: its first 64 inputs came from b2
   BRTM_HIP(upsample_bwd(u->dy_cat2.as<float>(), 96, u->dy_b2.as<float>(), C3, C3, v3, st));
-  U_TRY(layer_bwd(u, 4, u->dy_b2.as<float>(), C3, act(u->b2, C3, C3), act(u->b1, C3, C3),
+  U_TRY(layer_bwd(u, 4, u->dy_b2.as<float>(), C3, act(u->b2, C3, C3), act(u->b1, C3, C3), none,
                   u->dy_b1.as<float>(), v3));
-  U_TRY(layer_bwd(u, 3, u->dy_b1.as<float>(), C3, act(u->b1, C3, C3), act(u->p2, C2, C2),
+  U_TRY(layer_bwd(u, 3, u->dy_b1.as<float>(), C3, act(u->b1, C3, C3), act(u->p2, C2, C2), none,
                   u->dy_p2.as<float>(), v3));
-  // e2b (cat2[64:96]) gets the skip gradient plus the pooled path
+  // e2b gets the skip gradient plus the pooled path
   BRTM_HIP(avgpool_bwd(u->dy_p2.as<float>(), C2, u->dy_cat2.as<float>() + 64, 96, C2, v2, st));
-  U_TRY(layer_bwd(u, 2, u->dy_cat2.as<float>() + 64, 96, act(u->cat2, C2, 96, 64),
-                  act(u->e2a, C2, C2), u->dy_e2a.as<float>(), v2));
-  U_TRY(layer_bwd(u, 1, u->dy_e2a.as<float>(), C2, act(u->e2a, C2, C2), act(u->p1, C1, C1),
+  U_TRY(layer_bwd(u, 2, u->dy_cat2.as<float>() + 64, 96, s2,
+                  act(u->e2a, C2, C2), none, u->dy_e2a.as<float>(), v2));
+  U_TRY(layer_bwd(u, 1, u->dy_e2a.as<float>(), C2, act(u->e2a, C2, C2), act(u->p1, C1, C1), none,
                   u->dy_p1.as<float>(), v2));
   BRTM_HIP(avgpool_bwd(u->dy_p1.as<float>(), C1, u->dy_cat1.as<float>() + 32, 48, C1, v1, st));
-  U_TRY(layer_bwd(u, 0, u->dy_cat1.as<float>() + 32, 48, act(u->cat1, C1, 48, 32),
-                  act(u->e1a, C1, C1), u->dy_e1a.as<float>(), v1));
+  U_TRY(layer_bwd(u, 0, u->dy_cat1.as<float>() + 32, 48, s1,
+                  act(u->e1a, C1, C1), none, u->dy_e1a.as<float>(), v1));
   // first layer: ReLU backward then weight gradient (no input gradient)
   Act dp = act(u->dpre, C1, C1);
   BRTM_HIP(relu_bwd(u->dy_e1a.as<float>(), C1, act(u->e1a, C1, C1), dp, v1, st));
@@ -333,10 +363,10 @@ int brtm_unet_create(brtm_ctx *ctx, int batch, int patch, unsigned long long see
   }
   A(u->gscratch, f4 * kGradScratch);
   A(u->e1a, bf * B * P3 * C1);
-  A(u->cat1, bf * B * P3 * 48);
+  A(u->skip1, bf * B * P3 * C1);
   A(u->p1, bf * B * P3b * C1);
   A(u->e2a, bf * B * P3b * C2);
-  A(u->cat2, bf * B * P3b * 96);
+  A(u->skip2, bf * B * P3b * C2);
   A(u->p2, bf * B * P3c * C2);
   A(u->b1, bf * B * P3c * C3);
   A(u->b2, bf * B * P3c * C3);
@@ -472,47 +502,28 @@ static int apply_signed(brtm_unet *u, const brtm_vec *g, brtm_vec *z, int m1, in
   U_TRY(brtm_vec_dot(g, g, &gg));
   const long n = brtm_vec_size(g);
   const double rms = std::sqrt(gg / (double)n);
-  BRTM_HIP(hipMemsetAsync(brtm_vec_data(z), 0, sizeof(float) * n, u->ctx->stream));
-  if (rms == 0) return BRTM_OK;
-  const int S = u->P - 2 * ov;
-  const int k1 = (m1 + S - 1) / S, k2 = (m2 + S - 1) / S, k3 = (m3 + S - 1) / S;
-  std::vector<int> orig;
-  for (int c = 0; c < k3; ++c)
-    for (int b = 0; b < k2; ++b)
-      for (int a = 0; a < k1; ++a) {
-        orig.push_back(a * S - ov);
-        orig.push_back(b * S - ov);
-        orig.push_back(c * S - ov);
-      }
-  const int np = (int)orig.size() / 3;
   const float *gp = static_cast<const float *>(brtm_vec_data(const_cast<brtm_vec *>(g)));
   float *zp = static_cast<float *>(brtm_vec_data(z));
   hipStream_t st = u->ctx->stream;
+  if (rms == 0) {
+    BRTM_HIP(hipMemsetAsync(zp, 0, sizeof(float) * n, st));
+    return BRTM_OK;
+  }
+  // the blocks cover the volume: every cell of z is written
+  const int S = u->P - 2 * ov;
+  const int k1 = (m1 + S - 1) / S, k2 = (m2 + S - 1) / S, k3 = (m3 + S - 1) / S;
+  const Blocks blk{m1, m2, m3, u->P, ov, k1, k2};
+  const int np = k1 * k2 * k3;
   const int per = odd ? u->B / 2 : u->B;  // patches per forward pass
+  const int ge = (int)(u->P3 / 1024), gi = (int)(((long)S * S * S + 255) / 256);
   for (int p0 = 0; p0 < np; p0 += per) {
     const int nb = std::min(per, np - p0);
-    for (int k = 0; k < nb; ++k) {
-      const int *o = &orig[3 * (p0 + k)];
-      k_extract<<<1024, 256, 0, st>>>(gp, m1, m2, m3, o[0], o[1], o[2],
-                                      sign * (float)(1.0 / rms),
-                                      u->xpatch.as<float>() + k * u->P3, u->P);
-      if (odd)
-        k_extract<<<1024, 256, 0, st>>>(gp, m1, m2, m3, o[0], o[1], o[2],
-                                        -sign * (float)(1.0 / rms),
-                                        u->xpatch.as<float>() + (nb + k) * u->P3, u->P);
-    }
+    k_extract_all<<<dim3(ge, nb), 256, 0, st>>>(gp, blk, p0, sign * (float)(1.0 / rms), odd,
+                                                u->xpatch.as<float>());
     BRTM_HIP(hipGetLastError());
     U_TRY(forward(u, u->xpatch.as<float>(), odd ? 2 * nb : nb));
-    for (int k = 0; k < nb; ++k) {
-      const int *o = &orig[3 * (p0 + k)];
-      const float *out = u->out.as<float>();
-      if (odd)
-        k_insert_odd<<<1024, 256, 0, st>>>(out + k * u->P3, out + (nb + k) * u->P3, u->P, ov, zp,
-                                           m1, m2, m3, o[0], o[1], o[2], sign * (float)rms);
-      else
-        k_insert<<<1024, 256, 0, st>>>(out + k * u->P3, u->P, ov, zp, m1, m2, m3, o[0], o[1],
-                                       o[2], sign * (float)rms);
-    }
+    k_insert_all<<<dim3(gi, nb), 256, 0, st>>>(u->out.as<float>(), blk, p0, sign * (float)rms,
+                                               odd, zp);
     BRTM_HIP(hipGetLastError());
   }
   return BRTM_OK;
