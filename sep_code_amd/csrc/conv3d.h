@@ -20,23 +20,33 @@ struct Vol {          // spatial shape (per batch item)
   long spatial() const { return (long)d * h * w; }
 };
 
-// y = ReLU(conv3x3x3(x, W) + b), zero padding 1; out_f32: y is FP32 (no bias,
-// no ReLU: the input gradient).
+// y = ReLU(conv3x3x3(x, W) + b), zero padding 1.
 // up: the first input channels when they come from a volume of half the size
 // through nearest-neighbour upsampling (channels contiguous), or no channels.
 hipError_t conv3d_fwd(const Act &x, const Act &up, const uint16_t *W, const float *bias, Act y,
-                      Vol v, bool out_f32, hipStream_t st);
+                      Vol v, hipStream_t st);
+// Input gradient: the convolution of dy with the transposed weights, FP32
+// into dx; with act (the input itself, an activation), through its ReLU
+// (dx = 0 where act <= 0) as BF16.
+hipError_t conv3d_bwd(const Act &dy, const uint16_t *Wt, const Act &act, Act dx, Vol v,
+                      hipStream_t st);
 // dW[tap][co][ci] = sum_p dy[p][co] x[p + tap][ci] (FP32, [27][cout][cin]);
 // db[co] = sum_p dy[p][co].  scratch holds kGradScratch floats.
 constexpr long kGradScratch = 8L << 20;
 hipError_t conv3d_wgrad(const Act &x, const Act &up, const Act &dy, float *dW, float *db, Vol v,
                         float *scratch, hipStream_t st);
-// Weights of the transposed convolution: Wt[tap][ci][co] = W[26-tap][co][ci]
-// (cin/cout swapped, pads to 32 on the new input channels).
-hipError_t conv3d_flip_weights(const uint16_t *W, uint16_t *Wt, int cin, int cout,
-                               hipStream_t st);
-// FP32 master weights [27][cout][cin] -> BF16 padded [27][cout][cin_pad].
-hipError_t pack_weights(const float *Wf, uint16_t *W, int cin, int cout, hipStream_t st);
+// BF16 weights of a layer from the FP32 masters w [27][cout][cin]: W
+// [27][cout][cin_pad], and those of the transposed convolution Wt[tap][ci][co]
+// = W[26-tap][co][ci] (channels padded to 32).
+struct PackLayer {
+  const float *w;
+  uint16_t *W, *Wt;
+  int cin, cout;
+};
+struct PackTable {
+  PackLayer l[9];
+};
+hipError_t pack_weights(const PackTable &t, int layers, hipStream_t st);
 
 // First layer: 1 FP32 input channel -> cout BF16 channels, ReLU.
 hipError_t conv3d_first_fwd(const float *x, const float *W, const float *b, Act y, Vol v,
@@ -47,22 +57,19 @@ hipError_t conv3d_first_wgrad(const float *x, const Act &dy, float *dW, float *d
 // Head: 1x1x1 conv cin -> 1 FP32 plus the residual input: out = x0 + W.y + b.
 hipError_t head_fwd(const Act &y, const float *W, const float *b, const float *x0, float *out,
                     Vol v, hipStream_t st);
-// Head backward: dy[p][c] = g[p] W[c] (FP32 act gradient), dW, db sums.
-hipError_t head_bwd(const Act &y, const float *W, const float *g, float *dy, int dy_cs,
-                    float *dW, float *db, Vol v, hipStream_t st);
+// Head backward: dpre = g W through the ReLU of y (BF16), dW and db.
+hipError_t head_bwd(const Act &y, const float *W, const float *g, Act dpre, float *dW, float *db,
+                    Vol v, float *scratch, hipStream_t st);
 
-// dpre = dy * (y > 0) as BF16 (ReLU backward into an MFMA operand).
-hipError_t relu_bwd(const float *dy, int dy_cs, const Act &y, Act dpre, Vol v,
-                    hipStream_t st);
-// 2x2x2 average pool (v is the input shape) and its adjoint (accumulates).
+// 2x2x2 average pool (v is the input shape).
 hipError_t avgpool_fwd(const Act &x, Act y, Vol v, hipStream_t st);
-hipError_t avgpool_bwd(const float *dy, int dy_cs, float *dx, int dx_cs, int c, Vol v,
-                       hipStream_t st);
-// Adjoint of nearest x2 upsampling (v is the coarse shape; accumulates).
-hipError_t upsample_bwd(const float *dy, int dy_cs, float *dx, int dx_cs, int c, Vol v,
-                        hipStream_t st);
-// dst (FP32, stride dcs) += src (FP32, stride scs) over c channels.
-hipError_t add_channels(const float *src, int scs, float *dst, int dcs, int c, long npos,
+// Gradient of a pooled activation y that also is a skip connection: dskip
+// plus the pool's adjoint of dpool, through y's ReLU.
+hipError_t avgpool_bwd(const float *dskip, int dskip_cs, const float *dpool, const Act &y,
+                       Act dpre, Vol v, hipStream_t st);
+// Gradient of an activation y (of shape v) that was upsampled x2: the adjoint
+// of the upsampling, through y's ReLU.
+hipError_t upsample_bwd(const float *dy, int dy_cs, const Act &y, Act dpre, Vol v,
                         hipStream_t st);
 // Adam step on FP32 parameters.
 hipError_t adam_step(float *p, const float *g, float *m, float *v, long n, float lr, float b1,

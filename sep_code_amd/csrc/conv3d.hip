@@ -59,8 +59,18 @@ __device__ __forceinline__ int opaque(int v) {
   return v;
 }
 
+// Two gradients through the ReLU of two BF16 activations, as BF16.
+__device__ __forceinline__ uint32_t masked2(uint32_t act, float g0, float g1) {
+  g0 = __uint_as_float(act << 16) > 0.f ? g0 : 0.f;
+  g1 = __uint_as_float(act & 0xffff0000u) > 0.f ? g1 : 0.f;
+  return (uint32_t)f2bf(g0) | ((uint32_t)f2bf(g1) << 16);
+}
+
 // What happens to a finished output tile.
-enum { OUT_ACT = 0, OUT_GRAD = 1 };  // bias + ReLU to BF16; FP32 as it is
+// OUT_ACT: bias and ReLU, BF16.  OUT_GRAD: FP32 as it is.  OUT_MASK: an input
+// gradient through the ReLU that made that input, BF16 (zero where the
+// activation aux is not positive).
+enum { OUT_ACT = 0, OUT_GRAD = 1, OUT_MASK = 2 };
 
 // A workgroup sweeps z over zl output planes of a tile of 16 WX positions by
 // YT WY rows.  Each input plane of the tile (with its halo, zeros outside the
@@ -87,7 +97,8 @@ enum { OUT_ACT = 0, OUT_GRAD = 1 };  // bias + ReLU to BF16; FP32 as it is
 template <int CIN, int CU, int COUT, int MTW, int YT, int WX, int WY, bool WL, int OUT>
 __global__ void __launch_bounds__(64 * WX * WY * (COUT / 16 / MTW), 2)
 k_conv(const uint16_t *__restrict__ x, int xcs, const uint16_t *__restrict__ up,
-       const uint16_t *__restrict__ W, const float *__restrict__ bias, void *y, int ycs, int zl, int D, int H, int Wd) {
+       const uint16_t *__restrict__ W, const void *__restrict__ aux, void *y, int ycs, int zl,
+       int D, int H, int Wd) {
   constexpr int CIN_P = (CIN + 31) / 32 * 32;
   constexpr int NT = 64 * WX * WY * (COUT / 16 / MTW);
   constexpr int NC = CIN / 32;          // 32-channel chunks
@@ -180,8 +191,12 @@ k_conv(const uint16_t *__restrict__ x, int xcs, const uint16_t *__restrict__ up,
         const f32x4 v = acc[2][m][t];
         if constexpr (OUT == OUT_GRAD) {
           *reinterpret_cast<f32x4 *>(static_cast<float *>(y) + o + c0) = v;
+        } else if constexpr (OUT == OUT_MASK) {
+          const uint2 a = *reinterpret_cast<const uint2 *>(static_cast<const uint16_t *>(aux) + o + c0);
+          *reinterpret_cast<uint2 *>(static_cast<uint16_t *>(y) + o + c0) =
+              make_uint2(masked2(a.x, v[0], v[1]), masked2(a.y, v[2], v[3]));
         } else {
-          const float4 b = *reinterpret_cast<const float4 *>(bias + c0);
+          const float4 b = *reinterpret_cast<const float4 *>(static_cast<const float *>(aux) + c0);
           const float v0 = fmaxf(v[0] + b.x, 0.f), v1 = fmaxf(v[1] + b.y, 0.f);
           const float v2 = fmaxf(v[2] + b.z, 0.f), v3 = fmaxf(v[3] + b.w, 0.f);
           *reinterpret_cast<uint2 *>(static_cast<uint16_t *>(y) + o + c0) =
@@ -457,27 +472,22 @@ k_grad_sum(const float *__restrict__ part, int S, int nw, int nb, float *dW, flo
   }
 }
 
-__global__ void k_flip(const uint16_t *W, uint16_t *Wt, int cin, int cout) {
-  // W [27][cout][cin_p] -> Wt [27][cin][cout_p]
-  const int cin_p = cpad(cin), cout_p = cpad(cout);
-  const long n = 27L * cin * cout_p;
-  for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (long)gridDim.x * blockDim.x) {
-    const int co = (int)(i % cout_p);
-    const int ci = (int)((i / cout_p) % cin);
-    const int tap = (int)(i / ((long)cout_p * cin));
-    Wt[i] = co < cout ? W[((long)(26 - tap) * cout + co) * cin_p + ci] : (uint16_t)0;
-  }
-}
-
-__global__ void k_pack(const float *Wf, uint16_t *W, int cin, int cout) {
-  const int cin_p = cpad(cin);
-  const long n = 27L * cout * cin_p;
-  for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (long)gridDim.x * blockDim.x) {
-    const int ci = (int)(i % cin_p);
-    const long r = i / cin_p;  // tap*cout + co
-    W[i] = ci < cin ? f2bf(Wf[r * cin + ci]) : (uint16_t)0;
+// BF16 weights of every layer, forward [27][cout][cin_p] and transposed
+// [27][cin][cout_p], from the FP32 parameters: one launch (two for each layer
+// before, 47 us of a training step).
+__global__ void __launch_bounds__(256) k_pack(PackTable t) {
+  const PackLayer l = t.l[blockIdx.y];
+  const int cin_p = cpad(l.cin), cout_p = cpad(l.cout);
+  const int n = 27 * l.cout * cin_p, nt = 27 * l.cin * cout_p;
+  for (int i = blockIdx.x * 256 + threadIdx.x; i < n + nt; i += gridDim.x * 256) {
+    if (i < n) {
+      const int ci = i % cin_p, r = i / cin_p;  // r = tap * cout + co
+      l.W[i] = ci < l.cin ? f2bf(l.w[(long)r * l.cin + ci]) : (uint16_t)0;
+    } else {
+      const int j = i - n, co = j % cout_p, ci = j / cout_p % l.cin, tap = j / (cout_p * l.cin);
+      l.Wt[j] = co < l.cout ? f2bf(l.w[((long)(26 - tap) * l.cout + co) * l.cin + ci])
+                            : (uint16_t)0;
+    }
   }
 }
 
@@ -690,47 +700,48 @@ __global__ void k_head_fwd(const uint16_t *__restrict__ y, int ycs, int c,
   }
 }
 
-__global__ void k_head_bwd(const uint16_t *__restrict__ y, int ycs, int c,
-                           const float *__restrict__ W, const float *__restrict__ g, float *dy,
-                           int dycs, float *dW, float *db, long npos) {
-  float acc[17];
-  for (int k = 0; k <= c; ++k) acc[k] = 0.f;
-  for (long p = (long)blockIdx.x * blockDim.x + threadIdx.x; p < npos;
-       p += (long)gridDim.x * blockDim.x) {
+// Head backward: the gradient g W of the last activation y through its ReLU,
+// and the head's own gradient (16 channels and the bias) as one partial sum
+// per workgroup.  One position of 16 channels per thread in 16-byte moves;
+// writing the gradient in FP32 one channel at a time, to be masked in another
+// pass, took 181 + 35 us at 4 x 64^3, now 16.
+__global__ void __launch_bounds__(256)
+k_head_bwd(const uint16_t *__restrict__ y, const float *__restrict__ W,
+           const float *__restrict__ g, uint16_t *__restrict__ dpre, float *__restrict__ part,
+           long npos) {
+  float acc[17] = {};
+  for (long p = (long)blockIdx.x * 256 + threadIdx.x; p < npos; p += (long)gridDim.x * 256) {
     const float gv = g[p];
-    for (int k = 0; k < c; ++k) {
-      dy[p * dycs + k] = gv * W[k];
-      acc[k] = fmaf(gv, bf2f(y[p * ycs + k]), acc[k]);
+    const uint4 *src = reinterpret_cast<const uint4 *>(y + p * 16);
+    const uint4 u[2] = {src[0], src[1]};
+    uint32_t o[8];
+#pragma unroll
+    for (int h = 0; h < 8; ++h) {
+      const uint4 q = u[h / 4];
+      const uint32_t a = h % 4 == 0 ? q.x : h % 4 == 1 ? q.y : h % 4 == 2 ? q.z : q.w;
+      o[h] = masked2(a, gv * W[2 * h], gv * W[2 * h + 1]);
+      acc[2 * h] = fmaf(gv, __uint_as_float(a << 16), acc[2 * h]);
+      acc[2 * h + 1] = fmaf(gv, __uint_as_float(a & 0xffff0000u), acc[2 * h + 1]);
     }
-    acc[c] += gv;
+    uint4 *dst = reinterpret_cast<uint4 *>(dpre + p * 16);
+    dst[0] = make_uint4(o[0], o[1], o[2], o[3]);
+    dst[1] = make_uint4(o[4], o[5], o[6], o[7]);
+    acc[16] += gv;
   }
-  __shared__ float red[256];
-  for (int k = 0; k <= c; ++k) {
-    red[threadIdx.x] = acc[k];
-    __syncthreads();
-    for (int o = blockDim.x / 2; o > 0; o >>= 1) {
-      if ((int)threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
-      __syncthreads();
-    }
-    if (threadIdx.x == 0) atomicAdd(k < c ? dW + k : db, red[0]);
-    __syncthreads();
+  __shared__ float red[4][17];
+#pragma unroll
+  for (int k = 0; k < 17; ++k) {
+#pragma unroll
+    for (int m = 32; m > 0; m >>= 1) acc[k] += __shfl_xor(acc[k], m);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6][k] = acc[k];
   }
+  __syncthreads();
+  if (threadIdx.x < 17)
+    part[blockIdx.x * 17 + threadIdx.x] = (red[0][threadIdx.x] + red[1][threadIdx.x]) +
+                                          (red[2][threadIdx.x] + red[3][threadIdx.x]);
 }
 
 // ----------------------------------------------------------- elementwise
-__global__ void k_relu_bwd(const float *__restrict__ dy, int dycs,
-                           const uint16_t *__restrict__ y, int ycs, uint16_t *dpre, int dcs,
-                           int c, long npos) {
-  const long n = npos * c;
-  for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (long)gridDim.x * blockDim.x) {
-    const long p = i / c;
-    const int k = (int)(i % c);
-    const float g = bf2f(y[p * ycs + k]) > 0.f ? dy[p * dycs + k] : 0.f;
-    dpre[p * dcs + k] = f2bf(g);
-  }
-}
-
 // 2x2x2 average of 8 channels of one coarse position per thread, 16 bytes a
 // load (memory bound: 28.7 us with one channel per thread at 8 x 64^3 x 16,
 // now 9.4).
@@ -767,56 +778,65 @@ k_pool_fwd(const uint16_t *__restrict__ x, int xcs, uint16_t *__restrict__ y, in
   *reinterpret_cast<uint4 *>(y + p * ycs + k) = make_uint4(w[0], w[1], w[2], w[3]);
 }
 
-__global__ void k_pool_bwd(const float *__restrict__ dy, int dycs, float *dx, int dxcs, int c,
-                           int N, int D, int H, int Wd) {
-  const long n = (long)N * D * H * Wd * c;  // over fine positions
-  for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (long)gridDim.x * blockDim.x) {
-    const int k = (int)(i % c);
-    long r = i / c;
-    const int xx = (int)(r % Wd);
-    long t = r / Wd;
-    const int yv = (int)(t % H);
-    t /= H;
-    const int zv = (int)(t % D);
-    const int nn = (int)(t / D);
-    const long q = (((long)nn * (D / 2) + zv / 2) * (H / 2) + yv / 2) * (Wd / 2) + xx / 2;
-    dx[r * dxcs + k] += 0.125f * dy[q * dycs + k];
-  }
+// Gradient of a skip activation y: that of the decoder (FP32, stride dycs)
+// plus a 1/8 of the pooled one's, through the ReLU that made y, as BF16.
+// Four channels of a fine position per thread (memory bound; adding the
+// pooled gradient in place and masking in a second pass took 46 + 26 us on
+// average of the two levels at 4 x 64^3, now 23).
+__global__ void __launch_bounds__(256)
+k_pool_bwd(const float *__restrict__ dskip, int dscs, const float *__restrict__ dpool,
+           const uint16_t *__restrict__ y, uint16_t *__restrict__ dpre, int c4, long n, int H,
+           int Wd) {
+  const long i = (long)blockIdx.x * 256 + threadIdx.x;
+  if (i >= n) return;
+  const int k = (int)(i % c4) * 4;
+  const long p = i / c4;
+  const int xx = (int)(p % Wd);
+  long r = p / Wd;
+  const int yv = (int)(r % H);
+  r /= H;  // fine plane of the batch
+  const long q = ((r >> 1) * (H / 2) + yv / 2) * (Wd / 2) + xx / 2;
+  const float4 s = *reinterpret_cast<const float4 *>(dskip + p * dscs + k);
+  const float4 d = *reinterpret_cast<const float4 *>(dpool + q * 4 * c4 + k);
+  const uint2 a = *reinterpret_cast<const uint2 *>(y + p * 4 * c4 + k);
+  *reinterpret_cast<uint2 *>(dpre + p * 4 * c4 + k) =
+      make_uint2(masked2(a.x, s.x + 0.125f * d.x, s.y + 0.125f * d.y),
+                 masked2(a.y, s.z + 0.125f * d.z, s.w + 0.125f * d.w));
 }
 
-__global__ void k_up_bwd(const float *__restrict__ dy, int dycs, float *dx, int dxcs, int c,
-                         int N, int D, int H, int Wd) {
-  const long n = (long)N * D * H * Wd * c;  // over coarse positions
-  for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (long)gridDim.x * blockDim.x) {
-    const int k = (int)(i % c);
-    long r = i / c;
-    const int xx = (int)(r % Wd);
-    long t = r / Wd;
-    const int yv = (int)(t % H);
-    t /= H;
-    const int zv = (int)(t % D);
-    const int nn = (int)(t / D);
-    float s = 0.f;
-    for (int o = 0; o < 8; ++o) {
-      const long q = (((long)nn * 2 * D + 2 * zv + (o >> 2)) * 2 * H + 2 * yv + ((o >> 1) & 1)) *
-                         2 * Wd + 2 * xx + (o & 1);
-      s += dy[q * dycs + k];
-    }
-    dx[r * dxcs + k] += s;
+// Gradient of an upsampled activation y: the sum over its eight fine
+// positions, through the ReLU that made y, as BF16 (27 us on average of the
+// two levels at 4 x 64^3 with one channel per thread, the mask and the
+// clearing of the sums in other passes, now 20).
+__global__ void __launch_bounds__(256)
+k_up_bwd(const float *__restrict__ dy, int dycs, const uint16_t *__restrict__ y,
+         uint16_t *__restrict__ dpre, int c4, long n, int H, int Wd) {
+  const long i = (long)blockIdx.x * 256 + threadIdx.x;
+  if (i >= n) return;
+  const int k = (int)(i % c4) * 4;
+  const long p = i / c4;
+  const int xx = (int)(p % Wd);
+  long r = p / Wd;
+  const int yv = (int)(r % H);
+  r /= H;  // coarse plane of the batch
+  float4 v[8];
+#pragma unroll
+  for (int o = 0; o < 8; ++o) {
+    const long q =
+        ((2 * r + (o >> 2)) * 2 * H + 2 * yv + ((o >> 1) & 1)) * 2 * Wd + 2 * xx + (o & 1);
+    v[o] = *reinterpret_cast<const float4 *>(dy + q * dycs + k);
   }
-}
-
-__global__ void k_add_ch(const float *__restrict__ src, int scs, float *dst, int dcs, int c,
-                         long npos) {
-  const long n = npos * c;
-  for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (long)gridDim.x * blockDim.x) {
-    const long p = i / c;
-    const int k = (int)(i % c);
-    dst[p * dcs + k] += src[p * scs + k];
+  float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+  for (int o = 0; o < 8; ++o) {
+    s.x += v[o].x;
+    s.y += v[o].y;
+    s.z += v[o].z;
+    s.w += v[o].w;
   }
+  const uint2 a = *reinterpret_cast<const uint2 *>(y + p * 4 * c4 + k);
+  *reinterpret_cast<uint2 *>(dpre + p * 4 * c4 + k) =
+      make_uint2(masked2(a.x, s.x, s.y), masked2(a.y, s.z, s.w));
 }
 
 __global__ void k_adam(float *p, const float *__restrict__ g, float *m, float *v, long n,
@@ -833,8 +853,8 @@ __global__ void k_adam(float *p, const float *__restrict__ g, float *m, float *v
 }
 
 // Output planes per sweep: as many as leave two workgroups for a compute unit.
-template <int CIN, int CU, int COUT, int MTW, int YT, int WX, int WY, bool WL>
-hipError_t conv_t(const Act &x, const uint16_t *up, const uint16_t *W, const float *b, Act y, Vol v, bool f32,
+template <int OUT, int CIN, int CU, int COUT, int MTW, int YT, int WX, int WY, bool WL>
+hipError_t conv_t(const Act &x, const uint16_t *up, const uint16_t *W, const void *aux, Act y, Vol v,
                   hipStream_t st) {
   if (v.w % (16 * WX) || v.h % (YT * WY)) return hipErrorInvalidValue;
   constexpr int NT = 64 * WX * WY * (COUT / 16 / MTW);
@@ -842,12 +862,8 @@ hipError_t conv_t(const Act &x, const uint16_t *up, const uint16_t *W, const flo
   int zl = 16;
   while (zl > 1 && (v.d % zl || tiles * (v.d / zl) < (NT > 256 ? 256 : 512))) zl /= 2;
   const int grid = (int)(tiles * (v.d / zl));
-  if (f32)
-    k_conv<CIN, CU, COUT, MTW, YT, WX, WY, WL, OUT_GRAD><<<grid, NT, 0, st>>>(
-        (const uint16_t *)x.p, x.cs, up, W, b, y.p, y.cs, zl, v.d, v.h, v.w);
-  else
-    k_conv<CIN, CU, COUT, MTW, YT, WX, WY, WL, OUT_ACT><<<grid, NT, 0, st>>>(
-        (const uint16_t *)x.p, x.cs, up, W, b, y.p, y.cs, zl, v.d, v.h, v.w);
+  k_conv<CIN, CU, COUT, MTW, YT, WX, WY, WL, OUT><<<grid, NT, 0, st>>>(
+      (const uint16_t *)x.p, x.cs, up, W, aux, y.p, y.cs, zl, v.d, v.h, v.w);
   return hipGetLastError();
 }
 
@@ -875,30 +891,44 @@ hipError_t wgrad_t(const Act &x, const uint16_t *up, const Act &dy, float *dW, f
   X(16, 0, 16, 64, 8) X(48, 32, 16, 64, 8) X(16, 0, 32, 32, 8) X(32, 0, 32, 32, 8) \
   X(96, 64, 32, 32, 4) X(32, 0, 64, 16, 8) X(64, 0, 64, 16, 8)
 
-// The forward convolutions and the transposed ones (input gradients): (cin,
-// of these upsampled, cout, output tiles and rows per wave, waves in x and y,
-// weights in LDS).
-#define BRTM_CONV_SHAPES(X)                                                                \
-  X(16, 0, 16, 1, 8, 4, 2, true) X(48, 32, 16, 1, 8, 4, 2, true) X(16, 0, 48, 3, 4, 4, 2, true) \
-  X(16, 0, 32, 2, 4, 2, 2, true) X(32, 0, 32, 2, 4, 2, 4, true) X(32, 0, 16, 1, 4, 2, 4, true) \
-  X(96, 64, 32, 2, 4, 2, 2, false) X(32, 0, 96, 3, 4, 2, 2, false)                          \
-  X(32, 0, 64, 2, 4, 1, 2, false) X(64, 0, 64, 2, 4, 1, 2, false) X(64, 0, 32, 1, 4, 1, 2, false)
+// The forward convolutions (ACT) and the transposed ones (MASK, GRAD): (out,
+// cin, of these upsampled, cout, output tiles and rows per wave, waves in x
+// and y, weights in LDS).
+#define BRTM_CONV_SHAPES(X)                                                          \
+  X(ACT, 16, 0, 16, 1, 8, 4, 2, true) X(ACT, 48, 32, 16, 1, 8, 4, 2, true)           \
+  X(ACT, 16, 0, 32, 2, 4, 2, 2, true) X(ACT, 32, 0, 32, 2, 4, 2, 4, true)            \
+  X(ACT, 96, 64, 32, 2, 4, 2, 2, false) X(ACT, 32, 0, 64, 2, 4, 1, 2, false)         \
+  X(ACT, 64, 0, 64, 2, 4, 1, 2, false) X(MASK, 16, 0, 16, 1, 8, 4, 2, true)          \
+  X(MASK, 32, 0, 32, 2, 4, 2, 4, true) X(MASK, 64, 0, 64, 2, 4, 1, 2, false)         \
+  X(GRAD, 16, 0, 48, 3, 4, 4, 2, true) X(GRAD, 32, 0, 96, 3, 4, 2, 2, false)         \
+  X(GRAD, 32, 0, 16, 1, 4, 2, 4, true) X(GRAD, 64, 0, 32, 1, 4, 1, 2, false)
 
 // Whether (x, up) are CI input channels of which the first CU are upsampled.
 static bool is_input(const Act &x, const Act &up, int ci, int cu) {
   return up.c == cu && x.c == ci - cu && (cu == 0 || up.cs == cu);
 }
 
-hipError_t conv3d_fwd(const Act &x, const Act &up, const uint16_t *W, const float *bias, Act y,
-                      Vol v, bool out_f32, hipStream_t st) {
+static hipError_t conv(const Act &x, const Act &up, const uint16_t *W, const void *aux, Act y,
+                       Vol v, int out, hipStream_t st) {
   if (x.cs % 8 || y.cs % 4) return hipErrorInvalidValue;
-#define X(CI, CU, CO, MTW, YT, WX, WY, WL)                                                \
-  if (is_input(x, up, CI, CU) && y.c == CO)                                               \
-    return conv_t<CI, CU, CO, MTW, YT, WX, WY, WL>(x, (const uint16_t *)up.p, W, bias, y, v, \
-                                                   out_f32, st);
+#define X(O, CI, CU, CO, MTW, YT, WX, WY, WL)                                               \
+  if (out == OUT_##O && is_input(x, up, CI, CU) && y.c == CO)                               \
+    return conv_t<OUT_##O, CI, CU, CO, MTW, YT, WX, WY, WL>(x, (const uint16_t *)up.p, W, aux, y, \
+                                                            v, st);
   BRTM_CONV_SHAPES(X)
 #undef X
   return hipErrorInvalidValue;
+}
+
+hipError_t conv3d_fwd(const Act &x, const Act &up, const uint16_t *W, const float *bias, Act y,
+                      Vol v, hipStream_t st) {
+  return conv(x, up, W, bias, y, v, OUT_ACT, st);
+}
+
+hipError_t conv3d_bwd(const Act &dy, const uint16_t *Wt, const Act &act, Act dx, Vol v,
+                      hipStream_t st) {
+  if (act.p && act.cs != dx.cs) return hipErrorInvalidValue;
+  return conv(dy, Act{nullptr, 0, 0}, Wt, act.p, dx, v, act.p ? OUT_MASK : OUT_GRAD, st);
 }
 
 hipError_t conv3d_wgrad(const Act &x, const Act &up, const Act &dy, float *dW, float *db, Vol v,
@@ -912,14 +942,8 @@ hipError_t conv3d_wgrad(const Act &x, const Act &up, const Act &dy, float *dW, f
   return hipErrorInvalidValue;
 }
 
-hipError_t conv3d_flip_weights(const uint16_t *W, uint16_t *Wt, int cin, int cout,
-                               hipStream_t st) {
-  k_flip<<<grid1(27L * cin * cpad(cout)), 256, 0, st>>>(W, Wt, cin, cout);
-  return hipGetLastError();
-}
-
-hipError_t pack_weights(const float *Wf, uint16_t *W, int cin, int cout, hipStream_t st) {
-  k_pack<<<grid1(27L * cout * cpad(cin)), 256, 0, st>>>(Wf, W, cin, cout);
+hipError_t pack_weights(const PackTable &t, int layers, hipStream_t st) {
+  k_pack<<<dim3(64, layers), 256, 0, st>>>(t);
   return hipGetLastError();
 }
 
@@ -956,19 +980,12 @@ hipError_t head_fwd(const Act &y, const float *W, const float *b, const float *x
   return hipGetLastError();
 }
 
-hipError_t head_bwd(const Act &y, const float *W, const float *g, float *dy, int dy_cs,
-                    float *dW, float *db, Vol v, hipStream_t st) {
-  if (y.c > 16) return hipErrorInvalidValue;
+hipError_t head_bwd(const Act &y, const float *W, const float *g, Act dpre, float *dW, float *db,
+                    Vol v, float *scratch, hipStream_t st) {
+  if (y.c != 16 || y.cs != 16 || dpre.cs != 16) return hipErrorInvalidValue;
   const long npos = (long)v.n * v.spatial();
-  k_head_bwd<<<512, 256, 0, st>>>((const uint16_t *)y.p, y.cs, y.c, W, g, dy, dy_cs, dW, db,
-                                  npos);
-  return hipGetLastError();
-}
-
-hipError_t relu_bwd(const float *dy, int dy_cs, const Act &y, Act dpre, Vol v, hipStream_t st) {
-  const long npos = (long)v.n * v.spatial();
-  k_relu_bwd<<<grid1(npos * y.c), 256, 0, st>>>(dy, dy_cs, (const uint16_t *)y.p, y.cs,
-                                                (uint16_t *)dpre.p, dpre.cs, y.c, npos);
+  k_head_bwd<<<1024, 256, 0, st>>>((const uint16_t *)y.p, W, g, (uint16_t *)dpre.p, scratch, npos);
+  k_grad_sum<<<1, 256, 0, st>>>(scratch, 1024, 16, 1, dW, db);
   return hipGetLastError();
 }
 
@@ -981,23 +998,22 @@ hipError_t avgpool_fwd(const Act &x, Act y, Vol v, hipStream_t st) {
   return hipGetLastError();
 }
 
-hipError_t avgpool_bwd(const float *dy, int dy_cs, float *dx, int dx_cs, int c, Vol v,
-                       hipStream_t st) {
-  k_pool_bwd<<<grid1((long)v.n * v.spatial() * c), 256, 0, st>>>(dy, dy_cs, dx, dx_cs, c, v.n,
-                                                                   v.d, v.h, v.w);
+hipError_t avgpool_bwd(const float *dskip, int dskip_cs, const float *dpool, const Act &y,
+                       Act dpre, Vol v, hipStream_t st) {
+  if (y.c % 4 || y.cs != y.c || dpre.cs != y.c || dskip_cs % 4) return hipErrorInvalidValue;
+  const long n = (long)v.n * v.spatial() * (y.c / 4);
+  k_pool_bwd<<<(int)((n + 255) / 256), 256, 0, st>>>(dskip, dskip_cs, dpool,
+                                                     (const uint16_t *)y.p, (uint16_t *)dpre.p,
+                                                     y.c / 4, n, v.h, v.w);
   return hipGetLastError();
 }
 
-hipError_t upsample_bwd(const float *dy, int dy_cs, float *dx, int dx_cs, int c, Vol v,
+hipError_t upsample_bwd(const float *dy, int dy_cs, const Act &y, Act dpre, Vol v,
                         hipStream_t st) {
-  k_up_bwd<<<grid1((long)v.n * v.spatial() * c), 256, 0, st>>>(dy, dy_cs, dx, dx_cs, c, v.n,
-                                                                 v.d, v.h, v.w);
-  return hipGetLastError();
-}
-
-hipError_t add_channels(const float *src, int scs, float *dst, int dcs, int c, long npos,
-                        hipStream_t st) {
-  k_add_ch<<<grid1(npos * c), 256, 0, st>>>(src, scs, dst, dcs, c, npos);
+  if (y.c % 4 || y.cs != y.c || dpre.cs != y.c || dy_cs % 4) return hipErrorInvalidValue;
+  const long n = (long)v.n * v.spatial() * (y.c / 4);
+  k_up_bwd<<<(int)((n + 255) / 256), 256, 0, st>>>(dy, dy_cs, (const uint16_t *)y.p,
+                                                   (uint16_t *)dpre.p, y.c / 4, n, v.h, v.w);
   return hipGetLastError();
 }
 

@@ -155,8 +155,7 @@ struct brtm_unet {
   DevBuf wbf[9], wtf[9];
   DevBuf gscratch;  // partial weight gradients
   DevBuf e1a, skip1, p1, e2a, skip2, p2, b1, b2, d2a, d2b, d1a, d1b, out;
-  DevBuf g_out, dy_d1b, dy_d1a, dy_cat1, dy_d2b, dy_d2a, dy_cat2, dy_b2, dy_b1, dy_p2, dy_e2a,
-      dy_p1, dy_e1a, dpre;
+  DevBuf g_out, dy_cat1, dy_cat2, dy_p2, dy_p1, dpre[2];
   DevBuf partials, lossv, xpatch, ypatch;
   int step = 0;
   int gm1 = 0, gm2 = 0, gm3 = 0, gov = 8;
@@ -185,13 +184,11 @@ Act act(const DevBuf &b, int c, int cs, int c0 = 0) {
 }
 
 int repack(brtm_unet *u) {
-  hipStream_t st = u->ctx->stream;
-  for (int l = 0; l < 9; ++l) {
-    BRTM_HIP(pack_weights(u->prm() + u->wl[l], u->wbf[l].as<uint16_t>(), kConv[l].cin,
-                          kConv[l].cout, st));
-    BRTM_HIP(conv3d_flip_weights(u->wbf[l].as<uint16_t>(), u->wtf[l].as<uint16_t>(),
-                                 kConv[l].cin, kConv[l].cout, st));
-  }
+  PackTable t;
+  for (int l = 0; l < 9; ++l)
+    t.l[l] = {u->prm() + u->wl[l], u->wbf[l].as<uint16_t>(), u->wtf[l].as<uint16_t>(),
+              kConv[l].cin, kConv[l].cout};
+  BRTM_HIP(pack_weights(t, 9, u->ctx->stream));
   return BRTM_OK;
 }
 
@@ -205,7 +202,7 @@ int forward(brtm_unet *u, const float *x, int nb) {
   BRTM_HIP(conv3d_first_fwd(x, pr + u->w0, pr + u->b0, act(u->e1a, C1, C1), v1, st));
   // layer l, from x (and up, of half the size) to y
   auto conv = [&](int l, const Act &x, const Act &up, const Act &y, const Vol &v) {
-    return conv3d_fwd(x, up, W(l), Bv(l), y, v, false, st);
+    return conv3d_fwd(x, up, W(l), Bv(l), y, v, st);
   };
   const Act none{nullptr, 0, 0};
   const Act s1 = act(u->skip1, C1, C1), s2 = act(u->skip2, C2, C2), b2 = act(u->b2, C3, C3),
@@ -225,22 +222,16 @@ int forward(brtm_unet *u, const float *x, int nb) {
   return BRTM_OK;
 }
 
-// Backward of one MFMA layer l: given the FP32 gradient of its (ReLU) output
-// gy (stride gcs) and its output activation y, write its parameter
-// gradients from its input (x and, of half the size, up) and (if gx) write
-// the input gradient gx (FP32, all cin channels, stride cin).
-int layer_bwd(brtm_unet *u, int l, const float *gy, int gcs, const Act &y, const Act &x,
-              const Act &up, float *gx, const Vol &v) {
+// Backward of one MFMA layer l: from the gradient dp of its output before the
+// ReLU (BF16), its parameter gradients, with its input x and, of half the
+// size, up; and the input gradient dx: with act (the input), through that
+// activation's ReLU as BF16, else FP32.
+int layer_bwd(brtm_unet *u, int l, const Act &dp, const Act &x, const Act &up, const Act &act,
+              const Act &dx, const Vol &v) {
   hipStream_t st = u->ctx->stream;
-  const int cin = kConv[l].cin, cout = kConv[l].cout;
-  Act dp = act(u->dpre, cout, cout);
-  BRTM_HIP(relu_bwd(gy, gcs, y, dp, v, st));
   float *G = u->grads.as<float>();
   BRTM_HIP(conv3d_wgrad(x, up, dp, G + u->wl[l], G + u->bl[l], v, u->gscratch.as<float>(), st));
-  if (gx) {
-    Act out{gx, cin, cin};
-    BRTM_HIP(conv3d_fwd(dp, Act{nullptr, 0, 0}, u->wtf[l].as<uint16_t>(), nullptr, out, v, true, st));
-  }
+  BRTM_HIP(conv3d_bwd(dp, u->wtf[l].as<uint16_t>(), act, dx, v, st));
   return BRTM_OK;
 }
 
@@ -248,49 +239,36 @@ int backward(brtm_unet *u, const float *x, int nb) {
   hipStream_t st = u->ctx->stream;
   const int P = u->P;
   const Vol v1{nb, P, P, P}, v2{nb, P / 2, P / 2, P / 2}, v3{nb, P / 4, P / 4, P / 4};
-  const long n1 = (long)nb * v1.spatial(), n2 = (long)nb * v2.spatial(),
-             n3 = (long)nb * v3.spatial();
   float *G = u->grads.as<float>();
   const float *pr = u->prm();
-  // the head's gradient accumulates; every other one is written whole
-  BRTM_HIP(hipMemsetAsync(G + u->wh, 0, sizeof(float) * (C1 + 1), st));
-  BRTM_HIP(hipMemsetAsync(u->dy_d2b.ptr, 0, sizeof(float) * n2 * C2, st));
-  BRTM_HIP(hipMemsetAsync(u->dy_b2.ptr, 0, sizeof(float) * n3 * C3, st));
-  const Act none{nullptr, 0, 0}, s1 = act(u->skip1, C1, C1), s2 = act(u->skip2, C2, C2);
-  // head
-  BRTM_HIP(head_bwd(act(u->d1b, C1, C1), pr + u->wh, u->g_out.as<float>(),
-                    u->dy_d1b.as<float>(), C1, G + u->wh, G + u->bh, v1, st));
-  // d1b, d1a
-  U_TRY(layer_bwd(u, 8, u->dy_d1b.as<float>(), C1, act(u->d1b, C1, C1), act(u->d1a, C1, C1), none,
-                  u->dy_d1a.as<float>(), v1));
-  U_TRY(layer_bwd(u, 7, u->dy_d1a.as<float>(), C1, act(u->d1a, C1, C1), s1, act(u->d2b, C2, C2),
-                  u->dy_cat1.as<float>(), v1));
-  // up1: its first 32 inputs came from d2b
-  BRTM_HIP(upsample_bwd(u->dy_cat1.as<float>(), 48, u->dy_d2b.as<float>(), C2, C2, v2, st));
-  U_TRY(layer_bwd(u, 6, u->dy_d2b.as<float>(), C2, act(u->d2b, C2, C2), act(u->d2a, C2, C2), none,
-                  u->dy_d2a.as<float>(), v2));
-  U_TRY(layer_bwd(u, 5, u->dy_d2a.as<float>(), C2, act(u->d2a, C2, C2), s2, act(u->b2, C3, C3),
-                  u->dy_cat2.as<float>(), v2));
-  // up2: its first 64 inputs came from b2
-  BRTM_HIP(upsample_bwd(u->dy_cat2.as<float>(), 96, u->dy_b2.as<float>(), C3, C3, v3, st));
-  U_TRY(layer_bwd(u, 4, u->dy_b2.as<float>(), C3, act(u->b2, C3, C3), act(u->b1, C3, C3), none,
-                  u->dy_b1.as<float>(), v3));
-  U_TRY(layer_bwd(u, 3, u->dy_b1.as<float>(), C3, act(u->b1, C3, C3), act(u->p2, C2, C2), none,
-                  u->dy_p2.as<float>(), v3));
-  // e2b gets the skip gradient plus the pooled path
-  BRTM_HIP(avgpool_bwd(u->dy_p2.as<float>(), C2, u->dy_cat2.as<float>() + 64, 96, C2, v2, st));
-  U_TRY(layer_bwd(u, 2, u->dy_cat2.as<float>() + 64, 96, s2,
-                  act(u->e2a, C2, C2), none, u->dy_e2a.as<float>(), v2));
-  U_TRY(layer_bwd(u, 1, u->dy_e2a.as<float>(), C2, act(u->e2a, C2, C2), act(u->p1, C1, C1), none,
-                  u->dy_p1.as<float>(), v2));
-  BRTM_HIP(avgpool_bwd(u->dy_p1.as<float>(), C1, u->dy_cat1.as<float>() + 32, 48, C1, v1, st));
-  U_TRY(layer_bwd(u, 0, u->dy_cat1.as<float>() + 32, 48, s1,
-                  act(u->e1a, C1, C1), none, u->dy_e1a.as<float>(), v1));
-  // first layer: ReLU backward then weight gradient (no input gradient)
-  Act dp = act(u->dpre, C1, C1);
-  BRTM_HIP(relu_bwd(u->dy_e1a.as<float>(), C1, act(u->e1a, C1, C1), dp, v1, st));
-  BRTM_HIP(conv3d_first_wgrad(x, dp, G + u->w0, G + u->b0, v1, u->gscratch.as<float>(), st));
-  (void)n1;
+  const Act none{nullptr, 0, 0};
+  const Act e1a = act(u->e1a, C1, C1), s1 = act(u->skip1, C1, C1), p1 = act(u->p1, C1, C1),
+            e2a = act(u->e2a, C2, C2), s2 = act(u->skip2, C2, C2), p2 = act(u->p2, C2, C2),
+            b1 = act(u->b1, C3, C3), b2 = act(u->b2, C3, C3), d2a = act(u->d2a, C2, C2),
+            d2b = act(u->d2b, C2, C2), d1a = act(u->d1a, C1, C1), d1b = act(u->d1b, C1, C1);
+  // the gradient before each layer's ReLU, in two buffers by turns
+  auto dp = [&](int i, int c) { return act(u->dpre[i], c, c); };
+  auto gr = [](const DevBuf &b, int c) { return Act{b.ptr, c, c}; };
+  float *cat1 = u->dy_cat1.as<float>(), *cat2 = u->dy_cat2.as<float>();
+  BRTM_HIP(head_bwd(d1b, pr + u->wh, u->g_out.as<float>(), dp(0, C1), G + u->wh, G + u->bh, v1,
+                    u->gscratch.as<float>(), st));
+  U_TRY(layer_bwd(u, 8, dp(0, C1), d1a, none, d1a, dp(1, C1), v1));
+  U_TRY(layer_bwd(u, 7, dp(1, C1), s1, d2b, none, gr(u->dy_cat1, 48), v1));
+  // layer 7's first 32 inputs came from d2b
+  BRTM_HIP(upsample_bwd(cat1, 48, d2b, dp(0, C2), v2, st));
+  U_TRY(layer_bwd(u, 6, dp(0, C2), d2a, none, d2a, dp(1, C2), v2));
+  U_TRY(layer_bwd(u, 5, dp(1, C2), s2, b2, none, gr(u->dy_cat2, 96), v2));
+  // layer 5's first 64 inputs came from b2
+  BRTM_HIP(upsample_bwd(cat2, 96, b2, dp(0, C3), v3, st));
+  U_TRY(layer_bwd(u, 4, dp(0, C3), b1, none, b1, dp(1, C3), v3));
+  U_TRY(layer_bwd(u, 3, dp(1, C3), p2, none, none, gr(u->dy_p2, C2), v3));
+  BRTM_HIP(avgpool_bwd(cat2 + 64, 96, u->dy_p2.as<float>(), s2, dp(0, C2), v2, st));
+  U_TRY(layer_bwd(u, 2, dp(0, C2), e2a, none, e2a, dp(1, C2), v2));
+  U_TRY(layer_bwd(u, 1, dp(1, C2), p1, none, none, gr(u->dy_p1, C1), v2));
+  BRTM_HIP(avgpool_bwd(cat1 + 32, 48, u->dy_p1.as<float>(), s1, dp(0, C1), v1, st));
+  U_TRY(layer_bwd(u, 0, dp(0, C1), e1a, none, e1a, dp(1, C1), v1));
+  BRTM_HIP(conv3d_first_wgrad(x, dp(1, C1), G + u->w0, G + u->b0, v1, u->gscratch.as<float>(),
+                              st));
   return BRTM_OK;
 }
 
@@ -376,19 +354,12 @@ int brtm_unet_create(brtm_ctx *ctx, int batch, int patch, unsigned long long see
   A(u->d1b, bf * B * P3 * C1);
   A(u->out, f4 * B * P3);
   A(u->g_out, f4 * B * P3);
-  A(u->dy_d1b, f4 * B * P3 * C1);
-  A(u->dy_d1a, f4 * B * P3 * C1);
   A(u->dy_cat1, f4 * B * P3 * 48);
-  A(u->dy_d2b, f4 * B * P3b * C2);
-  A(u->dy_d2a, f4 * B * P3b * C2);
   A(u->dy_cat2, f4 * B * P3b * 96);
-  A(u->dy_b2, f4 * B * P3c * C3);
-  A(u->dy_b1, f4 * B * P3c * C3);
   A(u->dy_p2, f4 * B * P3c * C2);
-  A(u->dy_e2a, f4 * B * P3b * C2);
   A(u->dy_p1, f4 * B * P3b * C1);
-  A(u->dy_e1a, f4 * B * P3 * C1);
-  A(u->dpre, bf * B * P3 * C1);
+  A(u->dpre[0], bf * B * P3 * C1);
+  A(u->dpre[1], bf * B * P3 * C1);
   A(u->partials, sizeof(double) * 256);
   A(u->lossv, sizeof(double));
   A(u->xpatch, f4 * B * P3);
