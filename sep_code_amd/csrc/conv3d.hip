@@ -41,6 +41,12 @@ __device__ __forceinline__ i16x4 ld4h(const uint16_t *p) {
 }
 __device__ __forceinline__ i16x4 zero4h() { return __builtin_bit_cast(i16x4, make_uint2(0, 0)); }
 
+// v, in a form that the compiler cannot move out of a loop.
+__device__ __forceinline__ int opaque(int v) {
+  asm volatile("" : "+v"(v));
+  return v;
+}
+
 __host__ __device__ inline int cpad(int c) { return (c + 31) / 32 * 32; }
 int grid1(long n, int bs = 256) {
   long g = (n + bs - 1) / bs;
@@ -52,12 +58,6 @@ int grid1(long n, int bs = 256) {
 // a 16-byte read are that far apart, and strides of an odd number of 16-byte
 // units or of at most 64 bytes spread them over all banks.
 __host__ __device__ constexpr int pos_stride(int c) { return c > 48 ? c + 8 : c; }
-
-// v, in a form that the compiler cannot move out of a loop.
-__device__ __forceinline__ int opaque(int v) {
-  asm volatile("" : "+v"(v));
-  return v;
-}
 
 // Two gradients through the ReLU of two BF16 activations, as BF16.
 __device__ __forceinline__ uint32_t masked2(uint32_t act, float g0, float g1) {
@@ -308,8 +308,12 @@ k_conv(const uint16_t *__restrict__ x, int xcs, const uint16_t *__restrict__ up,
 // bias gradient is one more product, dy by ones, on the wave of the centre
 // tap.  Before this a workgroup per tap re-read both tensors 27 times and
 // transposed them with 2-byte LDS stores: 2.00 ms for 16->16 and 3.79 ms for
-// 48->16 at 4 x 64^3, now 0.055 and 0.22 ms (two workgroups of 80 KB of LDS
-// per CU, the stage and the products in turn).
+// 48->16 at 4 x 64^3, now 0.039 and 0.094 ms.  The next unit is loaded into
+// registers while a unit's products run (loading it only when they were done,
+// 0.055 and 0.20 ms: the loads' latency was most of the time), and WGS
+// workgroups per compute unit are launched, all resident at once (a third
+// part more of them than fit 48->16: another 9 %).  What bounds it now: LDS
+// reads and writes of the staged tile, and three waves on four matrix units.
 //
 // SEG positions per K run: 64 on the full-resolution level, 32 and 16 on the
 // coarser ones (their row lengths are multiples of these for every patch).
@@ -342,8 +346,8 @@ struct GradFrag {
   }
 };
 
-template <int CIN, int CU, int COUT, int SEG, int R>
-__global__ void __launch_bounds__(192)
+template <int CIN, int CU, int COUT, int SEG, int R, int WGS>
+__global__ void __launch_bounds__(192, WGS * 3 >= 5 ? 2 : 1)
 k_wgrad(const uint16_t *__restrict__ x, int xcs, const uint16_t *__restrict__ up,
         const uint16_t *__restrict__ dy, int dycs,
         float *__restrict__ part, int D, int H, int Wd, long units) {
@@ -369,40 +373,91 @@ k_wgrad(const uint16_t *__restrict__ x, int xcs, const uint16_t *__restrict__ up
   Frag one;
   one.ones();
   const int nseg = Wd / SEG, nyc = H / R;
-  for (long u = blockIdx.x; u < units; u += gridDim.x) {
+  // 16-byte chunks of a unit: upsampled channels, the others, dy
+  constexpr int UC = CU / 8, XC = CIN / 8 - UC, DC = COUT / 8;
+  constexpr int NU = (R + 2) * XP * UC, NX = (R + 2) * XP * XC, ND = R * SEG * DC;
+  constexpr int PU = (NU + 191) / 192, PX = (NX + 191) / 192, PD = (ND + 191) / 192;
+  uint4 pu[PU + 1], px[PX], pd[PD];
+  const uint32_t xbytes = ((uint32_t)(H * Wd - 1) * xcs + 8 * XC) * 2;
+  const uint32_t ubytes = (uint32_t)(H / 2) * (Wd / 2) * CU * 2;
+  const uint32_t dbytes = ((uint32_t)(R * Wd - 1) * dycs + COUT) * 2;
+  // the first unit from u on whose input plane is inside the volume
+  auto valid = [&](long u) {
+    for (; u < units; u += gridDim.x) {
+      const int z2 = (int)(u / ((long)nseg * nyc) % D) + dz - 1;
+      if (z2 >= 0 && z2 < D) break;
+    }
+    return u;
+  };
+  auto fetch = [&](long u) {
     const int xs = (int)(u % nseg) * SEG;
     long r = u / nseg;
     const int y0 = (int)(r % nyc) * R;
     r /= nyc;
-    const int z = (int)(r % D), z2 = z + dz - 1;
-    const long nn = r / D;
-    if (z2 < 0 || z2 >= D) continue;  // the whole workgroup: a zero plane
-    __syncthreads();                  // the previous unit has been read
-    const uint16_t *xp = x + (nn * D + z2) * H * Wd * xcs;
-    const uint16_t *upl = up + ((nn * D + z2) >> 1) * (H / 2) * (Wd / 2) * CU;
-    constexpr int XC = CIN / 8, NX = (R + 2) * XP * XC;
-#pragma unroll 4
-    for (int i = tid; i < NX; i += 192) {
-      const int c = i % XC, p = (i / XC) % XP, rr = i / (XC * XP);
-      const int yy = y0 + rr - 1, xx = xs + p - 1;
-      uint4 v = make_uint4(0, 0, 0, 0);
-      if (yy >= 0 && yy < H && xx >= 0 && xx < Wd) {
-        const uint16_t *s = xp + ((long)yy * Wd + xx) * xcs + 8 * c - CU;
-        if (CU > 0 && c < CU / 8)  // the upsampled channels (k_conv)
-          s = upl + ((long)(yy >> 1) * (Wd >> 1) + (xx >> 1)) * CU + 8 * c;
-        v = *reinterpret_cast<const uint4 *>(s);
+    const long z = r, z2 = r + dz - 1;  // planes of the batch
+    const int t_ = opaque(tid);
+    auto load = [&](const uint16_t *base, uint32_t bytes, uint32_t off) {
+      return __builtin_bit_cast(
+          uint4, __builtin_amdgcn_raw_buffer_load_b128(
+                     __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(base), 0, bytes,
+                                                       0x00020000),
+                     off, 0, 0));
+    };
+    if constexpr (CU > 0) {
+#pragma unroll
+      for (int i = 0; i < PU; ++i) {
+        const int e = t_ + i * 192, c = e % UC, p = (e / UC) % XP, rr = e / (UC * XP);
+        const int yy = y0 + rr - 1, xx = xs + p - 1;
+        const bool ok = e < NU && yy >= 0 && yy < H && xx >= 0 && xx < Wd;
+        pu[i] = load(up + (z2 >> 1) * (H / 2) * (Wd / 2) * CU, ubytes,
+                     ok ? (uint32_t)((yy >> 1) * (Wd >> 1) + (xx >> 1)) * CU * 2 + 16 * c
+                        : 0x80000000u);
       }
-      *reinterpret_cast<uint4 *>(&Xs[rr][p][8 * c]) = v;
     }
-    const uint16_t *dp = dy + (((nn * D + z) * H + y0) * Wd + xs) * dycs;
-    constexpr int DC = COUT / 8, ND = R * SEG * DC;
-#pragma unroll 4
-    for (int i = tid; i < ND; i += 192) {
-      const int c = i % DC, p = (i / DC) % SEG, rr = i / (DC * SEG);
-      *reinterpret_cast<uint4 *>(&Ds[rr][p][8 * c]) =
-          *reinterpret_cast<const uint4 *>(dp + ((long)rr * Wd + p) * dycs + 8 * c);
+#pragma unroll
+    for (int i = 0; i < PX; ++i) {
+      const int e = t_ + i * 192, c = e % XC, p = (e / XC) % XP, rr = e / (XC * XP);
+      const int yy = y0 + rr - 1, xx = xs + p - 1;
+      const bool ok = e < NX && yy >= 0 && yy < H && xx >= 0 && xx < Wd;
+      px[i] = load(x + z2 * H * Wd * xcs, xbytes,
+                   ok ? (uint32_t)(yy * Wd + xx) * xcs * 2 + 16 * c : 0x80000000u);
+    }
+#pragma unroll
+    for (int i = 0; i < PD; ++i) {
+      const int e = t_ + i * 192, c = e % DC, p = (e / DC) % SEG, rr = e / (DC * SEG);
+      pd[i] = load(dy + (z * H + y0) * Wd * dycs, dbytes,
+                   e < ND ? (uint32_t)(rr * Wd + xs + p) * dycs * 2 + 16 * c : 0x80000000u);
+    }
+  };
+  long u = valid(blockIdx.x);
+  if (u < units) fetch(u);
+  while (u < units) {
+    __syncthreads();                  // the previous unit has been read
+    {
+      const int t_ = opaque(tid);
+      if constexpr (CU > 0) {
+#pragma unroll
+        for (int i = 0; i < PU; ++i) {
+          const int e = t_ + i * 192;
+          if (e < NU)
+            *reinterpret_cast<uint4 *>(&Xs[0][0][0] + e / UC * XS + e % UC * 8) = pu[i];
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < PX; ++i) {
+        const int e = t_ + i * 192;
+        if (e < NX)
+          *reinterpret_cast<uint4 *>(&Xs[0][0][0] + e / XC * XS + e % XC * 8 + CU) = px[i];
+      }
+#pragma unroll
+      for (int i = 0; i < PD; ++i) {
+        const int e = t_ + i * 192;
+        if (e < ND) *reinterpret_cast<uint4 *>(&Ds[0][0][0] + e / DC * DS + e % DC * 8) = pd[i];
+      }
     }
     __syncthreads();
+    u = valid(u + gridDim.x);
+    if (u < units) fetch(u);  // while this one's products run
     Frag a[3][KS][MT];
 #pragma unroll
     for (int xr = 0; xr < R + 2; ++xr) {
@@ -867,16 +922,17 @@ hipError_t conv_t(const Act &x, const uint16_t *up, const uint16_t *W, const voi
   return hipGetLastError();
 }
 
-// Workgroups of a weight gradient: up to 256 (times the three dz), fewer
-// where the volume has fewer units or the partials would pass kGradScratch.
-template <int CIN, int CU, int COUT, int SEG, int R>
-hipError_t wgrad_t(const Act &x, const uint16_t *up, const Act &dy, float *dW, float *db, Vol v, float *scratch,
-                   hipStream_t st) {
+// Workgroups of a weight gradient: with the three dz up to WGS per compute
+// unit, fewer where the volume has fewer units or the partials would pass
+// kGradScratch.
+template <int CIN, int CU, int COUT, int SEG, int R, int WGS>
+hipError_t wgrad_t(const Act &x, const uint16_t *up, const Act &dy, float *dW, float *db, Vol v,
+                   float *scratch, hipStream_t st) {
   constexpr int NW = 27 * CIN * COUT;
   if (v.w % SEG || v.h % R) return hipErrorInvalidValue;
   const long units = (long)v.n * v.d * (v.h / R) * (v.w / SEG);
-  const int S = (int)std::min({units, 256L, kGradScratch / (NW + COUT)});
-  k_wgrad<CIN, CU, COUT, SEG, R><<<dim3(S, 3), 192, 0, st>>>(
+  const int S = (int)std::min({units, 256L * WGS / 3, kGradScratch / (NW + COUT)});
+  k_wgrad<CIN, CU, COUT, SEG, R, WGS><<<dim3(S, 3), 192, 0, st>>>(
       (const uint16_t *)x.p, x.cs, up, (const uint16_t *)dy.p, dy.cs, scratch, v.d, v.h, v.w, units);
   k_grad_sum<<<(NW + COUT + 63) / 64, 256, 0, st>>>(scratch, S, NW, COUT, dW, db);
   return hipGetLastError();
@@ -885,11 +941,13 @@ hipError_t wgrad_t(const Act &x, const uint16_t *up, const Act &dy, float *dW, f
 }  // namespace
 
 // The weight gradients of the network: (cin, of these upsampled, cout,
-// positions per K run, rows per unit).  The level fixes the run; 96 input
-// channels take four rows so that two workgroups fit a CU's LDS.
-#define BRTM_WGRAD_SHAPES(X)                                                    \
-  X(16, 0, 16, 64, 8) X(48, 32, 16, 64, 8) X(16, 0, 32, 32, 8) X(32, 0, 32, 32, 8) \
-  X(96, 64, 32, 32, 4) X(32, 0, 64, 16, 8) X(64, 0, 64, 16, 8)
+// positions per K run, rows per unit, workgroups per CU).  The level fixes the
+// run; 96 input channels take four rows so that two workgroups fit a CU's LDS;
+// 64->64 has 228 sums in registers and is alone on its CU (24 us at 4 x 16^3;
+// two of them, with spills, 54).
+#define BRTM_WGRAD_SHAPES(X)                                                               \
+  X(16, 0, 16, 64, 8, 3) X(48, 32, 16, 64, 8, 2) X(16, 0, 32, 32, 8, 3) X(32, 0, 32, 32, 8, 2) \
+  X(96, 64, 32, 32, 4, 2) X(32, 0, 64, 16, 8, 2) X(64, 0, 64, 16, 8, 1)
 
 // The forward convolutions (ACT) and the transposed ones (MASK, GRAD): (out,
 // cin, of these upsampled, cout, output tiles and rows per wave, waves in x
@@ -934,9 +992,9 @@ hipError_t conv3d_bwd(const Act &dy, const uint16_t *Wt, const Act &act, Act dx,
 hipError_t conv3d_wgrad(const Act &x, const Act &up, const Act &dy, float *dW, float *db, Vol v,
                         float *scratch, hipStream_t st) {
   if (x.cs % 8 || dy.cs % 8) return hipErrorInvalidValue;
-#define X(CI, CU, CO, SEG, R)                                                                \
+#define X(CI, CU, CO, SEG, R, WGS)                                                            \
   if (is_input(x, up, CI, CU) && dy.c == CO)                                                 \
-    return wgrad_t<CI, CU, CO, SEG, R>(x, (const uint16_t *)up.p, dy, dW, db, v, scratch, st);
+    return wgrad_t<CI, CU, CO, SEG, R, WGS>(x, (const uint16_t *)up.p, dy, dW, db, v, scratch, st);
   BRTM_WGRAD_SHAPES(X)
 #undef X
   return hipErrorInvalidValue;
