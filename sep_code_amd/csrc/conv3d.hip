@@ -125,6 +125,7 @@ k_conv(const uint16_t *__restrict__ x, int xcs, const uint16_t *__restrict__ up,
   // 16-byte chunks of a plane: the upsampled channels first, then the others
   constexpr int UC = CU / 8, XC = CIN / 8 - UC, NP = (R + 2) * (X + 2);
   constexpr int NU = NP * UC, NX = NP * XC, PU = (NU + NT - 1) / NT, PT = (NX + NT - 1) / NT;
+  constexpr bool BOTH = PU + PT <= 8 && MTW < 3;
   uint4 preu[PU + 1], pre[PT];
   const long plane = (long)H * Wd * xcs, uplane = (long)(H / 2) * (Wd / 2) * CU;
   const uint32_t bytes = ((uint32_t)(H * Wd - 1) * xcs + 8 * XC) * 2;
@@ -143,7 +144,7 @@ k_conv(const uint16_t *__restrict__ x, int xcs, const uint16_t *__restrict__ up,
         const int e = t_ + i * NT;
         const int c = e % UC, p = (e / UC) % (X + 2), rr = e / (UC * (X + 2));
         const int yy = y0 + rr - 1, xx = x0 + p - 1;
-        const bool ok = e < NU && yy >= 0 && yy < H && xx >= 0 && xx < Wd;
+        const bool ok = ((i + 1) * NT <= NU || e < NU) & ((unsigned)yy < (unsigned)H) & ((unsigned)xx < (unsigned)Wd);
         const uint32_t off =
             ok ? (uint32_t)((yy >> 1) * (Wd >> 1) + (xx >> 1)) * CU * 2 + 16 * c : 0x80000000u;
         preu[i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(ru, off, 0, 0));
@@ -154,7 +155,7 @@ k_conv(const uint16_t *__restrict__ x, int xcs, const uint16_t *__restrict__ up,
       const int e = t_ + i * NT;
       const int c = e % XC, p = (e / XC) % (X + 2), rr = e / (XC * (X + 2));
       const int yy = y0 + rr - 1, xx = x0 + p - 1;
-      const bool ok = e < NX && yy >= 0 && yy < H && xx >= 0 && xx < Wd;
+      const bool ok = ((i + 1) * NT <= NX || e < NX) & ((unsigned)yy < (unsigned)H) & ((unsigned)xx < (unsigned)Wd);
       const uint32_t off = ok ? (uint32_t)(yy * Wd + xx) * xcs * 2 + 16 * c : 0x80000000u;
       pre[i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rs, off, 0, 0));
     }
@@ -265,18 +266,21 @@ k_conv(const uint16_t *__restrict__ x, int xcs, const uint16_t *__restrict__ up,
 #pragma unroll
       for (int i = 0; i < PU; ++i) {
         const int e = t_ + i * NT;
-        if (e < NU) *reinterpret_cast<uint4 *>(&Xs[e / UC * PS + e % UC * 8]) = preu[i];
+        if ((i + 1) * NT <= NU || e < NU) *reinterpret_cast<uint4 *>(&Xs[e / UC * PS + e % UC * 8]) = preu[i];
       }
     }
 #pragma unroll
     for (int i = 0; i < PT; ++i) {
       const int e = t_ + i * NT;
-      if (e < NX) *reinterpret_cast<uint4 *>(&Xs[e / XC * PS + e % XC * 8 + CU]) = pre[i];
+      if ((i + 1) * NT <= NX || e < NX) *reinterpret_cast<uint4 *>(&Xs[e / XC * PS + e % XC * 8 + CU]) = pre[i];
     }
     __syncthreads();
     if (zp < ze) fetch(zp + 1);
     const bool on0 = zp + 1 < z0 + zl, on1 = zp >= z0 && zp < z0 + zl, on2 = zp > z0;
-    products(on0, on1, on2);
+    if (BOTH && on0 && on1 && on2)
+      products(true, true, true);
+    else
+      products(on0, on1, on2);
     if (on2) store(zp - 1);
 #pragma unroll
     for (int m = 0; m < MTW; ++m)
@@ -408,7 +412,7 @@ k_wgrad(const uint16_t *__restrict__ x, int xcs, const uint16_t *__restrict__ up
       for (int i = 0; i < PU; ++i) {
         const int e = t_ + i * 192, c = e % UC, p = (e / UC) % XP, rr = e / (UC * XP);
         const int yy = y0 + rr - 1, xx = xs + p - 1;
-        const bool ok = e < NU && yy >= 0 && yy < H && xx >= 0 && xx < Wd;
+        const bool ok = ((i + 1) * 192 <= NU || e < NU) & ((unsigned)yy < (unsigned)H) & ((unsigned)xx < (unsigned)Wd);
         pu[i] = load(up + (z2 >> 1) * (H / 2) * (Wd / 2) * CU, ubytes,
                      ok ? (uint32_t)((yy >> 1) * (Wd >> 1) + (xx >> 1)) * CU * 2 + 16 * c
                         : 0x80000000u);
@@ -418,7 +422,7 @@ k_wgrad(const uint16_t *__restrict__ x, int xcs, const uint16_t *__restrict__ up
     for (int i = 0; i < PX; ++i) {
       const int e = t_ + i * 192, c = e % XC, p = (e / XC) % XP, rr = e / (XC * XP);
       const int yy = y0 + rr - 1, xx = xs + p - 1;
-      const bool ok = e < NX && yy >= 0 && yy < H && xx >= 0 && xx < Wd;
+      const bool ok = ((i + 1) * 192 <= NX || e < NX) & ((unsigned)yy < (unsigned)H) & ((unsigned)xx < (unsigned)Wd);
       px[i] = load(x + z2 * H * Wd * xcs, xbytes,
                    ok ? (uint32_t)(yy * Wd + xx) * xcs * 2 + 16 * c : 0x80000000u);
     }
@@ -426,7 +430,7 @@ k_wgrad(const uint16_t *__restrict__ x, int xcs, const uint16_t *__restrict__ up
     for (int i = 0; i < PD; ++i) {
       const int e = t_ + i * 192, c = e % DC, p = (e / DC) % SEG, rr = e / (DC * SEG);
       pd[i] = load(dy + (z * H + y0) * Wd * dycs, dbytes,
-                   e < ND ? (uint32_t)(rr * Wd + xs + p) * dycs * 2 + 16 * c : 0x80000000u);
+                   (i + 1) * 192 <= ND || e < ND ? (uint32_t)(rr * Wd + xs + p) * dycs * 2 + 16 * c : 0x80000000u);
     }
   };
   long u = valid(blockIdx.x);
@@ -439,20 +443,20 @@ k_wgrad(const uint16_t *__restrict__ x, int xcs, const uint16_t *__restrict__ up
 #pragma unroll
         for (int i = 0; i < PU; ++i) {
           const int e = t_ + i * 192;
-          if (e < NU)
+          if ((i + 1) * 192 <= NU || e < NU)
             *reinterpret_cast<uint4 *>(&Xs[0][0][0] + e / UC * XS + e % UC * 8) = pu[i];
         }
       }
 #pragma unroll
       for (int i = 0; i < PX; ++i) {
         const int e = t_ + i * 192;
-        if (e < NX)
+        if ((i + 1) * 192 <= NX || e < NX)
           *reinterpret_cast<uint4 *>(&Xs[0][0][0] + e / XC * XS + e % XC * 8 + CU) = px[i];
       }
 #pragma unroll
       for (int i = 0; i < PD; ++i) {
         const int e = t_ + i * 192;
-        if (e < ND) *reinterpret_cast<uint4 *>(&Ds[0][0][0] + e / DC * DS + e % DC * 8) = pd[i];
+        if ((i + 1) * 192 <= ND || e < ND) *reinterpret_cast<uint4 *>(&Ds[0][0][0] + e / DC * DS + e % DC * 8) = pd[i];
       }
     }
     __syncthreads();
