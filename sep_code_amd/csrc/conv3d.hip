@@ -13,6 +13,7 @@
 #include "conv3d.h"
 
 #include <algorithm>
+#include <utility>
 
 namespace brtm {
 namespace {
@@ -24,6 +25,12 @@ __device__ __forceinline__ uint16_t f2bf(float x) {
   uint32_t u = __float_as_uint(x);
   u += 0x7fffu + ((u >> 16) & 1u);
   return (uint16_t)(u >> 16);
+}
+// two of them in one conversion (round to nearest even, as f2bf)
+__device__ __forceinline__ uint32_t f2bf2(float lo, float hi) {
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{lo, hi}, bf16x2));
 }
 __device__ __forceinline__ float bf2f(uint16_t h) { return __uint_as_float(((uint32_t)h) << 16); }
 
@@ -54,16 +61,38 @@ int grid1(long n, int bs = 256) {
 }
 
 // ------------------------------------------------------------- forward GEMM
-// Elements between two positions (or two weight rows) in LDS: lanes 0..15 of
-// a 16-byte read are that far apart, and strides of an odd number of 16-byte
-// units or of at most 64 bytes spread them over all banks.
-__host__ __device__ constexpr int pos_stride(int c) { return c > 48 ? c + 8 : c; }
+// Elements between two positions (or two weight rows) in LDS.  Sixteen rows
+// are read at once, 16 bytes (or, for 16 channels, 8) of each by the four lane
+// groups: free of bank conflicts where the stride is an odd multiple of 32
+// bytes (of 16 for 16 channels), measured 4.1 clocks for a 16-byte read of a
+// wave against 8.2 at 64 bytes and 16 at 128.
+__host__ __device__ constexpr int pos_stride(int c) {
+  return c == 16 ? 24 : c / 16 % 2 ? c : c + 16;
+}
+
+// Where lane group kq finds its 4 channels of the 16-channel remainder behind
+// 32 channels: the two 16-byte halves change places every four positions,
+// which keeps the 8-byte reads at that stride free of bank conflicts.
+__device__ __forceinline__ int remainder_at(int kq, int pos) {
+  return ((kq >> 1) ^ (pos >> 2 & 1)) * 8 + (kq & 1) * 4;
+}
+
+template <int V>
+struct Int {
+  static constexpr int value = V;
+};
+
+// f(Int<0>()), f(Int<1>()), ...: a loop unrolled whatever its length
+template <class F, int... K>
+__device__ __forceinline__ void unrolled(F &&f, std::integer_sequence<int, K...>) {
+  (f(Int<K>()), ...);
+}
 
 // Two gradients through the ReLU of two BF16 activations, as BF16.
 __device__ __forceinline__ uint32_t masked2(uint32_t act, float g0, float g1) {
   g0 = __uint_as_float(act << 16) > 0.f ? g0 : 0.f;
   g1 = __uint_as_float(act & 0xffff0000u) > 0.f ? g1 : 0.f;
-  return (uint32_t)f2bf(g0) | ((uint32_t)f2bf(g1) << 16);
+  return f2bf2(g0, g1);
 }
 
 // What happens to a finished output tile.
@@ -89,11 +118,16 @@ enum { OUT_ACT = 0, OUT_GRAD = 1, OUT_MASK = 2 };
 // tensor is never stored: 28 us a layer for writing it, and its reads).
 //
 // What bounds it: the matrix unit (46 us for 48->16 at 8 x 64^3, the K = 16
-// products at half rate) and the LDS reads that feed it.  A wave that loaded
-// its rows from the vector cache for each dz, dx and chunk moved three times
-// the fragments through a 64-byte-per-clock cache: at 8 x 64^3 48->16 took 219
-// us, now 117; 16->16 93, now 50; 96->32 (32^3) 108, now 73; 32->32 41, now
-// 23; 64->64 (16^3) 62, now 23; 32->64 21, now 18.
+// products at half rate) and what it waits for between planes: a workgroup's
+// waves write, wait and finish outputs together.  A wave that loaded its rows
+// from the vector cache for each dz, dx and chunk moved three times the
+// fragments through a 64-byte-per-clock cache: 48->16 at 8 x 64^3 took 219 us,
+// now 90; 16->16 93, now 44; 96->32 (32^3) 108, now 54; 32->32 41, now 21;
+// 64->64 (16^3) 62, now 20; 32->64 21, now 11; and 16->48 at 4 x 64^3 106 with
+// 12 sums of 16 x 16 outputs a wave and output plane, now 71 with six.  A wave
+// has few sums (MTW YT is 4 to 6) so that more waves than two are resident on
+// a matrix unit and no register is spilled: eight sums took 97 us for 48->16
+// and 81 for 96->32.
 template <int CIN, int CU, int COUT, int MTW, int YT, int WX, int WY, bool WL, int OUT>
 __global__ void __launch_bounds__(64 * WX * WY * (COUT / 16 / MTW), 2)
 k_conv(const uint16_t *__restrict__ x, int xcs, const uint16_t *__restrict__ up,
@@ -105,6 +139,8 @@ k_conv(const uint16_t *__restrict__ x, int xcs, const uint16_t *__restrict__ up,
   constexpr bool R16 = CIN % 32 == 16;  // and a 16-channel remainder
   constexpr int R = YT * WY, X = 16 * WX, PS = pos_stride(CIN), RS = (X + 2) * PS;
   constexpr int WS = WL ? PS : CIN_P;
+  constexpr bool SWZ = R16 && NC > 0;  // the remainder's halves are swapped (remainder_at)
+  static_assert(!SWZ || (CU == NC * 32 && WL), "the remainder is its own source");
   __shared__ __attribute__((aligned(16))) uint16_t Xs[(R + 2) * RS];
   __shared__ __attribute__((aligned(16))) uint16_t Ws[WL ? 27 * COUT * PS : 8];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -125,7 +161,6 @@ k_conv(const uint16_t *__restrict__ x, int xcs, const uint16_t *__restrict__ up,
   // 16-byte chunks of a plane: the upsampled channels first, then the others
   constexpr int UC = CU / 8, XC = CIN / 8 - UC, NP = (R + 2) * (X + 2);
   constexpr int NU = NP * UC, NX = NP * XC, PU = (NU + NT - 1) / NT, PT = (NX + NT - 1) / NT;
-  constexpr bool BOTH = PU + PT <= 8 && MTW < 3;
   uint4 preu[PU + 1], pre[PT];
   const long plane = (long)H * Wd * xcs, uplane = (long)(H / 2) * (Wd / 2) * CU;
   const uint32_t bytes = ((uint32_t)(H * Wd - 1) * xcs + 8 * XC) * 2;
@@ -165,11 +200,16 @@ k_conv(const uint16_t *__restrict__ x, int xcs, const uint16_t *__restrict__ up,
   fetch(zf);
   if constexpr (WL) {
     constexpr int WC = CIN / 8;
-    for (int i = tid; i < 27 * COUT * WC; i += NT)
-      *reinterpret_cast<uint4 *>(&Ws[i / WC * PS + i % WC * 8]) =
-          *reinterpret_cast<const uint4 *>(W + (long)(i / WC) * CIN_P + i % WC * 8);
+    for (int i = tid; i < 27 * COUT * WC; i += NT) {
+      const int r = i / WC, c = i % WC, sw = SWZ && c >= NC * 4 ? r >> 2 & 1 : 0;
+      *reinterpret_cast<uint4 *>(&Ws[r * PS + (c ^ sw) * 8]) =
+          *reinterpret_cast<const uint4 *>(W + (long)r * CIN_P + c * 8);
+    }
   }
-  const uint16_t *wb = (WL ? Ws : W) + (wm * MTW * 16 + col) * WS;
+  static_assert(WL || !R16, "a remainder's weights wait in LDS");
+  const __amdgpu_buffer_rsrc_t wrs = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint16_t *>(W), 0, 27 * COUT * CIN_P * 2, 0x00020000);
+  const int wrem = SWZ ? remainder_at(kq, col) : 4 * kq;
   const uint16_t *xb = Xs + (wy * YT) * RS + (wx * 16 + col) * PS;
 
   f32x4 acc[3][MTW][YT];  // outputs zp + 1, zp, zp - 1 of input plane zp
@@ -201,62 +241,75 @@ k_conv(const uint16_t *__restrict__ x, int xcs, const uint16_t *__restrict__ up,
           const float v0 = fmaxf(v[0] + b.x, 0.f), v1 = fmaxf(v[1] + b.y, 0.f);
           const float v2 = fmaxf(v[2] + b.z, 0.f), v3 = fmaxf(v[3] + b.w, 0.f);
           *reinterpret_cast<uint2 *>(static_cast<uint16_t *>(y) + o + c0) =
-              make_uint2((uint32_t)f2bf(v0) | ((uint32_t)f2bf(v1) << 16),
-                         (uint32_t)f2bf(v2) | ((uint32_t)f2bf(v3) << 16));
+              make_uint2(f2bf2(v0, v1), f2bf2(v2, v3));
         }
       }
     }
   };
 
-  // products of the staged plane; on[d]: output zp + 1 - d is this sweep's
-  auto products = [&](bool on0, bool on1, bool on2) {
-    const uint16_t *wq = wb + opaque(0);  // no weights kept over the plane loop
+  // Products of the staged plane for the outputs zp + 1 - dz whose bit of MASK
+  // is set, in steps of one weight fragment per output tile; the fragments are
+  // read AHEAD steps before their products, which the compiler left next to
+  // them.
+  constexpr int NPC = NC + R16, AHEAD = WL ? 1 : 3;
+  auto products = [&](auto mask) {
+    constexpr int MASK = decltype(mask)::value;
+    constexpr int ND = (MASK & 1) + (MASK >> 1 & 1) + (MASK >> 2), K = 9 * NPC * ND;
+    // no weights kept over the plane loop
+    const uint16_t *wq = Ws + ((wm * MTW * 16 + col) * WS + opaque(0)) * WL;
+    const int wlane = ((wm * MTW * 16 + col) * WS + 8 * kq + opaque(0)) * 2;
+    bf16x8 b[YT + 2], a[AHEAD + 1][MTW];
+    i16x4 bh[YT + 2], ah[AHEAD + 1][MTW];
+    // step k: x tap, chunk, z tap, y tap
+    auto tap = [](int k) constexpr {
+      const int d = k / 3 % ND, lo = MASK & 1 ? 0 : MASK & 2 ? 1 : 2;
+      return (lo + d) * 9 + k % 3 * 3 + k / (3 * ND * NPC);
+    };
+    auto weights = [&](int k) __attribute__((always_inline)) {
+      const int pc = k / (3 * ND) % NPC, o = tap(k) * COUT;
 #pragma unroll
-    for (int dx = 0; dx < 3; ++dx) {
-#pragma unroll
-      for (int cg = 0; cg < NC; ++cg) {
-        const int c = cg * 32 + 8 * kq;
-        bf16x8 bv[YT + 2];
-#pragma unroll
-        for (int i = 0; i < YT + 2; ++i) bv[i] = ld8(xb + i * RS + dx * PS + c);
-#pragma unroll
-        for (int dz = 0; dz < 3; ++dz) {
-          if (!(dz == 0 ? on0 : dz == 1 ? on1 : on2)) continue;
-#pragma unroll
-          for (int dy = 0; dy < 3; ++dy)
-#pragma unroll
-            for (int m = 0; m < MTW; ++m) {
-              const bf16x8 a = ld8(wq + ((dz * 9 + dy * 3 + dx) * COUT + m * 16) * WS + c);
-#pragma unroll
-              for (int t = 0; t < YT; ++t)
-                acc[dz][m][t] =
-                    __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bv[t + dy], acc[dz][m][t], 0, 0, 0);
-            }
-        }
-        __builtin_amdgcn_sched_barrier(0);
+      for (int m = 0; m < MTW; ++m) {
+        if (!WL)  // one register of lane offsets, the rest in the scalar offset
+          a[k % (AHEAD + 1)][m] = __builtin_bit_cast(
+              bf16x8, __builtin_amdgcn_raw_buffer_load_b128(
+                          wrs, wlane, ((o + m * 16) * WS + pc * 32) * 2, 0));
+        else if (pc < NC)
+          a[k % (AHEAD + 1)][m] = ld8(wq + (o + m * 16) * WS + pc * 32 + 8 * kq);
+        else
+          ah[k % (AHEAD + 1)][m] = ld4h(wq + (o + m * 16) * WS + NC * 32 + wrem);
       }
-      if constexpr (R16) {
-        const int c = NC * 32 + 4 * kq;
-        i16x4 bv[YT + 2];
+    };
 #pragma unroll
-        for (int i = 0; i < YT + 2; ++i) bv[i] = ld4h(xb + i * RS + dx * PS + c);
+    for (int k = 0; k < AHEAD; ++k) weights(k);
+    auto step = [&](auto kk) __attribute__((always_inline)) {
+      constexpr int k = decltype(kk)::value;
+      constexpr int pc = k / (3 * ND) % NPC, dx = k / (3 * ND * NPC), t9 = tap(k);
+      if (k % (3 * ND) == 0) {
+        const uint16_t *xr = xb + dx * PS;
+        const int rem = NC * 32 + (SWZ ? remainder_at(kq, col + dx) : 4 * kq);
 #pragma unroll
-        for (int dz = 0; dz < 3; ++dz) {
-          if (!(dz == 0 ? on0 : dz == 1 ? on1 : on2)) continue;
-#pragma unroll
-          for (int dy = 0; dy < 3; ++dy)
-#pragma unroll
-            for (int m = 0; m < MTW; ++m) {
-              const i16x4 a = ld4h(wq + ((dz * 9 + dy * 3 + dx) * COUT + m * 16) * WS + c);
-#pragma unroll
-              for (int t = 0; t < YT; ++t)
-                acc[dz][m][t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, bv[t + dy],
-                                                                          acc[dz][m][t], 0, 0, 0);
-            }
+        for (int i = 0; i < YT + 2; ++i) {
+          if (pc < NC) b[i] = ld8(xr + i * RS + pc * 32 + 8 * kq);
+          else bh[i] = ld4h(xr + i * RS + rem);
         }
-        __builtin_amdgcn_sched_barrier(0);
       }
-    }
+      if (k + AHEAD < K) weights(k + AHEAD);
+      __builtin_amdgcn_sched_barrier(0);
+      constexpr int dz = t9 / 9, dy = t9 / 3 % 3;
+#pragma unroll
+      for (int m = 0; m < MTW; ++m)
+#pragma unroll
+        for (int t = 0; t < YT; ++t) {
+          if (pc < NC)
+            acc[dz][m][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                a[k % (AHEAD + 1)][m], b[t + dy], acc[dz][m][t], 0, 0, 0);
+          else
+            acc[dz][m][t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(
+                ah[k % (AHEAD + 1)][m], bh[t + dy], acc[dz][m][t], 0, 0, 0);
+        }
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    unrolled(step, std::make_integer_sequence<int, K>());
   };
 
   for (int zp = zf; zp <= ze; ++zp) {
@@ -272,15 +325,23 @@ k_conv(const uint16_t *__restrict__ x, int xcs, const uint16_t *__restrict__ up,
 #pragma unroll
     for (int i = 0; i < PT; ++i) {
       const int e = t_ + i * NT;
-      if ((i + 1) * NT <= NX || e < NX) *reinterpret_cast<uint4 *>(&Xs[e / XC * PS + e % XC * 8 + CU]) = pre[i];
+      if ((i + 1) * NT <= NX || e < NX) {
+        const int p = e / XC, sw = SWZ ? p % (X + 2) >> 2 & 1 : 0;
+        *reinterpret_cast<uint4 *>(&Xs[p * PS + ((e % XC) ^ sw) * 8 + CU]) = pre[i];
+      }
     }
     __syncthreads();
-    if (zp < ze) fetch(zp + 1);
+    if (WL && zp < ze) fetch(zp + 1);
     const bool on0 = zp + 1 < z0 + zl, on1 = zp >= z0 && zp < z0 + zl, on2 = zp > z0;
-    if (BOTH && on0 && on1 && on2)
-      products(true, true, true);
-    else
-      products(on0, on1, on2);
+    if (on0 && on1 && on2) products(Int<7>());
+    else if (on0 && on1) products(Int<3>());
+    else if (on1 && on2) products(Int<6>());
+    else if (on0) products(Int<1>());
+    else if (on1) products(Int<2>());
+    else products(Int<4>());
+    // where the weights come through the vector cache the next plane is loaded
+    // behind them (loads return in order), while the other workgroup computes
+    if (!WL && zp < ze) fetch(zp + 1);
     if (on2) store(zp - 1);
 #pragma unroll
     for (int m = 0; m < MTW; ++m)
@@ -656,8 +717,7 @@ k_first_fwd4(const float *__restrict__ x, const float *__restrict__ W,
       uint32_t w[4];
 #pragma unroll
       for (int h = 0; h < 4; ++h)
-        w[h] = (uint32_t)f2bf(fmaxf(s[j][2 * h], 0.f)) |
-               ((uint32_t)f2bf(fmaxf(s[j][2 * h + 1], 0.f)) << 16);
+        w[h] = f2bf2(fmaxf(s[j][2 * h], 0.f), fmaxf(s[j][2 * h + 1], 0.f));
       *reinterpret_cast<uint4 *>(o + j * ycs + c0) = make_uint4(w[0], w[1], w[2], w[3]);
     }
   }
@@ -832,7 +892,7 @@ k_pool_fwd(const uint16_t *__restrict__ x, int xcs, uint16_t *__restrict__ y, in
       lo += __uint_as_float(u << 16);
       hi += __uint_as_float(u & 0xffff0000u);
     }
-    w[h] = (uint32_t)f2bf(0.125f * lo) | ((uint32_t)f2bf(0.125f * hi) << 16);
+    w[h] = f2bf2(0.125f * lo, 0.125f * hi);
   }
   *reinterpret_cast<uint4 *>(y + p * ycs + k) = make_uint4(w[0], w[1], w[2], w[3]);
 }
@@ -957,13 +1017,13 @@ hipError_t wgrad_t(const Act &x, const uint16_t *up, const Act &dy, float *dW, f
 // cin, of these upsampled, cout, output tiles and rows per wave, waves in x
 // and y, weights in LDS).
 #define BRTM_CONV_SHAPES(X)                                                          \
-  X(ACT, 16, 0, 16, 1, 8, 4, 2, true) X(ACT, 48, 32, 16, 1, 8, 4, 2, true)           \
-  X(ACT, 16, 0, 32, 2, 4, 2, 2, true) X(ACT, 32, 0, 32, 2, 4, 2, 4, true)            \
-  X(ACT, 96, 64, 32, 2, 4, 2, 2, false) X(ACT, 32, 0, 64, 2, 4, 1, 2, false)         \
-  X(ACT, 64, 0, 64, 2, 4, 1, 2, false) X(MASK, 16, 0, 16, 1, 8, 4, 2, true)          \
-  X(MASK, 32, 0, 32, 2, 4, 2, 4, true) X(MASK, 64, 0, 64, 2, 4, 1, 2, false)         \
-  X(GRAD, 16, 0, 48, 3, 4, 4, 2, true) X(GRAD, 32, 0, 96, 3, 4, 2, 2, false)         \
-  X(GRAD, 32, 0, 16, 1, 4, 2, 4, true) X(GRAD, 64, 0, 32, 1, 4, 1, 2, false)
+  X(ACT, 16, 0, 16, 1, 4, 4, 1, true) X(ACT, 48, 32, 16, 1, 4, 4, 2, true)           \
+  X(ACT, 16, 0, 32, 1, 4, 2, 2, true) X(ACT, 32, 0, 32, 1, 4, 2, 2, true)            \
+  X(ACT, 96, 64, 32, 1, 4, 2, 2, false) X(ACT, 32, 0, 64, 1, 4, 1, 2, false)         \
+  X(ACT, 64, 0, 64, 1, 4, 1, 2, false) X(MASK, 16, 0, 16, 1, 4, 4, 1, true)          \
+  X(MASK, 32, 0, 32, 1, 4, 2, 2, true) X(MASK, 64, 0, 64, 1, 4, 1, 2, false)         \
+  X(GRAD, 16, 0, 48, 3, 2, 4, 2, true) X(GRAD, 32, 0, 96, 3, 2, 2, 2, false)         \
+  X(GRAD, 32, 0, 16, 1, 4, 2, 4, true) X(GRAD, 64, 0, 32, 1, 4, 1, 1, false)
 
 // Whether (x, up) are CI input channels of which the first CU are upsampled.
 static bool is_input(const Act &x, const Act &up, int ci, int cu) {
