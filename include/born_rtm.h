@@ -180,26 +180,29 @@ int brtm_set_tuning(brtm_ctx *ctx, int ty_tile, int target_blocks);
 
 /* Cells per lane along x for VL-form steps: 1 (64-wide tiles, 4-byte
  * accesses), 2 (128-wide tiles, 8-byte accesses; n1 even) or 4 (256-wide
- * tiles, 16-byte accesses; n1 % 4 == 0); 0 (the default) picks the widest
- * whose tiles keep at least 3/4 of the lanes busy.  A grid that does not
- * allow the width asked for uses the widest one it allows.  Results agree
- * to FP32 rounding. */
+ * tiles, 16-byte accesses; n1 % 4 == 0); 0 (the default) picks by the grid:
+ * a four-cell kernel without LDS up to 10 M cells (16 M where n1 % 4 != 0),
+ * whose reuse the caches serve; above, with n1 % 4 == 0, the four-cell ring in
+ * the tile shape whose rounds of workgroups cost least; else the one-cell or
+ * two-cell tiles.  A grid that does not allow the width asked for uses the
+ * widest one it allows.  Results agree to FP32 rounding. */
 int brtm_set_x_per_lane(brtm_ctx *ctx, int cells);
 
 /* One- and four-cell VL steps staged through a ring of six LDS planes whose
  * halos are loaded together with the z-queue (on = 1), or through the
  * two-plane buffer that loads each halo one slice ahead (on = 0); -1, the
- * default, uses the ring for the four-cell kernel (3 % faster at 512^3) and
- * not for the one-cell kernel.  Same results. */
+ * default, uses the ring for the four-cell tiles (3 % faster at 512^3) and
+ * not for the one-cell kernel; 0 or 1 also keeps the steps on tiles where the
+ * automatic choice would take the kernel without LDS.  Same results. */
 int brtm_set_halo_ring(brtm_ctx *ctx, int on);
 
 /* Receivers and sources inside the step (no counterpart in the reference):
  * when the active receivers share one depth plane with at most one receiver
- * per cell, the four-cell ring step injects the data (RTM adjoint) or
- * extracts it (Born modelling) on that plane itself instead of a separate
- * launch per step; the source points likewise.  on = 1 (the default) allows
- * it, 0 keeps the separate kernels.  The same results, to FP32 rounding of
- * the imaging term. */
+ * per cell, the four-cell ring step and the kernel without LDS inject the data
+ * (RTM adjoint) or extract it (Born modelling) on that plane themselves
+ * instead of a separate launch per step; the source points likewise.  on = 1
+ * (the default) allows it, 0 keeps the separate kernels.  The same results, to
+ * FP32 rounding of the imaging term. */
 int brtm_set_receiver_fusion(brtm_ctx *ctx, int on);
 
 /* Global-load lookahead of the plain four-cell ring step, in z slices: 1

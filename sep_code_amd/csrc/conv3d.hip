@@ -373,7 +373,7 @@ k_conv(const uint16_t *__restrict__ x, int xcs, const uint16_t *__restrict__ up,
 // bias gradient is one more product, dy by ones, on the wave of the centre
 // tap.  Before this a workgroup per tap re-read both tensors 27 times and
 // transposed them with 2-byte LDS stores: 2.00 ms for 16->16 and 3.79 ms for
-// 48->16 at 4 x 64^3, now 0.039 and 0.094 ms.  The next unit is loaded into
+// 48->16 at 4 x 64^3, now 0.035 and 0.082 ms.  The next unit is loaded into
 // registers while a unit's products run (loading it only when they were done,
 // 0.055 and 0.20 ms: the loads' latency was most of the time), and WGS
 // workgroups per compute unit are launched, all resident at once (a third
