@@ -971,7 +971,9 @@ __global__ void k_adam(float *p, const float *__restrict__ g, float *m, float *v
   }
 }
 
-// Output planes per sweep: as many as leave two workgroups for a compute unit.
+// Output planes per sweep: as many as leave two workgroups of four waves, or
+// one of eight, for a compute unit (each sweep stages two planes more than it
+// writes: with 1024 workgroups 16->16 took 48.4 us at 8 x 64^3, 44.5 with 512).
 template <int OUT, int CIN, int CU, int COUT, int MTW, int YT, int WX, int WY, bool WL>
 hipError_t conv_t(const Act &x, const uint16_t *up, const uint16_t *W, const void *aux, Act y, Vol v,
                   hipStream_t st) {
