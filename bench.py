@@ -54,11 +54,8 @@ BYTES_PER_CELL = 16.0
 # FETCH_SIZE / WRITE_SIZE scaled by the copy-kernel calibration (2.0 / 1.0):
 # profiles/stencil512_traffic.md.  Used for the default configuration only.
 TRAFFIC_X4R_512 = (2.0 * 794832 + 508032) * 1024.0
-# The library's ring step reads the data it uses once with nontemporal loads
-# when a step moves more than this many bytes (16 per cell).
-STREAM_MIN_STEP_BYTES = 512 * 2 ** 20
-# ... and launches its propagation loops as graphs on grids of at most this
-# many cells (brtm_set_graphs, automatic).
+# The library launches its propagation loops as graphs on grids of at most
+# this many cells (brtm_set_graphs, automatic).
 GRAPH_MAX_CELLS = 1 << 22
 
 
@@ -99,9 +96,9 @@ def rtm_shot(dev, w):
 
 
 def cells_per_lane(n1, want):
-    """The forward-form kernel the library runs for this n1: cells per lane
-    asked for (1, 2, 4) where n1 allows it, or automatically (0) the widest
-    whose tiles keep at least 3/4 of the lanes busy."""
+    """Cells per lane of the forward-form tiles for this n1: those asked for
+    (1, 2, 4) where n1 allows them, or (0) the widest whose tiles keep at
+    least 3/4 of the lanes busy."""
     if want == 0:
         want = 1
         for k in (4, 2):
@@ -117,10 +114,11 @@ def cells_per_lane(n1, want):
 
 
 def plain_step_kernel(n, want):
-    """(cells per lane, tile rows) of the plain forward step the library
-    runs on grid n = (n1, n2, n3) with automatic tiles: the default shape,
-    or 64-wide 8-row tiles when that shape would leave some of MI355X's 256
-    compute units without a workgroup."""
+    """(cells per lane, tile rows) of the plain forward step on the tiled
+    kernels on grid n = (n1, n2, n3): the default shape, or 64-wide 8-row
+    tiles when that shape would leave some of MI355X's 256 compute units
+    without a workgroup.  The library's automatic choice has other kernels
+    and shapes as well: plain_step_label asks it."""
     xl = cells_per_lane(n[0], want)
     ty, tb = {4: (16, 256), 2: (16, 2048), 1: (32, 1024)}[xl]
     if want == 0:
@@ -130,6 +128,12 @@ def plain_step_kernel(n, want):
         if tiles * -(-nz // zc) < 256:
             return 1, 8
     return xl, ty
+
+
+def plain_step_label(dev):
+    """The kernel that the plain forward step of dev's grid and settings runs
+    on (the shot's sources and receivers inside the step), from the library."""
+    return f"brtm::{dev.step_kernel(0, 0, 0, 1)}, VL, fused sponge"
 
 
 def cpu_model() -> str:
@@ -330,6 +334,7 @@ def lsrtm_main(a):
     # stream (the solves launch it millions of times)
     kcount = 200
     k_ms = dev.time_step(0, 1, 3, kcount)
+    step_name = dev.step_kernel(0, 1, 3)
     achieved = 26.0 * w.ncell / (k_ms * 1e-3) / 1e9
     fp = out.get("fpcg", {})
     cpu = None
@@ -356,7 +361,7 @@ def lsrtm_main(a):
         "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
                      "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
                      "traffic": None,
-                     "kernel": "brtm::k_step_x4r VL step with fused imaging from FP16 "
+                     "kernel": f"brtm::{step_name}, VL step with fused imaging from FP16 "
                                "snapshots (26 B per cell)",
                      "kernel_ms": round(k_ms, 4), "launches": kcount},
         "cpu_baseline": cpu, "lsrtm": out,
@@ -456,22 +461,15 @@ def main():
     default_cfg = w.n == (512, 512, 512) and a.x_per_lane in (0, 4) and a.ty == 0
     if traffic is None and default_cfg:
         traffic = TRAFFIC_X4R_512
-    kxl, kty = plain_step_kernel(w.n, a.x_per_lane) if a.ty == 0 else (
-        cells_per_lane(w.n[0], a.x_per_lane), a.ty)
     roof = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
             "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
             "traffic": traffic,
             "traffic_source": ("--traffic-bytes of this run" if a.traffic_bytes else
                                "rocprofv3 FETCH_SIZE x 2.0 + WRITE_SIZE x 1.0 per launch of "
-                               "this kernel at this shape, from a separate counter run of the "
-                               "same build (profiles/stencil512_traffic.md), not measured in "
-                               "this run" if traffic else "not measured for this shape"),
-            "kernel": {1: "brtm::k_step (VL, fused sponge)",
-                       2: "brtm::k_step_x2 (VL, 2 cells/lane, fused sponge)",
-                       4: "brtm::k_step_x4r (VL, 4 cells/lane, six-plane halo ring, fused sponge)"
-                       }[kxl] + f", {kty}-row tiles" + (
-                           " + streaming loads" if kxl == 4 and 16 * ncell > STREAM_MIN_STEP_BYTES
-                           else ""),
+                               "this kernel at this shape, from a separate counter run "
+                               "(profiles/stencil512_traffic.md names the build), not "
+                               "measured in this run" if traffic else "not measured for this shape"),
+            "kernel": plain_step_label(dev),
             "kernel_ms": round(k_ms, 4), "launches": kcount,
             "kernel_timing": ("HIP events around every launch in the timed shots" if not graphs
                               else "HIP events around every launch of one extra, eagerly "

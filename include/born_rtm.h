@@ -162,6 +162,13 @@ int brtm_propagate(brtm_ctx *ctx, int form, int nsteps, float *p_cur, float *p_o
  * format (none, FP32, BF16, FP16; none exactly when act is none). */
 int brtm_time_step(brtm_ctx *ctx, int form, int act, int fmt, int nrep, double *avg_ms);
 
+/* Name and tile shape of the kernel such a step runs on with the context's
+ * grid and settings; rec: 0 without receivers inside the step, 1 injected,
+ * 2 extracted (receivers on one plane).  name receives at most len bytes,
+ * terminated; BRTM_EINVAL if they do not hold it.  No counterpart in the
+ * reference. */
+int brtm_step_kernel(brtm_ctx *ctx, int form, int act, int fmt, int rec, char *name, int len);
+
 /* Born modelling path: 0 (default) advances u = V.w.q with the forward-form
  * kernel (the transpose-form step equals D^-1 A_VL D, D = V.w); 1 runs the
  * transpose-form kernel on q directly (cross-check). */

@@ -62,6 +62,7 @@ SIGNATURES = {
     "brtm_get_snapshot": [_P, _I, _P],
     "brtm_propagate": [_P, _I, _I, _P, _P],
     "brtm_time_step": [_P, _I, _I, _I, _I, C.POINTER(_D)],
+    "brtm_step_kernel": [_P, _I, _I, _I, _I, C.c_char_p, _I],
     "brtm_set_tuning": [_P, _I, _I],
     "brtm_set_x_per_lane": [_P, _I],
     "brtm_set_halo_ring": [_P, _I],

@@ -155,18 +155,6 @@ constexpr int kAutoPrefetch = 1;
 // launches, which the hint would forfeit: 11 % slower at 256^3.
 constexpr double kStreamMinStepBytes = 512.0 * 1024 * 1024;
 
-// Largest grids of the VL step without LDS.  Its taps go through L1 and L2,
-// which pays while the fields stay in the Infinity Cache.  Plain / FP32
-// imaging / FP16 imaging / FP16 Born steps in us, before and with it: 48^3 8.8
-// / 9.6 / 11.6 / 11.5 and 3.2 / 3.6 / 3.6 / 3.5; 128^3 10.6 / 11.9 / 16.3 / 15.8
-// and 8.4 / 11.1 / 10.6 / 9.8; 208^3 (9.0 M cells) 31 / 63 / 47 / 45 and 26 / 40
-// / 37 / 33.  At 288 x 240 x 208 (14.4 M) it takes 41 / 77 / 61 / 57, the ring's
-// 64 x 16 tiles 36 / 62 / 63 / 55.  Where n1 is no multiple of 4 the
-// alternative is the one- or two-cell kernel: 257 x 201 x 233 (12 M) 41 / 66 /
-// 60 / 52 against 36 / 54 / 51 / 44, 301^3 (27 M) 100 / 173 / 172 / 150 against
-// 113 / 178 / 174 / 149.
-constexpr long kDirectMaxCells = 10L << 20, kDirectMaxCellsOdd = 16L << 20;
-
 #define BRTM_TRY(x)              \
   do {                           \
     int rc_ = (x);               \
@@ -194,6 +182,15 @@ static int ktime_end(brtm_ctx *c, bool timed) {
   return BRTM_OK;
 }
 
+static StepSetting step_setting(const brtm_ctx *c) {
+  return {c->n1, c->n2, c->n3, c->ncu, c->ty_tile, c->target_blocks, c->x_per_lane, c->halo_ring};
+}
+
+static bool streams(const brtm_ctx *c) {
+  return c->stream_loads < 0 ? 16.0 * (double)c->ncell > kStreamMinStepBytes
+                             : c->stream_loads != 0;
+}
+
 int step(brtm_ctx *c, int form, int act, int fmt, const float *p, const float *po, float *pn,
          const void *snap, const float *sscale, float *img, const float *m, int rec, int it,
          int jt, const float *rscale, bool *fused) {
@@ -215,56 +212,20 @@ int step(brtm_ctx *c, int form, int act, int fmt, const float *p, const float *p
   P.m = m;
   P.cimg = c->cimg;
   P.pf = c->prefetch == 0 ? kAutoPrefetch : c->prefetch;
-  P.stream = c->stream_loads < 0 ? (16.0 * (double)c->ncell > kStreamMinStepBytes)
-                                 : c->stream_loads != 0;
-  // The automatic choice: the kernel without LDS while the fields stay in the
-  // caches, the four-cell ring where n1 allows it, else as below.
-  const bool autosel =
-      form == FORM_VL && c->ty_tile == 0 && c->x_per_lane == 0 && c->halo_ring < 0;
-  const bool direct =
-      autosel && c->ncell <= (c->n1 % 4 == 0 ? kDirectMaxCells : kDirectMaxCellsOdd);
-  const bool auto4 = autosel && !direct && c->n1 % 4 == 0;
-  // Tile rows / workgroup target per variant (measured on MI355X at 512^3):
-  // plain steps prefer tall tiles, 16-bit snapshot variants short ones.
-  int ty = c->ty_tile, tb = c->target_blocks;
-  // cells per lane: 4 or 2 where asked for and n1 allows, else 1; automatic
-  // (0): the widest whose tiles keep at least 3/4 of the lanes busy
-  int xl = 1;
-  if (form == FORM_VL) {
-    int want = c->x_per_lane;
-    if (want == 0) {
-      want = 1;
-      for (int k : {4, 2}) {
-        const int w = 64 * k, used = ((c->n1 + w - 1) / w) * w;
-        if (c->n1 % k == 0 && 4 * c->n1 >= 3 * used) { want = k; break; }
-      }
-    }
-    if (want == 4 && c->n1 % 4 == 0) xl = 4;
-    else if (want >= 2 && c->n1 % 2 == 0) xl = 2;
-  }
-  // halo ring: automatic (-1) means on for the 4-cell kernel
-  const bool ring = c->halo_ring < 0 ? xl == 4 : c->halo_ring != 0;
-  if (ty == 0) {
-    if (xl == 4) { ty = (ring && act == ACT_IMG && fmt == FMT_F32) ? 8 : 16; tb = 256; }
-    else if (xl == 2) { ty = 16; tb = 2048; }
-    else if (act == ACT_NONE) { ty = 32; tb = 1024; }
-    else if (fmt == FMT_F32) { ty = 16; tb = 8192; }
-    else { ty = 8; tb = 8192; }
-  }
-  if (xl == 4 && ty == 32) ty = 16;  // the 4-cell kernel's tiles are 8 or 16 rows
-  plan_step(P, ty, tb, 64 * xl);
+  P.stream = streams(c);
   const bool timed =
       c->ktime_on && form == c->ktime_form && act == c->ktime_act && fmt == c->ktime_fmt;
-  BRTM_TRY(ktime_begin(c, timed));
-  // receivers inside the step: the four-cell ring kernel, the kernel without
-  // LDS, or the one-cell kernel's 8-row shape; one receiver plane
+  // receivers inside the step, where the kernel takes them: one plane
   const bool src = rec == REC_SOURCE;
-  const bool rec_kernel =
-      direct || auto4 || (xl == 4 && ring) || (xl == 1 && !ring && ty == 8);
-  const bool in_step = rec != REC_NONE && fused && c->rec_fusion && rec_kernel &&
-                       form == FORM_VL &&
-                       (src ? c->src_plane && c->nsrc > 0 : c->rec_plane && c->nrec > 0);
-  if (in_step) {
+  const bool plane = rec != REC_NONE && fused && c->rec_fusion && form == FORM_VL &&
+                     (src ? c->src_plane && c->nsrc > 0 : c->rec_plane && c->nrec > 0);
+  const StepChoice ch = choose_step(step_setting(c), form, act, fmt,
+                                    !plane ? REC_NONE : src ? REC_INJECT : rec);
+  P.ntx = ch.ntx;
+  P.nty = ch.nty;
+  P.ntz = ch.ntz;
+  P.zc = ch.zc;
+  if (ch.rec != REC_NONE) {
     P.rz = src ? c->src_z : c->rec_z;
     P.nrec = src ? c->nsrc : c->nrec;
     P.rsp = src ? c->ntr_s : 1;
@@ -275,23 +236,29 @@ int step(brtm_ctx *c, int form, int act, int fmt, const float *p, const float *p
     P.rscale = rec == REC_EXTRACT ? rscale : nullptr;
     std::memcpy(P.rsinc, &c->sinc[src ? 0 : 1][8 * (it % jt)], sizeof(P.rsinc));
   }
-  const int kmode = !in_step ? REC_NONE : (src ? REC_INJECT : rec);
-  if (direct) {
-    // two slices per thread once that still leaves 12 waves per compute unit
-    const long waves2 = ((c->n1 - 5L) / 4) * (c->n2 - 8) * ((c->n3 - 7) / 2) / 64;
-    BRTM_HIP(launch_step_direct(act, fmt, P, waves2 >= 12L * c->ncu ? 2 : 1, c->stream, kmode));
-  } else if (auto4)
-    BRTM_HIP(launch_step_auto4(act, fmt, P, c->ncu, c->stream, kmode));
-  else if (xl == 1 && form == FORM_VL && ring)
-    BRTM_HIP(launch_step_ring(act, fmt, P, ty, c->stream));
-  else if (xl == 4)
-    BRTM_HIP(launch_step_x4(act, fmt, P, ty, ring, c->stream, kmode));
-  else if (xl == 2)
-    BRTM_HIP(launch_step_x2(act, fmt, P, ty, c->stream));
-  else
-    BRTM_HIP(launch_step(form, act, fmt, P, ty, c->stream, kmode));
+  BRTM_TRY(ktime_begin(c, timed));
+  switch (ch.kernel) {
+    case STEP_DIRECT:
+      BRTM_HIP(launch_step_direct(act, fmt, P, c->stream, ch.rec));
+      break;
+    case STEP_X4R:
+      BRTM_HIP(launch_step_x4r(act, fmt, P, ch.tw, ch.ty, c->stream, ch.rec));
+      break;
+    case STEP_X4:
+      BRTM_HIP(launch_step_x4(act, fmt, P, ch.ty, c->stream));
+      break;
+    case STEP_X2:
+      BRTM_HIP(launch_step_x2(act, fmt, P, ch.ty, c->stream));
+      break;
+    case STEP_RING:
+      BRTM_HIP(launch_step_ring(act, fmt, P, ch.ty, c->stream));
+      break;
+    case STEP_TILES:
+      BRTM_HIP(launch_step(form, act, fmt, P, ch.ty, c->stream, ch.rec));
+      break;
+  }
   BRTM_TRY(ktime_end(c, timed));
-  if (fused) *fused = in_step;
+  if (fused) *fused = ch.rec != REC_NONE;
   return BRTM_OK;
 }
 
@@ -1236,6 +1203,21 @@ int brtm_propagate(brtm_ctx *c, int form, int nsteps, float *p_cur, float *p_old
   BRTM_HIP(launch_zero_halo(cur, c->ncell, 1, c->n1, c->n2, c->n3, c->stream));
   BRTM_HIP(launch_zero_halo(old, c->ncell, 1, c->n1, c->n2, c->n3, c->stream));
   BRTM_HIP(hipStreamSynchronize(c->stream));
+  return BRTM_OK;
+}
+
+int brtm_step_kernel(brtm_ctx *c, int form, int act, int fmt, int rec, char *name, int len) {
+  BRTM_REQUIRE(c && name && len > 0, BRTM_EINVAL, "bad arguments");
+  BRTM_REQUIRE((form == FORM_VL || form == FORM_LV) && act >= ACT_NONE && act <= ACT_BORN &&
+                   fmt >= FMT_NONE && fmt <= FMT_F16 && rec >= REC_NONE && rec <= REC_EXTRACT &&
+                   (act == ACT_NONE) == (fmt == FMT_NONE),
+               BRTM_EINVAL, "no such step");
+  BRTM_REQUIRE(c->have_space, BRTM_ESTATE, "brtm_create_space has not been called");
+  const StepChoice ch = choose_step(step_setting(c), form, act, fmt, rec);
+  std::string s = step_kernel_name(ch);
+  if (ch.kernel == STEP_X4R && streams(c)) s += " + streaming loads";
+  BRTM_REQUIRE((int)s.size() < len, BRTM_EINVAL, "name does not fit");
+  std::memcpy(name, s.c_str(), s.size() + 1);
   return BRTM_OK;
 }
 

@@ -4,22 +4,9 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-namespace brtm {
+#include "step_choice.h"
 
-// Storage format of a source-wavefield snapshot.
-enum SnapFmt { FMT_NONE = 0, FMT_F32 = 1, FMT_BF16 = 2, FMT_F16 = 3 };
-// Step form: VL = V.L(p) (Born/wave_fkernel.3d8o.cu:31), LV = L(V.p) (:109).
-enum StepForm { FORM_VL = 0, FORM_LV = 1 };
-// What the step does with the snapshot s besides the update:
-//   ACT_IMG  img += cimg . s . p_new        (zero-lag imaging, VL only)
-//   ACT_BORN p_new += cimg . s . m          (Born secondary source)
-enum StepAct { ACT_NONE = 0, ACT_IMG = 1, ACT_BORN = 2 };
-// Receivers handled inside the step (the four-cell ring kernel, the kernel
-// without LDS, and the one-cell kernel's 8-row shape):
-//   REC_INJECT   pn += sum_k rsinc[k] rtr(r, rid+k) before imaging and the store
-//   REC_EXTRACT  rtr(r, rid+k) += rsinc[k] . pn . (rscale[r] or 1)
-// for the cells of plane rz whose rmap entry is a receiver index r >= 0.
-enum RecMode { REC_NONE = 0, REC_INJECT = 1, REC_EXTRACT = 2 };
+namespace brtm {
 
 constexpr int kWMax = 256;  // longest sponge table the kernels accept
 
@@ -72,18 +59,16 @@ hipError_t launch_step(int form, int act, int fmt, StepParams P, int ty_tile, hi
 hipError_t launch_step_ring(int act, int fmt, StepParams P, int ty_tile, hipStream_t st);
 // The VL step with two consecutive x per lane (128-wide tiles, n1 even).
 hipError_t launch_step_x2(int act, int fmt, StepParams P, int ty_tile, hipStream_t st);
-// The VL step with four consecutive x per lane (256-wide tiles, n1 % 4 == 0),
-// on the two-plane buffer or (ring) the six-plane halo ring; rec (RecMode,
-// ring only) handles the receivers inside the step.
-hipError_t launch_step_x4(int act, int fmt, StepParams P, int ty_tile, bool ring,
-                          hipStream_t st, int rec = REC_NONE);
-// The four-cell ring step in the tile shape and z chunks that fill ncu
-// compute units best (plans P itself).
-hipError_t launch_step_auto4(int act, int fmt, const StepParams &P, int ncu, hipStream_t st,
-                             int rec = REC_NONE);
-// The VL step without LDS for grids that stay in the caches (any n1): zc
+// The VL step with four consecutive x per lane on the two-plane buffer
+// (256-wide tiles, n1 % 4 == 0).
+hipError_t launch_step_x4(int act, int fmt, const StepParams &P, int ty_tile, hipStream_t st);
+// ... on the six-plane halo ring, in tiles of tw x ty cells (256 x 8, 256 x 16,
+// 128 x 24 or 64 x 16); rec (RecMode): the receivers inside the step.
+hipError_t launch_step_x4r(int act, int fmt, const StepParams &P, int tw, int ty, hipStream_t st,
+                           int rec = REC_NONE);
+// The VL step without LDS for grids that stay in the caches (any n1), P.zc
 // (1 or 2) slices per thread; rec as above.
-hipError_t launch_step_direct(int act, int fmt, const StepParams &P, int zc, hipStream_t st,
+hipError_t launch_step_direct(int act, int fmt, const StepParams &P, hipStream_t st,
                               int rec = REC_NONE);
 // Two consecutive plain VL steps in one pass: p^{n+1} = step(p = p^n,
 // po = p^{n-1}) into pn and p^{n+2} = step(p^{n+1}, p^n) into pn2, with the
@@ -93,10 +78,6 @@ hipError_t launch_step_direct(int act, int fmt, const StepParams &P, int zc, hip
 // not alias p, po or each other (other tiles read p and po around their
 // own).  n1 % 4 == 0.  Fills the tile geometry itself.
 hipError_t launch_step2(StepParams P, int target_blocks, hipStream_t st, int rec = REC_NONE);
-// Tile / chunk geometry chosen for a grid (fills ntx..zc of P); xw is the
-// tile width in x (64, 128 or 256 for the 1-, 2- and 4-cell kernels).
-void plan_step(StepParams &P, int ty_tile, int target_blocks, int xw = 64);
-
 // p[loc_j] += scale * sum_k sinc8[k] tr(j, id+k), tr(j,t) = tr[j*sp + t*st].
 // When img != null: img[loc_j] += cimg * s[loc_j] * (added amount).
 struct InjectParams {

@@ -2456,79 +2456,28 @@ hipError_t launch_step_ring(int act, int fmt, StepParams P, int ty_tile, hipStre
   return launch_ring_t<16, 4>(act, fmt, P, st);
 }
 
-hipError_t launch_step_x4(int act, int fmt, StepParams P, int ty_tile, bool ring,
-                          hipStream_t st, int rec) {
+static bool rec_ok(const StepParams &P, int rec) {
+  return rec == REC_NONE ||
+         (P.rmap && P.rtr && P.nrec > 0 && P.rz >= 4 && P.rz < P.n3 - 4);
+}
+
+hipError_t launch_step_x4(int act, int fmt, const StepParams &P, int ty_tile, hipStream_t st) {
   if (P.nw > kWMax || P.n3 < 9 || P.n2 < 9 || P.n1 < 12 || (P.n1 & 3)) return hipErrorInvalidValue;
-  if (rec != REC_NONE && (!P.rmap || !P.rtr || P.nrec <= 0 || P.rz < 4 || P.rz >= P.n3 - 4))
-    return hipErrorInvalidValue;
-  // 8-row tiles with one row per thread, or 16-row tiles with two (ty_tile
-  // 16 or 32); four cells per lane leave no registers for taller tiles.
-  if (ring) {
-    if (ty_tile == 8) return by_action<RingShapeOf<64, 8, 1>::L>(act, fmt, P, st, rec);
-    return by_action<RingShapeOf<64, 8, 2>::L>(act, fmt, P, st, rec);
-  }
-  if (rec != REC_NONE) return hipErrorInvalidValue;
+  // 8-row tiles with one row per thread, or 16-row tiles with two; four cells
+  // per lane leave no registers for taller tiles.
   if (ty_tile == 8) return by_action<FlatShapeOf<8, 1>::L>(act, fmt, P, st);
   return by_action<FlatShapeOf<16, 2>::L>(act, fmt, P, st);
 }
 
-// z chunks of a ring step whose workgroups run `capacity` at a time: a round
-// of workgroups takes a chunk's slices plus about nine for its prologue, so
-// the chunk count that fills one to four rounds with the fewest slices wins.
-// Returns the slices all rounds take together.
-static long plan_rounds(StepParams &P, int ty, int xw, int capacity) {
-  P.ntx = (P.n1 + xw - 1) / xw;
-  P.nty = (P.n2 + ty - 1) / ty;
-  const int nz = P.n3 - 8;
-  const long tiles = (long)P.ntx * P.nty;
-  long best = -1;
-  for (int r = 1; r <= 4; ++r) {
-    const long want = std::max(1L, std::min((long)nz, capacity * (long)r / tiles));
-    const int zc = (int)((nz + want - 1) / want), ntz = (nz + zc - 1) / zc;
-    const long rounds = (tiles * ntz + capacity - 1) / capacity;
-    const long cost = rounds * (zc + 9);
-    if (best < 0 || cost < best) {
-      best = cost;
-      P.zc = zc;
-      P.ntz = ntz;
-    }
-  }
-  return best;
-}
-
-hipError_t launch_step_auto4(int act, int fmt, const StepParams &P, int ncu, hipStream_t st,
-                             int rec) {
-  if (P.nw > kWMax || P.n3 < 9 || P.n2 < 9 || P.n1 < 12 || (P.n1 & 3)) return hipErrorInvalidValue;
-  if (rec != REC_NONE && (!P.rmap || !P.rtr || P.nrec <= 0 || P.rz < 4 || P.rz >= P.n3 - 4))
+hipError_t launch_step_x4r(int act, int fmt, const StepParams &P, int tw, int ty, hipStream_t st,
+                           int rec) {
+  if (P.nw > kWMax || P.n3 < 9 || P.n2 < 9 || P.n1 < 12 || (P.n1 & 3) || !rec_ok(P, rec))
     return hipErrorInvalidValue;
-  // Tile shapes, and what a slice of one round of workgroups costs next to a
-  // slice of 256 x 8 tiles (plain steps at 256^3 to 512^3):
-  //   256 x 8   1.00  one 8-wave workgroup per CU
-  //   256 x 16  1.66  the same with two rows per thread, plain steps only (in
-  //                   the others its second row costs twice: FP16 imaging at
-  //                   512^3 630 us against 590 us in 256 x 8)
-  //   128 x 24  1.33  one 12-wave workgroup per CU
-  //   64 x 16   1.38  three 4-wave workgroups per CU
-  // The shape whose rounds cost least is taken: where 256-wide tiles fit the
-  // rows they win (256^3: plain 38.6 us against 39.9 us in 128 x 24 and 42.0
-  // us in the 256 x 16 tiles used there before; 512^3 256 x 16), elsewhere the
-  // narrow ones: 384^3 149 us in 128 x 24 (287-323 us in 256 x 16 with a
-  // second round of 32 workgroups before), 320^3 101 us and 288 x 240 x 208 36
-  // us in 64 x 16 (120 and 46 us in the two-cell kernel before).
-  // (imaging and Born steps move more per slice, which the narrow shapes' finer
-  // halos cost more: FP32 imaging at 512^3 640 us in 256 x 8, 750 us in 64 x 16)
-  const bool plain = act == ACT_NONE;
-  StepParams Q[4] = {P, P, P, P};
-  const double cost[4] = {1.00 * plan_rounds(Q[0], 8, 256, ncu),
-                          plain ? 1.66 * plan_rounds(Q[1], 16, 256, ncu) : 1e30,
-                          (plain ? 1.33 : 1.45) * plan_rounds(Q[2], 24, 128, ncu),
-                          (plain ? 1.38 : 1.60) * plan_rounds(Q[3], 16, 64, 3 * ncu)};
-  switch (std::min_element(cost, cost + 4) - cost) {
-    case 0: return by_action<RingShapeOf<64, 8, 1>::L>(act, fmt, Q[0], st, rec);
-    case 1: return by_action<RingShapeOf<64, 8, 2>::L>(act, fmt, Q[1], st, rec);
-    case 2: return by_action<RingShapeOf<32, 12, 1>::L>(act, fmt, Q[2], st, rec);
-    default: return by_action<RingShapeOf<16, 4, 1>::L>(act, fmt, Q[3], st, rec);
-  }
+  if (tw == 256 && ty == 8) return by_action<RingShapeOf<64, 8, 1>::L>(act, fmt, P, st, rec);
+  if (tw == 256 && ty == 16) return by_action<RingShapeOf<64, 8, 2>::L>(act, fmt, P, st, rec);
+  if (tw == 128 && ty == 24) return by_action<RingShapeOf<32, 12, 1>::L>(act, fmt, P, st, rec);
+  if (tw == 64 && ty == 16) return by_action<RingShapeOf<16, 4, 1>::L>(act, fmt, P, st, rec);
+  return hipErrorInvalidValue;
 }
 
 template <int ZC, int FMT, int ACT, int REC>
@@ -2559,22 +2508,12 @@ struct DirectOf {
   };
 };
 
-template <int ZC>
-hipError_t launch_direct_t(int act, int fmt, StepParams P, hipStream_t st, int rec) {
-  const long groups = (long)((P.n1 - 5) / 4) * (P.n2 - 8);
-  P.ntx = (int)((groups + 255) / 256);
-  P.ntz = (P.n3 - 8 + ZC - 1) / ZC;
-  if ((long)P.ntx * P.ntz > 0x7fffffffL) return hipErrorInvalidValue;
-  return by_action<DirectOf<ZC>::template L>(act, fmt, P, st, rec);
-}
-
-hipError_t launch_step_direct(int act, int fmt, const StepParams &P, int zc, hipStream_t st,
-                              int rec) {
-  if (P.nw > kWMax || P.n3 < 9 || P.n2 < 9 || P.n1 < 9) return hipErrorInvalidValue;
-  if (rec != REC_NONE && (!P.rmap || !P.rtr || P.nrec <= 0 || P.rz < 4 || P.rz >= P.n3 - 4))
+hipError_t launch_step_direct(int act, int fmt, const StepParams &P, hipStream_t st, int rec) {
+  if (P.nw > kWMax || P.n3 < 9 || P.n2 < 9 || P.n1 < 9 || !rec_ok(P, rec))
     return hipErrorInvalidValue;
-  if (zc == 1) return launch_direct_t<1>(act, fmt, P, st, rec);
-  return launch_direct_t<2>(act, fmt, P, st, rec);
+  if (P.zc == 1) return by_action<DirectOf<1>::L>(act, fmt, P, st, rec);
+  if (P.zc == 2) return by_action<DirectOf<2>::L>(act, fmt, P, st, rec);
+  return hipErrorInvalidValue;
 }
 
 template <int REC>
@@ -2594,21 +2533,14 @@ hipError_t launch_step2(StepParams P, int target_blocks, hipStream_t st, int rec
   if (rec != REC_NONE &&
       (rec != REC_INJECT || !P.rmap || !P.rtr || P.nrec <= 0 || P.rz < 4 || P.rz >= P.n3 - 4))
     return hipErrorInvalidValue;
-  plan_step(P, 32, target_blocks, 64);
+  StepChoice c{};
+  plan_tiles(c, {P.n1, P.n2, P.n3}, 64, 32, target_blocks);
+  P.ntx = c.ntx;
+  P.nty = c.nty;
+  P.ntz = c.ntz;
+  P.zc = c.zc;
   if (rec == REC_INJECT) return launch_step2_r<REC_INJECT>(P, st);
   return launch_step2_r<REC_NONE>(P, st);
-}
-
-void plan_step(StepParams &P, int ty_tile, int target_blocks, int xw) {
-  P.ntx = (P.n1 + xw - 1) / xw;
-  P.nty = (P.n2 + ty_tile - 1) / ty_tile;
-  const int nz = P.n3 - 8;
-  const long tiles = (long)P.ntx * P.nty;
-  long zc = (tiles * nz + target_blocks - 1) / target_blocks;
-  if (zc < 8) zc = 8;
-  if (zc > nz) zc = nz;
-  P.zc = (int)zc;
-  P.ntz = (nz + P.zc - 1) / P.zc;
 }
 
 hipError_t launch_step(int form, int act, int fmt, StepParams P, int ty_tile, hipStream_t st,

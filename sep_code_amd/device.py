@@ -164,6 +164,13 @@ class BornDevice:
         call("brtm_time_step", self.h, int(form), int(act), int(fmt), int(nrep), C.byref(ms))
         return ms.value
 
+    def step_kernel(self, form=0, act=0, fmt=0, rec=0):
+        """Name and tile shape of the kernel such a step runs on here (rec: 0,
+        or receivers inside the step: 1 injected, 2 extracted)."""
+        name = C.create_string_buffer(128)
+        call("brtm_step_kernel", self.h, int(form), int(act), int(fmt), int(rec), name, len(name))
+        return name.value.decode()
+
     def copy_bench(self, nbytes, nrep=10):
         ms = C.c_double()
         call("brtm_copy_bench", self.h, float(nbytes), int(nrep), C.byref(ms))
