@@ -102,7 +102,8 @@ inline long plan_rounds(StepChoice &c, const StepSetting &s, int tw, int ty, int
 //   256 x 8   1.00  one 8-wave workgroup per CU
 //   256 x 16  1.66  the same with two rows per thread, plain steps only (in
 //                   the others its second row costs twice: FP16 imaging at
-//                   512^3 630 us against 590 us in 256 x 8)
+//                   512^3 630 us against 590 us in 256 x 8); 1.55 where the
+//                   step extracts receivers
 //   128 x 24  1.33  one 12-wave workgroup per CU
 //   64 x 16   1.38  three 4-wave workgroups per CU
 // The shape whose rounds cost least is taken: where 256-wide tiles fit the
@@ -113,12 +114,22 @@ inline long plan_rounds(StepChoice &c, const StepSetting &s, int tw, int ty, int
 // us in 64 x 16 (120 and 46 us in the two-cell kernel before).
 // (imaging and Born steps move more per slice, which the narrow shapes' finer
 // halos cost more: FP32 imaging at 512^3 640 us in 256 x 8, 750 us in 64 x 16)
-inline void choose_ring_tiles(StepChoice &c, const StepSetting &s, int act) {
+// Steps that extract receivers (Born modelling) take 256 x 16 earlier: where
+// several contexts model by turns, which overlaps their steps, the 256 x 8 tiles'
+// twofold y halo costs more than the second round that 256 x 16 may leave, and
+// alone the two are even.  A modelling of two shots at 256^3 (FP16 snapshots
+// every 4 of 120 steps), three contexts by turns / one alone: 13.07 / 11.53 ms
+// in 256 x 8, 12.65 / 11.75 in 256 x 16 (12.68 / 12.40 before 256 x 8 was
+// introduced); one shot of 100 steps at 240^3 4.85 / 4.46 against 4.70 / 4.38,
+// at 256 x 224 x 288 5.88 / 5.02 against 5.78 / 5.02, at 512 x 160 x 208 6.00 /
+// 5.29 against 5.95 / 5.29.  Steps that inject keep the line above (adjoint at
+// 256^3 12.83 / 12.05 in 256 x 8, 12.72 / 12.50 in 256 x 16).
+inline void choose_ring_tiles(StepChoice &c, const StepSetting &s, int act, int rec) {
   const bool plain = act == ACT_NONE;
   StepChoice q[4] = {c, c, c, c};
   const double cost[4] = {
       1.00 * plan_rounds(q[0], s, 256, 8, s.ncu),
-      plain ? 1.66 * plan_rounds(q[1], s, 256, 16, s.ncu) : 1e30,
+      plain ? (rec == REC_EXTRACT ? 1.55 : 1.66) * plan_rounds(q[1], s, 256, 16, s.ncu) : 1e30,
       (plain ? 1.33 : 1.45) * plan_rounds(q[2], s, 128, 24, s.ncu),
       (plain ? 1.38 : 1.60) * plan_rounds(q[3], s, 64, 16, 3 * s.ncu)};
   c = q[std::min_element(cost, cost + 4) - cost];
@@ -148,7 +159,7 @@ inline StepChoice choose_step(const StepSetting &s, int form, int act, int fmt, 
   if (autosel && s.n1 % 4 == 0) {
     c.kernel = STEP_X4R;
     c.rec = rec;
-    choose_ring_tiles(c, s, act);
+    choose_ring_tiles(c, s, act, rec);
     return c;
   }
   // cells per lane: 4 or 2 where asked for and n1 allows, else 1; automatic

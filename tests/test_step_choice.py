@@ -62,6 +62,16 @@ def test_automatic_kernels(choose, n, act, fmt, kernel, tile):
     assert (c[3] if kernel == "k_step_direct" else (c[1], c[2])) == tile, name
 
 
+@pytest.mark.parametrize("n", [(256, 256, 256), (240, 240, 240), (512, 160, 208)])
+def test_extracting_steps_take_taller_tiles(choose, n):
+    """Plain steps of Born modelling, which extract receivers, run in 16-row
+    tiles where the others take 8 rows or narrow tiles; steps with an action
+    keep their shape."""
+    assert choose(n, rec=EXTRACT)[1][1:3] == [256, 16]
+    assert choose(n, rec=INJECT)[1][1:3] == choose(n)[1][1:3] != [256, 16]
+    assert choose(n, BORN, F16, EXTRACT)[1][1:3] == choose(n, BORN, F16)[1][1:3] == [256, 8]
+
+
 @pytest.mark.parametrize("xl,ring,ty,kernel,tile", [
     (1, -1, 0, "k_step", (64, 32)), (1, 1, 16, "k_step_ring", (64, 16)),
     (2, -1, 0, "k_step_x2", (128, 16)), (4, 0, 0, "k_step_x4", (256, 16)),
