@@ -992,6 +992,11 @@ k_step_x4r(const StepParams P) {
   constexpr int HY = (8 * LX + NT - 1) / NT, NH = HY + RPT;
   constexpr int LW = TW + 8;
   constexpr int NR = 6;
+  // FP32 imaging in 256-wide tiles issues a slice's loads in one uniform branch,
+  // all masked by exec, without the wait below: 61.0 us at 256^3, 155.5 at 512 x
+  // 256 x 256 (62.6 and 156.4 with its snapshot and image through buffer
+  // loads and the wait, as the 16-bit formats have them).
+  constexpr bool ONE_BRANCH = LX == 64 && ACT == ACT_IMG && FMT == FMT_F32;
   __shared__ __attribute__((aligned(16))) float ring[NR][TY + 8][LW];
   __shared__ float wsh[kWMax];
 
@@ -1078,7 +1083,11 @@ k_step_x4r(const StepParams P) {
       // an FP32 snapshot streams at every size (64.6 against 70.4 us for
       // FP32 imaging at 256^3); 16-bit ones only with STREAM (BF16 imaging
       // at 256^3: 77.4 against 74.6 us)
-      if constexpr (FMT == FMT_F32) {
+      if constexpr (ONE_BRANCH) {
+#pragma unroll
+        for (int r = 0; r < RPT; ++r)
+          oS[r] = plane_ld4<true>(plane(static_cast<const float *>(P.snap), z), lo[r], on);
+      } else if constexpr (FMT == FMT_F32) {
         const plane_rsrc rs = plane_of(plane(static_cast<const float *>(P.snap), z), pb);
 #pragma unroll
         for (int r = 0; r < RPT; ++r) oS[r] = buffer_ld4<true>(rs, lo[r]);
@@ -1095,9 +1104,14 @@ k_step_x4r(const StepParams P) {
       // the image streams at every size (FP32 / BF16 imaging at 256^3:
       // 62.3 / 71.6 against 65.2 / 74.6 us); the model only with STREAM
       // (the Born step at 256^3: 66.0 against 64.5 us)
-      const plane_rsrc rx = plane_of(plane(ACT == ACT_IMG ? P.img : P.m, z), pb);
+      if constexpr (ONE_BRANCH) {
 #pragma unroll
-      for (int r = 0; r < RPT; ++r) oX[r] = buffer_ld4 < STREAM || ACT == ACT_IMG > (rx, lo[r]);
+        for (int r = 0; r < RPT; ++r) oX[r] = plane_ld4<true>(plane(P.img, z), lo[r], on);
+      } else {
+        const plane_rsrc rx = plane_of(plane(ACT == ACT_IMG ? P.img : P.m, z), pb);
+#pragma unroll
+        for (int r = 0; r < RPT; ++r) oX[r] = buffer_ld4 < STREAM || ACT == ACT_IMG > (rx, lo[r]);
+      }
     }
   };
 
@@ -1142,7 +1156,7 @@ k_step_x4r(const StepParams P) {
     // costs less in the plain step (320^3: 102 against 109 us) and in
     // 256-wide tiles, and more in the narrow tiles' imaging and Born steps
     // (384^3, FP32 imaging: 282 against 270 us), which leave it out.
-    if constexpr (LX == 64 || ACT == ACT_NONE) __builtin_amdgcn_s_waitcnt(0x0f70);
+    if constexpr (ACT == ACT_NONE || (LX == 64 && !ONE_BRANCH)) __builtin_amdgcn_s_waitcnt(0x0f70);
     {
       f32x4 c[RPT];
 #pragma unroll
@@ -1154,10 +1168,17 @@ k_step_x4r(const StepParams P) {
     const int zf = on ? z + PF : z;
     f32x4 nq[RPT], nh[NH];
     f32x4 npo[RPT], nV[RPT], nS[RPT], nX[RPT];
+    auto load_next = [&](bool in) {
 #pragma unroll
-    for (int r = 0; r < RPT; ++r) nq[r] = plane_ld4<false>(plane(P.p, zf + 4), lo[r], on);
-    load_halo(zf + 4, on, nh);
-    load_center(zf, on, npo, nV, nS, nX);
+      for (int r = 0; r < RPT; ++r) nq[r] = plane_ld4<false>(plane(P.p, zf + 4), lo[r], in);
+      load_halo(zf + 4, in, nh);
+      load_center(zf, in, npo, nV, nS, nX);
+    };
+    if constexpr (ONE_BRANCH) {
+      if (on) load_next(true);
+    } else {
+      load_next(on);
+    }
     __syncthreads();
 
     float(*pl)[LW] = ring[z % NR];
