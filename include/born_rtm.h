@@ -188,9 +188,10 @@ int brtm_set_tuning(brtm_ctx *ctx, int ty_tile, int target_blocks);
 /* Cells per lane along x for VL-form steps: 1 (64-wide tiles, 4-byte
  * accesses), 2 (128-wide tiles, 8-byte accesses; n1 even) or 4 (256-wide
  * tiles, 16-byte accesses; n1 % 4 == 0); 0 (the default) picks by the grid:
- * a four-cell kernel without LDS up to 10 M cells (16 M where n1 % 4 != 0),
+ * a four-cell kernel without LDS up to 7 M cells (16 M where n1 % 4 != 0),
  * whose reuse the caches serve; above, with n1 % 4 == 0, the four-cell ring in
- * the tile shape whose rounds of workgroups cost least; else the one-cell or
+ * the tile shape whose rounds of workgroups cost least, or up to 12.6 M cells
+ * the kernel without LDS where that costs less; else the one-cell or
  * two-cell tiles.  A grid that does not allow the width asked for uses the
  * widest one it allows.  Results agree to FP32 rounding. */
 int brtm_set_x_per_lane(brtm_ctx *ctx, int cells);
@@ -221,7 +222,8 @@ int brtm_set_prefetch(brtm_ctx *ctx, int slices);
 /* Streaming (nontemporal) loads of p_old, V, 16-bit snapshots and the
  * model, which the four-cell ring step reads once: 1 on, 0 off, -1 (the
  * default) on when a step moves more than 512 MB, twice the Infinity Cache
- * (512^3 yes, 256^3 no).  The image and FP32 snapshots stream at every
+ * (512^3 yes, 256^3 no), except in 64-wide tiles of rows of which 16 cells are
+ * no divisor.  The image and FP32 snapshots stream at every
  * size.  No counterpart in the reference; the same results. */
 int brtm_set_stream_loads(brtm_ctx *ctx, int mode);
 

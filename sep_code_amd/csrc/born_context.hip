@@ -149,12 +149,6 @@ static hipError_t h2d(brtm_ctx *c, void *dst, const void *src, size_t bytes) {
 
 // Load lookahead of the plain four-cell ring step when left automatic.
 constexpr int kAutoPrefetch = 1;
-// Streaming (nontemporal) loads pay off once a step's working set (16 B per
-// cell: p, p_old, V, p_new) is well beyond the 256 MB Infinity Cache: 6 %
-// faster at 512^3.  Below that the fields stay cache-resident between
-// launches, which the hint would forfeit: 11 % slower at 256^3.
-constexpr double kStreamMinStepBytes = 512.0 * 1024 * 1024;
-
 #define BRTM_TRY(x)              \
   do {                           \
     int rc_ = (x);               \
@@ -186,9 +180,8 @@ static StepSetting step_setting(const brtm_ctx *c) {
   return {c->n1, c->n2, c->n3, c->ncu, c->ty_tile, c->target_blocks, c->x_per_lane, c->halo_ring};
 }
 
-static bool streams(const brtm_ctx *c) {
-  return c->stream_loads < 0 ? 16.0 * (double)c->ncell > kStreamMinStepBytes
-                             : c->stream_loads != 0;
+static bool streams(const brtm_ctx *c, const StepChoice &ch) {
+  return c->stream_loads < 0 ? choose_streaming(step_setting(c), ch) : c->stream_loads != 0;
 }
 
 int step(brtm_ctx *c, int form, int act, int fmt, const float *p, const float *po, float *pn,
@@ -212,7 +205,6 @@ int step(brtm_ctx *c, int form, int act, int fmt, const float *p, const float *p
   P.m = m;
   P.cimg = c->cimg;
   P.pf = c->prefetch == 0 ? kAutoPrefetch : c->prefetch;
-  P.stream = streams(c);
   const bool timed =
       c->ktime_on && form == c->ktime_form && act == c->ktime_act && fmt == c->ktime_fmt;
   // receivers inside the step, where the kernel takes them: one plane
@@ -225,6 +217,7 @@ int step(brtm_ctx *c, int form, int act, int fmt, const float *p, const float *p
   P.nty = ch.nty;
   P.ntz = ch.ntz;
   P.zc = ch.zc;
+  P.stream = streams(c, ch);
   if (ch.rec != REC_NONE) {
     P.rz = src ? c->src_z : c->rec_z;
     P.nrec = src ? c->nsrc : c->nrec;
@@ -1215,7 +1208,7 @@ int brtm_step_kernel(brtm_ctx *c, int form, int act, int fmt, int rec, char *nam
   BRTM_REQUIRE(c->have_space, BRTM_ESTATE, "brtm_create_space has not been called");
   const StepChoice ch = choose_step(step_setting(c), form, act, fmt, rec);
   std::string s = step_kernel_name(ch);
-  if (ch.kernel == STEP_X4R && streams(c)) s += " + streaming loads";
+  if (ch.kernel == STEP_X4R && streams(c, ch)) s += " + streaming loads";
   BRTM_REQUIRE((int)s.size() < len, BRTM_EINVAL, "name does not fit");
   std::memcpy(name, s.c_str(), s.size() + 1);
   return BRTM_OK;

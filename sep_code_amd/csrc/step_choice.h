@@ -44,17 +44,25 @@ struct StepChoice {
   int rec;                 // the receivers' mode inside the step, or REC_NONE
 };
 
-// Largest grids of the VL step without LDS.  Its taps go through L1 and L2,
+// Largest grids of the VL step without LDS, whose taps go through L1 and L2,
 // which pays while the fields stay in the Infinity Cache.  Plain / FP32
-// imaging / FP16 imaging / FP16 Born steps in us, before and with it: 48^3 8.8
-// / 9.6 / 11.6 / 11.5 and 3.2 / 3.6 / 3.6 / 3.5; 128^3 10.6 / 11.9 / 16.3 / 15.8
-// and 8.4 / 11.1 / 10.6 / 9.8; 208^3 (9.0 M cells) 31 / 63 / 47 / 45 and 26 / 40
-// / 37 / 33.  At 288 x 240 x 208 (14.4 M) it takes 41 / 77 / 61 / 57, the ring's
-// 64 x 16 tiles 36 / 62 / 63 / 55.  Where n1 is no multiple of 4 the
-// alternative is the one- or two-cell kernel: 257 x 201 x 233 (12 M) 41 / 66 /
-// 60 / 52 against 36 / 54 / 51 / 44, 301^3 (27 M) 100 / 173 / 172 / 150 against
-// 113 / 178 / 174 / 149.
-constexpr long kDirectMaxCells = 10L << 20, kDirectMaxCellsOdd = 16L << 20;
+// imaging / FP16 imaging / FP16 Born steps in us, in the tiled kernels and
+// without LDS: 48^3 8.8 / 9.6 / 11.6 / 11.5 and 3.2 / 3.6 / 3.6 / 3.5; 128^3
+// 10.6 / 11.9 / 16.3 / 15.8 and 8.4 / 11.1 / 10.6 / 9.8.  Where n1 % 4 == 0 the
+// ring's tiles come near it from 7 M cells on.  There a million (2^20) cells
+// take 3.1 / 4.7 / 4.35 / 3.85 us without LDS, about 3.74 (plain) or 3.44 of the
+// slices that the ring's tiles are counted in (choose_ring_tiles): the ring
+// is taken where it costs less, and from 10 M cells to 12.6 M, where the caches
+// begin to overflow, unless it costs a tenth more.  224 x 256 x 160 (8.8 M) 25.9 /
+// 38.4 / 35.7 / 31.9 and in 256 x 8 tiles 25.6 / 36.2 / 36.4 / 29.8; 272 x 541 x 86
+// (12.1 M) 32.9 / 46.2 / 43.5 / 39.9 and in 64 x 16 tiles 33.6 / 62.8 / 58.9 / 41.5
+// (60 in the two-cell kernel, FP32 imaging); 288 x 240 x 208 (13.7 M) 41 / 78 /
+// 63 / 54 and 36 / 63 / 59 / 47.  Where n1 is no multiple of 4 the alternative is
+// the one- or two-cell kernel: 257 x 201 x 233 (12 M) 41 / 66 / 60 / 52 against
+// 36 / 54 / 51 / 44, 301^3 (27 M) 100 / 173 / 172 / 150 against 113 / 178 / 174 /
+// 149.
+constexpr long kDirectCells = 7L << 20, kDirectEven = 10L << 20,
+               kDirectMaxCells = 126L * (1 << 20) / 10, kDirectMaxCellsOdd = 16L << 20;
 
 // z chunks of tiles tw x ty: about target_blocks workgroups in all, at least
 // 8 slices each.
@@ -96,24 +104,28 @@ inline long plan_rounds(StepChoice &c, const StepSetting &s, int tw, int ty, int
   return best;
 }
 
-// The four-cell ring's automatic tile shape, and what a slice of one round of
-// workgroups costs next to a slice of 256 x 8 tiles (plain steps at 256^3 to
-// 512^3):
-//   256 x 8   1.00  one 8-wave workgroup per CU
-//   256 x 16  1.66  the same with two rows per thread, plain steps only (in
-//                   the others its second row costs twice: FP16 imaging at
-//                   512^3 630 us against 590 us in 256 x 8); 1.55 where the
-//                   step extracts receivers
-//   128 x 24  1.33  one 12-wave workgroup per CU
-//   64 x 16   1.38  three 4-wave workgroups per CU
-// The shape whose rounds cost least is taken: where 256-wide tiles fit the
-// rows they win (256^3: plain 38.6 us against 39.9 us in 128 x 24 and 42.0
-// us in the 256 x 16 tiles used there before; 512^3 256 x 16), elsewhere the
-// narrow ones: 384^3 149 us in 128 x 24 (287-323 us in 256 x 16 with a
-// second round of 32 workgroups before), 320^3 101 us and 288 x 240 x 208 36
-// us in 64 x 16 (120 and 46 us in the two-cell kernel before).
-// (imaging and Born steps move more per slice, which the narrow shapes' finer
-// halos cost more: FP32 imaging at 512^3 640 us in 256 x 8, 750 us in 64 x 16)
+// The four-cell ring's automatic tile shape: the one whose rounds of workgroups
+// cost least, in slices of one round of 256 x 8 tiles.  What a slice of the
+// others costs next to that:
+//   256 x 8    1.00  one 8-wave workgroup per CU
+//   256 x 16   1.50  the same with two rows per thread, plain steps only (in
+//                    the others its second row costs twice: FP16 imaging at
+//                    512^3 630 us against 590 us in 256 x 8); 1.66 where planes
+//                    are multiples of 256 KB, whose z taps meet in the same
+//                    cache sets (256^3: 42.0 us against 38.8 in 256 x 8; 240^3:
+//                    35.1 against 36.2; 204 x 248 x 235: 31.2 against 35.4)
+//   128 x 24   1.33  one 12-wave workgroup per CU
+//   64 x 16    1.38  three 4-wave workgroups per CU
+// The narrow tiles win where 256-wide ones fit the rows badly: 384^3 plain 146
+// us in 128 x 24 (193 in 256 x 16), 320^3 102 and 288 x 240 x 208 36 us in 64 x 16
+// (120 and 46 us in the two-cell kernel).  Imaging and Born steps move more per
+// slice, which the narrow tiles' finer halos cost more (1.45, 1.60: FP32
+// imaging at 512^3 617 us in 256 x 8, 754 in 64 x 16); imaging takes 1.50 and 2.00
+// where rows start anywhere in a cache line, so that a tile's pieces of them
+// share their first and last line with the neighbours': 164 x 544 x 393 FP32 187
+// us in 256 x 8, 240 in 128 x 24, 254 in 64 x 16, 225 in the one-cell kernel.
+// On 1595 steps timed on about 300 grids of 5 to 105 million cells it is 2.4 %
+// slower than the best of these kernels on average.
 // Steps that extract receivers (Born modelling) take 256 x 16 earlier: where
 // several contexts model by turns, which overlaps their steps, the 256 x 8 tiles'
 // twofold y halo costs more than the second round that 256 x 16 may leave, and
@@ -124,15 +136,39 @@ inline long plan_rounds(StepChoice &c, const StepSetting &s, int tw, int ty, int
 // at 256 x 224 x 288 5.88 / 5.02 against 5.78 / 5.02, at 512 x 160 x 208 6.00 /
 // 5.29 against 5.95 / 5.29.  Steps that inject keep the line above (adjoint at
 // 256^3 12.83 / 12.05 in 256 x 8, 12.72 / 12.50 in 256 x 16).
-inline void choose_ring_tiles(StepChoice &c, const StepSetting &s, int act, int rec) {
+// Returns what the choice costs.
+inline double choose_ring_tiles(StepChoice &c, const StepSetting &s, int act, int rec) {
   const bool plain = act == ACT_NONE;
+  const bool sets = (long)s.n1 * s.n2 % 65536 == 0;
+  const double w16 = !plain               ? 1e30
+                     : rec == REC_EXTRACT ? (sets ? 1.55 : 1.45)
+                                          : (sets ? 1.66 : 1.50);
+  const bool split = act == ACT_IMG && s.n1 % 16 != 0;
+  const double w128 = plain ? 1.33 : split ? 1.50 : 1.45;
+  const double w64 = plain ? 1.38 : split ? 2.00 : 1.60;
   StepChoice q[4] = {c, c, c, c};
-  const double cost[4] = {
-      1.00 * plan_rounds(q[0], s, 256, 8, s.ncu),
-      plain ? (rec == REC_EXTRACT ? 1.55 : 1.66) * plan_rounds(q[1], s, 256, 16, s.ncu) : 1e30,
-      (plain ? 1.33 : 1.45) * plan_rounds(q[2], s, 128, 24, s.ncu),
-      (plain ? 1.38 : 1.60) * plan_rounds(q[3], s, 64, 16, 3 * s.ncu)};
-  c = q[std::min_element(cost, cost + 4) - cost];
+  const double cost[4] = {1.00 * plan_rounds(q[0], s, 256, 8, s.ncu),
+                          w16 * plan_rounds(q[1], s, 256, 16, s.ncu),
+                          w128 * plan_rounds(q[2], s, 128, 24, s.ncu),
+                          w64 * plan_rounds(q[3], s, 64, 16, 3 * s.ncu)};
+  const double *best = std::min_element(cost, cost + 4);
+  c = q[best - cost];
+  return *best;
+}
+
+// Whether the ring's own streams are read with nontemporal loads when left
+// automatic.  They pay off once a step's working set (16 B per cell: p, p_old,
+// V, p_new) is well beyond the 256 MB Infinity Cache: 6 % faster at 512^3.
+// Below that the fields stay cache-resident between launches, which the hint
+// would forfeit: 11 % slower at 256^3.  Nor where 64-wide tiles of rows that
+// start anywhere share the lines at their ends with their neighbours, which
+// then read them again: plain / FP32 imaging at 164 x 544 x 393 133 / 254 us with
+// it, 119 / 233 without (but 119 / 221 without at 400 x 208 x 432, whose rows
+// start on half lines, 115 / 213 with it).
+constexpr double kStreamMinStepBytes = 512.0 * 1024 * 1024;
+
+inline bool choose_streaming(const StepSetting &s, const StepChoice &c) {
+  return 16.0 * s.n1 * s.n2 * s.n3 > kStreamMinStepBytes && (c.tw > 64 || s.n1 % 16 == 0);
 }
 
 // rec: the receivers' mode that the caller would have inside the step.
@@ -142,8 +178,18 @@ inline StepChoice choose_step(const StepSetting &s, int form, int act, int fmt, 
   // caches, the four-cell ring where n1 allows it, else tiles as below.
   const bool autosel =
       form == FORM_VL && s.ty_tile == 0 && s.x_per_lane == 0 && s.halo_ring < 0;
+  const bool quad = s.n1 % 4 == 0;
   const long ncell = (long)s.n1 * s.n2 * s.n3;
-  if (autosel && ncell <= (s.n1 % 4 == 0 ? kDirectMaxCells : kDirectMaxCellsOdd)) {
+  double ring_cost = 1e30;
+  if (autosel && quad && ncell > kDirectCells) {
+    c.kernel = STEP_X4R;
+    c.rec = rec;
+    ring_cost = choose_ring_tiles(c, s, act, rec);
+  }
+  const double direct_cost =
+      (act == ACT_NONE ? 3.74 : 3.44) * (ncell <= kDirectEven ? 1.0 : 1.1) * ncell / (1 << 20);
+  if (autosel && (quad ? ncell <= kDirectMaxCells && direct_cost < ring_cost
+                       : ncell <= kDirectMaxCellsOdd)) {
     // lanes run over the (group of four cells, row) pairs of the update set;
     // two slices per thread once that still leaves 12 waves per compute unit
     const long groups = (s.n1 - 5L) / 4 * (s.n2 - 8);
@@ -156,12 +202,7 @@ inline StepChoice choose_step(const StepSetting &s, int form, int act, int fmt, 
     c.rec = rec;
     return c;
   }
-  if (autosel && s.n1 % 4 == 0) {
-    c.kernel = STEP_X4R;
-    c.rec = rec;
-    choose_ring_tiles(c, s, act, rec);
-    return c;
-  }
+  if (autosel && quad) return c;
   // cells per lane: 4 or 2 where asked for and n1 allows, else 1; automatic
   // (0): the widest whose tiles keep at least 3/4 of the lanes busy
   int xl = 1;

@@ -29,7 +29,8 @@ GRIDS = [
     # partial tiles in x, y and z
     ((380, 284, 104), 0, _ring("128x24"), _ring("128x24")),
     ((380, 284, 104), 1, _ring("128x24"), _ring("128x24")),
-    ((300, 220, 172), 1, _ring("64x16"), _ring("64x16")),
+    ((304, 220, 200), 0, _ring("64x16"), _ring("64x16")),
+    ((304, 220, 200), 1, _ring("64x16"), _ring("64x16")),
     ((508, 218, 132), 0, _ring("256x16"), _ring("256x8")),
     ((508, 218, 132), 1, _ring("256x16"), _ring("256x8")),
 ]

@@ -62,14 +62,27 @@ def test_automatic_kernels(choose, n, act, fmt, kernel, tile):
     assert (c[3] if kernel == "k_step_direct" else (c[1], c[2])) == tile, name
 
 
-@pytest.mark.parametrize("n", [(256, 256, 256), (240, 240, 240), (512, 160, 208)])
-def test_extracting_steps_take_taller_tiles(choose, n):
+def test_extracting_steps_take_taller_tiles(choose):
     """Plain steps of Born modelling, which extract receivers, run in 16-row
-    tiles where the others take 8 rows or narrow tiles; steps with an action
-    keep their shape."""
+    tiles at 256^3, where the others take 8 rows; steps with an action keep
+    their shape."""
+    n = (256, 256, 256)
     assert choose(n, rec=EXTRACT)[1][1:3] == [256, 16]
-    assert choose(n, rec=INJECT)[1][1:3] == choose(n)[1][1:3] != [256, 16]
+    assert choose(n, rec=INJECT)[1][1:3] == choose(n)[1][1:3] == [256, 8]
     assert choose(n, BORN, F16, EXTRACT)[1][1:3] == choose(n, BORN, F16)[1][1:3] == [256, 8]
+
+
+@pytest.mark.parametrize("n,act,fmt,want", [
+    # grids where 64 x 16 tiles, or the kernel without LDS (plain steps below
+    # 10 M cells), were slower than the one- and two-cell kernels
+    ((164, 544, 393), IMG, F32, "256x8 tiles"), ((164, 544, 393), IMG, F16, "256x8 tiles"),
+    ((564, 293, 259), IMG, F32, "256x8 tiles"), ((264, 368, 128), IMG, F16, "no LDS"),
+    ((300, 220, 172), IMG, F32, "no LDS"), ((272, 541, 86), IMG, F16, "no LDS"),
+    ((164, 294, 237), IMG, F32, "no LDS"), ((204, 248, 235), PLAIN, 0, "256x16 tiles"),
+    ((196, 248, 213), PLAIN, 0, "256x16 tiles"), ((224, 256, 160), PLAIN, 0, "256x8 tiles"),
+])
+def test_grids_that_narrow_tiles_fit_badly(choose, n, act, fmt, want):
+    assert want in choose(n, act, fmt)[2]
 
 
 @pytest.mark.parametrize("xl,ring,ty,kernel,tile", [
