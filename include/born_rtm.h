@@ -280,8 +280,16 @@ int brtm_dot_noalloc(brtm_ctx *ctx, const float *a, const float *b, long n, doub
  * reference, whose calls return after their last copy). */
 int brtm_sync(brtm_ctx *ctx);
 
-/* Bytes of device memory the context currently holds (no counterpart in
- * the reference). */
+/* Give back the memory that the context keeps of destroyed vectors for its
+ * next ones.  (All contexts on a device together keep at most a sixteenth of
+ * its memory, a context without vectors at most 64 MB; destroying the
+ * context, giving it a new grid, and an allocation of this library that finds
+ * no memory give it back as well.)  For programs that share the device with
+ * another allocator.  No counterpart in the reference. */
+int brtm_trim(brtm_ctx *ctx);
+
+/* Bytes of device memory the context currently holds, vectors in use not
+ * counted (no counterpart in the reference). */
 int brtm_device_bytes(brtm_ctx *ctx, double *bytes);
 
 #ifdef __cplusplus

@@ -78,6 +78,7 @@ SIGNATURES = {
     "brtm_stream_bench": [_P, _I, _D, _I, _I, C.POINTER(_D)],
     "brtm_dot_noalloc": [_P, _P, _P, C.c_long, C.POINTER(_D)],
     "brtm_sync": [_P],
+    "brtm_trim": [_P],
     "brtm_device_bytes": [_P, C.POINTER(_D)],
 }
 _RESTYPES = {"brtm_last_error": C.c_char_p, "brtm_version": C.c_char_p}

@@ -32,17 +32,33 @@ void set_error(const std::string &msg) { g_err = msg; }
 std::shared_mutex g_capturing;
 
 namespace {
-std::mutex g_live_mu;
-std::vector<brtm_ctx *> g_live;  // contexts whose pools may hold memory
+constexpr int kMaxDevices = 64;
+constexpr size_t kPoolBuffers = 256;  // kept by one context at most
 
-void flush_pools() {
-  std::lock_guard<std::mutex> lock(g_live_mu);
-  for (brtm_ctx *c : g_live) c->pool.flush();
-}
+std::mutex g_pool_mu;               // guards every pool and the two below
+std::vector<VecPool *> g_pools;     // open pools
+size_t g_pool_bytes[kMaxDevices];   // kept on each device
 }  // namespace
 
+void VecPool::open(int device, size_t cap) {
+  std::lock_guard<std::mutex> lock(g_pool_mu);
+  device_ = device;
+  cap_ = cap;
+  free_.reserve(kPoolBuffers);
+  g_pools.push_back(this);
+}
+
+void VecPool::close() {
+  {
+    std::lock_guard<std::mutex> lock(g_pool_mu);
+    cap_ = 0;
+    g_pools.erase(std::remove(g_pools.begin(), g_pools.end(), this), g_pools.end());
+  }
+  flush();
+}
+
 bool VecPool::take(size_t n, DevBuf *out) {
-  std::lock_guard<std::mutex> lock(mu_);
+  std::lock_guard<std::mutex> lock(g_pool_mu);
   size_t best = free_.size();
   for (size_t i = 0; i < free_.size(); ++i)
     if (free_[i].bytes >= n && free_[i].bytes - n <= n / 8 &&
@@ -50,37 +66,62 @@ bool VecPool::take(size_t n, DevBuf *out) {
       best = i;
   if (best == free_.size()) return false;
   bytes_ -= free_[best].bytes;
+  g_pool_bytes[device_] -= free_[best].bytes;
   *out = std::move(free_[best]);
   free_.erase(free_.begin() + best);
   return true;
 }
 
-void VecPool::put(DevBuf &&b) {
-  if (!b.ptr) return;
-  DevBuf gone;  // freed outside the lock
-  std::unique_lock<std::shared_mutex> quiet(g_capturing, std::try_to_lock);
-  if (!quiet || hipDeviceSynchronize() != hipSuccess) {
-    gone = std::move(b);
-    return;
-  }
-  std::lock_guard<std::mutex> lock(mu_);
-  if (bytes_ + b.bytes > cap) {
-    gone = std::move(b);
-    return;
-  }
-  bytes_ += b.bytes;
-  free_.push_back(std::move(b));
+void VecPool::created() {
+  std::lock_guard<std::mutex> lock(g_pool_mu);
+  ++vectors_;
 }
 
-void VecPool::flush() {
+void VecPool::put(DevBuf &&b) {
+  if (!b.ptr) return;
+  DevBuf gone;  // freed outside the locks
+  bool idle = false;
+  {
+    std::unique_lock<std::shared_mutex> quiet(g_capturing, std::try_to_lock);
+    const bool waited = quiet && hipDeviceSynchronize() == hipSuccess;
+    std::lock_guard<std::mutex> lock(g_pool_mu);
+    idle = --vectors_ == 0;
+    if (!waited || free_.size() >= kPoolBuffers || cap_ == 0 ||
+        g_pool_bytes[device_] + b.bytes > cap_) {
+      gone = std::move(b);
+    } else {
+      bytes_ += b.bytes;
+      g_pool_bytes[device_] += b.bytes;
+      free_.push_back(std::move(b));
+    }
+  }
+  if (idle) trim(kPoolIdleBytes);
+}
+
+// g_pool_mu is held; the last that came goes first.
+void VecPool::shrink(size_t keep, std::vector<DevBuf> &gone) {
+  while (bytes_ > keep) {
+    bytes_ -= free_.back().bytes;
+    g_pool_bytes[device_] -= free_.back().bytes;
+    gone.push_back(std::move(free_.back()));
+    free_.pop_back();
+  }
+}
+
+void VecPool::trim(size_t keep) {
+  std::vector<DevBuf> gone;  // freed after the lock is
+  std::lock_guard<std::mutex> lock(g_pool_mu);
+  shrink(keep, gone);
+}
+
+void VecPool::flush_all() {
   std::vector<DevBuf> gone;
-  std::lock_guard<std::mutex> lock(mu_);
-  gone.swap(free_);
-  bytes_ = 0;
+  std::lock_guard<std::mutex> lock(g_pool_mu);
+  for (VecPool *p : g_pools) p->shrink(0, gone);
 }
 
 size_t VecPool::held() {
-  std::lock_guard<std::mutex> lock(mu_);
+  std::lock_guard<std::mutex> lock(g_pool_mu);
   return bytes_;
 }
 
@@ -91,7 +132,7 @@ int DevBuf::alloc(size_t n) {
   hipError_t e = hipMalloc(&ptr, n);
   if (e == hipErrorOutOfMemory) {  // what the pools keep is given back first
     (void)hipGetLastError();
-    flush_pools();
+    VecPool::flush_all();
     e = hipMalloc(&ptr, n);
   }
   if (e != hipSuccess) {
@@ -777,7 +818,6 @@ int dot(brtm_ctx *c, const float *a, const float *b, long n, double *out) {
 }
 
 namespace {
-constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mu;
 double *g_scratch[kMaxDevices] = {};  // address of `scratch` on each device
 
@@ -851,11 +891,8 @@ int brtm_create(int device, brtm_ctx **out) {
     return rc;
   }
   size_t mfree = 0, mtotal = 0;
-  if (hipMemGetInfo(&mfree, &mtotal) == hipSuccess) c->pool.cap = mtotal / 16;
-  {
-    std::lock_guard<std::mutex> lock(g_live_mu);
-    g_live.push_back(c);
-  }
+  if (hipMemGetInfo(&mfree, &mtotal) != hipSuccess) mtotal = 0;
+  c->pool.open(device, mtotal / 16);
   *out = c;
   return BRTM_OK;
 }
@@ -865,14 +902,9 @@ int brtm_destroy(brtm_ctx *c) {
   BRTM_REQUIRE(!c->destroyed, BRTM_ESTATE, "brtm_destroy called twice on one context");
   (void)hipSetDevice(c->device);
   if (c->stream) (void)hipStreamSynchronize(c->stream);
-  {
-    std::lock_guard<std::mutex> lock(g_live_mu);
-    g_live.erase(std::remove(g_live.begin(), g_live.end(), c), g_live.end());
-  }
   // The device memory goes now; objects still alive on the context keep
   // only its host record (stream, events) until they are destroyed.
-  c->pool.cap = 0;
-  c->pool.flush();
+  c->pool.close();
   c->stores.clear();
   for (DevBuf *b : {&c->d_wtab, &c->V, &c->fa, &c->fb, &c->fc, &c->fd, &c->img, &c->mdl,
                     &c->seg, &c->mvw, &c->rscale, &c->partials, &c->dotv, &c->gram, &c->encmax, &c->slocs, &c->strc,
@@ -1417,6 +1449,14 @@ int brtm_set_two_step(brtm_ctx *c, int mode) {
 int brtm_set_graphs(brtm_ctx *c, int mode) {
   BRTM_REQUIRE(c && mode >= -1 && mode <= 1, BRTM_EINVAL, "mode must be -1, 0 or 1");
   c->graphs = mode;
+  return BRTM_OK;
+}
+
+int brtm_trim(brtm_ctx *c) {
+  BRTM_REQUIRE(c, BRTM_EINVAL, "ctx is NULL");
+  BRTM_LIVE(c);
+  BRTM_HIP(hipSetDevice(c->device));
+  c->pool.flush();
   return BRTM_OK;
 }
 

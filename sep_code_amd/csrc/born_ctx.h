@@ -54,23 +54,35 @@ struct DevBuf {
 // Buffers of destroyed vectors, kept for the next ones of about their size:
 // allocating and freeing the vectors of a solver (22 of them, 2.3 GB, at 16 M
 // samples and history 8) took 9 to 47 ms per solve, several times the
-// solve's kernels.  Holds at most a sixteenth of the device's memory; given
-// back when the context is destroyed, gets a new grid, or any allocation of
-// the library finds no memory.  A context's vectors are used on its stream,
-// so a buffer taken again is ordered after its last use there, and put()
-// waits for the device first, as freeing it would have.
+// solve's kernels.  All contexts on a device together keep at most a sixteenth
+// of its memory; a context without vectors keeps at most kPoolIdleBytes, and
+// everything is given back when the context is destroyed, gets a new grid or
+// is trimmed (brtm_trim), or when any allocation of the library finds no
+// memory.  A context's vectors are used on its stream, so a buffer taken again
+// is ordered after its last use there, and put() waits for the device first,
+// as freeing it would have.  Safe with several threads and contexts: one mutex
+// guards all pools, and nothing is freed under it.
+constexpr size_t kPoolIdleBytes = 64u << 20;
+
 class VecPool {
  public:
+  void open(int device, size_t cap);  // cap: bytes kept on the device in all
+  void close();                       // flush, and keep nothing from here on
+  // a buffer for a new vector of n bytes; false: none kept fits
   bool take(size_t n, DevBuf *out);
-  void put(DevBuf &&b);  // frees b when it does not fit
-  void flush();
+  void put(DevBuf &&b);  // the buffer of a destroyed vector: kept or freed
+  void created();        // a vector with a buffer of its own exists
+  void flush() { trim(0); }
+  static void flush_all();  // every context's
   size_t held();
-  size_t cap = 0;
 
  private:
-  std::mutex mu_;
+  void trim(size_t keep);
+  void shrink(size_t keep, std::vector<DevBuf> &gone);
   std::vector<DevBuf> free_;
-  size_t bytes_ = 0;
+  size_t bytes_ = 0, cap_ = 0;
+  long vectors_ = 0;
+  int device_ = -1;
 };
 
 // Held shared while a propagation loop is being captured: a device-wide wait

@@ -63,6 +63,7 @@ int vec_create(brtm_ctx *ctx, long n, bool zero, brtm_vec **out) {
     set_error(hipGetErrorString(e));
     return BRTM_EHIP;
   }
+  ctx->pool.created();
   *out = v;
   return BRTM_OK;
 }

@@ -237,6 +237,10 @@ class BornDevice:
     def sync(self):
         call("brtm_sync", self.h)
 
+    def trim(self):
+        """Give back the memory kept of destroyed vectors for the next ones."""
+        call("brtm_trim", self.h)
+
     def device_bytes(self):
         b = C.c_double()
         call("brtm_device_bytes", self.h, C.byref(b))
