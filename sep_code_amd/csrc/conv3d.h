@@ -23,18 +23,19 @@ struct Vol {          // spatial shape (per batch item)
 // y = ReLU(conv3x3x3(x, W) + b), zero padding 1.
 // up: the first input channels when they come from a volume of half the size
 // through nearest-neighbour upsampling (channels contiguous), or no channels.
+// ncu (here and below): compute units of the device.
 hipError_t conv3d_fwd(const Act &x, const Act &up, const uint16_t *W, const float *bias, Act y,
-                      Vol v, hipStream_t st);
+                      Vol v, int ncu, hipStream_t st);
 // Input gradient: the convolution of dy with the transposed weights, FP32
 // into dx; with act (the input itself, an activation), through its ReLU
 // (dx = 0 where act <= 0) as BF16.
-hipError_t conv3d_bwd(const Act &dy, const uint16_t *Wt, const Act &act, Act dx, Vol v,
+hipError_t conv3d_bwd(const Act &dy, const uint16_t *Wt, const Act &act, Act dx, Vol v, int ncu,
                       hipStream_t st);
 // dW[tap][co][ci] = sum_p dy[p][co] x[p + tap][ci] (FP32, [27][cout][cin]);
 // db[co] = sum_p dy[p][co].  scratch holds kGradScratch floats.
 constexpr long kGradScratch = 8L << 20;
 hipError_t conv3d_wgrad(const Act &x, const Act &up, const Act &dy, float *dW, float *db, Vol v,
-                        float *scratch, hipStream_t st);
+                        float *scratch, int ncu, hipStream_t st);
 // BF16 weights of a layer from the FP32 masters w [27][cout][cin]: W
 // [27][cout][cin_pad], and those of the transposed convolution Wt[tap][ci][co]
 // = W[26-tap][co][ci] (channels padded to 32).
@@ -53,7 +54,7 @@ hipError_t conv3d_first_fwd(const float *x, const float *W, const float *b, Act 
                             hipStream_t st);
 // Its weight and bias gradient (16 channels; overwrites dW [27][16] and db).
 hipError_t conv3d_first_wgrad(const float *x, const Act &dy, float *dW, float *db, Vol v,
-                              float *scratch, hipStream_t st);
+                              float *scratch, int ncu, hipStream_t st);
 // Head: 1x1x1 conv cin -> 1 FP32 plus the residual input: out = x0 + W.y + b.
 hipError_t head_fwd(const Act &y, const float *W, const float *b, const float *x0, float *out,
                     Vol v, hipStream_t st);

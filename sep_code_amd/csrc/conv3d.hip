@@ -12,6 +12,8 @@
 // operands are read from LDS with the transposing read (k_wgrad).
 #include "conv3d.h"
 
+#include "conv_plan.h"
+
 #include <algorithm>
 #include <utility>
 
@@ -971,33 +973,26 @@ __global__ void k_adam(float *p, const float *__restrict__ g, float *m, float *v
   }
 }
 
-// Output planes per sweep: as many as leave two workgroups of four waves, or
-// one of eight, for a compute unit (each sweep stages two planes more than it
-// writes: with 1024 workgroups 16->16 took 48.4 us at 8 x 64^3, 44.5 with 512).
 template <int OUT, int CIN, int CU, int COUT, int MTW, int YT, int WX, int WY, bool WL>
 hipError_t conv_t(const Act &x, const uint16_t *up, const uint16_t *W, const void *aux, Act y, Vol v,
-                  hipStream_t st) {
+                  int ncu, hipStream_t st) {
   if (v.w % (16 * WX) || v.h % (YT * WY)) return hipErrorInvalidValue;
   constexpr int NT = 64 * WX * WY * (COUT / 16 / MTW);
   const long tiles = (long)v.n * (v.h / (YT * WY)) * (v.w / (16 * WX));
-  int zl = 16;
-  while (zl > 1 && (v.d % zl || tiles * (v.d / zl) < (NT > 256 ? 256 : 512))) zl /= 2;
+  const int zl = sweep_planes(tiles, v.d, NT, ncu);
   const int grid = (int)(tiles * (v.d / zl));
   k_conv<CIN, CU, COUT, MTW, YT, WX, WY, WL, OUT><<<grid, NT, 0, st>>>(
       (const uint16_t *)x.p, x.cs, up, W, aux, y.p, y.cs, zl, v.d, v.h, v.w);
   return hipGetLastError();
 }
 
-// Workgroups of a weight gradient: with the three dz up to WGS per compute
-// unit, fewer where the volume has fewer units or the partials would pass
-// kGradScratch.
 template <int CIN, int CU, int COUT, int SEG, int R, int WGS>
 hipError_t wgrad_t(const Act &x, const uint16_t *up, const Act &dy, float *dW, float *db, Vol v,
-                   float *scratch, hipStream_t st) {
+                   float *scratch, int ncu, hipStream_t st) {
   constexpr int NW = 27 * CIN * COUT;
   if (v.w % SEG || v.h % R) return hipErrorInvalidValue;
   const long units = (long)v.n * v.d * (v.h / R) * (v.w / SEG);
-  const int S = (int)std::min({units, 256L * WGS / 3, kGradScratch / (NW + COUT)});
+  const int S = grad_groups(units, ncu, WGS, kGradScratch / (NW + COUT));
   k_wgrad<CIN, CU, COUT, SEG, R, WGS><<<dim3(S, 3), 192, 0, st>>>(
       (const uint16_t *)x.p, x.cs, up, (const uint16_t *)dy.p, dy.cs, scratch, v.d, v.h, v.w, units);
   k_grad_sum<<<(NW + COUT + 63) / 64, 256, 0, st>>>(scratch, S, NW, COUT, dW, db);
@@ -1033,34 +1028,35 @@ static bool is_input(const Act &x, const Act &up, int ci, int cu) {
 }
 
 static hipError_t conv(const Act &x, const Act &up, const uint16_t *W, const void *aux, Act y,
-                       Vol v, int out, hipStream_t st) {
+                       Vol v, int out, int ncu, hipStream_t st) {
   if (x.cs % 8 || y.cs % 4) return hipErrorInvalidValue;
 #define X(O, CI, CU, CO, MTW, YT, WX, WY, WL)                                               \
   if (out == OUT_##O && is_input(x, up, CI, CU) && y.c == CO)                               \
     return conv_t<OUT_##O, CI, CU, CO, MTW, YT, WX, WY, WL>(x, (const uint16_t *)up.p, W, aux, y, \
-                                                            v, st);
+                                                            v, ncu, st);
   BRTM_CONV_SHAPES(X)
 #undef X
   return hipErrorInvalidValue;
 }
 
 hipError_t conv3d_fwd(const Act &x, const Act &up, const uint16_t *W, const float *bias, Act y,
-                      Vol v, hipStream_t st) {
-  return conv(x, up, W, bias, y, v, OUT_ACT, st);
+                      Vol v, int ncu, hipStream_t st) {
+  return conv(x, up, W, bias, y, v, OUT_ACT, ncu, st);
 }
 
-hipError_t conv3d_bwd(const Act &dy, const uint16_t *Wt, const Act &act, Act dx, Vol v,
+hipError_t conv3d_bwd(const Act &dy, const uint16_t *Wt, const Act &act, Act dx, Vol v, int ncu,
                       hipStream_t st) {
   if (act.p && act.cs != dx.cs) return hipErrorInvalidValue;
-  return conv(dy, Act{nullptr, 0, 0}, Wt, act.p, dx, v, act.p ? OUT_MASK : OUT_GRAD, st);
+  return conv(dy, Act{nullptr, 0, 0}, Wt, act.p, dx, v, act.p ? OUT_MASK : OUT_GRAD, ncu, st);
 }
 
 hipError_t conv3d_wgrad(const Act &x, const Act &up, const Act &dy, float *dW, float *db, Vol v,
-                        float *scratch, hipStream_t st) {
+                        float *scratch, int ncu, hipStream_t st) {
   if (x.cs % 8 || dy.cs % 8) return hipErrorInvalidValue;
 #define X(CI, CU, CO, SEG, R, WGS)                                                            \
   if (is_input(x, up, CI, CU) && dy.c == CO)                                                 \
-    return wgrad_t<CI, CU, CO, SEG, R, WGS>(x, (const uint16_t *)up.p, dy, dW, db, v, scratch, st);
+    return wgrad_t<CI, CU, CO, SEG, R, WGS>(x, (const uint16_t *)up.p, dy, dW, db, v, scratch, ncu, \
+                                         st);
   BRTM_WGRAD_SHAPES(X)
 #undef X
   return hipErrorInvalidValue;
@@ -1087,10 +1083,10 @@ hipError_t conv3d_first_fwd(const float *x, const float *W, const float *b, Act 
 }
 
 hipError_t conv3d_first_wgrad(const float *x, const Act &dy, float *dW, float *db, Vol v,
-                              float *scratch, hipStream_t st) {
+                              float *scratch, int ncu, hipStream_t st) {
   if (dy.c != 16 || dy.cs % 8 || v.w % 64 || v.h % 8) return hipErrorInvalidValue;
   const long units = (long)v.n * v.d * (v.h / 8) * (v.w / 64);
-  const int S = (int)std::min(units, 512L);
+  const int S = (int)std::min(units, 2L * ncu);
   k_first_wgrad<<<S, 256, 0, st>>>(x, (const uint16_t *)dy.p, dy.cs, scratch, v.d, v.h, v.w,
                                    units);
   k_grad_sum<<<7, 256, 0, st>>>(scratch, S, 27 * 16, 16, dW, db);

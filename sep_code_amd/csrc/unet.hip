@@ -202,7 +202,7 @@ int forward(brtm_unet *u, const float *x, int nb) {
   BRTM_HIP(conv3d_first_fwd(x, pr + u->w0, pr + u->b0, act(u->e1a, C1, C1), v1, st));
   // layer l, from x (and up, of half the size) to y
   auto conv = [&](int l, const Act &x, const Act &up, const Act &y, const Vol &v) {
-    return conv3d_fwd(x, up, W(l), Bv(l), y, v, st);
+    return conv3d_fwd(x, up, W(l), Bv(l), y, v, u->ctx->ncu, st);
   };
   const Act none{nullptr, 0, 0};
   const Act s1 = act(u->skip1, C1, C1), s2 = act(u->skip2, C2, C2), b2 = act(u->b2, C3, C3),
@@ -230,8 +230,10 @@ int layer_bwd(brtm_unet *u, int l, const Act &dp, const Act &x, const Act &up, c
               const Act &dx, const Vol &v) {
   hipStream_t st = u->ctx->stream;
   float *G = u->grads.as<float>();
-  BRTM_HIP(conv3d_wgrad(x, up, dp, G + u->wl[l], G + u->bl[l], v, u->gscratch.as<float>(), st));
-  BRTM_HIP(conv3d_bwd(dp, u->wtf[l].as<uint16_t>(), act, dx, v, st));
+  const int ncu = u->ctx->ncu;
+  BRTM_HIP(conv3d_wgrad(x, up, dp, G + u->wl[l], G + u->bl[l], v, u->gscratch.as<float>(), ncu,
+                        st));
+  BRTM_HIP(conv3d_bwd(dp, u->wtf[l].as<uint16_t>(), act, dx, v, ncu, st));
   return BRTM_OK;
 }
 
@@ -268,7 +270,7 @@ int backward(brtm_unet *u, const float *x, int nb) {
   BRTM_HIP(avgpool_bwd(cat1 + 32, 48, u->dy_p1.as<float>(), s1, dp(0, C1), v1, st));
   U_TRY(layer_bwd(u, 0, dp(0, C1), e1a, none, e1a, dp(1, C1), v1));
   BRTM_HIP(conv3d_first_wgrad(x, dp(1, C1), G + u->w0, G + u->b0, v1, u->gscratch.as<float>(),
-                              st));
+                              u->ctx->ncu, st));
   return BRTM_OK;
 }
 
