@@ -87,6 +87,49 @@ def test_shots_on_the_larger_kernels(dev, n, stream, plain, action, store):
         dev.set_stream_loads(-1)
 
 
+@pytest.mark.parametrize("store", ["f32", "f16"])
+@pytest.mark.parametrize("n", [(53, 44, 40), (131, 37, 29)])
+def test_one_cell_tiles_with_receivers_inside(dev, n, store):
+    """The one-cell step's 64 x 8 tiles, which take receivers inside the step:
+    traces bit-identical to the separate extraction, images to FP32 rounding
+    of the separate injection."""
+    print(f"one-cell tiles {n} {store}", file=sys.stderr, flush=True)
+    r = _setup(dev, n, 12)
+    n1, n2, n3 = n
+    nt, ntr = 6, 14
+    tab = np.zeros((1, 8), np.float32)
+    tab[0, 3] = 1
+    dev.set_sinc_table(0, tab)
+    dev.set_sinc_table(1, tab)
+    dev.set_source(np.array([n1 // 2 + n1 * (n2 // 2) + n1 * n2 * (n3 // 2)], np.int32),
+                   r.standard_normal((1, ntr)).astype(np.float32))
+    yy, xx = np.meshgrid(np.arange(n2), np.arange(n1), indexing="ij")
+    rl = (xx + yy * n1 + 4 * n1 * n2).astype(np.int32).ravel()
+    data = r.standard_normal((len(rl), ntr)).astype(np.float32)
+    model = r.standard_normal(n[::-1]).astype(np.float32)
+    out = []
+    try:
+        dev.set_x_per_lane(1)
+        dev.set_tuning(8, 2048)
+        assert dev.step_kernel(0, 1, 1, 1) == "k_step, 64x8 tiles"
+        for fuse in (0, 1):
+            dev.set_receiver_fusion(fuse)
+            dev.set_receivers(rl, data, nx=n1, ny=n2)
+            dev.source_prop(1, nt, 1, store=store)
+            dev.zero_image()
+            dev.rtm_adjoint(1, nt, 1)
+            img = dev.get_image()
+            dev.set_model(model)
+            dev.rtm_forward(1, nt, 1)
+            out.append((img, dev.get_receivers()))
+    finally:
+        dev.set_receiver_fusion(1)
+        dev.set_tuning(0, 2048)
+        dev.set_x_per_lane(0)
+    np.testing.assert_array_equal(out[1][1], out[0][1])
+    _close(out[1][0], out[0][0])
+
+
 @pytest.mark.parametrize("n,kernel", [((128, 128, 128), "k_step_direct"),
                                       ((288, 240, 208), "64x16 tiles"),
                                       ((512, 218, 132), "256x16 tiles")])
