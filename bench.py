@@ -53,7 +53,7 @@ BYTES_PER_CELL = 16.0
 # HBM bytes per launch of the plain VL step (k_step_x4r, 512^3) from rocprofv3
 # FETCH_SIZE / WRITE_SIZE scaled by the copy-kernel calibration (2.0 / 1.0):
 # profiles/stencil512_traffic.md.  Used for the default configuration only.
-TRAFFIC_X4R_512 = (2.0 * 794832 + 508032) * 1024.0
+TRAFFIC_X4R_512 = (2.0 * 794960 + 508032) * 1024.0
 # The library launches its propagation loops as graphs on grids of at most
 # this many cells (brtm_set_graphs, automatic).
 GRAPH_MAX_CELLS = 1 << 22

@@ -414,11 +414,16 @@ static int check_ready(brtm_ctx *c, int jt, int nt, int jimg) {
 }
 
 // ---------------------------------------------------------------------------
-// Graph launch of a propagation loop.  On small grids a step is short, and
-// the time between two dependent launches (about 4 us at 128^3, against 12-16
-// us steps) is a fifth of the loop.  A loop whose launches are captured into
-// one graph and launched together avoids most of it.  Everything a loop
-// enqueues is a kernel launch: no memset, copy, event or synchronisation.
+// Graph launch of a propagation loop: its launches are captured into one graph
+// and launched together.  Everything a loop enqueues is a kernel launch: no
+// memset, copy, event or synchronisation.  The line dates from steps of 12-16
+// us at 128^3, with about 4 us between two dependent launches, when a shot of
+// 1000 steps each way took 31.2 ms as graphs and 36.6 ms eager.  With today's
+// steps of 3-11 us, whose capture and instantiation come before a loop's first
+// kernel, eager launches are the faster: 300 steps each way take, eager / as
+// graphs, 2.9 / 3.4 ms at 48^3, 4.3 / 5.0 at 96^3, 7.9 / 8.6 at 128^3 and, above
+// the line, 12.7 / 13.4 at 160^3 (with PyTorch's HIP runtime 3.4 / 3.6, 4.6 /
+// 5.0, 7.9 / 8.5, 12.7 / 13.4).
 // ---------------------------------------------------------------------------
 constexpr long kGraphMaxCells = 1L << 22;  // automatic: grids of up to 4 M cells
 

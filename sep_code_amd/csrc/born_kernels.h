@@ -52,7 +52,7 @@ struct StepParams {
 };
 
 // rec (RecMode): the receivers or source points of one plane inside the
-// step; VL form with 8-row tiles (the small-grid shape) only.
+// step; VL form with 8-row tiles only.
 hipError_t launch_step(int form, int act, int fmt, StepParams P, int ty_tile, hipStream_t st,
                        int rec = REC_NONE);
 // The VL step with a six-plane LDS ring (halos loaded with the z-queue).

@@ -936,7 +936,7 @@ k_step_x4(const StepParams P) {
 //     workgroup per CU;
 //   LX 32, 12 waves: 128 x 24 (102 KB), one workgroup per CU, and LX 16, 4
 //     waves: 64 x 16 (41 KB), three per CU: for rows that 256-wide tiles fit
-//     badly (launch_step_auto4 chooses).
+//     badly (choose_ring_tiles in step_choice.h).
 // ---------------------------------------------------------------------------
 // A lane's accesses to one x-y plane: its byte offset inside the plane is
 // fixed for the whole z sweep, and kOff marks a lane that has none (the load
@@ -2443,7 +2443,7 @@ hipError_t launch_step_t(int act, int fmt, const StepParams &P, hipStream_t st) 
   return hipErrorInvalidValue;
 }
 
-// The small-grid shape (VL, 8-row tiles) with the receivers or the source
+// 64 x 8 tiles of the one-cell VL step with the receivers or the source
 // points of one plane inside the step.
 template <int REC>
 hipError_t launch_step_rec_t(int act, int fmt, const StepParams &P, hipStream_t st) {

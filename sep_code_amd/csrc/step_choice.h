@@ -124,7 +124,7 @@ inline long plan_rounds(StepChoice &c, const StepSetting &s, int tw, int ty, int
 // where rows start anywhere in a cache line, so that a tile's pieces of them
 // share their first and last line with the neighbours': 164 x 544 x 393 FP32 187
 // us in 256 x 8, 240 in 128 x 24, 254 in 64 x 16, 225 in the one-cell kernel.
-// On 1595 steps timed on about 300 grids of 5 to 105 million cells it is 2.4 %
+// On 1595 steps timed on about 300 grids of 5 to 105 million cells it is 2.3 %
 // slower than the best of these kernels on average.
 // Steps that extract receivers (Born modelling) take 256 x 16 earlier: where
 // several contexts model by turns, which overlaps their steps, the 256 x 8 tiles'
