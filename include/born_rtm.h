@@ -216,15 +216,15 @@ int brtm_set_receiver_fusion(brtm_ctx *ctx, int on);
 /* Global-load lookahead of the plain four-cell ring step, in z slices: 1
  * (inputs of slice z+1 loaded while slice z computes), 2 (two slices ahead,
  * 36 more registers per lane) or 0 (the default: the faster of the two on
- * MI355X).  No counterpart in the reference; the same results. */
+ * MI355X).  Tiles narrower than 256 cells always load one slice ahead.  No
+ * counterpart in the reference; the same results. */
 int brtm_set_prefetch(brtm_ctx *ctx, int slices);
 
 /* Streaming (nontemporal) loads of p_old, V, 16-bit snapshots and the
  * model, which the four-cell ring step reads once: 1 on, 0 off, -1 (the
  * default) on when a step moves more than 512 MB, twice the Infinity Cache
- * (512^3 yes, 256^3 no), except in 64-wide tiles of rows of which 16 cells are
- * no divisor.  The image and FP32 snapshots stream at every
- * size.  No counterpart in the reference; the same results. */
+ * (512^3 yes, 256^3 no), except in 64-wide tiles where n1 is no multiple of
+ * 16.  The image and FP32 snapshots stream at every size.  No counterpart in the reference; the same results. */
 int brtm_set_stream_loads(brtm_ctx *ctx, int mode);
 
 /* Launch each propagation loop (source propagation, Born modelling, the
